@@ -1,14 +1,14 @@
 // K6: temperature / top-k / top-p / multinomial sampling, sort-free.
 //
-// One 1024-thread workgroup per batch row, logits read with 16-byte loads from L2/HBM:
-//   * temperature == 0          → arg-max (lowest index on ties), one pass.
-//   * top_k == 0 && top_p >= 1  → Gumbel-max draw  argmax_i(x_i / T + g_i), one pass (shift invariant,
-//                                  so neither the row max nor the softmax sum is needed).
-//   * otherwise                 → threshold search instead of a sort: the fp32 logit is mapped to an
-//                                  order-preserving 32-bit key and the cut-off key is found by a 4-pass
-//                                  radix descent (8 bits per pass, 256-bin LDS histogram of *counts*
-//                                  for top-k, of *probability mass* for top-p); then the Gumbel-max
-//                                  draw runs over the surviving keys only.
+//   * temperature == 0          → arg-max (lowest index on ties).
+//   * top_k == 0 && top_p >= 1  → Gumbel-max draw  argmax_i(x_i / T + g_i) (shift invariant, so neither the row max nor the
+//                                  softmax sum is needed).
+//   * otherwise                 → a cut-off on the logit instead of a sort, then the Gumbel-max draw over what reaches it.
+//
+// Serving path (bf16 rows of up to 131072 logits, 16-byte aligned): sample_cut_kernel finds the cut-off key of the rows that need
+// one, sample_draw_kernel draws with a row's slices spread over the chip.  Other rows (fp32, unaligned, longer) take
+// sample_kernel: one 1024-thread workgroup per row, cut-off by a 4-pass radix descent (8 bits per pass, 256-bin LDS histogram of
+// *counts* for top-k, of *probability mass* for top-p).
 // Gumbel noise comes from Philox4x32-10 keyed by the request seed, counter = (element/4, step), so a
 // request's draw is independent of the batch it happens to share; a `noise` tensor can be supplied
 // instead (tests: bit-exact comparison against the torch reference with the same uniforms).
@@ -203,13 +203,11 @@ __global__ __launch_bounds__(SNT) void sample_kernel(const T* __restrict__ logit
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// bf16 fast path (the serving path: logits come out of the LM-head GEMM in bf16, V ≤ 131072, V % 8 == 0).
-// The whole row lives in registers — thread t holds 16-byte chunks t, t+1024, … (8 logits each, packed) — so
-// every later pass (max, mass, radix, draw) is register work and the row is read from memory exactly once.
-// A bf16 logit has only 16 key bits, so the radix descent takes TWO 8-bit passes (not four), and a thread adds
-// runs of equal bins to the LDS histogram with one atomic (softmax-shaped rows put most of a thread's elements
-// in the same two or three bins; per-element atomics on them serialise the whole workgroup).
-// The Philox counter of element i is i/4 exactly as in the generic kernel: both paths draw the same token.
+// bf16 serving path (logits come out of the LM-head GEMM in bf16, V ≤ 131072, V % 8 == 0).
+//
+// A draw without a cut-off is bound by Philox (≈ 45 µs of integer multiplies when one compute unit does a 128k row) and a cut-off by
+// the LDS atomics of its histogram, so neither fits one kernel of a workgroup per row, which leaves most of the chip idle at
+// decode batch sizes: B = 57, V = 128256 with a quarter each of greedy, plain, top-p and top-k rows took 239 µs that way.
 // ---------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t okey16(uint32_t h) { return (h & 0x8000u) ? (~h & 0xFFFFu) : (h | 0x8000u); }
 __device__ __forceinline__ uint32_t half_of(const uint4& c, int e) {   // e-th bf16 (0..7) of a chunk, compile-time e
@@ -217,6 +215,7 @@ __device__ __forceinline__ uint32_t half_of(const uint4& c, int e) {   // e-th b
   return (e & 1) ? (w >> 16) : (w & 0xFFFFu);
 }
 
+// The row of a cut-off lives in registers — thread t holds 16-byte chunks t, t+1024, … (8 logits each, packed).
 // Every pass re-derives keys and weights from the packed row.  Without this fence the compiler keeps the 128 unpacked
 // keys of a thread alive from one pass to the next (CSE) and spills; the empty asm makes the registers opaque.
 template <int NCH>
@@ -252,6 +251,8 @@ __device__ __forceinline__ void pick_bin(const float* hist, float remaining, uin
   }
 }
 
+// Exact for any row, two 8-bit passes over the 16-bit keys; the fallback of cut_by_counts.  A thread adds runs of equal bins to the
+// LDS histogram with one atomic.
 template <int NCH, bool MASS>
 __device__ __forceinline__ uint32_t radix_cut16(uint4 (&regs)[NCH], float inv_t_log2, float zmax, float target, uint32_t floor_key,
                                 float* hist, uint32_t* s_pick, float* s_rem) {
@@ -297,19 +298,104 @@ __device__ __forceinline__ uint32_t radix_cut16(uint4 (&regs)[NCH], float inv_t_
   return prefix;
 }
 
+// ---- cut-off by counting.  One pass adds every logit of the row to a histogram of COUNTS with a bin per bf16 value: magnitudes from
+// the row's largest down 32 octaves (MBINS = 32 · 128 mantissa steps) for either sign, smaller ones share the bin at zero.  Logits
+// spread over hundreds of such bins, so the LDS atomics hardly collide (bins of the upper 8 key bits put a softmax-shaped row
+// into five or six), and a bin's probability mass is count · exp2(z − zmax): top-k and top-p read the same histogram, each sum in a
+// fixed order.  A cut-off inside the shared bin, or a row with infinities or NaN, is left to radix_cut16.  The atomics and the row's
+// arrival at one compute unit bound it: 23 µs a launch at V = 128256 up to 256 filtered rows (radix descents of the whole row: 235).
+// Position d runs from the largest value down: positive magnitude index c at MBINS − 1 − c, negative at MBINS + c.
+constexpr int MBINS = 4096;
+constexpr int BINS_PER_THREAD = 2 * MBINS / SNT;
+// LDS word of position d: thread t scans positions 8 t … 8 t + 7, rotated so that the lanes of a read fall on different banks
+__device__ __forceinline__ int bin_word(int d) { return (d & ~7) | ((d + (d >> 3)) & 7); }
+
+struct CutScratch {
+  float wave_tot[SNT / 64];
+  int first;
+  int pick;
+};
+
+// position of the first bin where the running weight of the bins up to position d_last reaches `target` (FRACTION: that share of
+// their total), or −1
+template <bool MASS, bool FRACTION>
+__device__ __forceinline__ int scan_cut(const uint32_t* counts, int lo, float inv_t_log2, float zmax, float target, int d_last,
+                                        CutScratch* s) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  float w[BINS_PER_THREAD], local = 0.f;
+#pragma unroll
+  for (int j = 0; j < BINS_PER_THREAD; ++j) {
+    const int d = t * BINS_PER_THREAD + j;
+    const uint32_t n = d <= d_last ? counts[bin_word(d)] : 0u;
+    const int c = d < MBINS ? MBINS - 1 - d : d - MBINS;
+    const float x = bf2f((uint16_t)(c + lo)) * (d < MBINS ? inv_t_log2 : -inv_t_log2);
+    w[j] = n == 0u ? 0.f : MASS ? (float)n * fast_exp2(x - zmax) : (float)n;
+    local += w[j];
+  }
+  float incl = local;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float up = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += up;
+  }
+  if (lane == 63) s->wave_tot[wave] = incl;
+  if (t == 0) { s->first = SNT; s->pick = -1; }
+  __syncthreads();
+  float before = 0.f, total = 0.f;
+#pragma unroll
+  for (int k = 0; k < SNT / 64; ++k) {
+    const float x = s->wave_tot[k];
+    before += k < wave ? x : 0.f;
+    total += x;
+  }
+  const float want = FRACTION ? target * total : target;
+  const bool reached = before + incl >= want && local > 0.f;
+  const uint64_t hit = __ballot(reached);
+  if (hit != 0 && lane == 0) atomicMin(&s->first, wave * 64 + __ffsll((long long)hit) - 1);
+  __syncthreads();
+  if (t == s->first) {
+    float acc = before + (incl - local);
+    int pick = -1;
+#pragma unroll
+    for (int j = 0; j < BINS_PER_THREAD; ++j) {
+      if (w[j] > 0.f && (pick < 0 || acc < want)) pick = t * BINS_PER_THREAD + j;   // `want` was not reached in front of it
+      acc += w[j];
+    }
+    s->pick = pick;
+  }
+  __syncthreads();
+  const int r = s->pick;
+  __syncthreads();
+  return r;
+}
+
+// per row of the launch: what the draw needs to know, and the words its slices meet in (a cache line each: the atomics of eight rows on
+// one line wait for each other)
+struct alignas(128) SampleRow {
+  unsigned long long best;     // (ordered value, ~index) of the best candidate so far
+  uint32_t cut;                // smallest 16-bit key that takes part
+  uint32_t done;               // slices that have delivered
+};
+
 template <int NCH>
-__global__ __launch_bounds__(SNT) void sample_bf16_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
-                                                          const float* __restrict__ temperature, const float* __restrict__ top_p,
-                                                          const int* __restrict__ top_k, const int64_t* __restrict__ seeds,
-                                                          const int64_t* __restrict__ steps, const float* __restrict__ noise,
-                                                          int64_t* __restrict__ out) {
+__global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
+                                                         const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                         const int* __restrict__ top_k, SampleRow* __restrict__ rows) {
+  __shared__ uint32_t counts[2 * MBINS];
   __shared__ float sv[SNT / 64];
-  __shared__ int si[SNT / 64];
-  __shared__ float hist[256];
+  __shared__ CutScratch cs;
   __shared__ uint32_t s_pick;
   __shared__ float s_rem;
 
   const int b = blockIdx.x;
+  const float temp = temperature[b];
+  const float p = top_p[b];
+  int k = top_k[b];
+  if (k <= 0 || k > V) k = V;
+  if (temp <= 0.f || (k >= V && !(p < 1.f))) {              // nothing to cut
+    if (threadIdx.x == 0) rows[b] = SampleRow{0ull, 0u, 0u};
+    return;
+  }
   const uint4* row = reinterpret_cast<const uint4*>(logits + (int64_t)b * row_stride);
   const int nchunks = V >> 3;
   uint4 regs[NCH];
@@ -318,34 +404,52 @@ __global__ __launch_bounds__(SNT) void sample_bf16_kernel(const uint16_t* __rest
     const int idx = c * SNT + threadIdx.x;
     regs[c] = idx < nchunks ? row[idx] : make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);   // -inf padding
   }
-  const float temp = temperature[b];
-
-  if (temp <= 0.f) {
-    ArgMax a{-3.0e38f, 0x7fffffff};
-#pragma clang loop unroll(full)
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        a = amax(a, ArgMax{bf2f((uint16_t)half_of(regs[c], e)), (c * SNT + (int)threadIdx.x) * 8 + e});
-    a = block_argmax(a, sv, si);
-    if (threadIdx.x == 0) out[b] = valid_token(a.i, V);
-    return;
-  }
+  for (int i = threadIdx.x; i < 2 * MBINS; i += SNT) counts[i] = 0u;
 
   const float inv_t_log2 = 1.4426950408889634f / temp;    // z = x / T in log2 units
-  const float p = top_p[b];
-  int k = top_k[b];
-  if (k <= 0 || k > V) k = V;
-  uint32_t floor_key = 0;                                  // 16-bit key of the raw bf16 logit (x → x/T is monotone)
-
-  if (k < V || p < 1.f) {
-    float zmax = -3.0e38f;
+  float vmax = -3.0e38f;
+  uint32_t mag_max = 0;
+#pragma clang loop unroll(full)
+  for (int c = 0; c < NCH; ++c) {
+    const bool in = c * SNT + (int)threadIdx.x < nchunks;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t h = half_of(regs[c], e);
+      vmax = fmaxf(vmax, bf2f((uint16_t)h));
+      mag_max = max(mag_max, in ? h & 0x7FFFu : 0u);
+    }
+  }
+  const float zmax = block_max(vmax, sv) * inv_t_log2;
+  const int top = (int)block_max((float)mag_max, sv);       // (a 15-bit whole number is exact in fp32)
+  uint32_t floor_key = 0;                                   // 16-bit key of the raw bf16 logit (x → x/T is monotone)
+  bool exact = top <= 0x7F7F;                               // every logit finite
+  if (exact) {
+    const int lo = max(top - (MBINS - 1), 0);
     opaque(regs);
 #pragma clang loop unroll(full)
-    for (int c = 0; c < NCH; ++c)
+    for (int c = 0; c < NCH; ++c) {
+      if (c * SNT + (int)threadIdx.x < nchunks) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) zmax = fmaxf(zmax, bf2f((uint16_t)half_of(regs[c], e)));
-    zmax = block_max(zmax, sv) * inv_t_log2;
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t h = half_of(regs[c], e);
+          const int m = max((int)(h & 0x7FFFu) - lo, 0);
+          atomicAdd(&counts[bin_word((h & 0x8000u) ? MBINS + m : MBINS - 1 - m)], 1u);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);      // one chunk at a time: keeps the row registers the only long-lived ones
+    }
+    __syncthreads();
+    int d = 2 * MBINS - 1;
+    if (k < V) d = scan_cut<false, false>(counts, lo, inv_t_log2, zmax, (float)k, d, &cs);
+    exact = d >= 0 && !(lo > 0 && (d == MBINS - 1 || d == MBINS));
+    if (exact && p < 1.f) {
+      d = scan_cut<true, true>(counts, lo, inv_t_log2, zmax, p, d, &cs);
+      exact = d >= 0 && !(lo > 0 && (d == MBINS - 1 || d == MBINS));
+    }
+    if (exact) floor_key = d < MBINS ? 0x8000u | (uint32_t)(MBINS - 1 - d + lo) : 0x7FFFu - (uint32_t)(d - MBINS + lo);
+  }
+  if (!exact) {
+    float* hist = reinterpret_cast<float*>(counts);
     if (k < V) floor_key = radix_cut16<NCH, false>(regs, inv_t_log2, zmax, (float)k, 0u, hist, &s_pick, &s_rem);
     if (p < 1.f) {
       float tot = 0.f;                                     // mass of what survived top-k
@@ -368,19 +472,53 @@ __global__ __launch_bounds__(SNT) void sample_bf16_kernel(const uint16_t* __rest
       floor_key = radix_cut16<NCH, true>(regs, inv_t_log2, zmax, p * tot, floor_key, hist, &s_pick, &s_rem);
     }
   }
+  if (threadIdx.x == 0) rows[b] = SampleRow{0ull, floor_key, 0u};
+}
 
-  const uint64_t seed = (uint64_t)seeds[b];
-  const uint64_t step = (uint64_t)steps[b];
-  const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
+// ---- draw.  Grid (slices, B): a 256-thread workgroup takes 256 · NC chunks of 8 logits.  Its best candidate goes into the row's
+// 64-bit maximum (value in the order-preserving 32 bits, then the lowest index); the slice that delivers last reads the result.
+// The Philox counter of element i is i/4 exactly as in sample_kernel: both paths draw the same token.  V = 128256, a quarter of the rows
+// without cut-off: 12 µs at B = 57, 20 at 120.
+constexpr int DNT = 256;
+template <int NC>
+__global__ __launch_bounds__(DNT) void sample_draw_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
+                                                          const float* __restrict__ temperature, const int64_t* __restrict__ seeds,
+                                                          const int64_t* __restrict__ steps, const float* __restrict__ noise,
+                                                          SampleRow* __restrict__ rows, int64_t* __restrict__ out) {
+  __shared__ ArgMax sa[DNT / 64];
+  const int b = blockIdx.y;
+  const uint4* row = reinterpret_cast<const uint4*>(logits + (int64_t)b * row_stride);
+  const int nchunks = V >> 3, first = blockIdx.x * (DNT * NC) + threadIdx.x;
+  uint4 regs[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) regs[c] = first + c * DNT < nchunks ? row[first + c * DNT] : make_uint4(0, 0, 0, 0);
+  const float temp = temperature[b];
   ArgMax a{-3.0e38f, 0x7fffffff};
-  const float ln2 = 0.6931471805599453f;
-  opaque(regs);
-#pragma clang loop unroll(full)
-  for (int c = 0; c < NCH; ++c) {
-    const int chunk = c * SNT + (int)threadIdx.x;
-    if (chunk < nchunks) {
+  if (temp <= 0.f) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (first + c * DNT < nchunks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a = amax(a, ArgMax{bf2f((uint16_t)half_of(regs[c], e)), (first + c * DNT) * 8 + e});
+      }
+    }
+  } else {
+    const float inv_t_log2 = 1.4426950408889634f / temp;
+    const float ln2 = 0.6931471805599453f;
+    const uint32_t floor_key = rows[b].cut;
+    const uint64_t seed = (uint64_t)seeds[b];
+    const uint64_t step = (uint64_t)steps[b];
+    const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int chunk = first + c * DNT;
+      if (chunk >= nchunks) break;
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
+        bool any = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) any = any || okey16(half_of(regs[c], half * 4 + e)) >= floor_key;
+        if (!any) continue;                                // behind a cut-off most groups of four draw nothing
         const int i4 = chunk * 2 + half;
         uint4 r = make_uint4(0, 0, 0, 0);
         if (noise == nullptr) r = philox4x32_10(make_uint4((uint32_t)i4, (uint32_t)step, (uint32_t)(step >> 32), 0x5A17u), key);
@@ -394,31 +532,65 @@ __global__ __launch_bounds__(SNT) void sample_bf16_kernel(const uint16_t* __rest
             a = amax(a, ArgMax{bf2f((uint16_t)h) * inv_t_log2 * ln2 + gumbel(u), i});
           }
         }
-        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
-  a = block_argmax(a, sv, si);
-  if (threadIdx.x == 0) out[b] = valid_token(a.i, V);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a = amax(a, ArgMax{__shfl_xor(a.v, o, 64), __shfl_xor(a.i, o, 64)});
+  if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int w = 1; w < DNT / 64; ++w) a = amax(a, sa[w]);
+  SampleRow* r = rows + b;
+  // The two words are only ever touched by atomics at the memory side, so the order "maximum, then count" is all it takes, and the wait
+  // for the maximum's old value gives it.  (A release / acquire count writes back and empties the die's L2 once per workgroup: 340 µs
+  // instead of 67 at B = 512, V = 128256.)
+  if ((unsigned)a.i < (unsigned)V) {                       // a slice without a candidate delivers none; + 0: −0 ties with +0
+    const unsigned long long old = __hip_atomic_fetch_max(&r->best, (unsigned long long)okey(a.v + 0.f) << 32 | (uint32_t)~a.i,
+                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"((uint32_t)old), "v"((uint32_t)(old >> 32)) : "memory");
+  }
+  const uint32_t before = __hip_atomic_fetch_add(&r->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (before == gridDim.x - 1) {
+    const unsigned long long best = __hip_atomic_fetch_max(&r->best, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    out[b] = best == 0ull ? 0 : valid_token((int)~(uint32_t)best, V);
+  }
 }
 
+bool sample_by_slices(bool logits_fp32, const void* logits, int64_t row_stride, int B, int V) {
+  return !logits_fp32 && V % 8 == 0 && V > 0 && V <= 16 * SNT * 8 && row_stride % 8 == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0 &&
+         B <= 65535;
+}
+
+size_t sample_workspace_bytes(int B) { return (size_t)B * sizeof(SampleRow); }
+
+// `ws`: sample_workspace_bytes(B) where sample_by_slices says so (contents do not matter), else not read.
 void launch_sample(const void* logits, bool logits_fp32, int64_t row_stride, int B, int V, const float* temperature,
                    const float* top_p, const int* top_k, const int64_t* seeds, const int64_t* steps, const float* noise,
-                   int64_t* out, hipStream_t stream) {
+                   int64_t* out, void* ws, hipStream_t stream) {
   if (B == 0) return;
-  const bool rows16 = V % 8 == 0 && row_stride % 8 == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
-  if (logits_fp32)
+  if (sample_by_slices(logits_fp32, logits, row_stride, B, V)) {
+    const uint16_t* x = (const uint16_t*)logits;
+    SampleRow* rows = (SampleRow*)ws;
+    if (V <= 4 * SNT * 8)
+      hipLaunchKernelGGL(sample_cut_kernel<4>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
+    else
+      hipLaunchKernelGGL(sample_cut_kernel<16>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
+    // slices of 8192 logits where they keep all compute units busy several times over (half the atomics), of 2048 below: B = 57 18 → 16 µs
+    const int wide = (V / 8 + DNT * 4 - 1) / (DNT * 4);
+    if ((int64_t)wide * B >= 2048)
+      hipLaunchKernelGGL(sample_draw_kernel<4>, dim3(wide, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, seeds, steps, noise, rows, out);
+    else
+      hipLaunchKernelGGL(sample_draw_kernel<1>, dim3((V / 8 + DNT - 1) / DNT, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, seeds,
+                         steps, noise, rows, out);
+  } else if (logits_fp32) {
     hipLaunchKernelGGL(sample_kernel<float>, dim3(B), dim3(SNT), 0, stream, (const float*)logits, row_stride, V,
                        temperature, top_p, top_k, seeds, steps, noise, out);
-  else if (rows16 && V <= 4 * SNT * 8)
-    hipLaunchKernelGGL(sample_bf16_kernel<4>, dim3(B), dim3(SNT), 0, stream, (const uint16_t*)logits, row_stride, V,
-                       temperature, top_p, top_k, seeds, steps, noise, out);
-  else if (rows16 && V <= 16 * SNT * 8)
-    hipLaunchKernelGGL(sample_bf16_kernel<16>, dim3(B), dim3(SNT), 0, stream, (const uint16_t*)logits, row_stride, V,
-                       temperature, top_p, top_k, seeds, steps, noise, out);
-  else
+  } else {
     hipLaunchKernelGGL(sample_kernel<uint16_t>, dim3(B), dim3(SNT), 0, stream, (const uint16_t*)logits, row_stride, V,
                        temperature, top_p, top_k, seeds, steps, noise, out);
+  }
 }
 
 // Pipelined stepping: a decode row whose input id was sampled by the step still in flight reads it from the

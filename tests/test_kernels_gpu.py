@@ -279,6 +279,40 @@ def test_sampler_matches_reference_with_shared_noise(V, dtype):
     assert agree >= rounds * B - 2, f"only {agree}/{rounds * B} draws agree with the reference"
 
 
+@pytest.mark.parametrize("B,V", [(1, 8), (7, 2040), (24, 2056), (12, 32768), (12, 32776), (64, 65536), (12, 131064)])
+def test_sampler_slices_draw_what_the_row_kernel_draws(B, V):
+    """bf16 rows (histogram cut-off, slices of a row over the chip) against the same values in fp32 (one workgroup per row, radix
+    descent): the formulas of value and noise are the same, so every id is — nothing but a nucleus boundary within rounding of ``p``
+    (~1e-6 of the mass) could differ.  Rows that are hard for the histogram among them: equal logits, signed zeros, masked tokens, a
+    cut-off among values 33 octaves below the largest, an infinity."""
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn(B, V, generator=g) * torch.tensor([0.02, 1.0, 3.0, 12.0])[torch.arange(B) % 4, None]).to(torch.bfloat16)
+    if B > 8:
+        logits[1] = 0.5
+        logits[2, ::2], logits[2, 1::2] = 0.0, -0.0
+        logits[3, V // 3:] = float("-inf")
+        logits[4] = (torch.randn(V, generator=g) * 2.0 ** -40).to(torch.bfloat16)
+        logits[4, 11] = 2.0
+        logits[6, V - 1] = float("inf")
+        logits[7] = torch.finfo(torch.bfloat16).min
+        logits[7, 5] = 1.0
+    i = torch.arange(B)
+    temp = torch.where(i % 6 == 5, 0.0, 0.5 + 0.25 * (i % 4)).float().to(DEV)
+    top_p = torch.where(i % 3 == 0, 1.0, 0.35 + 0.07 * (i % 9)).float().to(DEV)
+    top_k = torch.where(i % 2 == 0, 0, 1 + (i * i * 3) % (V - 1)).int().to(DEV)
+    seeds, steps = (i * 7919 + 3).to(DEV), (i * 31).to(DEV)
+    x = logits.to(DEV)
+    if B > 8:
+        assert ops.sample(x[6:7], temp[1:2] + 1, top_p[1:2], top_k[:1], seeds[:1], steps[:1]).item() == V - 1
+    for r in range(4):
+        got = ops.sample(x, temp, top_p, top_k, seeds, steps + r)
+        want = ops.sample(x.float(), temp, top_p, top_k, seeds, steps + r)
+        keep = torch.ones(B, dtype=torch.bool)
+        if B > 8:
+            keep[6] = False                                       # (an infinite maximum: inf - inf in the mass)
+        assert torch.equal(got.cpu()[keep], want.cpu()[keep]), (r, got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_sampler_nan_row_yields_a_valid_token(dtype):
     """A NaN row (a bug upstream) must not turn into an out-of-range token id: the next step embeds it."""
