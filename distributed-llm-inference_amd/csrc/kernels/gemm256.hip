@@ -422,6 +422,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
+// slabs [n_slabs][M][N] → out [M, N] (swiglu: [M, N / 2])
+void launch_splitk_reduce(bool swiglu, const float* slabs, int n_slabs, int M, int N, void* out, int64_t out_stride, hipStream_t stream) {
+  const int n_out = swiglu ? N / 2 : N;
+  const int blocks = (int)std::min<int64_t>(((int64_t)M * (n_out / 4) + 255) / 256, 2048);
+  hipLaunchKernelGGL(swiglu ? splitk_reduce_kernel<true> : splitk_reduce_kernel<false>, dim3(blocks), dim3(256), 0, stream, slabs, n_slabs,
+                     (int64_t)M * N, (int64_t)N, M, n_out, (uint16_t*)out, out_stride);
+}
+
 // out tile (tile, col_block) of the range = Σ_s compact slab_s, epilogue applied: the reduce pass of the RANGE-mode tail
 // (one workgroup per quarter tile: 64 rows)
 template <bool SWIGLU>
@@ -497,13 +505,7 @@ void launch_dense_gemm256(bool swiglu, const void* x, int64_t x_stride, const vo
     const int grid = (n_tiles * n_col_blocks * k_splits + 7) / 8 * 8;
     if (swiglu) G256_DENSE(EPI_SWIGLU_SPLITK, grid, workspace, ldc, k_splits, slab, 0, 0);
     else G256_DENSE(EPI_PLAIN_SPLITK, grid, workspace, ldc, k_splits, slab, 0, 0);
-    const int blocks = (int)std::min<int64_t>(((int64_t)M * (N_out / 4) + 255) / 256, 2048);
-    if (swiglu)
-      hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3(blocks), dim3(256), 0, stream, workspace, k_splits, slab, ldc, M, N_out,
-                         (uint16_t*)out, out_stride);
-    else
-      hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3(blocks), dim3(256), 0, stream, workspace, k_splits, slab, ldc, M, N_out,
-                         (uint16_t*)out, out_stride);
+    launch_splitk_reduce(swiglu, workspace, k_splits, M, (int)ldc, out, out_stride, stream);
     return;
   }
   int r = 0, s = 0;

@@ -65,6 +65,14 @@ void launch_grouped_gemm256(int epilogue, const void* A, int64_t a_stride, const
 void launch_dense_gemm256(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M,
                           int K, int N_out, int k_splits, float* workspace, bool split_tail, hipStream_t stream);
 void dense_gemm256_tail_plan(int M, int K, int N_out, bool swiglu, int* tail_tiles, int* tail_slices);
+// activation rows 17 … 256: weight-streaming tiles (stream_gemm.hip)
+void launch_stream_gemm(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M, int K, int N,
+                        int k_splits, hipStream_t stream);
+void launch_grouped_stream_gemm(int epilogue, int tile_rows, const void* A, int64_t a_stride, const void* W, int64_t w_expert_stride,
+                                const int* sorted_ids, const int* tile_expert, const int* meta, const float* topk_w, int top_k, void* out,
+                                int64_t out_stride, int K, int N_out, int max_tiles, int k_splits, int64_t slab_elems, hipStream_t stream,
+                                float act_limit);
+void launch_splitk_reduce(bool swiglu, const float* slabs, int n_slabs, int M, int N, void* out, int64_t out_stride, hipStream_t stream);
 void launch_moe_sum(const void* y, bool y_fp32, int n_slabs, int64_t slab_elems, const int* ids, int expert_offset, int E_local,
                     int top_k, int T, int H, void* out, hipStream_t stream);
 

@@ -326,11 +326,43 @@ Tensor dense_gemm256(const Tensor& x, const Tensor& w, bool swiglu, int64_t k_sp
   return out;
 }
 
-// row tile of the grouped GEMM: 256 from this many routed rows per expert on (DLI_MOE_TILE=128|256 forces one).
-// Measured crossover at Mixtral shapes (profiles/kernels_moe_tile_crossover_r2z.txt): 96 rows per expert → 128-row tiles
-// win by 8 %, from 128 rows per expert on the 256-row tile wins by 1.2–1.37 ×.
+// y = x · Wᵀ on the weight-streaming tiles (stream_gemm.hip), swiglu as for dense_gemm256.  k_splits = 0: as many K slices as it takes
+// to give every compute unit a workgroup.
+Tensor stream_gemm(const Tensor& x, const Tensor& w, bool swiglu, int64_t k_splits, const c10::optional<Tensor>& out_) {
+  check_bf16_rows(x, "x");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 && w.is_contiguous() && w.size(1) == K,
+              "stream_gemm: weight must be a contiguous bf16 [N, K] GPU tensor with K = ", K);
+  TORCH_CHECK(M >= 1 && M <= 256 && K >= 64 && K % 64 == 0 && N >= 128 && N % 128 == 0, "stream_gemm: 1..256 rows, K % 64 == 0, N % 128 == 0; got M=", M,
+              " N=", N, " K=", K);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "stream_gemm: weight must be 16-byte aligned");
+  if (k_splits == 0) {
+    // never a second, partly filled round of one workgroup (M > 64) or two (M ≤ 64) per compute unit; at least 8 steps each
+    const int64_t blocks = (M + 127) / 128 * (N / 128);
+    k_splits = std::max<int64_t>(1, std::min<int64_t>({256 / blocks, K / 512, 8}));
+  }
+  TORCH_CHECK(k_splits >= 1 && k_splits <= 32 && k_splits <= K / 64, "stream_gemm: k_splits must be in [1, min(32, K / 64)]");
+  Tensor out = take_out(out_, M, swiglu ? N / 2 : N, x);
+  if (k_splits == 1) {
+    dli::launch_stream_gemm(swiglu, x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0), (int)M, (int)K, (int)N, 1, cur_stream(x));
+  } else {
+    Tensor ws = at::empty({k_splits, M, N}, x.options().dtype(at::kFloat));
+    dli::launch_stream_gemm(swiglu, x.data_ptr(), x.stride(0), w.data_ptr(), ws.data_ptr(), N, (int)M, (int)K, (int)N, (int)k_splits, cur_stream(x));
+    dli::launch_splitk_reduce(swiglu, ws.data_ptr<float>(), (int)k_splits, (int)M, (int)N, out.data_ptr(), out.stride(0), cur_stream(x));
+  }
+  return out;
+}
+
+// Row tile of the experts' GEMMs by the rows an expert gets under uniform routing, 2-of-8 routing at Mixtral shapes, µs a layer:
+//   rows       8     16     25     32     50     64    100    113    128
+//   32        455    453    518    606    804    897                         streaming tiles (stream_gemm.hip): their weights pass by
+//   64        479    479    497    484    500    651                         once, a second tile of an expert fetches them again
+//   128       558    560    564    567    606    612    641    843    818    128 × 128 tiles (moe.hip)
+//   256       557    561    565    567    574    576    612    622    643    256² tiles (gemm256.hip)
+// (20 rows on average are seldom more than 32, 53 seldom more than 64.)  The 128 × 128 tiles stay for shapes that the 256² tiles do not
+// take.  DLI_MOE_TILE=32|64|128|256 forces one.
 const int64_t g_moe_tile_force = std::getenv("DLI_MOE_TILE") ? std::atoll(std::getenv("DLI_MOE_TILE")) : 0;
-const int64_t g_moe_tile256_min_rows = std::getenv("DLI_MOE_TILE256_MIN_ROWS") ? std::atoll(std::getenv("DLI_MOE_TILE256_MIN_ROWS")) : 128;
+const int64_t g_moe_tile64_min_rows = 21, g_moe_tile256_min_rows = std::getenv("DLI_MOE_TILE256_MIN_ROWS") ? std::atoll(std::getenv("DLI_MOE_TILE256_MIN_ROWS")) : 54;
 
 const int64_t g_moe_splitk_min_blocks256 = std::getenv("DLI_MOE_SPLITK_MIN_BLOCKS256") ? std::atoll(std::getenv("DLI_MOE_SPLITK_MIN_BLOCKS256")) : 512;
 
@@ -338,33 +370,48 @@ const int64_t g_moe_splitk_min_blocks256 = std::getenv("DLI_MOE_SPLITK_MIN_BLOCK
 const int64_t g_moe_skinny_max_t = std::getenv("DLI_NO_SKINNY_MOE") ? 0
                                    : std::getenv("DLI_SKINNY_MOE_MAX_T") ? std::atoll(std::getenv("DLI_SKINNY_MOE_MAX_T")) : 32;
 
+// workgroups a streaming down projection should have (K slices below): one per compute unit; twice as many slices cost 1 % more in slabs
+const int64_t g_moe_stream_min_blocks = 256;
+int64_t moe_tile_rows(int64_t rows, bool fits256) {
+  if (g_moe_tile_force == 256) return fits256 ? 256 : 128;
+  if (g_moe_tile_force) return g_moe_tile_force;
+  if (rows >= g_moe_tile256_min_rows) return fits256 ? 256 : 128;
+  return rows >= g_moe_tile64_min_rows ? 64 : 32;
+}
+
 // align → grouped GEMM (SwiGLU epilogue) → grouped GEMM (weighted scatter) → sum over the slots of a token, for (token,
 // slot) pairs whose expert ids / gate weights are already on the device (``ids`` < 0 or outside the local range: skipped).
 // ``out``: [T, H] bf16 (any device memory: the expert-parallel path hands in its IPC-visible result buffer).
 void moe_experts_forward(const Tensor& x, const Tensor& ids, const Tensor& wts, const Tensor& w13, const Tensor& w2, int64_t top_k,
-                         int64_t expert_offset, bool big, void* out, hipStream_t stream, float act_limit = 0.f) {
+                         int64_t expert_offset, int64_t TR, void* out, hipStream_t stream, float act_limit = 0.f) {
   const int64_t T = x.size(0), H = x.size(1), El = w13.size(0), I = w13.size(1) / 2;
   const int64_t n = T * top_k;
   auto i32 = x.options().dtype(at::kInt);
-  const int64_t TR = big ? 256 : 128;
   const int64_t capacity = (n + TR - 1) / TR * TR + El * TR;
   const int64_t max_tiles = capacity / TR;
   Tensor sorted = at::empty({capacity}, i32), tile_expert = at::empty({max_tiles}, i32), meta = at::empty({2}, i32);
   Tensor act = at::empty({capacity, I}, x.options());
-  // Down projection: with few row tiles (decode-sized batches) a (row tile × 128 columns) grid cannot fill 256 CUs and
-  // every block would stream a 3.7 MB weight panel through a 16 KB-deep pipeline, so K is cut into slices whose fp32
+  // Down projection: with few row tiles a (row tile × 128 columns) grid cannot fill 256 CUs, so K is cut into slices whose fp32
   // partial slabs are summed (in fixed order) by moe_sum.  The slice count depends on T only: static under hipGraph.
-  const int64_t col_blocks2 = H / TR, nk2 = I / 64;
+  // (512-thread 256² tiles run one per CU: two full rounds of the chip are enough; the 128² tiles run 2–3 per CU; of the streaming tiles
+  // about one an expert has rows)
+  const int64_t nk2 = I / 64;
+  const bool stream_tiles = TR <= 64;
+  const int64_t blocks = stream_tiles ? (std::min(n, El) + n / TR) * (H / 128) : max_tiles * (H / TR);
+  const int64_t want_blocks = stream_tiles ? g_moe_stream_min_blocks : TR == 256 ? g_moe_splitk_min_blocks256 : 1024;
   int64_t k_splits = 1;
-  // (512-thread 256² tiles run one per CU: two full rounds of the chip are enough; the 128² tiles run 2–3 per CU)
-  const int64_t want_blocks = big ? g_moe_splitk_min_blocks256 : 1024;
-  if (max_tiles * col_blocks2 < want_blocks)
-    k_splits = std::min<int64_t>({(want_blocks + max_tiles * col_blocks2 - 1) / (max_tiles * col_blocks2), 16, nk2});
-  const bool split = k_splits > 1;
+  if (blocks < want_blocks)
+    k_splits = std::max<int64_t>(1, std::min<int64_t>({(want_blocks + blocks - 1) / blocks, 16, stream_tiles ? nk2 / 8 : nk2}));
+  const bool split = k_splits > 1 || stream_tiles;           // (few rows: the slots of a token are added in fp32 whatever the slice count)
   Tensor y = split ? at::empty({k_splits, n, H}, x.options().dtype(at::kFloat)) : at::empty({n, H}, x.options());
   dli::launch_moe_align(ids.data_ptr<int>(), (int)n, (int)expert_offset, (int)El, sorted.data_ptr<int>(),
                         tile_expert.data_ptr<int>(), meta.data_ptr<int>(), (int)capacity, (int)TR, stream);
-  auto gg = big ? dli::launch_grouped_gemm256 : dli::launch_grouped_gemm;
+  auto gg = [&](int epi, const void* A, int64_t a_stride, const void* W, int64_t w_stride, const int* ids_, const int* te, const int* mt,
+                const float* tw, int k_, void* o, int64_t os, int K, int N_out, int tiles, int splits, int64_t slab, hipStream_t st, float limit) {
+    if (TR == 256) dli::launch_grouped_gemm256(epi, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
+    else if (TR == 128) dli::launch_grouped_gemm(epi, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
+    else dli::launch_grouped_stream_gemm(epi, (int)TR, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
+  };
   gg(0, x.data_ptr(), H, w13.data_ptr(), 2 * I * H, sorted.data_ptr<int>(), tile_expert.data_ptr<int>(), meta.data_ptr<int>(),
      wts.data_ptr<float>(), (int)top_k, act.data_ptr(), I, (int)H, (int)I, (int)max_tiles, 1, 0, stream, act_limit);
   gg(split ? 2 : 1, act.data_ptr(), I, w2.data_ptr(), H * I, sorted.data_ptr<int>(), tile_expert.data_ptr<int>(),
@@ -381,11 +428,10 @@ void moe_apply(const Tensor& x, const Tensor& ids, const Tensor& wts, const Tens
   const int64_t T = x.size(0), H = x.size(1), El = w13.size(0), I = w13.size(1) / 2;
   auto i32 = x.options().dtype(at::kInt);
   const int64_t n = T * top_k;
-  // 256-row tiles when the experts see enough rows to fill them (and the shapes divide): gemm256.hip
-  bool big = n / E >= g_moe_tile256_min_rows;               // expected rows per expert (local or not) under uniform routing
-  if (g_moe_tile_force) big = g_moe_tile_force == 256;
-  if (tile_rows) big = tile_rows == 256;                     // A/B measurements in one process
-  big = big && I % 128 == 0 && H % 256 == 0 && n * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
+  const bool fits256 = I % 128 == 0 && H % 256 == 0 && n * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
+  int64_t rows = tile_rows;                                  // given: A/B measurements and tests in one process
+  if (rows == 0 || (rows == 256 && !fits256)) rows = moe_tile_rows(n / E, fits256);   // (local experts or not)
+  TORCH_CHECK(rows == 32 || rows == 64 || rows == 128 || rows == 256, "fused_moe: tile_rows must be 0, 32, 64, 128 or 256");
   if (T <= std::min<int64_t>(g_moe_skinny_max_t, 128) && I % 128 == 0 && tile_rows == 0) {
     // Decode-sized batch: an expert sees ≤ 16 rows (at T ≤ 32 and 2-of-8 routing: nearly always; more rows cost an
     // extra pass over that expert's weights from cache), so both projections are pure weight streams — the
@@ -408,7 +454,7 @@ void moe_apply(const Tensor& x, const Tensor& ids, const Tensor& wts, const Tens
                         (int)H, out.data_ptr(), stream);
     return;
   }
-  moe_experts_forward(x, ids, wts, w13, w2, top_k, expert_offset, big, out.data_ptr(), stream, act_limit);
+  moe_experts_forward(x, ids, wts, w13, w2, top_k, expert_offset, rows, out.data_ptr(), stream, act_limit);
 }
 
 // ---- MoE: route → align → grouped GEMM (SwiGLU epilogue) → grouped GEMM (weighted scatter) → sum ----
@@ -507,10 +553,9 @@ Tensor ep_moe(int64_t st, const Tensor& x_l, const Tensor& router_logits_l, cons
   TORCH_CHECK(rc == 0, "ep_moe: dispatch launch rejected");
   // local experts on the received rows: one "slot" per row, gate weight applied here, output straight into the IPC result buffer.
   // Row tile: the expected rows per local expert under uniform routing (what arrives is ≈ r_cap / world of the capacity)
-  bool big = (n_cap * world / std::max<int64_t>(world, 1)) / std::max<int64_t>(El, 1) >= g_moe_tile256_min_rows;
-  if (g_moe_tile_force) big = g_moe_tile_force == 256;
-  big = big && I % 128 == 0 && H % 256 == 0 && r_cap * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
-  moe_experts_forward(recv_x, ids_local, w_local, w13, w2, 1, rank * El, big, dli::ep_result_ptr(state), stream);
+  const bool fits256 = I % 128 == 0 && H % 256 == 0 && r_cap * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
+  const int64_t rows = moe_tile_rows(n_cap / std::max<int64_t>(El, 1), fits256);
+  moe_experts_forward(recv_x, ids_local, w_local, w13, w2, 1, rank * El, rows, dli::ep_result_ptr(state), stream);
   Tensor y_back = at::empty({std::max<int64_t>(n, 1), H}, w13.options());
   rc = dli::launch_ep_combine(state, ids.data_ptr<int>(), slot.data_ptr<int>(), (int)n, (int)n_cap, (int)H, (int)El, y_back.data_ptr(),
                               blocks, stream);
@@ -712,6 +757,7 @@ TORCH_LIBRARY(dli, m) {
   m.def("rms_norm_quant(Tensor x, Tensor(a!)? residual, Tensor weight, float eps) -> (Tensor, Tensor)", &rms_norm_quant);
   m.def("skinny_linear(Tensor x, Tensor w, Tensor? bias, bool swiglu=False, Tensor? out=None, Tensor? w_scale=None) -> Tensor", &skinny_linear);
   m.def("dense_gemm256(Tensor x, Tensor w, bool swiglu=False, int k_splits=1, Tensor? out=None, bool split_tail=False) -> Tensor", &dense_gemm256);
+  m.def("stream_gemm(Tensor x, Tensor w, bool swiglu=False, int k_splits=0, Tensor? out=None) -> Tensor", &stream_gemm);
   m.def("ar_staging_tensor(int state, int rows, int cols, Tensor like) -> Tensor", &ar_staging_tensor);
   m.def("ar_all_reduce_add_norm(int state, Tensor staged, Tensor(a!) residual, Tensor weight, float eps, Tensor(b!) out, int blocks=0) -> ()",
         &ar_all_reduce_add_norm);

@@ -264,15 +264,35 @@ def _tile_operand_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and x.shape[0] * x.stride(0) * 2 < 2 ** 32 and weight.numel() * 2 < 2 ** 32)
 
 
+def stream_rows_ok(m: int, n: int, k: int) -> bool:
+    """Row counts and shapes for which the weight-streaming tiles (``csrc/kernels/stream_gemm.hip``) beat both the library GEMM and the
+    split-K 256² tile: one row tile (up to 128 rows) over at least 64 MiB of weights — with less, the ramp of a launch and the slabs'
+    reduce pass weigh as much as the stream (6144 × 4096: 22.0 against 22.6 µs at 96 rows, 18.6 against 17.6 at 64) — and two row
+    tiles where the columns are few enough to be cut along K anyway (4096 × 14336 at 192 rows 43 against 102 µs, 7168 × 8192 44 against 65;
+    28672 × 4096 76 against 67)."""
+    return 0 < m <= 256 and n * k >= 1 << 25 and n % 128 == 0 and k % 64 == 0 and (m <= 128 or n <= 8192)
+
+
+def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> bool:
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2):
+        return False
+    if not stream_rows_ok(x.shape[0], weight.shape[0], weight.shape[1]) or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
+        return False
+    return (weight.is_contiguous() and weight.data_ptr() % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and (out is None or (out.is_contiguous() and out.data_ptr() % 16 == 0)))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weightᵀ + bias``.  Decode-sized GPU inputs take the weight-streaming MFMA kernel
-    (``csrc/kernels/skinny_gemm.hip``); above that the start-up measurement (``ops/gemm_plan.py``) says, per layer shape
-    and row count, whether the library GEMM (hipBLASLt through torch) or the own 256² tile — with K cut into slices at
+    (``csrc/kernels/skinny_gemm.hip``), decode batches of large layers the streaming tiles (``stream_rows_ok``); above that the
+    start-up measurement (``ops/gemm_plan.py``) says, per layer shape and row count, whether the library GEMM (hipBLASLt through torch) or the own 256² tile — with K cut into slices at
     mid-M — runs; shapes it never measured go to the library.  ``out``: 2-D result buffer to write into (the row-parallel
     layers pass a view of the all-reduce's IPC staging buffer)."""
     if _skinny_ok(x, weight, 16):
         return hip().skinny_linear(x, weight, bias, False, out)
+    if bias is None and _stream_ok(x, weight, out):
+        return hip().stream_gemm(x, weight, False, 0, out)
     if bias is None and _PLAN.table and x.is_cuda and x.dim() == 2:
         s = _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], False)
         if s and _tile_operand_ok(x, weight):
@@ -369,10 +389,12 @@ def gemm256_swiglu_ok(m: int, n_out: int, k: int) -> bool:
 
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``silu(x @ W_gateᵀ) * (x @ W_upᵀ)`` for a fused ``weight = [W_gate; W_up]``: one kernel at decode size
-    (SwiGLU in the epilogue of the weight-streaming GEMM) and at prefill size (SwiGLU in the epilogue of the 256² tile
+    (SwiGLU in the epilogue of the weight-streaming GEMMs) and at prefill size (SwiGLU in the epilogue of the 256² tile
     GEMM: the ``[T, 2·I]`` intermediate never exists), library GEMM + ``silu_and_mul`` in between."""
     if _skinny_ok(x, weight, 32):
         return hip().skinny_linear(x, weight, None, True)
+    if _stream_ok(x, weight):
+        return hip().stream_gemm(x, weight, True)
     if _PLAN.table and x.is_cuda and x.dim() == 2:          # measured at start-up for this shape and row count
         s = _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], True)
         if s is not None:

@@ -441,6 +441,66 @@ def test_fused_moe_256_row_half_tiles_match_reference(counts, H, I):
         assert torch.equal(ops.hip().fused_moe(x, logits, w13, w2, 2, 0, 256).float(), got)
 
 
+@pytest.mark.parametrize("rows,counts,H,I", [(32, [31, 32, 33, 1, 0, 5], 512, 192), (64, [63, 64, 65, 2, 0, 40], 256, 448),
+                                             (32, [100, 8], 4096, 1792), (64, [1, 127], 128, 64)])
+def test_fused_moe_streaming_tiles_match_reference(rows, counts, H, I):
+    """The experts' GEMMs on the weight-streaming tiles (stream_gemm.hip): full, one-over, one-row and empty tiles; inner sizes of one
+    K step, of odd numbers of steps and of several K slices.  Same tolerances as the other tilings: bf16 operands and results."""
+    E = len(counts)
+    T, order = sum(counts), torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    logits = torch.full((T, E), -4.0)
+    logits[torch.arange(T), order] = 3.0
+    logits = logits[torch.randperm(T, generator=torch.Generator().manual_seed(3))].to(DEV).bfloat16()
+    x = _bf(T, H, seed=58)
+    w13, w2 = _bf(E, 2 * I, H, seed=59, scale=0.03), _bf(E, H, I, seed=60, scale=0.03)
+    got = ops.hip().fused_moe(x, logits, w13, w2, 1, 0, rows)
+    want = ref.moe_ref(x.float(), logits.float(), w13.float(), w2.float(), 1, 0).float()
+    scale = want.abs().max()
+    assert (got.float() - want).abs().max() / scale < 3e-2
+    assert (got.float() - ops.hip().fused_moe(x, logits, w13, w2, 1, 0, 128).float()).abs().max() / scale < 1.5e-2
+    for _ in range(3):
+        assert torch.equal(ops.hip().fused_moe(x, logits, w13, w2, 1, 0, rows), got)
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 128, 64, 1), (17, 256, 128, 1), (32, 384, 192, 3), (33, 128, 448, 1), (64, 256, 4096, 8), (65, 128, 320, 5),
+                                          (96, 512, 256, 2), (97, 256, 64, 1), (128, 128, 1024, 0), (129, 256, 512, 0), (200, 384, 192, 1),
+                                          (256, 8192, 4096, 0)])
+def test_stream_gemm_matches_fp32_reference(M, N, K, splits, swiglu):
+    """Weight-streaming tiles of 32 / 64 / 96 / 128 rows at their edges, one and two row tiles, one K step and odd numbers of them, K slices
+    whose step counts differ.  Both sides see the same bf16 operands: the error is the rounding of the result (2⁻⁸) and fp32 sums."""
+    x, w = _bf(M, K, seed=61), _bf(N, K, seed=62, scale=K ** -0.5)
+    got = ops.hip().stream_gemm(x, w, swiglu, splits).float()
+    want = x.float() @ w.float().t()
+    if swiglu:
+        want = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2e-3)
+
+
+def test_stream_gemm_dispatch():
+    """``linear`` / ``linear_swiglu`` take the streaming tiles for large layers — strided activation rows, a given result buffer — and what
+    these do not take goes where it went: a bias, a result that is a view of wider rows, gradients."""
+    M, N, K = 40, 8192, 4096
+    big = _bf(M, 2 * K, seed=63)
+    x, w, b = big[:, K:], _bf(N, K, seed=64, scale=K ** -0.5), _bf(N, seed=65)
+    want = x.float() @ w.float().t()
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    assert ops.linear(x, w, out=out).data_ptr() == out.data_ptr()
+    assert torch.equal(out, ops.hip().stream_gemm(x, w)) and torch.equal(ops.linear(x, w), out)
+    torch.testing.assert_close(out.float(), want, rtol=2 ** -7, atol=2e-3)
+    torch.testing.assert_close(ops.linear(x, w, b).float(), want + b.float(), rtol=2e-2, atol=2e-2)
+    wide = torch.empty(M, 2 * N, dtype=torch.bfloat16, device=DEV)
+    ops.linear(x, w, out=wide[:, :N])
+    torch.testing.assert_close(wide[:, :N].float(), want, rtol=2 ** -7, atol=2e-3)
+    assert torch.equal(ops.linear_swiglu(x, w), ops.hip().stream_gemm(x, w, True))
+    with torch.enable_grad():
+        leaf = x.clone().requires_grad_()
+        ops.linear(leaf, w).float().sum().backward()
+        assert leaf.grad is not None
+    with pytest.raises(RuntimeError):
+        ops.hip().stream_gemm(_bf(257, K, seed=1), w)
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 512, 256), (1000, 1024, 4096), (4096, 256, 512), (1, 256, 64), (300, 768, 1024),
                                    (513, 256, 192)])
 def test_dense_gemm256_matches_fp32_reference(M, N, K):
