@@ -151,7 +151,7 @@ __device__ __forceinline__ bf16x8 softmax_step(f32x4 (&s)[2], int tok0, int limi
 }
 
 // ==================================================================================================
-// Decode: 4 waves per workgroup; wave w takes pages w, w+4, … of the workgroup's page range of one (sequence, kv head).
+// Decode: NW waves per workgroup; wave w takes pages w, w + NW, … of the workgroup's page range of one (sequence, kv head).
 // The kv head is the fastest grid index: the 8 heads of a sequence (contiguous 64 KB per page) are read at the same
 // time by neighbouring workgroups, and a long sequence's work is spread over 8 workgroups that start together instead
 // of 8 that start num_seqs ids apart: +3–4 % on mixed-length batches (profiles/kernels_decode_r2aa.txt).
@@ -159,16 +159,16 @@ __device__ __forceinline__ bf16x8 softmax_step(f32x4 (&s)[2], int tok0, int limi
 // Two ways to say which pages a workgroup reads:
 //   WL = true   work list, grid (Hkv, items): `work[item] = {sequence, first page, end page, partial slot}` built by the
 //               host per step (ops.build_decode_work) — page ranges of about equal size whatever the sequence's length,
-//               so a 2048-token row and a 40-token row no longer get the same split count and the tail of the launch is
-//               one chunk long.  slot < 0: the range is the whole sequence, the result goes straight to `out`.  The
+//               so a 2048-token row and a 40-token row no longer get the same split count, longest range first, so the tail of
+//               the launch is made of short ones (B = 160 of 128 … 2048 tokens, 721 MB: 122 µs in row order, 110 sorted).  slot < 0: the range is the whole sequence, the result goes straight to `out`.  The
 //               number of valid items is read from DEVICE memory (`counts[0]`; extra workgroups exit), which is what
 //               lets a hipGraph with a fixed grid serve any batch.
 //   WL = false  uniform splits, grid (Hkv, num_seqs, num_splits): every sequence is cut into `num_splits` ranges.
 // Partial results: `part_o[(p·Hq + head)·128 + d]`, `part_ml[(p·Hq + head)·2 + {m, l}]` with p = slot (WL) or
 // seq·num_splits + split; decode_reduce_kernel combines them per sequence.
 // ==================================================================================================
-template <bool KV8, bool WL, bool NT = false>
-__global__ __launch_bounds__(256) void paged_decode_kernel(
+template <bool KV8, bool WL, int NW, bool NT = false>
+__global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, uint16_t* __restrict__ out,
     int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_splits,
@@ -227,9 +227,9 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
   // the block-table entry of the NEXT page of this wave is fetched one iteration ahead: the entry → page address → 16
   // fragment loads chain is otherwise paid in full at the top of every iteration
   int blk_next = b_begin + wave < b_end ? bt[b_begin + wave] : 0;
-  for (int b = b_begin + wave; b < b_end; b += 4) {
+  for (int b = b_begin + wave; b < b_end; b += NW) {
     const int blk_cur = blk_next;
-    if (b + 4 < b_end) blk_next = bt[b + 4];
+    if (b + NW < b_end) blk_next = bt[b + NW];
     const int64_t page = ((int64_t)blk_cur * Hkv + kvh) * (PAGE_ELEMS * ESZ);
     bf16x8 kf[2][4];
     KLoader<KV8>::template load<NT>(kc + page, col, g, kf);
@@ -257,13 +257,13 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
   }
   lsum = group_sum(lsum);
 
-  // ---- merge the 4 waves through LDS: [wave][G][128 + 4] fp32 + [wave][G] (m, l).  Rows are padded by one 16-byte
+  // ---- merge the waves through LDS: [wave][G][128 + 4] fp32 + [wave][G] (m, l).  Rows are padded by one 16-byte
   // slot: the G active lanes of a ds_write_b128 lane group hold the same d range of G different rows, and with
   // 512-byte rows they would all start on bank 0 (4-way conflict: 0.46 conflict cycles per LDS cycle in round 1).
   constexpr int HDP = HD + 4;
   float* sm_o = smem;
-  float* sm_m = smem + 4 * G * HDP;
-  float* sm_l = sm_m + 4 * G;
+  float* sm_m = smem + NW * G * HDP;
+  float* sm_l = sm_m + NW * G;
   if (col < G) {
     float* dst = sm_o + (wave * G + col) * HDP + 4 * g;
 #pragma unroll
@@ -271,14 +271,14 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
     if (g == 0) { sm_m[wave * G + col] = m; sm_l[wave * G + col] = lsum; }
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < G * HD; idx += 256) {
+  for (int idx = threadIdx.x; idx < G * HD; idx += NW * 64) {
     const int head = idx >> 7, d = idx & 127;
     float M = NEG_BIG;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, sm_m[w * G + head]);
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w * G + head]);
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = fast_exp2(sm_m[w * G + head] - M);
       num += f * sm_o[(w * G + head) * HDP + d];
       den += f * sm_l[w * G + head];
@@ -308,16 +308,28 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
     const int4 r = red[blockIdx.x];
     seq = r.x, first = r.y, n = r.z;
   }
-  const int qh = blockIdx.y, d = threadIdx.x;
+  const int qh = blockIdx.y, d = threadIdx.x, lane = threadIdx.x & 63;
   if (kv_scales != nullptr) v_scale = kv_scales[Hkv + qh / (Hq / Hkv)];
-  float M = NEG_BIG;
-  for (int s = 0; s < n; ++s) M = fmaxf(M, part_ml[((int64_t)(first + s) * Hq + qh) * 2]);
-  float num = 0.f, den = 0.f;
-  for (int s = 0; s < n; ++s) {
-    const int64_t slot = (int64_t)(first + s) * Hq + qh;
-    const float f = fast_exp2(part_ml[slot * 2] - M);
-    num += f * part_o[slot * HD + d];
-    den += f * part_ml[slot * 2 + 1];
+  // 64 partials at a time, a lane each: their (m, l) arrive together and the rows' loads do not wait for one another.  (One after the
+  // other — a load's latency per partial, twice — five partials took 4.5 µs.)
+  float M = NEG_BIG, num = 0.f, den = 0.f;
+  for (int s0 = 0; s0 < n; s0 += 64) {
+    const int k = min(n - s0, 64);
+    const int64_t slot0 = (int64_t)(first + s0) * Hq + qh;
+    const bool in = lane < k;
+    const f32x2 ml = in ? *reinterpret_cast<const f32x2*>(part_ml + (slot0 + (int64_t)lane * Hq) * 2) : f32x2{NEG_BIG, 0.f};
+    const float Mn = fmaxf(M, wave_max(ml[0])), old = fast_exp2(M - Mn);
+    const float f = in ? fast_exp2(ml[0] - Mn) : 0.f;
+    den = den * old + wave_sum(f * ml[1]);
+    num *= old;
+    M = Mn;
+    for (int s = 0; s < k; s += 8) {
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = part_o[(slot0 + (int64_t)min(s + j, k - 1) * Hq) * HD + d];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) num += s + j < k ? __shfl(f, s + j, 64) * x[j] : 0.f;
+    }
   }
   const float r = den > 0.f ? v_scale / den : 0.f;
   out[(int64_t)seq * out_stride + qh * HD + d] = f2bf(num * r);
@@ -580,6 +592,8 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_kernel(
 // trace's length mix at B = 1024 (profiles/ab_decode_nt_r3.jsonl).  DLI_DECODE_NT=0: plain loads (A/B knob).
 static const bool g_decode_nt = std::getenv("DLI_DECODE_NT") == nullptr || std::atoi(std::getenv("DLI_DECODE_NT")) != 0;
 
+static size_t decode_lds(int waves, int G) { return (size_t)(waves * G * (HD + 4) + 2 * waves * G) * sizeof(float); }
+
 void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
                          const int* block_tables, int max_blocks, const int* seq_lens, void* out, int64_t out_stride,
                          float* part_o, float* part_ml, int num_seqs, int Hq, int Hkv, int num_splits, float scale,
@@ -588,11 +602,10 @@ void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, c
   const int G = Hq / Hkv;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;        // the kernels read the per-head values themselves
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-  const size_t lds = (size_t)(4 * G * (HD + 4) + 8 * G) * sizeof(float);
   dim3 grid(Hkv, num_seqs, num_splits);
 #define DLI_DECODE_GO(KV8_, NT_)                                                                                              \
-  hipLaunchKernelGGL((paged_decode_kernel<KV8_, false, NT_>), grid, dim3(256), lds, stream, (const uint16_t*)q, q_stride, k_cache, \
-                     v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv,           \
+  hipLaunchKernelGGL((paged_decode_kernel<KV8_, false, 4, NT_>), grid, dim3(256), decode_lds(4, G), stream, (const uint16_t*)q, q_stride, \
+                     k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv,    \
                      num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, nullptr, nullptr)
   if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, true); else DLI_DECODE_GO(true, false); }
   else { if (g_decode_nt) DLI_DECODE_GO(false, true); else DLI_DECODE_GO(false, false); }
@@ -613,14 +626,18 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
   const int G = Hq / Hkv;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-  const size_t lds = (size_t)(4 * G * (HD + 4) + 8 * G) * sizeof(float);
   dim3 grid(Hkv, items);
-#define DLI_DECODE_GO(KV8_, NT_)                                                                                              \
-  hipLaunchKernelGGL((paged_decode_kernel<KV8_, true, NT_>), grid, dim3(256), lds, stream, (const uint16_t*)q, q_stride, k_cache,  \
-                     v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv, 1,        \
-                     scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work, counts)
-  if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, true); else DLI_DECODE_GO(true, false); }
-  else { if (g_decode_nt) DLI_DECODE_GO(false, true); else DLI_DECODE_GO(false, false); }
+#define DLI_DECODE_GO(KV8_, NW_, NT_)                                                                                         \
+  hipLaunchKernelGGL((paged_decode_kernel<KV8_, true, NW_, NT_>), grid, dim3(NW_ * 64), decode_lds(NW_, G), stream, (const uint16_t*)q, \
+                     q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq,  \
+                     Hkv, 1, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work, counts)
+  // bf16: eight waves a workgroup halve a whole row's serial pages; e4m3 pages take half the bytes a wave and the registers of the
+  // widening: four.  Sorted lists, 32/8 heads, µs, 4 against 8 waves — bf16, rows of up to 1500 / 2048 tokens: B = 100 55.9 / 52.6, 160 111.8 /
+  // 109.5, 300 199 / 199; e4m3: B = 100 30.0 / 32.6, 160 60.1 / 60.9, 300 104.6 / 112.4.
+  // Groups of more than 8 heads keep four: eight waves' merge buffers would pass 64 KB of LDS.
+  if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, 4, true); else DLI_DECODE_GO(true, 4, false); }
+  else if (G > 8) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
+  else { if (g_decode_nt) DLI_DECODE_GO(false, 8, true); else DLI_DECODE_GO(false, 8, false); }
 #undef DLI_DECODE_GO
   if (reds > 0)
     hipLaunchKernelGGL(decode_reduce_kernel, dim3(reds, Hq), dim3(128), 0, stream, part_o, part_ml, (uint16_t*)out,

@@ -153,7 +153,7 @@ def build_decode_work(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int = 
 
     Every sequence's pages are cut into ``ceil(pages / chunk)`` ranges of EQUAL size (rounded up to 4 pages), so a
     2048-token row becomes several workgroups per kv head and a 40-token row one.  Returns
-    ``work int32 [items, 4] = (row, first page, end page, partial slot | -1)``, ``red int32 [r, 4] = (row, first
+    ``work int32 [items, 4] = (row, first page, end page, partial slot | -1)``, longest ranges first, ``red int32 [r, 4] = (row, first
     partial, partials, 0)`` for the rows with more than one range, and the number of partial slots."""
     L = np.asarray(seq_lens, dtype=np.int64)
     n = len(L)
@@ -175,6 +175,7 @@ def build_decode_work(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int = 
     pfirst = np.cumsum(pk) - pk
     slot = np.where(multi[row], pfirst[row] + j, -1)
     work = np.stack([row, begin, end, slot], axis=1).astype(np.int32)
+    work = work[np.argsort(begin - end, kind="stable")]        # longest first: the launch ends on short ranges
     mrows = np.flatnonzero(multi)
     red = np.stack([mrows, pfirst[mrows], k[mrows], np.zeros_like(mrows)], axis=1).astype(np.int32)
     return work, red, int(pk.sum())

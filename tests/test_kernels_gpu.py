@@ -209,6 +209,26 @@ def test_decode_work_list_equals_uniform_splits_bitwise_on_single_range_rows():
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("Hq,Hkv,seq_lens,chunk", [(32, 4, [8500, 8192, 1, 260], 4), (8, 1, [255, 256, 257, 288, 225, 31], 16), (16, 1, [289, 33, 513], 8),
+                                                   (9, 1, [300, 64], 8), (4, 4, [8231, 2049], 4)])
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_decode_many_ranges_and_wave_remainders(Hq, Hkv, seq_lens, chunk, kv_dtype):
+    """The reduce past one wave of partials (8500 tokens in ranges of 4 pages: 67), pages that do not divide by the eight or four waves, and the
+    group size at which the merge buffer takes four waves.  Weights and results are rounded to bf16 (2^-9 each, |v| ≤ 4.5 here)."""
+    scales = (0.5, 0.25) if kv_dtype == torch.float8_e4m3fn else (1.0, 1.0)
+    kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=33, scales=scales)
+    B = len(seq_lens)
+    qkv = _bf(B, (Hq + 2 * Hkv) * 128, seed=34)
+    sl = torch.tensor(seq_lens, dtype=torch.int32, device=DEV)
+    qsl = torch.arange(B + 1, dtype=torch.int32, device=DEV)
+    meta = ops.AttnMetadata(num_decode=B, num_prefill=0, num_tokens=B, positions=None, slot_mapping=None,
+                            block_tables=bt, seq_lens=sl, query_start_loc=qsl)
+    ops.attach_decode_worklist(meta, np.array(seq_lens), Hq, Hkv, DEV, chunk_pages=chunk)
+    got = ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088, *scales).float()
+    want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(B, Hq, 128), kc, vc, bt, sl, qsl, 0.088, *scales).float()
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -9 * 4.5)
+
+
 def test_decode_softmax_rescale_branch():
     """One key dominates late in the sequence: forces a large running-max jump (guide rule 26)."""
     Hq, Hkv, L = 32, 8, 300
