@@ -97,6 +97,38 @@ def test_rope_and_cache(Hq, Hkv, kv_dtype, layout):
         torch.testing.assert_close(vc.float(), vc_ref.float(), rtol=0.13, atol=0.02)
 
 
+@pytest.mark.parametrize("T", [128, 129, 515])                    # one workgroup a token; v in groups of four slots
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_rope_and_cache_runs_of_slots(T, kv_dtype):
+    """Prompts that begin at batch rows and cache slots which are no multiples of four, runs shorter than a group, padding inside one, pages in
+    any order, and a step's last rows: v must come out as the reference packer writes it (a copy; e4m3: the same rounding)."""
+    Hq, Hkv, nblocks = 8, 2, 64
+    g = torch.Generator().manual_seed(T)
+    pages = torch.randperm(nblocks, generator=g)
+    lin = torch.arange(5, 5 + T)                                    # decode rows, then prompts of 1, 2, 3, 7, 37 … tokens from there on
+    slots = (pages[lin // 32] * 32 + lin % 32).to(torch.int32)
+    slots[3:23] = slots[3:23].flip(0)                               # twenty unrelated rows
+    for at in (40, 61, 62, T - 1):
+        slots[at] = -1
+    slots = slots.to(DEV)
+    qkv = _bf(T, (Hq + 2 * Hkv) * 128, seed=10)
+    pos = torch.randint(0, 4000, (T,), generator=g).to(torch.int32).to(DEV)
+    cs = ref.build_cos_sin_cache(4096, 128, 500000.0, DEV)
+    ks, vs = (0.05, 0.07) if kv_dtype == torch.float8_e4m3fn else (1.0, 1.0)
+    kc, vc = _caches(nblocks, Hkv, kv_dtype)
+    kc_ref, vc_ref = _caches(nblocks, Hkv, kv_dtype)
+    qkv_ref = qkv.clone()
+    ops.rope_and_cache(qkv, pos, cs, slots, kc, vc, Hq, Hkv, 128, ks, vs)
+    ref.rope_and_cache_ref(qkv_ref, pos, cs, slots, kc_ref, vc_ref, Hq, Hkv, 128, ks, vs)
+    torch.testing.assert_close(qkv.float(), qkv_ref.float(), rtol=2 ** -7, atol=2 ** -6)
+    if kv_dtype == torch.bfloat16:
+        assert torch.equal(vc, vc_ref)
+        torch.testing.assert_close(kc.float(), kc_ref.float(), rtol=2 ** -7, atol=2 ** -6)
+    else:                                                           # one e4m3 step = 12.5 %: a product and a quotient by the scale differ by it
+        torch.testing.assert_close(vc.float(), vc_ref.float(), rtol=0.13, atol=0.02)
+        torch.testing.assert_close(kc.float(), kc_ref.float(), rtol=0.13, atol=0.02)
+
+
 def test_fp8_cache_write_saturates_instead_of_nan():
     """Values past scale × 448 (activation outliers beyond the calibrated head-room) must store ±448, never the e4m3
     NaN pattern: one NaN key poisons every later softmax of its sequence (found with the 80 req/s fp8 bench)."""
