@@ -308,6 +308,31 @@ def test_paged_attention_prefill_and_mixed(Hq, Hkv, kv_dtype):
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("n", [1, 64, 65])                        # 8, 512 and 520 workgroups: two page groups, two, one
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
+    """Tiles of one page (the second group has none), of an odd and of an even number, with masked last pages; keys whose scores rise by more
+    and by less than the 2^8 that moves the running maximum.  Weights and results are rounded to bf16 (2^-9 each, |v| ≤ 4.5 here)."""
+    Hq = Hkv = 8
+    lens = [1, 31, 32, 33, 64, 65, 96, 97, 129, 300]
+    seq_lens = [lens[(i + 7) % 10] for i in range(n)]
+    qlens = [min(L, 1 + 13 * i % 120) for i, L in enumerate(seq_lens)]
+    scales = (0.5, 0.25) if kv_dtype == torch.float8_e4m3fn else (1.0, 1.0)
+    kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=23, scales=scales)
+    T = sum(qlens)
+    qkv = _bf(T, (Hq + 2 * Hkv) * 128, seed=24)
+    qkv[::3] *= 8                                                   # scores of ± 40: steps of the maximum past 2^8
+    sl = torch.tensor(seq_lens, dtype=torch.int32, device=DEV)
+    qsl = torch.tensor(np.concatenate([[0], np.cumsum(qlens)]), dtype=torch.int32, device=DEV)
+    ts, t0 = ops.build_prefill_tiles(np.array(qlens), 0, ops.prefill_tile_tokens(Hq, Hkv))
+    meta = ops.AttnMetadata(num_decode=0, num_prefill=n, num_tokens=T, positions=None, slot_mapping=None, block_tables=bt, seq_lens=sl,
+                            query_start_loc=qsl, decode_splits=1, prefill_tile_seq=torch.from_numpy(ts).to(DEV),
+                            prefill_tile_q0=torch.from_numpy(t0).to(DEV), num_prefill_tiles=len(ts))
+    got = ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088, *scales).float()
+    want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(T, Hq, 128), kc, vc, bt, sl, qsl, 0.088, *scales).float()
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -9 * 4.5)
+
+
 @pytest.mark.parametrize("V", [32000, 128256])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_sampler_matches_reference_with_shared_noise(V, dtype):
