@@ -141,6 +141,26 @@ __device__ __forceinline__ void shift_rows(const A* xr, float* st, int taps, int
   }
 }
 
+// decay and input weight of head h of token t (live: not a padding row)
+template <typename A>
+__device__ __forceinline__ void head_gate(const GateArgs<A>& gate, int64_t x_stride, int64_t t, int h, bool live) {
+  const int64_t at = t * gate.H + h;
+  if (!live) {
+    gate.decay[at] = gate.weight[at] = 0.f;
+    return;
+  }
+  const A* gr = gate.g + t * x_stride;
+  if (gate.kind == 3) {                                           // write strengths only
+    gate.decay[at] = 0.f;
+    gate.weight[at] = 1.f / (1.f + expf(-ldf<A>(gr + h)));
+    return;
+  }
+  const float z = ldf<A>(gr + (gate.kind == 1 ? gate.H + h : h)) + gate.bias[h];
+  const float sp = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));       // softplus
+  gate.decay[at] = -gate.rate[h] * sp;
+  gate.weight[at] = gate.kind == 1 ? 1.f / (1.f + expf(-ldf<A>(gr + h))) : sp;
+}
+
 template <typename A, typename O, int V>
 __global__ __launch_bounds__(NT) void causal_conv_kernel(const A* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
                                                          const float* __restrict__ bias, int taps, float* state,
@@ -154,7 +174,7 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const A* __restrict__ x
   if (seq < 0 || state_slots[seq] < 0) {                         // padding row
     for (int c = c0 + threadIdx.x; c < c1; c += NT) stf<O>(out + t * C + c, 0.f);
     if (gate.kind != 0 && blockIdx.y == 0)
-      for (int h = threadIdx.x; h < gate.H; h += NT) gate.decay[t * gate.H + h] = gate.weight[t * gate.H + h] = 0.f;
+      for (int h = threadIdx.x; h < gate.H; h += NT) head_gate(gate, x_stride, t, h, false);
     return;
   }
   const int p = positions[t];
@@ -178,20 +198,8 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const A* __restrict__ x
     for (int k = 0; k < V; ++k) o.v[k] = a.v[k];
     o.store(out + t * C + c);
   }
-  if (gate.kind != 0 && blockIdx.y == gridDim.y - 1) {
-    const A* gr = gate.g + t * x_stride;
-    for (int h = threadIdx.x; h < gate.H; h += NT) {
-      if (gate.kind == 3) {                                       // write strengths only
-        gate.decay[t * gate.H + h] = 0.f;
-        gate.weight[t * gate.H + h] = 1.f / (1.f + expf(-ldf<A>(gr + h)));
-        continue;
-      }
-      const float z = ldf<A>(gr + (gate.kind == 1 ? gate.H + h : h)) + gate.bias[h];
-      const float sp = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));  // softplus
-      gate.decay[t * gate.H + h] = -gate.rate[h] * sp;
-      gate.weight[t * gate.H + h] = gate.kind == 1 ? 1.f / (1.f + expf(-ldf<A>(gr + h))) : sp;
-    }
-  }
+  if (gate.kind != 0 && blockIdx.y == gridDim.y - 1)
+    for (int h = threadIdx.x; h < gate.H; h += NT) head_gate(gate, x_stride, t, h, true);
   if (c0 >= nu) return;
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -202,6 +210,120 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const A* __restrict__ x
     for (int i = lane; i < unit.d; i += 64) ss += row[i] * row[i];
     const float inv = (u < unit.scaled ? unit.scale : 1.f) / sqrtf(wave_sum(ss) + 1e-6f);
     for (int i = lane; i < unit.d; i += 64) stf<O>(out + t * C + u * unit.d + i, row[i] * inv);
+  }
+}
+
+// Four taps, RUN tokens of a step and 4 · NT channels per workgroup: a thread keeps its channels' four weights and the last three inputs in
+// registers, so a token costs its own row read and its result written instead of four rows of weights and four of inputs.  A sequence
+// that begins inside a run takes its inputs from its chunk or its state rows.  Vectors lie in d / 4 neighbouring lanes.  4096 channels, 3162
+// rows, state rows included: 39.2 → 22.2 µs (3.5 TB/s of the input and the result; bound by them and by how few workgroups a short step has;
+// runs of 8 tokens 23.8, of 16 41.1).
+constexpr int RUN = 4;
+template <typename A, typename O>
+__global__ __launch_bounds__(NT) void causal_conv_run_kernel(const A* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
+                                                             const float* __restrict__ bias, float* state,
+                                                             const int* __restrict__ positions, const int* __restrict__ token_seq,
+                                                             const int* __restrict__ qsl, const int* __restrict__ state_slots, int C,
+                                                             int rows, O* __restrict__ out, int silu, ConvUnit unit, GateArgs<A> gate) {
+  const int t0 = blockIdx.x * RUN, n = min(RUN, rows - t0);
+  const int c = (int)(blockIdx.y * NT + threadIdx.x) * 4;
+  if (gate.kind != 0 && blockIdx.y == gridDim.y - 1)
+    for (int i = threadIdx.x; i < n * gate.H; i += NT) {
+      const int t = t0 + i / gate.H, seq = token_seq[t];
+      head_gate(gate, x_stride, t, i % gate.H, seq >= 0 && state_slots[seq] >= 0);
+    }
+  if (c >= C) return;
+  Vec<A, 4> in[RUN];
+#pragma unroll
+  for (int i = 0; i < RUN; ++i) in[i].load(x + (int64_t)(t0 + min(i, n - 1)) * x_stride + c);
+  Vec<float, 4> wt[4], b, h1, h2, h3;                            // h_d: the input d tokens back
+#pragma unroll
+  for (int j = 0; j < 4; ++j) wt[j].load(w + (int64_t)j * C + c);
+  if (bias != nullptr) b.load(bias + c);
+  else
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b.v[k] = 0.f;
+  float a[RUN][4];
+  int cur = -1, p = 0;
+  bool live = false, single = false;
+  float* st = nullptr;
+#pragma unroll
+  for (int i = 0; i < RUN; ++i) {
+    const int t = t0 + min(i, n - 1);
+    const int seq = token_seq[t];
+    if (i < n && seq != cur) {
+      cur = seq;
+      const int slot = seq < 0 ? -1 : state_slots[seq];
+      live = slot >= 0;
+      if (live) {
+        const int q0 = qsl[seq], back = t - q0;
+        single = qsl[seq + 1] - q0 == 1;
+        p = positions[t];
+        st = state + (int64_t)slot * 3 * C + c;
+        const A* xr = x + (int64_t)t * x_stride + c;
+        auto before = [&](int d) {
+          Vec<float, 4> v;
+          if (d <= back) {
+            Vec<A, 4> xv;
+            xv.load(xr - (int64_t)d * x_stride);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v.v[k] = xv.v[k];
+          } else {
+            v.load(st + (int64_t)(3 - (d - back)) * C);
+          }
+          return v;
+        };
+        h1 = before(1);
+        h2 = before(2);
+        h3 = before(3);
+      }
+    }
+    if (i < n && live) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float s = b.v[k];                                         // taps that would reach before position 0 are skipped
+        if (p >= 3) s += wt[0].v[k] * h3.v[k];
+        if (p >= 2) s += wt[1].v[k] * h2.v[k];
+        if (p >= 1) s += wt[2].v[k] * h1.v[k];
+        s += wt[3].v[k] * in[i].v[k];
+        a[i][k] = silu ? s * sigmoid_f(s) : s;
+        h3.v[k] = h2.v[k];
+        h2.v[k] = h1.v[k];
+        h1.v[k] = in[i].v[k];
+      }
+      if (single) {                                               // the one token of a sequence also moves its state rows on
+        h3.store(st);
+        h2.store(st + C);
+        h1.store(st + 2 * (int64_t)C);
+      }
+      ++p;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[i][k] = 0.f;                 // padding row
+    }
+  }
+  if (c < unit.n * unit.d) {
+    float ss[RUN];
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) ss[i] = a[i][0] * a[i][0] + a[i][1] * a[i][1] + a[i][2] * a[i][2] + a[i][3] * a[i][3];
+    for (int m = unit.d >> 3; m > 0; m >>= 1)
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) ss[i] += __shfl_xor(ss[i], m, 64);
+    const float scale = c < unit.scaled * unit.d ? unit.scale : 1.f;
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+      const float inv = scale / sqrtf(ss[i] + 1e-6f);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[i][k] *= inv;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RUN; ++i) {
+    if (i >= n) break;
+    Vec<O, 4> o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o.v[k] = a[i][k];
+    o.store(out + (int64_t)(t0 + i) * C + c);
   }
 }
 
@@ -627,7 +749,18 @@ void launch_rm_causal_conv(const void* x, bool bf16, int64_t x_stride, const flo
                                                            qsl, state_slots, C, (O*)out, silu ? 1 : 0, unit,                          \
                                                            (GateArgs<A>{gate_kind, gate_heads, (const A*)gate, gate_rate, gate_bias,  \
                                                                         decay, weight}), span)))
-  if (C % 4 == 0 && nu % 4 == 0 && x_stride % 4 == 0 && al16(x) && al16(w) && al16(bias) && al16(state) && al16(out)) RM_CONV(4);
+  const bool wide = C % 4 == 0 && nu % 4 == 0 && x_stride % 4 == 0 && al16(x) && al16(w) && al16(bias) && al16(state) && al16(out);
+  // One workgroup per token below 128 rows, where its four times as many workgroups matter more than their bytes: 4096 / 8192 channels, µs, a token /
+  // a run each: 128 rows 7.1 / 6.9 and 11.0 / 7.8, 256 10.2 / 7.3 and 14.7 / 11.1, 1200 20.1 / 14.4 and 32.1 / 20.7; 17 rows 6.8 / 6.9.  Steps of
+  // single tokens only (no chunks) read four state rows a token whatever the split.
+  const bool vectors_in_lanes = nu == 0 || (unit_d >= 4 && unit_d <= 256 && (unit_d & (unit_d - 1)) == 0);
+  if (wide && taps == 4 && chunks && rows >= 128 && vectors_in_lanes)
+    RM_BF16(bf16, A, RM_BF16(out_bf16, O, hipLaunchKernelGGL((causal_conv_run_kernel<A, O>), dim3((rows + RUN - 1) / RUN, (C + 4 * NT - 1) / (4 * NT)), dim3(NT), 0,
+                                                             stream, (const A*)x, x_stride, w, bias, state, positions, token_seq, qsl,
+                                                             state_slots, C, rows, (O*)out, silu ? 1 : 0, unit,
+                                                             (GateArgs<A>{gate_kind, gate_heads, (const A*)gate, gate_rate, gate_bias,
+                                                                          decay, weight}))));
+  else if (wide) RM_CONV(4);
   else RM_CONV(1);
 #undef RM_CONV
   if (taps > 1 && seqs > 0 && chunks)

@@ -158,6 +158,40 @@ def test_scan_kernels_against_the_reference(delta, normaliser, H, G, D, Dv, dtyp
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,C,unit,gate", [([1, 1, 2, 3, 5, 500], 4 * 1024 + 128, (6, 128, 3, 0.5), "delta"), ([600, 1, 7, 8, 9, 1], 1020, (255, 4, 9, 2.0), "ssd"),
+                                              ([1, 700], 768, (3, 256, 1, 0.25), "beta"), ([121, 3], 64, None, None), ([122, 3], 512, (2, 128, 1, 1.0), "delta")])
+def test_convolution_runs_against_the_reference(lens, C, unit, gate, dtype):
+    """Four taps over sequences that begin, end and are single tokens anywhere in a run of tokens, chunks at positions 0 … 3 and later, three
+    padding rows, channels past the last whole workgroup, vectors of one to 64 lanes, 127 and 128 rows.  Two steps, so that the
+    state rows carry over.  Four products and a unit vector in fp32: a few 2^-23 of the largest sum; bf16 inputs enter exactly."""
+    from dli_amd.ops import seqmix
+    torch.manual_seed(7)
+    H = 4
+    w, bias, rate = torch.randn(4, C), torch.randn(C), torch.rand(H)
+    bias = bias if unit is None or unit[1] == 4 else None
+    cols = {"delta": 2 * H, "ssd": H, "beta": H, None: 0}[gate]
+    st_c = torch.randn(len(lens) + 4, 3, C)
+    st_g = st_c.cuda()
+    starts = [0, 1, 2, 3, 0, 9][:len(lens)]
+    for _ in range(2):
+        mc, T = _step(lens, starts, "cpu")
+        mg, _ = _step(lens, starts, "cuda")
+        mg.token_seq, mg.positions = (torch.nn.functional.pad(m, (0, 3), value=-1) for m in (mg.token_seq, mg.positions))
+        x = torch.randn(T + 3, C + cols).to(dtype)
+        run = lambda x, w, bias, st, m: seqmix.causal_conv(x[:, :C], w, bias, st, m, torch.float32, "silu" if unit else "none", unit,
+                                                           gates=(gate, x[:, C:], rate.to(x.device), rate.to(x.device)) if gate else None)
+        want = run(x, w, bias, st_c, mc)
+        got = run(x.cuda(), w.cuda(), None if bias is None else bias.cuda(), st_g, mg)
+        for a, b in (zip(got, want) if gate else ((got, want),)):
+            assert float((a[:T].cpu() - b[:T]).abs().max()) < 1e-5 * max(1.0, float(b[:T].abs().max()))
+            assert not a[T:].any()
+        starts = [s + n for s, n in zip(starts, lens)]
+        p1 = (mc.positions[(mc.query_start_loc[1:] - 1).long()] + 1).tolist()
+        for p, slot in zip(p1, mc.state_slots.tolist()):          # rows of positions before 0 are never read
+            assert torch.equal(st_g[slot, max(3 - p, 0):].cpu(), st_c[slot, max(3 - p, 0):])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_max_gates_against_the_reference(dtype):
     from dli_amd.ops import seqmix
     torch.manual_seed(5)
