@@ -883,8 +883,14 @@ __global__ __launch_bounds__(128) void map_merge_kernel(A* __restrict__ out, int
 // slot(t) = ((t & 15) >> 2)·8 + (t >> 4)·4 + (t & 3).  KSMAX / MTMAX: compile-time bounds of ceil(Dk / 32) and Dv / 16.
 // DIFF: every two groups of four waves are the two maps of one head — each with a key slice of its own, values shared; map 2's result
 // goes through LDS and map 1's waves write scale · d / rms(d), d = a1 - lam · a2.
-// Up to 256-wide keys (KSMAX ≤ 8) the next page is fetched into registers while this one is computed; the barriers wait for LDS only.
-template <int KSMAX, int MTMAX, int HW, bool DIFF>
+// Up to 256-wide keys (KSMAX ≤ 8) two pages alternate in LDS and the one after them is fetched into registers meanwhile: one barrier a page,
+// which waits for LDS only.
+// FULL: keys of 32 · KSMAX and values of 16 · MTMAX.  The steps are then free of conditions, so that a page's fragments are read ahead of their
+// products; otherwise every read is waited for where it is used.
+// Bound by a page's vector instructions (≈ 200 a wave of 16 queries with distance penalties, beside 24 products) and the chain through them.
+// 3200 tokens of four prompts, µs, before → now: 32/8 heads of 128 138 → 66, with cap 132 → 67, two maps of 128 161 → 71, 16/4 of 256 169 → 75, of
+// 192 (not FULL) 149 → 107, one group of 576 / 512 326 → 183; 400 tokens of 32/8 heads 30.4 → 21.4.
+template <int KSMAX, int MTMAX, int HW, bool DIFF, bool FULL>
 __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) void tile_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
     const uint16_t* __restrict__ q2, int64_t q2_ts, int64_t q2_hs, int D2, const uint16_t* __restrict__ kc, int rowk,
@@ -895,17 +901,21 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
     const uint16_t* __restrict__ gate, int64_t g_ts, const float* __restrict__ sink, AttnOpts opt) {
   extern __shared__ __align__(16) uint16_t tl[];
   const int ntiles = counts != nullptr ? min(counts[2], num_tiles) : num_tiles;
-  // the host walks causal tiles longest-first from the END of the list
-  const int tile = num_tiles - 1 - (int)blockIdx.x;
+  // HW heads of one key / value group per workgroup (4 waves each): the staged page serves all of them.  The heads of a tile are the fast
+  // block index, their group the fastest: the longest tiles of all heads start first (the host walks causal tiles longest-first from the
+  // END of the list), and with 8 groups an XCD serves one, whose pages its L2 holds
+  const int nh = H / HW, ng = DIFF ? G / 2 : G;
+  const int rank = (int)blockIdx.x / nh, slice = (int)blockIdx.x - rank * nh;
+  const int hblock = slice % ng * (nh / ng) + slice / ng;
+  const int tile = num_tiles - 1 - rank;
   if (tile >= ntiles) return;
-  // HW heads of one key / value group per workgroup (4 waves each): the staged page serves all of them
   constexpr int TNT = NT * HW;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int KROWS = DIFF ? 64 : 32;                   // staged key rows per page
   constexpr bool PREF = KSMAX <= 8;
   const int map = DIFF ? (wave_all >> 2) & 1 : 0, per = H / G;
   // DIFF: `head` counts (value head, head of its group); query heads are ordered (value head, map, head of its group)
-  const int head = DIFF ? (int)blockIdx.y * (HW / 2) + (wave_all >> 3) : (int)blockIdx.y * HW + (wave_all >> 2);
+  const int head = DIFF ? hblock * (HW / 2) + (wave_all >> 3) : hblock * HW + (wave_all >> 2);
   const int h = DIFF ? (head / per * 2 + map) * per + head % per : head;
   const int seq = tile_seq[tile], q0 = tile_q0[tile];
   const int t_begin = qsl[seq];
@@ -915,18 +925,21 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
   if (nq <= 0) return;
   const int wave = wave_all & 3;
   const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
-  const int Dk = D1 + D2;
+  const int Dk = FULL ? KSMAX * 32 : D1 + D2;
+  if (FULL) Dv = MTMAX * 16;
   const int KS = (Dk + 31) >> 5, MT = Dv >> 4;
   const int KST = KS * 32 + 8;                            // LDS row strides (elements): +16 bytes against bank conflicts
   constexpr int VST = 36;                                 // 18 dwords: 8-byte writes of eight 4-row groups × 8 columns hit all banks
   uint16_t* Ks = tl;                                      // [DIFF ? 2 maps : 1][32][KST]
   uint16_t* Vt = tl + KROWS * KST;
+  const int stage = KROWS * KST + Dv * VST;               // PREF: two of them, taken in turn
   const int g = h / per, gv = g / opt.vshare, g0 = g - map;    // g0: key head of the first staged slice
 
   // zero the K padding columns once (Dk not a multiple of 32): they are never staged over
   for (int i = threadIdx.x; i < KROWS * (KS * 32 - Dk); i += TNT) {
     const int row = i / (KS * 32 - Dk), col = Dk + i % (KS * 32 - Dk);
     Ks[row * KST + col] = 0;
+    if (PREF) Ks[stage + row * KST + col] = 0;
   }
 
   // this lane's query row as B fragments (zero past Dk and for rows past the tile)
@@ -966,12 +979,11 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 
   const int kchunks = Dk >> 3, vchunks = Dv >> 3;
   const bool vfromk = vc == kc && rowv == rowk && vhead == Dk;     // latent attention: one row is key and value
-  const uint16_t* Km = Ks + map * 32 * KST;
   // staging: keys in 16-byte pieces of a row; values in groups of 4 rows × 8 columns, whose slots are neighbours in Vt
   auto page_of = [&](int it) { return (int64_t)bt[it < kb_lo ? it - (kb_lo - kept_pages) : it] * kBlockTokens; };
-  auto put_values = [&](int i, bf16x8 v0, bf16x8 v1, bf16x8 v2, bf16x8 v3) {
+  auto put_values = [&](int i, int at, bf16x8 v0, bf16x8 v1, bf16x8 v2, bf16x8 v3) {
     const int rg = i & 7;
-    uint16_t* dst = Vt + (i >> 3) * 8 * VST + (rg & 3) * 8 + (rg >> 2) * 4;
+    uint16_t* dst = Vt + at + (i >> 3) * 8 * VST + (rg & 3) * 8 + (rg >> 2) * 4;
 #pragma unroll
     for (int j = 0; j < 8; ++j) *reinterpret_cast<bf16x4*>(dst + j * VST) = bf16x4{v0[j], v1[j], v2[j], v3[j]};
   };
@@ -1000,21 +1012,29 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
       }
     }
   };
-  if constexpr (PREF) fetch(page_of(kb_lo - kept_pages));
-  for (int it = kb_lo - kept_pages; it <= kb_hi; ++it) {
-    const int kb = it < kb_lo ? it - (kb_lo - kept_pages) : it;
+  auto put = [&](int at) {
+#pragma unroll
+    for (int u = 0; u < NKP; ++u)
+      if (kl[u] >= 0) *reinterpret_cast<bf16x8*>(Ks + at + kl[u]) = kr[u];
+#pragma unroll
+    for (int u = 0; u < NVP; ++u) {
+      const int i = threadIdx.x + u * TNT;
+      if (i < 8 * vchunks) put_values(i, at, vr[u][0], vr[u][1], vr[u][2], vr[u][3]);
+    }
+  };
+  const int it_lo = kb_lo - kept_pages;
+  if constexpr (PREF) {
+    fetch(page_of(it_lo));
+    put(0);
+    if (it_lo < kb_hi) fetch(page_of(it_lo + 1));
+    lds_barrier();
+  }
+  for (int it = it_lo; it <= kb_hi; ++it) {
+    const int kb = it < kb_lo ? it - it_lo : it;
+    const int at = PREF && ((it - it_lo) & 1) ? stage : 0;
     if constexpr (PREF) {
-      lds_barrier();                                      // everyone is done with the previous page
-#pragma unroll
-      for (int u = 0; u < NKP; ++u)
-        if (kl[u] >= 0) *reinterpret_cast<bf16x8*>(Ks + kl[u]) = kr[u];
-#pragma unroll
-      for (int u = 0; u < NVP; ++u) {
-        const int i = threadIdx.x + u * TNT;
-        if (i < 8 * vchunks) put_values(i, vr[u][0], vr[u][1], vr[u][2], vr[u][3]);
-      }
-      if (it < kb_hi) fetch(page_of(it + 1));
-      lds_barrier();
+      if (it < kb_hi) put(stage - at);                    // everyone passed the barrier after the page that was there
+      if (it + 1 < kb_hi) fetch(page_of(it + 2));
     } else {
       __syncthreads();                                    // everyone is done with the previous page
       const int64_t page_row = page_of(it);
@@ -1035,6 +1055,7 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
       __syncthreads();
     }
 
+    const uint16_t* Km = Ks + at + map * 32 * KST;
     f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KSMAX; ++s) {
@@ -1047,27 +1068,45 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
     }
     float sv[8];
     float mx = -INFINITY;
+    const int j0 = 32 * kb + 4 * g4;                      // this lane's keys: j0 … j0 + 3 and j0 + 16 … j0 + 19
+    auto key = [](int r) { return r < 4 ? r : 12 + r; };
     // a page every query of the tile sees whole (the common case far from the diagonal) needs no per-score masks
     const bool whole = nq == 64 && 32 * kb + 31 <= p_first && (32 * kb >= lo_last || 32 * kb + 31 < opt.keep);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int j = 32 * kb + (r < 4 ? 4 * g4 + r : 16 + 4 * g4 + (r - 4));
-      float v = (r < 4 ? sa[r] : sb[r - 4]) * qmul;
-      if (pen) v -= r1h * __builtin_amdgcn_logf(1.f + r2h * (float)max(pq - j, 0));
-      if (capped) v = capl - 2.f * capl * fast_rcp(fast_exp2(v) + 1.f);
-      if (!whole) {
-        const bool ok = qvalid && j <= pq && (j >= lo_q || j < opt.keep);
-        v = ok ? v : -INFINITY;
-      }
-      sv[r] = v;
-      mx = fmaxf(mx, v);
+    for (int r = 0; r < 8; ++r) sv[r] = (r < 4 ? sa[r] : sb[r - 4]) * qmul;
+    // one branch a page for each of these, not one a score
+    if (pen) {
+      const float far = (float)(pq - j0);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) sv[r] -= r1h * __builtin_amdgcn_logf(1.f + r2h * fmaxf(far - (float)key(r), 0.f));
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);
-    const float mu = mn == -INFINITY ? 0.f : mn;          // nothing visible yet: keep everything at zero
-    const float corr = fast_exp2(m - mu);
-    m = mn;
+    if (capped)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) sv[r] = capl - 2.f * capl * fast_rcp(fast_exp2(sv[r]) + 1.f);
+    if (!whole)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int j = j0 + key(r);
+        sv[r] = qvalid && j <= pq && (j >= lo_q || j < opt.keep) ? sv[r] : -INFINITY;
+      }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) mx = fmaxf(mx, sv[r]);
+    auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    // the maximum that a query's weights refer to moves only when a page passes it by more than 2^8 (for some query of the wave; then
+    // each takes its own): fp32 sums and the weights' head and remainder hold 2^8 as well, and most pages rescale nothing
+    // (Sizes below the bounds rescale each time: with their conditions per step the branch costs registers that they do not have.)
+    if (!FULL || __any(mx > m + 8.f)) {
+      const float mn = fmaxf(m, mx);
+      const float corr = fast_exp2(m - (mn == -INFINITY ? 0.f : mn));
+      m = mn;
+      l *= corr;
+#pragma unroll
+      for (int i = 0; i < MTMAX; ++i) acc[i] *= corr;
+    }
+    const float mu = m == -INFINITY ? 0.f : m;            // nothing visible yet: keep everything at zero
     bf16x8 ph, plo;
     float ps = 0.f;
 #pragma unroll
@@ -1078,18 +1117,16 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
       ph[r] = (short)hi;
       plo[r] = (short)f2bf(pv - bf2f(hi));
     }
-    l = l * corr + ps;
+    l += ps;
 #pragma unroll
     for (int i = 0; i < MTMAX; ++i) {
       if (i < MT) {
-        const bf16x4* vp = reinterpret_cast<const bf16x4*>(Vt + (16 * i + c) * VST + 8 * g4);
+        const bf16x4* vp = reinterpret_cast<const bf16x4*>(Vt + at + (16 * i + c) * VST + 8 * g4);
         const bf16x8 vf = __builtin_shufflevector(vp[0], vp[1], 0, 1, 2, 3, 4, 5, 6, 7);
-        f32x4 a = acc[i];
-        a[0] *= corr; a[1] *= corr; a[2] *= corr; a[3] *= corr;
-        a = mfma16(vf, ph, a);
-        acc[i] = mfma16(vf, plo, a);
+        acc[i] = mfma16(vf, plo, mfma16(vf, ph, acc[i]));
       }
     }
+    if constexpr (PREF) lds_barrier();                    // everyone is done with this page and has put the next one
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
@@ -1653,20 +1690,27 @@ bool launch_sm_tile_attention(void* out, int64_t o_ts, int64_t o_hs, const void*
   // for two heads
   const bool even = (H / G) % 2 == 0;
   const int hw = diff ? (even && KS <= 4 && MT <= 8 ? 4 : 2) : (even ? 2 : 1);
+  if (KS <= 8 && MT <= 16) lds *= 2;                      // two pages in turn
   if (diff) lds = std::max(lds, (size_t)hw / 2 * 64 * Dv * sizeof(float));
-  const dim3 grid(num_tiles, H / hw);
-#define SM_TILE_HW(KSM, MTM, HWV, DIFF)                                                                                                \
+  const dim3 grid(num_tiles * (H / hw));
+#define SM_TILE_GO(KSM, MTM, HWV, DIFF, FULL)                                                                                                \
   do {                                                                                                                           \
     static bool big = false;                                                                                                     \
     if (lds > 48 * 1024 && !big) {                                                                                               \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_attention_kernel<KSM, MTM, HWV, DIFF>),                      \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 100 * 1024);                                         \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_attention_kernel<KSM, MTM, HWV, DIFF, FULL>),                      \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);                                         \
       big = true;                                                                                                                \
     }                                                                                                                            \
-    hipLaunchKernelGGL((tile_attention_kernel<KSM, MTM, HWV, DIFF>), grid, dim3(NT * HWV), lds, stream, (uint16_t*)out, o_ts, o_hs,    \
+    hipLaunchKernelGGL((tile_attention_kernel<KSM, MTM, HWV, DIFF, FULL>), grid, dim3(NT * HWV), lds, stream, (uint16_t*)out, o_ts, o_hs,    \
                        (const uint16_t*)q1, q1_ts, q1_hs, D1, (const uint16_t*)q2, q2_ts, q2_hs, D2, (const uint16_t*)kc, rowk,  \
                        (const uint16_t*)vc, rowv, vhead, Dv, block_tables, max_blocks, seq_lens, qsl, tile_seq, tile_q0,        \
                        num_tiles, counts, H, G, scale, window, temp, r1, r2, (const uint16_t*)gate, g_ts, sink, opt);                       \
+  } while (0)
+// sizes that fill a variant's bounds take its form without conditions (32/8 heads, 3200 tokens: 128 wide 66 µs, 96 wide 69)
+#define SM_TILE_HW(KSM, MTM, HWV, DIFF)                                             \
+  do {                                                                              \
+    if (Dk == 32 * KSM && MT == MTM) SM_TILE_GO(KSM, MTM, HWV, DIFF, true);         \
+    else SM_TILE_GO(KSM, MTM, HWV, DIFF, false);                                    \
   } while (0)
 #define SM_TILE(KSM, MTM)              \
   do {                                 \
@@ -1684,6 +1728,7 @@ bool launch_sm_tile_attention(void* out, int64_t o_ts, int64_t o_hs, const void*
   else SM_TILE(18, 32);
 #undef SM_TILE
 #undef SM_TILE_HW
+#undef SM_TILE_GO
   return true;
 }
 

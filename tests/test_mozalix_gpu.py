@@ -246,6 +246,39 @@ def test_differential_attention_kernels_against_the_reference(H, G, D, Dv, windo
     assert oracle.F64 == torch.float64
 
 
+@pytest.mark.parametrize("H,G,D,Dv,maps", [(8, 2, 128, 128, 1), (6, 3, 128, 128, 1), (3, 3, 128, 128, 1), (4, 1, 256, 256, 1), (4, 1, 576, 512, 1), (4, 2, 120, 128, 1),
+                                          (4, 2, 128, 128, 2), (2, 2, 256, 256, 2)])
+@pytest.mark.parametrize("rise", [0.0, 0.15])
+def test_tiles_of_whole_sizes_against_the_reference(H, G, D, Dv, maps, rise):
+    """Sizes that fill the tile kernel's bounds, head blocks of one to eight groups, one page to many, distance penalties, and keys that grow along
+    the sequence: row maxima that pass the one in use by less and by more than 2^8.  Weights enter with 16 bits and results leave in bf16
+    (2^-9 of at most the largest value, twice that for a difference of two maps), beside fp32 sums."""
+    from dli_amd.ops import seqmix
+    torch.manual_seed(10)
+    lens, starts = [2, 70, 131, 33, 64], [64, 150, 0, 95, 0]
+    mc, T = _attention_step(starts, lens, "cpu")
+    mg, _ = _attention_step(starts, lens, "cuda")
+    latent = D == 576
+    kc, vc = torch.randn(96, 32, G * maps * D), None if latent else torch.randn(96, 32, G * Dv).to(torch.bfloat16)
+    B = len(lens)
+    kc *= 1.0 + rise * (torch.arange(96) // B * 32)[:, None, None].float() / 32 * 8
+    kc = kc.to(torch.bfloat16)
+    q = torch.randn(T, maps * H, D).to(torch.bfloat16)
+    cu = lambda t: t if t is None else t.cuda()
+    f32 = lambda t: t if t is None else t.float()
+    if maps == 2:
+        lam, want, got = torch.tensor([0.7]), torch.zeros(T, H * Dv), torch.zeros(T, H * Dv, dtype=torch.bfloat16, device="cuda")
+        seqmix.map_attention(want, q.float(), kc.float(), vc.float(), mc, G, Dv, D ** -0.5, 100, lam, 1e-5, 0.8)
+        seqmix.map_attention(got, cu(q), cu(kc), cu(vc), mg, G, Dv, D ** -0.5, 100, cu(lam), 1e-5, 0.8)
+    else:
+        r1, r2 = torch.rand(H), torch.rand(H)
+        r1[0] = 0.0                                                 # a head without penalty
+        want = seqmix.token_attention(torch.zeros(T, H, Dv), q.float(), None, kc.float(), f32(vc), mc, G, Dv, D ** -0.5, 0 if latent else 100, None, r1, r2)
+        got = seqmix.token_attention(torch.zeros(T, H, Dv, dtype=torch.bfloat16, device="cuda"), cu(q), None, cu(kc), cu(vc), mg, G, Dv, D ** -0.5,
+                                     0 if latent else 100, None, cu(r1), cu(r2))
+    assert float((got.cpu().float() - want).abs().max()) < 2 ** -8 * maps * max(float(want.abs().max()), 1.0)
+
+
 def test_generation_at_layer_sizes_of_a_real_model():
     """Random weights, heads of 128, hipGraph decode steps: the start-up self-test compares captured steps with eager ones."""
     from dli_amd.config import CacheConfig, EngineConfig, SamplingParams, SchedulerConfig, mozalix_config
