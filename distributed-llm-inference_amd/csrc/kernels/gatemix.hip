@@ -658,7 +658,8 @@ template <typename A> __device__ __forceinline__ typename Raw<A>::v4 raw4(const 
   return r;
 }
 // CHAN (delta rule, A = float): q, k and kᵀ come from the workspace with their channel decays in them (channel_block_kernel).
-template <typename A, bool DELTA, int DTMAX, int CT, bool CHAN>
+// FULL: D fills the DTMAX tiles, and no step of the loops over them has a condition in front of its reads.
+template <typename A, bool DELTA, int DTMAX, int CT, bool CHAN, bool FULL>
 __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, int64_t q_stride, const A* __restrict__ k, int64_t k_stride,
                                                        const A* __restrict__ v, int64_t v_stride, float* __restrict__ state,
                                                        const int* __restrict__ positions, const int* __restrict__ qsl,
@@ -674,7 +675,7 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
   if (slot < 0 || n < 2) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
   const int g = h / (H / G);
-  const int DT = (D + 15) >> 4, DS = DT * 16 + 4;
+  const int DT = FULL ? DTMAX : (D + 15) >> 4, DS = DT * 16 + 4;
   constexpr int DW = (DTMAX + 3) / 4;                     // state row tiles per wave: wave, wave + 4, …
   float* St = sh;                                         // [16·CT columns][DS]: the state at the block's start
   float* Rt = St + 16 * CT * DS;                          // [columns][BS]: right-hand sides of the delta rule
@@ -1039,13 +1040,16 @@ static void gated_scan(const A* q, int64_t q_stride, const A* k, int64_t k_strid
   const int DS = ((D + 15) / 16) * 16 + 4;
   const size_t lds = (size_t)16 * ct * (DS + (DELTA ? 3 : 2) * BS) * sizeof(float);
   const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
-#define GM_WALK(DT, CTV)                                                                                                               \
-  hipLaunchKernelGGL((scan_walk_kernel<A, DELTA, DT, CTV, false>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state,  \
+#define GM_WALK(DT, CTV, FULLV)                                                                                                               \
+  hipLaunchKernelGGL((scan_walk_kernel<A, DELTA, DT, CTV, false, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state,  \
                      positions, qsl, state_slots, counts, H, G, D, Dv, wide, q_scale, ws, out, nq)
-#define GM_WALK_D(DT)          \
-  do {                         \
-    if (ct == 2) GM_WALK(DT, 2); \
-    else GM_WALK(DT, 1);       \
+  // D that fills its bound, two column tiles: 32 heads of 128, whole scans, µs, with / without conditions: 799 rows, channel decays 117.8 / 110.1,
+  // 2048 rows 329.9 / 305.9.  One column tile has half the products a read and is no faster without (16 heads, 3162 rows: 213.8 / 220.2, 201.7 / 202.2).
+#define GM_WALK_D(DT)                                             \
+  do {                                                            \
+    if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
+    else if (ct == 2) GM_WALK(DT, 2, false);                      \
+    else GM_WALK(DT, 1, false);                                   \
   } while (0)
   if (D <= 64) GM_WALK_D(4);
   else if (D <= 128) GM_WALK_D(8);
@@ -1102,13 +1106,14 @@ void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, in
   const int DS = ((D + 15) / 16) * 16 + 4;
   const size_t lds = (size_t)16 * ct * (DS + 2 * BS) * sizeof(float);
   const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
-#define GM_WALK(DT, CTV)                                                                                                                \
-  hipLaunchKernelGGL((scan_walk_kernel<float, true, DT, CTV, true>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state, \
+#define GM_WALK(DT, CTV, FULLV)                                                                                                                \
+  hipLaunchKernelGGL((scan_walk_kernel<float, true, DT, CTV, true, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state, \
                      positions, qsl, state_slots, counts, H, G, D, Dv, wide, 1.f, ws, out, (float*)nullptr)
-#define GM_WALK_D(DT)          \
-  do {                         \
-    if (ct == 2) GM_WALK(DT, 2); \
-    else GM_WALK(DT, 1);       \
+#define GM_WALK_D(DT)                                             \
+  do {                                                            \
+    if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
+    else if (ct == 2) GM_WALK(DT, 2, false);                      \
+    else GM_WALK(DT, 1, false);                                   \
   } while (0)
   if (D <= 64) GM_WALK_D(4);
   else if (D <= 128) GM_WALK_D(8);

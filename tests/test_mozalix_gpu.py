@@ -135,6 +135,12 @@ def test_channel_scan_kernels_against_the_reference(H, G, D, Dv, dtype):
         starts = [s + n for s, n in zip(starts, lens)]
 
 
+@pytest.mark.parametrize("D", [64, 128, 115, 70])
+def test_channel_walk_of_two_column_tiles_and_whole_sizes(D):
+    """64 heads take two column tiles a workgroup; D fills its row tiles (70 does not)."""
+    test_channel_scan_kernels_against_the_reference(64, 8, D, 40, torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [256, 90, 4100])
 def test_norm_and_activation_kernels_against_the_reference(W, dtype):

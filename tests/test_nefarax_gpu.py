@@ -191,6 +191,12 @@ def test_convolution_runs_against_the_reference(lens, C, unit, gate, dtype):
             assert torch.equal(st_g[slot, max(3 - p, 0):].cpu(), st_c[slot, max(3 - p, 0):])
 
 
+@pytest.mark.parametrize("delta,D", [(True, 64), (True, 113), (True, 128), (False, 128), (True, 256), (False, 50)])
+def test_scan_walk_of_two_column_tiles_and_whole_sizes(delta, D):
+    """64 heads take two column tiles a workgroup; D fills its 4, 8 or 16 row tiles, also where the last of them is not whole."""
+    test_scan_kernels_against_the_reference(delta, False, 64, 4, D, 40, torch.float32)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_max_gates_against_the_reference(dtype):
     from dli_amd.ops import seqmix
