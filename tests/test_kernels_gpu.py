@@ -390,6 +390,41 @@ def test_sampler_slices_draw_what_the_row_kernel_draws(B, V):
         assert torch.equal(got.cpu()[keep], want.cpu()[keep]), (r, got, want)
 
 
+@pytest.mark.parametrize("V", [4096, 40000])
+@pytest.mark.parametrize("mask", [float("-inf"), torch.finfo(torch.bfloat16).min, -1e10, -3e9, -1e9, -1e4])
+def test_sampler_cut_ignores_masked_tokens(mask, V):
+    """Rows of which most tokens are masked with a large negative value: the cut-off is where float64 puts it.  200 logits a step of 1/16
+    apart (exact in bf16), mostly positive or mostly negative; the last token inside the cut-off gets a noise that wins over everything
+    but the first one outside, which gets a larger one.  ``p`` lies halfway between two cumulative masses, far from rounding."""
+    g = torch.Generator().manual_seed(5)
+    rows, params, noises, want = [], [], [], []
+    for first in (8.0, -0.5):
+        for temp, p, k in ((1.0, 0.5, 0), (1.0, 0.7, 0), (0.25, 0.7, 0), (2.5, 0.9, 0), (1.0, 1.0, 17), (2.0, 1.0, 150), (1.0, 0.8, 9), (2.0, 1.0, 1000), (1.0, 0.9, 1000)):
+            ids = torch.randperm(V, generator=g)[:200]
+            v = first - torch.arange(200).double() / 16
+            row = torch.full((V,), mask)
+            row[ids] = v.float()
+            n = min(k or 200, 200)
+            w = torch.exp((v[:n] - v[0]) / temp)
+            cum = torch.cumsum(w, 0) / w.sum()
+            last = n - 1
+            if p < 1.0:
+                last = int(torch.searchsorted(cum, torch.tensor(p, dtype=torch.float64)))
+                p = float((cum[last] + (cum[last - 1] if last else 0.0)) / 2)
+            u = torch.full((V,), 0.5)
+            u[ids[last]] = 1 - 2.0 ** -12                            # noise 8.3 and 13.9 beside 0.37: more than all logits differ by
+            if last + 1 < 200:
+                u[ids[last + 1]] = 1 - 2.0 ** -20
+            assert (v[0] - v[last]) / temp < 7
+            rows.append(row), params.append((temp, p, k)), noises.append(u)
+            want.append(int(ids[last]))
+    x = torch.stack(rows).to(torch.bfloat16).to(DEV)
+    temp, top_p, top_k = (torch.tensor(c) for c in zip(*params))
+    z = torch.zeros(len(rows), dtype=torch.int64, device=DEV)
+    got = ops.sample(x, temp.to(DEV), top_p.to(DEV), top_k.int().to(DEV), z, z, torch.stack(noises).to(DEV))
+    assert got.tolist() == want
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_sampler_nan_row_yields_a_valid_token(dtype):
     """A NaN row (a bug upstream) must not turn into an out-of-range token id: the next step embeds it."""
