@@ -359,10 +359,10 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
 //                          11 + 4 jj (v_slot, ops/kv_layout.py — the layout serves both MFMA shapes): exp2 and a bf16 pack of
 //                          those are the B fragment of k-step jj, one ds_read_b128 of the slot its A fragment;
 //   Oᵀ(128 d × 32 col)   = 4 d-tiles × 2 k-steps = 8 MFMAs.
-// A wave's page is ≈ 75 vector instructions beside the 16 products (205 with a rescale at every rise of a maximum and with the halves of
-// two V slots mixed into a fragment); one wave alone needs ≈ 0.7 µs for it, a serial chain of fragment reads, products, exponentials
-// and the issue of its share of the next page's DMA.  Whole steps, 32/8 heads: fresh prompts of up to 1333 tokens (4100 in all) 53 → 42 µs
-// (678 TFLOP/s), 4000 tokens 1.02 PFLOP/s.
+// A wave's page is ≈ 75 vector instructions beside the 16 products (and 64 where a maximum rises; 205 with the
+// halves of two V slots mixed into a fragment); one wave alone needs ≈ 0.7 µs for it, a serial chain of fragment reads, products,
+// exponentials and the issue of its share of the next page's DMA.  Whole steps, 32/8 heads: fresh prompts of up to 1333 tokens (4100 in all)
+// 56.4 → 55.2 µs, one of 4000 159 → 151 (0.99 PFLOP/s), two of 2048 87.9 → 85.4.
 // ==================================================================================================
 __device__ __forceinline__ int slot_swizzle(int row) { return (0x78 >> (2 * ((row >> 2) & 3))) & 3; }
 
@@ -542,11 +542,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
       float mx = (edge ? page_max32<true>(s, tok0, qpos) : page_max32<false>(s, tok0, qpos)) * scale_log2;
       auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      // The maximum that a column's weights refer to moves only when a page exceeds it by more than 2^8 (in some lane; then every column
-      // takes its own): until then weights reach 2^8, which the fp32 sums and the relative precision of bf16 hold as well.  With 32
-      // columns a wave nearly every page raises SOME maximum a little, and rescaling the 64 accumulators each time was a third of a
-      // page's vector instructions.
-      if (__any(mx > m + 8.f)) {
+      // The maximum moves with every page that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
+      // 2^8 saves these 64 products on most pages, 3 – 10 % of a launch, but rounds the largest weight like all others: relative error
+      // against 64 bits 0.00266 → 0.00272, e4m3 pages 0.00731 → 0.00734.)
+      if (__any(mx > m)) {
         asm volatile("" ::: "memory");
         const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
         m = mn;

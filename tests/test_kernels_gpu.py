@@ -311,8 +311,8 @@ def test_paged_attention_prefill_and_mixed(Hq, Hkv, kv_dtype):
 @pytest.mark.parametrize("n", [1, 64, 65])                        # 8, 512 and 520 workgroups: two page groups, two, one
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
-    """Tiles of one page (the second group has none), of an odd and of an even number, with masked last pages; keys whose scores rise by more
-    and by less than the 2^8 that moves the running maximum.  Weights and results are rounded to bf16 (2^-9 each, |v| ≤ 4.5 here)."""
+    """Tiles of one page (the second group has none), of an odd and of an even number, with masked last pages; keys whose scores rise by much and
+    by little along the row.  Weights and results are rounded to bf16 (2^-9 each, |v| ≤ 4.5 here)."""
     Hq = Hkv = 8
     lens = [1, 31, 32, 33, 64, 65, 96, 97, 129, 300]
     seq_lens = [lens[(i + 7) % 10] for i in range(n)]
@@ -321,7 +321,7 @@ def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
     kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=23, scales=scales)
     T = sum(qlens)
     qkv = _bf(T, (Hq + 2 * Hkv) * 128, seed=24)
-    qkv[::3] *= 8                                                   # scores of ± 40: steps of the maximum past 2^8
+    qkv[::3] *= 8                                                   # scores of ± 40
     sl = torch.tensor(seq_lens, dtype=torch.int32, device=DEV)
     qsl = torch.tensor(np.concatenate([[0], np.cumsum(qlens)]), dtype=torch.int32, device=DEV)
     ts, t0 = ops.build_prefill_tiles(np.array(qlens), 0, ops.prefill_tile_tokens(Hq, Hkv))
@@ -331,6 +331,36 @@ def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
     got = ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088, *scales).float()
     want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(T, Hq, 128), kc, vc, bt, sl, qsl, 0.088, *scales).float()
     torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -9 * 4.5)
+
+
+@pytest.mark.parametrize("n", [1, 65])                            # two page groups and one
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("peak", [7.5, 150.5, 197.5])
+def test_prefill_largest_weight_is_exact(n, kv_dtype, peak):
+    """One key, five pages in, scores log2(peak) above all others, and only its value is not zero: out = v·peak / (peak + others).  A
+    weight taken against the row's maximum is 1 there, so what remains is the rounding of the result (2^-8) and fp32 arithmetic; against a
+    maximum of earlier pages it is ``peak``, which bf16 holds only to another 2^-8 (150.5 becomes 150)."""
+    H, L, Q, top = 8, 190, 8, 140
+    kc, vc = _caches(6 * n, H, kv_dtype)
+    bt = torch.randperm(6 * n, generator=torch.Generator().manual_seed(1)).view(n, 6).to(torch.int32)
+    k, v = torch.zeros(n * L, H, 128), torch.zeros(n * L, H, 128)
+    at = torch.arange(n) * L + top
+    k[at, :, 3] = 1.0
+    v[at] = torch.randn(n, H, 128, generator=torch.Generator().manual_seed(2)).to(kv_dtype).float()
+    slots = (bt.long()[:, torch.arange(L) // 32] * 32 + torch.arange(L) % 32).reshape(-1).to(torch.int32)
+    from dli_amd.ops.kv_layout import write_kv_ref
+    write_kv_ref(k.to(torch.bfloat16).to(DEV), v.to(torch.bfloat16).to(DEV), slots.to(DEV), kc, vc, 1.0, 1.0)
+    qkv = torch.zeros(n * Q, 3 * H * 128, dtype=torch.bfloat16, device=DEV)
+    qkv[:, 3:H * 128:128] = 1.0
+    i32 = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    ts, t0 = ops.build_prefill_tiles(np.full(n, Q), 0, ops.prefill_tile_tokens(H, H))
+    meta = ops.AttnMetadata(num_decode=0, num_prefill=n, num_tokens=n * Q, positions=None, slot_mapping=None, block_tables=bt.to(DEV), seq_lens=i32([L] * n),
+                            query_start_loc=i32(np.arange(n + 1) * Q), decode_splits=1, prefill_tile_seq=i32(ts), prefill_tile_q0=i32(t0),
+                            num_prefill_tiles=len(ts))
+    got = ops.paged_attention(qkv, kc, vc, meta, H, H, 128, math.log(peak)).double().cpu().view(n, Q, H, 128)
+    others = (L - Q + torch.arange(Q)).double().view(1, Q, 1, 1)
+    want = v[at].double().view(n, 1, H, 128) * (peak / (peak + others))
+    assert ((got - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -13)).all()
 
 
 @pytest.mark.parametrize("V", [32000, 128256])
