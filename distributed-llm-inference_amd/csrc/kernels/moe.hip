@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const uint16_t* __restri
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int n, int expert_offset, int E_local,
                                                          int* __restrict__ sorted_ids, int* __restrict__ tile_expert,
                                                          int* __restrict__ meta, int capacity_rows, int tile_rows) {
-  const int BM = tile_rows;                               // row tile of the GEMM that consumes the alignment (128 or 256)
+  const int BM = tile_rows;                               // row tile of the GEMM that consumes the alignment (32, 64, 128 or 256)
   __shared__ int cnt[MOE_MAX_E], off[MOE_MAX_E + 1], pos[MOE_MAX_E];
   for (int e = threadIdx.x; e < MOE_MAX_E; e += blockDim.x) { cnt[e] = 0; pos[e] = 0; }
   __syncthreads();

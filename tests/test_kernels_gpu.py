@@ -604,6 +604,15 @@ def test_fused_moe_streaming_tiles_match_reference(rows, counts, H, I):
         assert torch.equal(ops.hip().fused_moe(x, logits, w13, w2, 1, 0, rows), got)
 
 
+def test_fused_moe_takes_any_tile_rows():
+    """Row counts that no kernel has mean 128, as they always did."""
+    x, logits = _bf(40, 256, seed=66), _bf(40, 4, seed=67)
+    w13, w2 = _bf(4, 2 * 192, 256, seed=68, scale=0.05), _bf(4, 256, 192, seed=69, scale=0.05)
+    want = ops.hip().fused_moe(x, logits, w13, w2, 2, 0, 128)
+    for rows in (1, 48, 96, 512, 256):                              # (256: 192 inner columns are no multiple of its 128)
+        assert torch.equal(ops.hip().fused_moe(x, logits, w13, w2, 2, 0, rows), want)
+
+
 @pytest.mark.parametrize("swiglu", [False, True])
 @pytest.mark.parametrize("M,N,K,splits", [(1, 128, 64, 1), (17, 256, 128, 1), (32, 384, 192, 3), (33, 128, 448, 1), (64, 256, 4096, 8), (65, 128, 320, 5),
                                           (96, 512, 256, 2), (97, 256, 64, 1), (128, 128, 1024, 0), (129, 256, 512, 0), (200, 384, 192, 1),
