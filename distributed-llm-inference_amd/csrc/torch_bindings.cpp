@@ -398,7 +398,8 @@ void moe_experts_forward(const Tensor& x, const Tensor& ids, const Tensor& wts, 
   // about one an expert has rows)
   const int64_t nk2 = I / 64;
   const bool stream_tiles = TR <= 64;
-  const int64_t blocks = stream_tiles ? (std::min(n, El) + n / TR) * (H / 128) : max_tiles * (H / TR);
+  // (no local expert, or a capacity of no rows: nothing to fill)
+  const int64_t blocks = std::max<int64_t>(1, stream_tiles ? (std::min(n, El) + n / TR) * (H / 128) : max_tiles * (H / TR));
   const int64_t want_blocks = stream_tiles ? g_moe_stream_min_blocks : TR == 256 ? g_moe_splitk_min_blocks256 : 1024;
   int64_t k_splits = 1;
   if (blocks < want_blocks)
@@ -428,6 +429,7 @@ void moe_apply(const Tensor& x, const Tensor& ids, const Tensor& wts, const Tens
                int64_t expert_offset, int64_t E, int64_t tile_rows, Tensor& out, hipStream_t stream, float act_limit = 0.f) {
   const int64_t T = x.size(0), H = x.size(1), El = w13.size(0), I = w13.size(1) / 2;
   auto i32 = x.options().dtype(at::kInt);
+  if (T == 0) return;
   const int64_t n = T * top_k;
   const bool fits256 = I % 128 == 0 && H % 256 == 0 && n * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
   const int64_t rows = moe_tile_rows(tile_rows, n / E, fits256);      // (tile_rows: A/B measurements and tests; local experts or not)

@@ -604,6 +604,16 @@ def test_fused_moe_streaming_tiles_match_reference(rows, counts, H, I):
         assert torch.equal(ops.hip().fused_moe(x, logits, w13, w2, 1, 0, rows), got)
 
 
+@pytest.mark.parametrize("I", [192, 256])                          # without and with the decode-sized path
+@pytest.mark.parametrize("rows", [0, 32, 64, 128, 256])
+def test_fused_moe_of_no_tokens(I, rows):
+    """A rank of an expert-parallel group may receive nothing: the share of the chip that no row fills is no divisor."""
+    x, logits = _bf(0, 256), _bf(0, 4)
+    w13, w2 = _bf(4, 2 * I, 256, seed=68), _bf(4, 256, I, seed=69)
+    assert ops.hip().fused_moe(x, logits, w13, w2, 2, 0, rows).shape == (0, 256)
+    torch.cuda.synchronize()
+
+
 def test_fused_moe_takes_any_tile_rows():
     """Row counts that no kernel has mean 128, as they always did."""
     x, logits = _bf(40, 256, seed=66), _bf(40, 4, seed=67)
