@@ -359,10 +359,20 @@ Tensor stream_gemm(const Tensor& x, const Tensor& w, bool swiglu, int64_t k_spli
 //   64        479    479    497    484    500    651                         once, a second tile of an expert fetches them again
 //   128       558    560    564    567    606    612    641    843    818    128 × 128 tiles (moe.hip)
 //   256       557    561    565    567    574    576    612    622    643    256² tiles (gemm256.hip)
-// (20 rows on average are seldom more than 32, 53 seldom more than 64.)  The 128 × 128 tiles stay for shapes that the 256² tiles do not
-// take.  DLI_MOE_TILE=32|64|128|256 forces one (any other value: 128).
+// (20 rows on average are seldom more than 32, 53 seldom more than 64.)  The 32- and 64-row tiles beat the 128 × 128 ones on every expert shape that was
+// timed (hidden × inner, experts, choices: 4096 × 1792 8/2, 2048 × 1408 64/4, 2048 × 768 64/8, 4096 × 2048 16/2, 1024 × 512 32/4, 2048 × 192 8/2; ratios
+// 1.2 – 1.7 at 20 rows).  Between 54 and 127 rows the 256² tiles win where the hidden size gives the down projection some columns:
+//   rows        64: 128 / 256     100: 128 / 256     127: 128 / 256
+//   4096 × 1792    134 / 128         148 / 139          155 / 153
+//   4096 × 2048    250 / 223         244 / 237          308 / 252
+//   2048 × 1408    311 / 301         382 / 325          420 / 349
+//   2048 × 768     217 / 218         240 / 239          292 / 258
+//   1024 × 512    71.0 / 74.5       84.9 / 86.9        90.6 / 94.9
+// so layers narrower than 2048 keep their line at 128 rows.  The 128 × 128 tiles also stay for shapes that the 256² tiles do not take.
+// DLI_MOE_TILE=32|64|128|256 forces one (any other value: 128), DLI_MOE_TILE256_MIN_ROWS moves the line of the 256² tiles.
 const int64_t g_moe_tile_force = std::getenv("DLI_MOE_TILE") ? std::atoll(std::getenv("DLI_MOE_TILE")) : 0;
-const int64_t g_moe_tile64_min_rows = 21, g_moe_tile256_min_rows = std::getenv("DLI_MOE_TILE256_MIN_ROWS") ? std::atoll(std::getenv("DLI_MOE_TILE256_MIN_ROWS")) : 54;
+const int64_t g_moe_tile64_min_rows = 21, g_moe_stream_max_rows = 53;
+const int64_t g_moe_tile256_min_rows = std::getenv("DLI_MOE_TILE256_MIN_ROWS") ? std::atoll(std::getenv("DLI_MOE_TILE256_MIN_ROWS")) : -1;
 
 const int64_t g_moe_splitk_min_blocks256 = std::getenv("DLI_MOE_SPLITK_MIN_BLOCKS256") ? std::atoll(std::getenv("DLI_MOE_SPLITK_MIN_BLOCKS256")) : 512;
 
@@ -373,10 +383,12 @@ const int64_t g_moe_skinny_max_t = std::getenv("DLI_NO_SKINNY_MOE") ? 0
 // workgroups a streaming down projection should have (K slices below): one per compute unit; twice as many slices cost 1 % more in slabs
 const int64_t g_moe_stream_min_blocks = 256;
 // `given`: the caller's choice (0: none), which goes before DLI_MOE_TILE.  Whatever is asked for, the result is a row count that a kernel has.
-int64_t moe_tile_rows(int64_t given, int64_t rows, bool fits256) {
+int64_t moe_tile_rows(int64_t given, int64_t rows, int64_t H, bool fits256) {
   if (given == 0) given = g_moe_tile_force;
   if (given != 0) return given == 32 || given == 64 ? given : given == 256 && fits256 ? 256 : 128;
-  if (rows >= g_moe_tile256_min_rows) return fits256 ? 256 : 128;
+  const int64_t from256 = g_moe_tile256_min_rows >= 0 ? g_moe_tile256_min_rows : H >= 2048 ? g_moe_stream_max_rows + 1 : 128;
+  if (rows >= from256 && fits256) return 256;
+  if (rows > g_moe_stream_max_rows) return 128;
   return rows >= g_moe_tile64_min_rows ? 64 : 32;
 }
 
@@ -432,7 +444,7 @@ void moe_apply(const Tensor& x, const Tensor& ids, const Tensor& wts, const Tens
   if (T == 0) return;
   const int64_t n = T * top_k;
   const bool fits256 = I % 128 == 0 && H % 256 == 0 && n * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
-  const int64_t rows = moe_tile_rows(tile_rows, n / E, fits256);      // (tile_rows: A/B measurements and tests; local experts or not)
+  const int64_t rows = moe_tile_rows(tile_rows, n / E, H, fits256);      // (tile_rows: A/B measurements and tests; local experts or not)
   if (T <= std::min<int64_t>(g_moe_skinny_max_t, 128) && I % 128 == 0 && tile_rows == 0) {
     // Decode-sized batch: an expert sees ≤ 16 rows (at T ≤ 32 and 2-of-8 routing: nearly always; more rows cost an
     // extra pass over that expert's weights from cache), so both projections are pure weight streams — the
@@ -555,7 +567,7 @@ Tensor ep_moe(int64_t st, const Tensor& x_l, const Tensor& router_logits_l, cons
   // local experts on the received rows: one "slot" per row, gate weight applied here, output straight into the IPC result buffer.
   // Row tile: the expected rows per local expert under uniform routing (what arrives is ≈ r_cap / world of the capacity)
   const bool fits256 = I % 128 == 0 && H % 256 == 0 && r_cap * std::max(H, I) * 2 < (int64_t(1) << 32) && 2 * I * H * 2 < (int64_t(1) << 32);
-  const int64_t rows = moe_tile_rows(0, n_cap / std::max<int64_t>(El, 1), fits256);
+  const int64_t rows = moe_tile_rows(0, n_cap / std::max<int64_t>(El, 1), H, fits256);
   moe_experts_forward(recv_x, ids_local, w_local, w13, w2, 1, rank * El, rows, dli::ep_result_ptr(state), stream);
   Tensor y_back = at::empty({std::max<int64_t>(n, 1), H}, w13.options());
   rc = dli::launch_ep_combine(state, ids.data_ptr<int>(), slot.data_ptr<int>(), (int)n, (int)n_cap, (int)H, (int)El, y_back.data_ptr(),
@@ -759,7 +771,7 @@ TORCH_LIBRARY(dli, m) {
   m.def("skinny_linear(Tensor x, Tensor w, Tensor? bias, bool swiglu=False, Tensor? out=None, Tensor? w_scale=None) -> Tensor", &skinny_linear);
   m.def("dense_gemm256(Tensor x, Tensor w, bool swiglu=False, int k_splits=1, Tensor? out=None, bool split_tail=False) -> Tensor", &dense_gemm256);
   m.def("stream_gemm(Tensor x, Tensor w, bool swiglu=False, int k_splits=0, Tensor? out=None) -> Tensor", &stream_gemm);
-  m.def("moe_tile_rows(int given, int rows, bool fits256) -> int", &moe_tile_rows);
+  m.def("moe_tile_rows(int given, int rows, int hidden, bool fits256) -> int", &moe_tile_rows);
   m.def("ar_staging_tensor(int state, int rows, int cols, Tensor like) -> Tensor", &ar_staging_tensor);
   m.def("ar_all_reduce_add_norm(int state, Tensor staged, Tensor(a!) residual, Tensor weight, float eps, Tensor(b!) out, int blocks=0) -> ()",
         &ar_all_reduce_add_norm);

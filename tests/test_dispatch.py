@@ -20,14 +20,18 @@ def _moe_rows(env, *args):
 @pytest.mark.parametrize("asked", ["96", "-5", "128"])
 def test_expert_row_tiles_are_ones_that_a_kernel_has(asked):
     """The experts' GEMMs align rows to this number and launch the tile of that size: any other value would be tiles past the rows."""
-    calls = (0, 8, True), (0, 4000, True), (0, 4000, False), (32, 4000, True), (64, 8, True), (256, 8, True), (256, 8, False)
+    H = 4096
+    calls = (0, 8, H, True), (0, 4000, H, True), (0, 4000, H, False), (32, 4000, H, True), (64, 8, H, True), (256, 8, H, True), (256, 8, H, False)
     assert _moe_rows({"DLI_MOE_TILE": asked}, *calls) == [128, 128, 128, 32, 64, 256, 128]
 
 
-def test_expert_row_tiles_by_rows_and_by_choice():
+@pytest.mark.parametrize("hidden", [512, 1920, 2048, 4096])
+def test_expert_row_tiles_by_rows_and_by_choice(hidden):
+    """Up to 53 rows the streaming tiles, from 128 the 256² ones where they fit; between the two those of 256 rows only for wide layers."""
     rule = ops.hip().moe_tile_rows
-    for rows in (0, 1, 20, 21, 53, 54, 127, 128, 10 ** 6):
-        assert rule(0, rows, True) in (32, 64, 256) and rule(0, rows, False) in (32, 64, 128)
+    between = 256 if hidden >= 2048 else 128
+    for rows, want in ((0, 32), (1, 32), (20, 32), (21, 64), (53, 64), (54, between), (127, between), (128, 256), (10 ** 6, 256)):
+        assert rule(0, rows, hidden, True) == want and rule(0, rows, hidden, False) == min(want, 128)
         for given in (32, 64, 128, 48, 7, -1):
-            assert rule(given, rows, True) == (given if given in (32, 64) else 128)
-        assert rule(256, rows, True) == 256 and rule(256, rows, False) == 128
+            assert rule(given, rows, hidden, True) == (given if given in (32, 64) else 128)
+        assert rule(256, rows, hidden, True) == 256 and rule(256, rows, hidden, False) == 128
