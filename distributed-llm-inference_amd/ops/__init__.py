@@ -274,13 +274,25 @@ def stream_rows_ok(m: int, n: int, k: int) -> bool:
     return 0 < m <= 256 and n * k >= 1 << 25 and n % 128 == 0 and k % 64 == 0 and (m <= 128 or n <= 8192)
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Ordinary tensors that nothing but the call looks at: no fake or other subclass, no trace, vmap, functional or forward-mode transform,
+    no gradient.  A kernel that takes addresses sees through all of these."""
+    return (not torch.compiler.is_compiling() and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None and torch.autograd.forward_ad._current_level < 0
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
+
+
 def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> bool:
     if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2):
         return False
-    if not stream_rows_ok(x.shape[0], weight.shape[0], weight.shape[1]) or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
+    m, (n, k) = x.shape[0], weight.shape
+    if not (stream_rows_ok(m, n, k) and (_plain(x, weight) if out is None else _plain(x, weight, out))):
         return False
-    return (weight.is_contiguous() and weight.data_ptr() % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and (out is None or (out.is_contiguous() and out.data_ptr() % 16 == 0)))
+    return (x.shape[1] == k and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and (out is None or (out.shape == (m, n) and out.dtype == torch.bfloat16 and out.device == x.device and out.is_contiguous()
+                                 and out.data_ptr() % 16 == 0)))
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,

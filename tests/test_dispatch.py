@@ -35,3 +35,45 @@ def test_expert_row_tiles_by_rows_and_by_choice(hidden):
         for given in (32, 64, 128, 48, 7, -1):
             assert rule(given, rows, hidden, True) == (given if given in (32, 64) else 128)
         assert rule(256, rows, hidden, True) == 256 and rule(256, rows, hidden, False) == 128
+
+
+class _Recorder:
+    """Stands in for the kernels: says which one a call came to."""
+
+    def __getattr__(self, name):
+        def call(*a):
+            raise RuntimeError(name)
+        return call
+
+
+def test_large_linear_layers_of_decode_batches_under_traces_and_transforms(monkeypatch):
+    """The streaming tiles take addresses, so only ordinary tensors go there; fake ones (shape propagation, export) stay with the library
+    operation at every row count, as they always did."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    monkeypatch.setattr(ops, "hip", _Recorder)
+    with FakeTensorMode():
+        w = torch.empty(8192, 5120, device="cuda", dtype=torch.bfloat16)
+        for m in (17, 40, 128, 200, 256, 320):
+            x = torch.empty(m, 5120, device="cuda", dtype=torch.bfloat16)
+            assert ops.stream_rows_ok(m, 8192, 5120) == (m <= 256) and not ops._stream_ok(x, w)
+            assert ops.linear(x, w).shape == (m, 8192)
+            with pytest.raises(RuntimeError, match="silu_and_mul"):        # (the library's product, then the activation kernel)
+                ops.linear_swiglu(x, w)
+
+
+def test_plain_tensors():
+    import torch.autograd.forward_ad as fw
+    t, seen = torch.zeros(4, 4), []
+    assert ops._plain(t) and ops._plain(t, torch.nn.Parameter(t, requires_grad=False))
+    with torch.no_grad():
+        assert ops._plain(torch.nn.Parameter(t))
+    with torch.enable_grad():
+        assert not ops._plain(t, torch.nn.Parameter(t))
+    look = lambda a: seen.append(ops._plain(a)) or a * 1
+    torch.func.vmap(look)(t)
+    torch.func.jvp(look, (t,), (t,))
+    torch.func.grad(lambda a: look(a).sum())(t)
+    with fw.dual_level():
+        look(fw.make_dual(t, t))
+    torch.jit.trace(look, (t,), check_trace=False)
+    assert seen == [False] * 5 and ops._plain(t)
