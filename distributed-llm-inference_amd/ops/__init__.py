@@ -265,13 +265,26 @@ def _tile_operand_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and x.shape[0] * x.stride(0) * 2 < 2 ** 32 and weight.numel() * 2 < 2 ** 32)
 
 
-def stream_rows_ok(m: int, n: int, k: int) -> bool:
-    """Row counts and shapes for which the weight-streaming tiles (``csrc/kernels/stream_gemm.hip``) beat both the library GEMM and the
-    split-K 256² tile: one row tile (up to 128 rows) over at least 64 MiB of weights — with less, the ramp of a launch and the slabs'
-    reduce pass weigh as much as the stream (6144 × 4096: 22.0 against 22.6 µs at 96 rows, 18.6 against 17.6 at 64) — and two row
-    tiles where the columns are few enough to be cut along K anyway (4096 × 14336 at 192 rows 43 against 102 µs, 7168 × 8192 44 against 65;
-    28672 × 4096 76 against 67)."""
-    return 0 < m <= 256 and n * k >= 1 << 25 and n % 128 == 0 and k % 64 == 0 and (m <= 128 or n <= 8192)
+def stream_rows_ok(m: int, n: int, k: int, swiglu: bool = False) -> bool:
+    """Row counts and shapes for which the weight-streaming tiles (``csrc/kernels/stream_gemm.hip``) beat the library GEMM (and its activation
+    pass), from 64 MiB of weights on: with less, a launch's ramp and the slabs' reduce pass weigh as much as the stream (6144 × 4096: 22.0 against
+    22.6 µs at 96 rows, 18.6 against 17.6 at 64).  By columns, which decide how K is cut and how the 256 compute units are filled (µs, library / tiles):
+
+    * up to 6144: always (4096 × 14336 at 96 rows 63 / 34, 3072 × 12288 at 64 35 / 24), but exactly 64 MiB only past 32 rows (4096 × 8192 at
+      17 rows 16.9 / 19.1, at 48 22.3 / 21.0);
+    * up to 10240, in two row tiles up to 8192: from 112 MiB (8192 × 8192 at 64 rows 32.7 / 31.4, at 128 48 / 39), with less where the library needs an
+      activation pass or falls off (8192 × 4096 at 40 rows 17.8 / 19.8, with SwiGLU at 48 20.7 / 19.7, at 192 rows 34.0 / 28.8);
+    * up to 16384: never — two K slices or half the chip (16384 × 2048 at 128 rows 20.6 / 28.3, 12288 × 4096 31.2 / 35.0, 14336 × 4096 33.4 / 37.7);
+    * more: no slices; up to 64 rows two workgroups a unit (17408 × 4096 at 17 36.4 / 29.6, at 64 40.5 / 37.3), up to 128 where the columns fill
+      three quarters of the units (28672 × 2048 32.0 / 30.9; 20480 × 3072 34.2 / 39.1) or the library needs its activation pass (22016 × 4096
+      49.8 / 46.2); not in two row tiles (28672 × 4096 at 192 rows 66 / 77)."""
+    if not (0 < m <= 256 and n % 128 == 0 and k % 64 == 0 and n * k >= 1 << 25):
+        return False
+    if n <= 6144:
+        return m > 32 or n * k > 1 << 25
+    if n <= (10240 if m <= 128 else 8192):
+        return swiglu or m >= 192 or n * k >= 7 << 23
+    return n > 16384 and (m <= 64 or (m <= 128 and (swiglu or n >= 24576)))
 
 
 def _plain(*tensors: torch.Tensor) -> bool:
@@ -283,11 +296,11 @@ def _plain(*tensors: torch.Tensor) -> bool:
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 
-def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> bool:
+def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
     if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2):
         return False
     m, (n, k) = x.shape[0], weight.shape
-    if not (stream_rows_ok(m, n, k) and (_plain(x, weight) if out is None else _plain(x, weight, out))):
+    if not (stream_rows_ok(m, n, k, swiglu) and (_plain(x, weight) if out is None else _plain(x, weight, out))):
         return False
     return (x.shape[1] == k and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
@@ -406,7 +419,7 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     GEMM: the ``[T, 2·I]`` intermediate never exists), library GEMM + ``silu_and_mul`` in between."""
     if _skinny_ok(x, weight, 32):
         return hip().skinny_linear(x, weight, None, True)
-    if _stream_ok(x, weight):
+    if _stream_ok(x, weight, swiglu=True):
         return hip().stream_gemm(x, weight, True)
     if _PLAN.table and x.is_cuda and x.dim() == 2:          # measured at start-up for this shape and row count
         s = _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], True)

@@ -37,6 +37,21 @@ def test_expert_row_tiles_by_rows_and_by_choice(hidden):
         assert rule(256, rows, hidden, True) == 256 and rule(256, rows, hidden, False) == 128
 
 
+@pytest.mark.parametrize("n,k,plain,swiglu", [
+    # rows 17, 32, 33, 64, 65, 128, 129, 192, 256, 257; 1: the streaming tiles
+    (4096, 14336, "1111111110", "1111111110"), (4096, 8192, "0011111110", "0011111110"), (6144, 6144, "1111111110", "1111111110"),
+    (6144, 4096, "0000000000", "0000000000"), (8192, 4096, "0000000110", "1111111110"), (8192, 8192, "1111111110", "1111111110"),
+    (10240, 4096, "0000000000", "1111110000"), (10240, 8192, "1111110000", "1111110000"), (12288, 4096, "0000000000", "0000000000"),
+    (16384, 4096, "0000000000", "0000000000"), (16512, 4096, "1111000000", "1111110000"), (24576, 2048, "1111110000", "1111110000"),
+    (128256, 4096, "1111110000", "1111110000"), (8192, 28672, "1111111110", "1111111110"), (4097, 14336, "0000000000", "0000000000"),
+    (4096, 14400, "1111111110", "1111111110"), (4096, 14337, "0000000000", "0000000000")])
+def test_shapes_of_the_streaming_tiles(n, k, plain, swiglu):
+    rows = (17, 32, 33, 64, 65, 128, 129, 192, 256, 257)
+    assert "".join(str(int(ops.stream_rows_ok(m, n, k))) for m in rows) == plain
+    assert "".join(str(int(ops.stream_rows_ok(m, n, k, True))) for m in rows) == swiglu
+    assert not ops.stream_rows_ok(0, n, k)
+
+
 class _Recorder:
     """Stands in for the kernels: says which one a call came to."""
 
@@ -52,10 +67,10 @@ def test_large_linear_layers_of_decode_batches_under_traces_and_transforms(monke
     from torch._subclasses.fake_tensor import FakeTensorMode
     monkeypatch.setattr(ops, "hip", _Recorder)
     with FakeTensorMode():
-        w = torch.empty(8192, 5120, device="cuda", dtype=torch.bfloat16)
+        w = torch.empty(8192, 8192, device="cuda", dtype=torch.bfloat16)
         for m in (17, 40, 128, 200, 256, 320):
-            x = torch.empty(m, 5120, device="cuda", dtype=torch.bfloat16)
-            assert ops.stream_rows_ok(m, 8192, 5120) == (m <= 256) and not ops._stream_ok(x, w)
+            x = torch.empty(m, 8192, device="cuda", dtype=torch.bfloat16)
+            assert ops.stream_rows_ok(m, 8192, 8192) == (m <= 256) and not ops._stream_ok(x, w)
             assert ops.linear(x, w).shape == (m, 8192)
             with pytest.raises(RuntimeError, match="silu_and_mul"):        # (the library's product, then the activation kernel)
                 ops.linear_swiglu(x, w)

@@ -641,7 +641,7 @@ def test_stream_gemm_matches_fp32_reference(M, N, K, splits, swiglu):
 def test_stream_gemm_dispatch():
     """``linear`` / ``linear_swiglu`` take the streaming tiles for large layers — strided activation rows, a given result buffer — and what
     these do not take goes where it went: a bias, a result that is a view of wider rows, gradients."""
-    M, N, K = 40, 8192, 4096
+    M, N, K = 40, 7168, 8192                                        # (8192 x 4096 is the library's: 17.8 against 19.8 µs at 40 rows)
     big = _bf(M, 2 * K, seed=63)
     x, w, b = big[:, K:], _bf(N, K, seed=64, scale=K ** -0.5), _bf(N, seed=65)
     want = x.float() @ w.float().t()
