@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import reference as ref
-from .gemm_plan import PLAN as _PLAN, TAIL as _TAIL
+from .gemm_plan import PLAN as _PLAN, STREAM as _STREAM, TAIL as _TAIL
 from .kv_layout import allocate_kv_cache, bytes_per_block, kv_cache_shapes  # noqa: F401
 from . import seqmix  # noqa: F401,E402  (heterogeneous stacks: norms with token shift, token-major attention, linear-attention scan)
 
@@ -296,32 +296,44 @@ def _plain(*tensors: torch.Tensor) -> bool:
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 
-def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
-    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2):
+def _stream_operands_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> bool:
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2
+            and (_plain(x, weight) if out is None else _plain(x, weight, out))):
         return False
     m, (n, k) = x.shape[0], weight.shape
-    if not (stream_rows_ok(m, n, k, swiglu) and (_plain(x, weight) if out is None else _plain(x, weight, out))):
-        return False
     return (x.shape[1] == k and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and (out is None or (out.shape == (m, n) and out.dtype == torch.bfloat16 and out.device == x.device and out.is_contiguous()
                                  and out.data_ptr() % 16 == 0)))
 
 
+def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False, plan: Optional[int] = None) -> bool:
+    """``plan``: what the start-up measurement says for this call (None: nothing, the rule decides)."""
+    if plan is None and not (x.dim() == 2 and weight.dim() == 2 and stream_rows_ok(x.shape[0], *weight.shape, swiglu)):
+        return False
+    return (plan is None or plan == _STREAM) and _stream_operands_ok(x, weight, out)
+
+
+def _planned(x: torch.Tensor, weight: torch.Tensor, swiglu: bool) -> Optional[int]:
+    if not (_PLAN.table and x.is_cuda and x.dim() == 2):
+        return None
+    return _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], swiglu)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weightᵀ + bias``.  Decode-sized GPU inputs take the weight-streaming MFMA kernel
-    (``csrc/kernels/skinny_gemm.hip``), decode batches of large layers the streaming tiles (``stream_rows_ok``); above that the
-    start-up measurement (``ops/gemm_plan.py``) says, per layer shape and row count, whether the library GEMM (hipBLASLt through torch) or the own 256² tile — with K cut into slices at
-    mid-M — runs; shapes it never measured go to the library.  ``out``: 2-D result buffer to write into (the row-parallel
+    (``csrc/kernels/skinny_gemm.hip``); above that the start-up measurement (``ops/gemm_plan.py``) says, per layer shape and row count, whether
+    the library GEMM (hipBLASLt through torch), the streaming tiles or the own 256² tile — with K cut into slices at mid-M — runs; what it
+    never measured goes to the streaming tiles where ``stream_rows_ok`` says so, else to the library.  ``out``: 2-D result buffer to write into (the row-parallel
     layers pass a view of the all-reduce's IPC staging buffer)."""
     if _skinny_ok(x, weight, 16):
         return hip().skinny_linear(x, weight, bias, False, out)
-    if bias is None and _stream_ok(x, weight, out):
-        return hip().stream_gemm(x, weight, False, 0, out)
-    if bias is None and _PLAN.table and x.is_cuda and x.dim() == 2:
-        s = _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], False)
-        if s and _tile_operand_ok(x, weight):
+    if bias is None:
+        s = _planned(x, weight, False)
+        if _stream_ok(x, weight, out, plan=s):
+            return hip().stream_gemm(x, weight, False, 0, out)
+        if s and s != _STREAM and _tile_operand_ok(x, weight):
             return hip().dense_gemm256(x, weight, False, 1, out, True) if s == _TAIL else hip().dense_gemm256(x, weight, False, s, out)
     if out is not None:
         return torch.mm(x, weight.t(), out=out) if bias is None else torch.addmm(bias, x, weight.t(), out=out)
@@ -419,14 +431,13 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     GEMM: the ``[T, 2·I]`` intermediate never exists), library GEMM + ``silu_and_mul`` in between."""
     if _skinny_ok(x, weight, 32):
         return hip().skinny_linear(x, weight, None, True)
-    if _stream_ok(x, weight, swiglu=True):
+    s = _planned(x, weight, True)
+    if _stream_ok(x, weight, swiglu=True, plan=s):
         return hip().stream_gemm(x, weight, True)
-    if _PLAN.table and x.is_cuda and x.dim() == 2:          # measured at start-up for this shape and row count
-        s = _PLAN.splits_for(x.shape[0], weight.shape[0], weight.shape[1], True)
-        if s is not None:
-            if s and _tile_operand_ok(x, weight):
-                return hip().dense_gemm256(x, weight, True, 1, None, True) if s == _TAIL else hip().dense_gemm256(x, weight, True, s)
-            return silu_and_mul(torch.nn.functional.linear(x, weight))
+    if s is not None:                                       # measured at start-up for this shape and row count
+        if s and s != _STREAM and _tile_operand_ok(x, weight):
+            return hip().dense_gemm256(x, weight, True, 1, None, True) if s == _TAIL else hip().dense_gemm256(x, weight, True, s)
+        return silu_and_mul(torch.nn.functional.linear(x, weight))
     if (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_contiguous()
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and gemm256_swiglu_ok(x.shape[0], weight.shape[0] // 2, weight.shape[1])

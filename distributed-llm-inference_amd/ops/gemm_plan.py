@@ -1,4 +1,4 @@
-"""Measured GEMM dispatch (VERDICT r2 item 6): which kernel runs a projection at which row count is decided by timing the
+"""Measured GEMM dispatch: which kernel runs a projection at which row count is decided by timing the
 candidates ON THIS GPU at start-up, per (layer shape, row count), instead of by thresholds guessed once.
 
 Why a table and not a rule: the hipGraph-timed sweep in ``profiles/midm_gemm_r3.md`` shows the vendor library 1.3–4.6 × off
@@ -11,9 +11,11 @@ token counts in multiples of 256), so the table is keyed by the exact M the grap
 the next bucket up.
 
 Candidates per (N, K, swiglu, M):  ``lib`` (hipBLASLt through torch, plus ``silu_and_mul`` for gate/up), ``tile:S`` —
-the 256² tile with S K-slices (S = 1: no slabs; with the SwiGLU epilogue fused for gate/up) — and ``tile+tail``: the tile
+the 256² tile with S K-slices (S = 1: no slabs; with the SwiGLU epilogue fused for gate/up) —, ``tile+tail``: the tile
 with only the REMAINDER of its last, partly filled round of one workgroup per CU cut into K-slices (a 7 × 112-tile
-gate/up GEMM is 3 rounds + 16 tiles: those 16 run as 128 slices next to each other instead of as a fourth round).  Weights rotate through all
+gate/up GEMM is 3 rounds + 16 tiles: those 16 run as 128 slices next to each other instead of as a fourth round), and up to 256 rows
+``stream``, the weight-streaming tiles of ``stream_gemm.hip``.  What was measured goes before ``ops.stream_rows_ok``, which speaks for
+shapes and row counts without an entry.  Weights rotate through all
 layers of the model while timing, so no candidate finds its matrix in the 256 MB infinity cache.  Rank 0's table is
 broadcast under TP: every rank of a group runs the same kernels.
 """
@@ -27,8 +29,10 @@ import torch
 
 ENABLED = os.environ.get("DLI_GEMM_TUNE", "1") != "0"
 CAPTURE_MODE = os.environ.get("DLI_CAPTURE_MODE", "thread_local")     # see ops.CAPTURE_MODE
-MIN_ROWS = 65                 # at and below 64 rows the weight-streaming kernel (skinny_gemm.hip) has its own rules
+MIN_ROWS = 65                 # at and below 64 rows the weight-streaming kernels have rules of their own (ops.skinny_rows_ok, ops.stream_rows_ok)
 TAIL = 100                    # table value: plain tiles for the whole rounds, K-split remainder (dense_gemm256 split_tail)
+STREAM = 200                  # table value: weight-streaming tiles (stream_gemm)
+STREAM_MAX_ROWS = 256
 NUM_CU = 256
 
 
@@ -39,7 +43,7 @@ class GemmPlan:
 
     # ------------------------------------------------------------------ lookup (hot path: two dict probes)
     def splits_for(self, m: int, n: int, k: int, swiglu: bool) -> Optional[int]:
-        """K-slices of the 256² tile for this call, 0 for the library path, None when the shape was never tuned."""
+        """K-slices of the 256² tile for this call (or ``TAIL``), ``STREAM``, 0 for the library path, None when the shape was never tuned."""
         rows = self.table.get((n, k, swiglu))
         if rows is None or m < MIN_ROWS:
             return None
@@ -50,7 +54,8 @@ class GemmPlan:
         for mm in ms:                                       # the next bucket up (same tile count or one more)
             if mm >= m:
                 return rows[mm]
-        return rows[ms[-1]]
+        last = rows[ms[-1]]
+        return None if last == STREAM and m > STREAM_MAX_ROWS else last
 
     # ------------------------------------------------------------------ tuning
     @staticmethod
@@ -80,6 +85,8 @@ class GemmPlan:
             s *= 2
         if GemmPlan.tail_slices(m, n, k, swiglu):
             out.append(TAIL)
+        if m <= STREAM_MAX_ROWS and n % 128 == 0 and k % 64 == 0:
+            out.append(STREAM)
         return out
 
     @torch.inference_mode()
@@ -108,6 +115,8 @@ class GemmPlan:
                         fn = (lambda w: silu_and_mul(F.linear(x, w))) if swiglu else (lambda w: F.linear(x, w))
                     elif s == TAIL:
                         fn = lambda w: lib.dense_gemm256(x, w, swiglu, 1, None, True)
+                    elif s == STREAM:
+                        fn = lambda w: lib.stream_gemm(x, w, swiglu)
                     else:
                         fn = lambda w, s=s: lib.dense_gemm256(x, w, swiglu, s)
                     times[s] = self._time(fn, weights)
@@ -116,7 +125,7 @@ class GemmPlan:
                     best = 0                                 # the library keeps ties: fewer moving parts
                 entry[m] = best
                 rep[m] = {"lib_us": round(times[0], 1), "best_us": round(times[best], 1),
-                          "best": "lib" if best == 0 else "tile+tail" if best == TAIL else f"tile:{best}"}
+                          "best": {0: "lib", TAIL: "tile+tail", STREAM: "stream"}.get(best, f"tile:{best}")}
                 if TAIL in times:
                     rep[m]["tail_us"], rep[m]["tile1_us"] = round(times[TAIL], 1), round(times[1], 1)
             if entry:

@@ -76,6 +76,36 @@ def test_large_linear_layers_of_decode_batches_under_traces_and_transforms(monke
                 ops.linear_swiglu(x, w)
 
 
+def test_the_plan_goes_before_the_rule(monkeypatch):
+    """A tuned entry decides also where the rule has an opinion; without one, and past the rows that a streaming entry can serve, the rule does."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from dli_amd.ops import gemm_plan
+    monkeypatch.setattr(ops, "hip", _Recorder)
+    monkeypatch.setattr(ops, "_plain", lambda *t: True)
+    plan = gemm_plan.GemmPlan()
+    monkeypatch.setattr(ops, "_PLAN", plan)
+    n, k = 8192, 8192
+
+    def route(m, swiglu, bias=None):
+        x, w = (torch.empty(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n))
+        try:
+            return "lib" if (ops.linear_swiglu(x, w) if swiglu else ops.linear(x, w, bias)) is not None else None
+        except RuntimeError as e:
+            return {"silu_and_mul": "lib"}.get(str(e), str(e))
+    with FakeTensorMode():
+        for swiglu in (False, True):
+            plan.load({})
+            assert [route(m, swiglu) for m in (40, 100, 256, 300)] == ["stream_gemm"] * 3 + ["lib"]
+            for value, kernel in ((0, "lib"), (4, "dense_gemm256"), (gemm_plan.TAIL, "dense_gemm256"), (gemm_plan.STREAM, "stream_gemm")):
+                plan.load({f"{n},{k},{int(swiglu)}": {"128": value}})
+                assert [route(m, swiglu) for m in (100, 128, 200)] == [kernel] * 3
+                assert route(40, swiglu) == "stream_gemm"                     # below the rows that are tuned
+                assert route(300, swiglu) == ("lib" if value == gemm_plan.STREAM else kernel)
+        assert route(100, False, torch.empty(n, device="cuda", dtype=torch.bfloat16)) == "lib"
+    assert [gemm_plan.STREAM in plan.candidates(m, n, k, False) for m in (65, 256, 257)] == [True, True, False]
+    assert plan.load(plan.export()) is None and plan.splits_for(128, n, k, True) == gemm_plan.STREAM
+
+
 def test_plain_tensors():
     import torch.autograd.forward_ad as fw
     t, seen = torch.zeros(4, 4), []

@@ -662,6 +662,29 @@ def test_stream_gemm_dispatch():
         ops.hip().stream_gemm(_bf(257, K, seed=1), w)
 
 
+def test_measured_dispatch_can_choose_the_streaming_tiles(monkeypatch):
+    """Start-up timing of a small layer, candidates streaming tiles included; then every table value gives the product by its own kernel."""
+    from dli_amd.ops import gemm_plan
+    N, K = 1024, 512
+    w = _bf(N, K, seed=71, scale=K ** -0.5)
+    plan = gemm_plan.GemmPlan()
+    monkeypatch.setattr(ops, "_PLAN", plan)
+    for swiglu in (False, True):
+        plan.tune([("layer", [w, w.clone()], swiglu)], [65, 96, 256, 512], DEV)
+        entry = plan.table[(N, K, swiglu)]
+        assert all(entry[m] in plan.candidates(m, N, K, swiglu) for m in (65, 96, 256, 512))
+        f = ops.linear_swiglu if swiglu else ops.linear
+        for m, value in ((96, gemm_plan.STREAM), (80, gemm_plan.STREAM), (96, 2), (96, 0), (300, gemm_plan.STREAM)):
+            plan.load({f"{N},{K},{int(swiglu)}": {"96": value}})
+            x = _bf(m, K, seed=72)
+            want = x.float() @ w.float().t()
+            want = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:] if swiglu else want
+            got = f(x, w)
+            torch.testing.assert_close(got.float(), want, rtol=2e-2, atol=2e-2)
+            if value == gemm_plan.STREAM and m <= 96:
+                assert torch.equal(got, ops.hip().stream_gemm(x, w, swiglu))
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 512, 256), (1000, 1024, 4096), (4096, 256, 512), (1, 256, 64), (300, 768, 1024),
                                    (513, 256, 192)])
 def test_dense_gemm256_matches_fp32_reference(M, N, K):
