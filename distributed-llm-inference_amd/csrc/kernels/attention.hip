@@ -636,6 +636,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
 // trace's length mix at B = 1024 (profiles/ab_decode_nt_r3.jsonl).  DLI_DECODE_NT=0: plain loads (A/B knob).
 static const bool g_decode_nt = std::getenv("DLI_DECODE_NT") == nullptr || std::atoi(std::getenv("DLI_DECODE_NT")) != 0;
 
+// Waves of a decode workgroup, the same for both launches, so that a row that is one range gets the same bits from either.
+// bf16: eight halve a whole row's serial pages; e4m3 pages take half the bytes a wave and the registers of the
+// widening: four.  Sorted lists, 32/8 heads, µs, 4 against 8 waves — bf16, rows of up to 1500 / 2048 tokens: B = 100 55.9 / 52.6, 160 111.8 /
+// 109.5, 300 199 / 199; e4m3: B = 100 30.0 / 32.6, 160 60.1 / 60.9, 300 104.6 / 112.4.  Rows cut into ranges of four pages and more, where
+// half of eight waves may have none, bf16: B = 1 of 620 tokens 7.9 / 7.6, 8 8.6 / 8.4, 1 of 2048 9.1 / 8.9, 8 13.3 / 14.3, 48 41.1 / 38.7.
+// Groups of more than 8 heads keep four: eight waves' merge buffers would pass 64 KB of LDS.
+static int decode_waves(bool kv_fp8, int G) { return kv_fp8 || G > 8 ? 4 : 8; }
 static size_t decode_lds(int waves, int G) { return (size_t)(waves * G * (HD + 4) + 2 * waves * G) * sizeof(float); }
 
 void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
@@ -647,12 +654,13 @@ void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, c
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;        // the kernels read the per-head values themselves
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
   dim3 grid(Hkv, num_seqs, num_splits);
-#define DLI_DECODE_GO(KV8_, NT_)                                                                                              \
-  hipLaunchKernelGGL((paged_decode_kernel<KV8_, false, 4, NT_>), grid, dim3(256), decode_lds(4, G), stream, (const uint16_t*)q, q_stride, \
-                     k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv,    \
+#define DLI_DECODE_GO(KV8_, NW_, NT_)                                                                                         \
+  hipLaunchKernelGGL((paged_decode_kernel<KV8_, false, NW_, NT_>), grid, dim3(NW_ * 64), decode_lds(NW_, G), stream, (const uint16_t*)q, \
+                     q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv, \
                      num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, nullptr, nullptr)
-  if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, true); else DLI_DECODE_GO(true, false); }
-  else { if (g_decode_nt) DLI_DECODE_GO(false, true); else DLI_DECODE_GO(false, false); }
+  if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, 4, true); else DLI_DECODE_GO(true, 4, false); }
+  else if (decode_waves(kv_fp8, G) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
+  else { if (g_decode_nt) DLI_DECODE_GO(false, 8, true); else DLI_DECODE_GO(false, 8, false); }
 #undef DLI_DECODE_GO
   if (num_splits > 1)
     hipLaunchKernelGGL(decode_reduce_kernel, dim3(num_seqs, Hq), dim3(128), 0, stream, part_o, part_ml, (uint16_t*)out,
@@ -675,12 +683,8 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
   hipLaunchKernelGGL((paged_decode_kernel<KV8_, true, NW_, NT_>), grid, dim3(NW_ * 64), decode_lds(NW_, G), stream, (const uint16_t*)q, \
                      q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq,  \
                      Hkv, 1, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work, counts)
-  // bf16: eight waves a workgroup halve a whole row's serial pages; e4m3 pages take half the bytes a wave and the registers of the
-  // widening: four.  Sorted lists, 32/8 heads, µs, 4 against 8 waves — bf16, rows of up to 1500 / 2048 tokens: B = 100 55.9 / 52.6, 160 111.8 /
-  // 109.5, 300 199 / 199; e4m3: B = 100 30.0 / 32.6, 160 60.1 / 60.9, 300 104.6 / 112.4.
-  // Groups of more than 8 heads keep four: eight waves' merge buffers would pass 64 KB of LDS.
   if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, 4, true); else DLI_DECODE_GO(true, 4, false); }
-  else if (G > 8) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
+  else if (decode_waves(kv_fp8, G) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
   else { if (g_decode_nt) DLI_DECODE_GO(false, 8, true); else DLI_DECODE_GO(false, 8, false); }
 #undef DLI_DECODE_GO
   if (reds > 0)

@@ -117,7 +117,7 @@ def choose_decode_splits(num_seqs: int, num_kv_heads: int, max_seq_len: int, num
     groups = max(num_seqs * num_kv_heads, 1)
     pages = max((max_seq_len + 31) // 32, 1)
     want = (2 * num_cus + groups - 1) // groups          # aim for ≥ 2 workgroups per CU
-    return int(max(1, min(want, (pages + 3) // 4, 16)))   # keep ≥ 4 pages (one per wave) per split
+    return int(max(1, min(want, (pages + 3) // 4, 16)))   # keep ≥ 4 pages per split (one per wave of four)
 
 
 def decode_chunk_pages(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int = 0, num_cus: int = 256) -> int:
@@ -126,7 +126,7 @@ def decode_chunk_pages(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int =
     5.73 TB/s, 32-page ranges 5.64, 16-page 5.40, 8-page 5.11 — per-workgroup fixed cost and the extra reduce pass
     outweigh the better balance; row order, longest first, is what recovers the tail), so big batches get ONE range per
     row.  Smaller batches cut the longest row into as many ranges as it takes to reach that fill (whole multiples of 4
-    pages: one per wave and iteration) — each row by its own length, a short row stays one range.  ``cap_items``:
+    pages: one per wave and iteration of an e4m3 workgroup's four; of a bf16 workgroup's eight half may have none, which costs nothing) — each row by its own length, a short row stays one range.  ``cap_items``:
     ranges are doubled until the list fits (the fixed grid of a hipGraph)."""
     pages = (np.asarray(seq_lens, dtype=np.int64) + 31) >> 5
     n, maxp = len(pages), max(int(pages.max()) if len(pages) else 1, 1)
@@ -149,7 +149,7 @@ def decode_launch_caps(rows: int, num_kv_heads: int, num_cus: int = 256):
 
 
 def build_decode_work(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int = 0, chunk_pages: int = 0):
-    """Host-side work list of the decode kernel (no launch-wide split count).
+    """Host-side work list of the decode kernel.
 
     Every sequence's pages are cut into ``ceil(pages / chunk)`` ranges of EQUAL size (rounded up to 4 pages), so a
     2048-token row becomes several workgroups per kv head and a 40-token row one.  Returns
@@ -162,7 +162,7 @@ def build_decode_work(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int = 
     pages = np.maximum((L + 31) >> 5, 1)
     c = chunk_pages or decode_chunk_pages(L, num_kv_heads, cap_items)
     k = (pages + c - 1) // c                                   # ranges per row
-    per = ((pages + k - 1) // k + 3) // 4 * 4                  # equal-size ranges, whole wave rounds
+    per = ((pages + k - 1) // k + 3) // 4 * 4                  # equal-size ranges, whole rounds of four waves
     k = (pages + per - 1) // per
     total = int(k.sum())
     row = np.repeat(np.arange(n), k)

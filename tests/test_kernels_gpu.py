@@ -241,6 +241,24 @@ def test_decode_work_list_equals_uniform_splits_bitwise_on_single_range_rows():
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (16, 1)])
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_decode_launches_give_whole_rows_the_same_bits(Hq, Hkv, kv_dtype):
+    """Rows of more pages than a workgroup has waves: the work list and the uniform launch deal the pages to as many waves."""
+    seq_lens = [5, 127, 128, 129, 260, 700, 2048]
+    kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=31)
+    B = len(seq_lens)
+    qkv = _bf(B, (Hq + 2 * Hkv) * 128, seed=32)
+    sl = torch.tensor(seq_lens, dtype=torch.int32, device=DEV)
+    qsl = torch.arange(B + 1, dtype=torch.int32, device=DEV)
+    m1 = ops.AttnMetadata(B, 0, B, None, None, bt, sl, qsl, decode_splits=1)
+    m2 = ops.attach_decode_worklist(ops.AttnMetadata(B, 0, B, None, None, bt, sl, qsl), np.array(seq_lens), Hq, Hkv, DEV, chunk_pages=64)
+    assert m2.decode_reds == 0
+    a = ops.paged_attention(qkv, kc, vc, m1, Hq, Hkv, 128, 0.088)
+    b = ops.paged_attention(qkv, kc, vc, m2, Hq, Hkv, 128, 0.088)
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("Hq,Hkv,seq_lens,chunk", [(32, 4, [8500, 8192, 1, 260], 4), (8, 1, [255, 256, 257, 288, 225, 31], 16), (16, 1, [289, 33, 513], 8),
                                                    (9, 1, [300, 64], 8), (4, 4, [8231, 2049], 4)])
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
