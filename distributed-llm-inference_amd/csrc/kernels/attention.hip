@@ -638,11 +638,15 @@ static const bool g_decode_nt = std::getenv("DLI_DECODE_NT") == nullptr || std::
 
 // Waves of a decode workgroup, the same for both launches, so that a row that is one range gets the same bits from either.
 // bf16: eight halve a whole row's serial pages; e4m3 pages take half the bytes a wave and the registers of the
-// widening: four.  Sorted lists, 32/8 heads, µs, 4 against 8 waves — bf16, rows of up to 1500 / 2048 tokens: B = 100 55.9 / 52.6, 160 111.8 /
-// 109.5, 300 199 / 199; e4m3: B = 100 30.0 / 32.6, 160 60.1 / 60.9, 300 104.6 / 112.4.  Rows cut into ranges of four pages and more, where
+// widening: four.  Sorted lists, 32/8 heads, µs, 4 against 8 waves — bf16, rows of up to 1500 tokens: B = 100 55.9 / 52.6; e4m3:
+// B = 100 30.0 / 32.6, 160 60.1 / 60.9, 300 104.6 / 112.4.  Rows cut into ranges of four pages and more, where
 // half of eight waves may have none, bf16: B = 1 of 620 tokens 7.9 / 7.6, 8 8.6 / 8.4, 1 of 2048 9.1 / 8.9, 8 13.3 / 14.3, 48 41.1 / 38.7.
+// Many workgroups keep four: the compute units are full anyway, and of a short row's eight waves half have no page.  Rows of up to 40 / 100 / 200 /
+// 1000 tokens, four against eight — B = 128 (1024 workgroups) 9.2 / 9.4, 11.0 / 10.8, 14.4 / 14.6, 45.0 / 44.6; B = 160 of up to
+// 2048 111.8 / 109.5, but of up to 40 10.0 / 11.5; B = 256 14.2 / 16.5, 17.6 / 19.6,
+// 24.6 / 25.1, 86.2 / 86.4; B = 512 26.8 / 31.8, 31.1 / 35.6, 44.9 / 46.4, 175 / 176.
 // Groups of more than 8 heads keep four: eight waves' merge buffers would pass 64 KB of LDS.
-static int decode_waves(bool kv_fp8, int G) { return kv_fp8 || G > 8 ? 4 : 8; }
+static int decode_waves(bool kv_fp8, int G, int64_t workgroups) { return kv_fp8 || G > 8 || workgroups > 1024 ? 4 : 8; }
 static size_t decode_lds(int waves, int G) { return (size_t)(waves * G * (HD + 4) + 2 * waves * G) * sizeof(float); }
 
 void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
@@ -659,7 +663,7 @@ void launch_paged_decode(const void* q, int64_t q_stride, const void* k_cache, c
                      q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq, Hkv, \
                      num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, nullptr, nullptr)
   if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, 4, true); else DLI_DECODE_GO(true, 4, false); }
-  else if (decode_waves(kv_fp8, G) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
+  else if (decode_waves(kv_fp8, G, (int64_t)Hkv * num_seqs * num_splits) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
   else { if (g_decode_nt) DLI_DECODE_GO(false, 8, true); else DLI_DECODE_GO(false, 8, false); }
 #undef DLI_DECODE_GO
   if (num_splits > 1)
@@ -684,7 +688,7 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
                      q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, (uint16_t*)out, out_stride, part_o, part_ml, Hq,  \
                      Hkv, 1, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work, counts)
   if (kv_fp8) { if (g_decode_nt) DLI_DECODE_GO(true, 4, true); else DLI_DECODE_GO(true, 4, false); }
-  else if (decode_waves(kv_fp8, G) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
+  else if (decode_waves(kv_fp8, G, (int64_t)Hkv * items) == 4) { if (g_decode_nt) DLI_DECODE_GO(false, 4, true); else DLI_DECODE_GO(false, 4, false); }
   else { if (g_decode_nt) DLI_DECODE_GO(false, 8, true); else DLI_DECODE_GO(false, 8, false); }
 #undef DLI_DECODE_GO
   if (reds > 0)

@@ -241,11 +241,11 @@ def test_decode_work_list_equals_uniform_splits_bitwise_on_single_range_rows():
     assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (16, 1)])
+@pytest.mark.parametrize("Hq,Hkv,n", [(32, 8, 1), (16, 1, 1), (32, 8, 18), (32, 8, 19)])      # 7 rows each; 1024 workgroups between the last two
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
-def test_decode_launches_give_whole_rows_the_same_bits(Hq, Hkv, kv_dtype):
+def test_decode_launches_give_whole_rows_the_same_bits(Hq, Hkv, n, kv_dtype):
     """Rows of more pages than a workgroup has waves: the work list and the uniform launch deal the pages to as many waves."""
-    seq_lens = [5, 127, 128, 129, 260, 700, 2048]
+    seq_lens = [5, 127, 128, 129, 260, 700, 2048 if n == 1 else 300] * n
     kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=31)
     B = len(seq_lens)
     qkv = _bf(B, (Hq + 2 * Hkv) * 128, seed=32)
@@ -257,6 +257,8 @@ def test_decode_launches_give_whole_rows_the_same_bits(Hq, Hkv, kv_dtype):
     a = ops.paged_attention(qkv, kc, vc, m1, Hq, Hkv, 128, 0.088)
     b = ops.paged_attention(qkv, kc, vc, m2, Hq, Hkv, 128, 0.088)
     assert torch.equal(a, b)
+    want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(B, Hq, 128), kc, vc, bt, sl, qsl, 0.088).float()
+    torch.testing.assert_close(a.float().view_as(want), want, rtol=2 ** -7, atol=2 ** -8 * 4.5)    # bf16 weights and results, |v| ≤ 4.5
 
 
 @pytest.mark.parametrize("Hq,Hkv,seq_lens,chunk", [(32, 4, [8500, 8192, 1, 260], 4), (8, 1, [255, 256, 257, 288, 225, 31], 16), (16, 1, [289, 33, 513], 8),
