@@ -21,6 +21,7 @@
 //
 // KV8: pages hold OCP e4m3 (K chunks are 64 wide, see kv_layout); values are widened to bf16 in
 // registers, the per-tensor scales are folded into the softmax scale (K) and the epilogue (V).
+#include <algorithm>
 #include <cstdlib>
 
 #include "common.h"
@@ -452,6 +453,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   const int my_nblk = last_pos < 0 ? 0 : (last_pos >> 5) + 1;
   const int tile_tokens = 16 * (8 / G);
   const int nblk = ((ctx + min(q0 + tile_tokens, n_new) - 1) >> 5) + 1;
+  // A tile of a few pages is done by one group alone, the other ends here (a barrier waits for the waves that are left): meeting at the end
+  // costs as much as a turn of four pages less saves (prompts of 64 tokens, µs, two groups / one / now 8.25 / 7.28 / 7.4, of 160 10.4 / 9.7 / 9.8,
+  // of 256 12.0 / 12.3 / 12.2).
+  const bool both = GROUPS == 2 && nblk > 7;
+  if (GROUPS == 2 && !both && grp == 1) return;
+  const int turns = both ? (nblk + 1) >> 1 : nblk;
+  const int step = both ? 2 : 1, start = both ? grp : 0;
 
   // Qᵀ fragments: k-step j covers d = 16 j + 8 hi … + 7 (fp8 pages keep d in 64-wide chunks: same d, other address)
   bf16x8 qf[8];
@@ -502,11 +510,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   const int v_off0 = c32 * 64 + ((hi ^ swz) << 4), v_off1 = c32 * 64 + (((2 + hi) ^ swz) << 4);
   const int v8_off = c32 * 32 + 8 * hi;
 
-  // group g walks pages g, g + GROUPS, … in a ring of its own; all groups pass the same barriers
-  const int turns = (nblk + GROUPS - 1) / GROUPS;
-  if (grp < nblk) DLI_STAGE(grp, 0);
-  if (grp + GROUPS < nblk) {
-    DLI_STAGE(grp + GROUPS, 1);
+  // group g walks pages g, g + 2, … in a ring of its own; both pass the same barriers
+  if (start < nblk) DLI_STAGE(start, 0);
+  if (start + step < nblk) {
+    DLI_STAGE(start + step, 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -514,10 +521,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   __syncthreads();
   int st = 0;
   for (int t = 0; t < turns; ++t) {
-    const int b = GROUPS * t + grp;
-    const bool ahead = b + 2 * GROUPS < nblk;
+    const int b = step * t + start;
+    const bool ahead = b + 2 * step < nblk;
     const int st2 = st == 0 ? NSTAGE - 1 : st - 1;
-    if (ahead) DLI_STAGE(b + 2 * GROUPS, st2);
+    if (ahead) DLI_STAGE(b + 2 * step, st2);
     if (b < my_nblk) {
       const char* kb = smem + st * 2 * PAGE_BYTES;
       const char* vb = kb + PAGE_BYTES;
@@ -579,38 +586,42 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   }
 
   if constexpr (GROUPS == 2) {
-    // the two groups of a column set swap halves of their sums: group 0 finishes d tiles 0 and 1, group 1 tiles 2 and 3
-    __shared__ float ml[2][4][2][64];
-    float* X = reinterpret_cast<float*>(smem_all) + wave * 2 * 2048;              // [wave][from group][32][64]
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) X[grp * 2048 + (n * 16 + r) * 64 + lane] = grp ? o[n][r] : o[n + 2][r];
-    ml[grp][wave][0][lane] = m;
-    ml[grp][wave][1][lane] = lsum;
-    __syncthreads();
-    const float m2 = ml[grp ^ 1][wave][0][lane], M = fmaxf(m, m2), f1 = fast_exp2(m - M), f2 = fast_exp2(m2 - M);
-    float l = lsum * f1 + ml[grp ^ 1][wave][1][lane] * f2;
-    {
-      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
-      l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-    }
-    if (valid) {
-      const float rcp = l > 0.f ? v_scale / l : 0.f;
-      const float r1 = f1 * rcp, r2 = f2 * rcp;
-      uint16_t* op = out + (int64_t)(qs + qtok) * out_stride + (kvh * G + head) * HD + 4 * hi + grp * 64;
+    if (both) {
+      // the two groups of a column set swap halves of their sums: group 0 finishes d tiles 0 and 1, group 1 tiles 2 and 3
+      __shared__ float ml[2][4][2][64];
+      float* X = reinterpret_cast<float*>(smem_all) + wave * 2 * 2048;              // [wave][from group][32][64]
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          bf16x4 w;
+        for (int r = 0; r < 16; ++r) X[grp * 2048 + (n * 16 + r) * 64 + lane] = grp ? o[n][r] : o[n + 2][r];
+      ml[grp][wave][0][lane] = m;
+      ml[grp][wave][1][lane] = lsum;
+      __syncthreads();
+      const float m2 = ml[grp ^ 1][wave][0][lane], M = fmaxf(m, m2), f1 = fast_exp2(m - M), f2 = fast_exp2(m2 - M);
+      float l = lsum * f1 + ml[grp ^ 1][wave][1][lane] * f2;
+      {
+        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+        l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+      }
+      if (valid) {
+        const float rcp = l > 0.f ? v_scale / l : 0.f;
+        const float r1 = f1 * rcp, r2 = f2 * rcp;
+        uint16_t* op = out + (int64_t)(qs + qtok) * out_stride + (kvh * G + head) * HD + 4 * hi + grp * 64;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            w[e] = (short)f2bf((grp ? o[n + 2][4 * r4 + e] : o[n][4 * r4 + e]) * r1 + X[(grp ^ 1) * 2048 + (n * 16 + 4 * r4 + e) * 64 + lane] * r2);
-          *reinterpret_cast<bf16x4*>(op + 32 * n + 8 * r4) = w;
-        }
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            bf16x4 w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              w[e] = (short)f2bf((grp ? o[n + 2][4 * r4 + e] : o[n][4 * r4 + e]) * r1 + X[(grp ^ 1) * 2048 + (n * 16 + 4 * r4 + e) * 64 + lane] * r2);
+            *reinterpret_cast<bf16x4*>(op + 32 * n + 8 * r4) = w;
+          }
+      }
+      return;
     }
-  } else {
+  }
+  {
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
     const float l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
     if (valid) {
@@ -696,20 +707,35 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
                        out_stride, Hq, 1, kv_fp8 ? v_scale : 1.f, kv_fp8 ? kv_scales : nullptr, Hkv, (const int4*)red, counts);
 }
 
+// Two groups where a compute unit gets one workgroup: a tile's pages are a serial chain of 0.7 µs each, and what the chip
+// has no second tile for, a second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: prompts of 1000 tokens (256
+// workgroups) 32.3 / 26.9, of 2000 with 8/1 heads (250) 57.8 / 45.7, 8 × 128 tokens behind 1000 (256) 37.9 / 34.5, 32 × 16 behind 300 15.0 / 15.3.
+// A unit holds one workgroup of two groups (100 KB of LDS), but three of one: past 256 the rest comes in a second round, whose
+// workgroups all start with 5 µs of latencies.  16 × 100 tokens (512) 12.5 / 17.2, 9 × 128 behind 1000 (288) 46.3 / 60.4, 3 × 600 (456) 25.0 /
+// 26.6.  It pays there only if the second round is made of short tiles: long prompts with little in front of them (one of 2000 (504) 62.2 / 56.1, two of
+// 600 (304) 23.7 / 19.4, one of 1300 behind 300 (328) 50.8 / 40.0).  With 5 µs + 0.0285 µs a token for one group, 5.5 + 0.0225 for two, and the
+// first tile of the second round at `second` tokens of context, that is what the last line says (fitted on 190 steps of equal prompts).
+// longest: tokens of context (new ones included) of the longest sequence, sequences: with new tokens; 0: not known, as for a captured launch of bounds.
+int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences) {
+  const int blocks = num_tiles * Hkv, tile_tokens = 16 * (8 / G);
+  if (blocks <= 256) return longest == 0 || longest > 224 ? 2 : 1;
+  if (blocks > 512 || longest <= 0 || sequences <= 0) return 1;
+  const float mean = std::min((float)longest, (float)num_tiles * tile_tokens / sequences);
+  const float second = longest - mean + mean * (blocks - 256) / blocks;
+  return second < 0.63f * longest - 180.f ? 2 : 1;
+}
+
 void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
                           const int* block_tables, int max_blocks, const int* seq_lens, const int* query_start_loc,
                           const int* tile_seq, const int* tile_q0, int num_tiles, void* out, int64_t out_stride, int Hq,
                           int Hkv, float scale, bool kv_fp8, float k_scale, float v_scale, const float* kv_scales,
-                          const int* counts, hipStream_t stream) {
+                          const int* counts, int longest, int sequences, hipStream_t stream) {
   if (num_tiles == 0) return;
+  const int G = Hq / Hkv;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-  // Two groups where a compute unit would get two workgroups or less: a tile's pages are a serial chain of 0.7 µs each, and what the chip
-  // has no second tile for, a second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: one prompt of
-  // 2048 (512 workgroups) 60.5 / 51.8, 100 tokens behind 1500 42.5 / 32.9, e4m3 2 × 1024 behind 1024 50.7 / 35.8; 592 workgroups 46.9 / 46.2,
-  // 1008 41.9 / 57.0.
-  const int blocks = num_tiles * Hkv, groups = blocks <= 512 ? 2 : 1;
-  dim3 grid((blocks + 7) / 8 * 8);
+  const int groups = prefill_page_groups(num_tiles, Hkv, G, longest, sequences);
+  dim3 grid((num_tiles * Hkv + 7) / 8 * 8);
 #define DLI_PREFILL_GO(KV8_, G_)                                                                                              \
   hipLaunchKernelGGL((paged_prefill_kernel<KV8_, G_>), grid, dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, v_cache, \
                      block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, Hq, Hkv, num_tiles, \

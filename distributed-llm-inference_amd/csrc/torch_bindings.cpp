@@ -239,7 +239,8 @@ void paged_attention_decode_worklist(Tensor out, const Tensor& q, const Tensor& 
 void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
                              const Tensor& seq_lens, const Tensor& query_start_loc, const Tensor& tile_seq, const Tensor& tile_q0,
                              int64_t num_tiles, int64_t Hq, int64_t Hkv, double scale, double k_scale, double v_scale,
-                             const c10::optional<Tensor>& kv_scales, const c10::optional<Tensor>& counts) {
+                             const c10::optional<Tensor>& kv_scales, const c10::optional<Tensor>& counts, int64_t longest,
+                             int64_t sequences) {
   check_bf16_rows(q, "q");
   check_bf16_rows(out, "out");
   check_i32(block_tables, "block_tables");
@@ -262,7 +263,7 @@ void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache,
                             (int)block_tables.size(1), seq_lens.data_ptr<int>(), query_start_loc.data_ptr<int>(),
                             tile_seq.data_ptr<int>(), tile_q0.data_ptr<int>(), (int)num_tiles, out.data_ptr(), out.stride(0),
                             (int)Hq, (int)Hkv, (float)scale, is_fp8(k_cache), (float)k_scale, (float)v_scale,
-                            scales_ptr(kv_scales, Hkv), cnt, cur_stream(q));
+                            scales_ptr(kv_scales, Hkv), cnt, (int)longest, (int)sequences, cur_stream(q));
 }
 
 void sample(Tensor out, const Tensor& logits, const Tensor& temperature, const Tensor& top_p, const Tensor& top_k,
@@ -784,7 +785,9 @@ TORCH_LIBRARY(dli, m) {
         "float v_scale, Tensor? kv_scales=None) -> ()", &paged_attention_decode);
   m.def("paged_attention_prefill(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor seq_lens, "
         "Tensor query_start_loc, Tensor tile_seq, Tensor tile_q0, int num_tiles, int num_heads, int num_kv_heads, float scale, "
-        "float k_scale, float v_scale, Tensor? kv_scales=None, Tensor? counts=None) -> ()", &paged_attention_prefill);
+        "float k_scale, float v_scale, Tensor? kv_scales=None, Tensor? counts=None, int longest=0, int sequences=0) -> ()", &paged_attention_prefill);
+  m.def("prefill_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences) -> int",
+        [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s) -> int64_t { return dli::prefill_page_groups((int)t, (int)h, (int)g, (int)l, (int)s); });
   m.def("paged_attention_decode_worklist(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor seq_lens, Tensor work, Tensor red, Tensor counts, int items, int reds, int max_parts, int Hq, int Hkv, float scale, "
         "Tensor workspace, float k_scale, float v_scale, Tensor? kv_scales=None) -> ()", &paged_attention_decode_worklist);

@@ -492,6 +492,7 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
             out = torch.empty(T, num_heads * head_dim, dtype=qkv.dtype, device=qkv.device)
         lib = hip()
         side = None
+        known = (0, 0) if meta.counts_on_device else (meta.max_seq_len, meta.num_prefill)    # a captured launch has bounds only
         if CONCURRENT_ATTN and meta.num_prefill_tiles > 0 and (meta.decode_items > 0 or meta.num_decode > 0):
             # mixed step: the prefill tiles (MFMA / VALU-bound, a few hundred workgroups) run on a side stream next to the
             # decode rows (HBM-bound) — disjoint rows of `out`; inside a capture the side stream forks from and joins the
@@ -503,7 +504,7 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                 lib.paged_attention_prefill(out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens,
                                             meta.query_start_loc, meta.prefill_tile_seq, meta.prefill_tile_q0,
                                             meta.num_prefill_tiles, num_heads, num_kv_heads, scale, k_scale, v_scale, kv_scales,
-                                            meta.counts if meta.counts_on_device else None)
+                                            meta.counts if meta.counts_on_device else None, *known)
         if meta.decode_items > 0:
             lib.paged_attention_decode_worklist(out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens,
                                                 meta.decode_work, meta.decode_red, meta.counts, meta.decode_items,
@@ -519,7 +520,7 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
             lib.paged_attention_prefill(out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens,
                                         meta.query_start_loc, meta.prefill_tile_seq, meta.prefill_tile_q0,
                                         meta.num_prefill_tiles, num_heads, num_kv_heads, scale, k_scale, v_scale, kv_scales,
-                                        meta.counts if meta.counts_on_device else None)
+                                        meta.counts if meta.counts_on_device else None, *known)
         return out
     B = meta.num_decode + meta.num_prefill
     if kv_scales is not None:

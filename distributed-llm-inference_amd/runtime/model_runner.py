@@ -513,6 +513,8 @@ class ModelRunner:
             self.stats["mixed_graph_steps"] += 1
             return self._fetch(S)
         meta = self._meta(B, T, nd, n_items, n_reds, n_tiles)
+        if not staged_on_device:
+            meta.max_seq_len = int(self.n_seq_lens[:B].max(initial=0))
         self._maybe_dump(self._forward_sample(T, S, meta))
         self.stats["eager_steps"] += 1
         return self._fetch(S)

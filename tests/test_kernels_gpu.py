@@ -328,10 +328,10 @@ def test_paged_attention_prefill_and_mixed(Hq, Hkv, kv_dtype):
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)
 
 
-@pytest.mark.parametrize("n", [1, 64, 65])                        # 8, 512 and 520 workgroups: two page groups, two, one
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65])                # 8, 256, 264, 512, 520 workgroups: two page groups up to 256, one above
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
-    """Tiles of one page (the second group has none), of an odd and of an even number, with masked last pages; keys whose scores rise by much and
+    """Tiles of one page to seven (one group alone), of an odd and of an even number of more, with masked last pages; keys whose scores rise by much and
     by little along the row.  Weights and results are rounded to bf16 (2^-9 each, |v| ≤ 4.5 here)."""
     Hq = Hkv = 8
     lens = [1, 31, 32, 33, 64, 65, 96, 97, 129, 300]
@@ -353,16 +353,39 @@ def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
     torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -9 * 4.5)
 
 
+@pytest.mark.parametrize("new,ctx,n", [(600, 0, 2), (1300, 300, 1), (1300, 2000, 1)])      # 304 and 328 workgroups: two groups, two, one
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_prefill_long_prompts_in_a_second_round(new, ctx, n, kv_dtype):
+    """Steps whose known lengths choose the page groups past 256 workgroups; the same bits from the form that a step of unknown lengths
+    takes where that is the same one.  Tolerances as above."""
+    Hq, Hkv = 32, 8
+    lens = [new + ctx] * n
+    kc, vc, bt = _fill_cache(Hq, Hkv, lens, kv_dtype, seed=25)
+    qkv = _bf(n * new, (Hq + 2 * Hkv) * 128, seed=26)
+    i32 = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    ts, t0 = ops.build_prefill_tiles(np.full(n, new), 0, ops.prefill_tile_tokens(Hq, Hkv), np.array(lens))
+    out = []
+    for longest in (new + ctx, 0):
+        meta = ops.AttnMetadata(num_decode=0, num_prefill=n, num_tokens=n * new, positions=None, slot_mapping=None, block_tables=bt, seq_lens=i32(lens),
+                                query_start_loc=i32(np.arange(n + 1) * new), max_seq_len=longest, prefill_tile_seq=i32(ts), prefill_tile_q0=i32(t0),
+                                num_prefill_tiles=len(ts))
+        out.append(ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088).float())
+    want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(n * new, Hq, 128), kc, vc, bt, i32(lens), i32(np.arange(n + 1) * new), 0.088).float()
+    for got in out:
+        torch.testing.assert_close(got.view_as(want), want, rtol=2 ** -7, atol=2 ** -8 * 4.5)
+    assert torch.equal(out[0], out[1]) == (ctx == 2000)
+
+
 @pytest.mark.parametrize("n", [1, 65])                            # two page groups and one
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("peak", [7.5, 150.5, 197.5])
 def test_prefill_largest_weight_is_exact(n, kv_dtype, peak):
-    """One key, five pages in, scores log2(peak) above all others, and only its value is not zero: out = v·peak / (peak + others).  A
+    """One key, seven pages in, scores log2(peak) above all others, and only its value is not zero: out = v·peak / (peak + others).  A
     weight taken against the row's maximum is 1 there, so what remains is the rounding of the result (2^-8) and fp32 arithmetic; against a
     maximum of earlier pages it is ``peak``, which bf16 holds only to another 2^-8 (150.5 becomes 150)."""
-    H, L, Q, top = 8, 190, 8, 140
-    kc, vc = _caches(6 * n, H, kv_dtype)
-    bt = torch.randperm(6 * n, generator=torch.Generator().manual_seed(1)).view(n, 6).to(torch.int32)
+    H, L, Q, top = 8, 318, 8, 204
+    kc, vc = _caches(10 * n, H, kv_dtype)
+    bt = torch.randperm(10 * n, generator=torch.Generator().manual_seed(1)).view(n, 10).to(torch.int32)
     k, v = torch.zeros(n * L, H, 128), torch.zeros(n * L, H, 128)
     at = torch.arange(n) * L + top
     k[at, :, 3] = 1.0
