@@ -2,13 +2,14 @@
 //
 // Work items are 8-element (16-byte) chunks: a q/k item owns
 // the pair (x[d0:d0+8], x[d0+64:d0+72]) of one head, so both halves of the rotation are produced by
-// the same thread; cos/sin come from a host-built fp32 table (no device trig), loaded once per (token, chunk) and
-// reused over the heads a thread walks.  Rotated k goes back
+// the same thread; cos/sin come from a host-built fp32 table (no device trig).  Rotated k goes back
 // into the qkv buffer (the prefill kernel reads everything from the cache, but the in-place result
 // keeps the op's semantics testable) and into the K page as one 16-byte store per chunk; v goes into
 // the transposed, slot-permuted V page (layout: ops/kv_layout.py).
 //
 // KV8 = true stores the cache as OCP e4m3 with per-tensor scales (value / scale, saturating).
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -18,12 +19,12 @@ constexpr int D = 128;
 
 __device__ __forceinline__ int v_slot(int t) { return ((t & 15) >> 2) * 8 + (t >> 4) * 4 + (t & 3); }
 
-// q/k of token t by one workgroup: thread = (chunk j of the half-row, head group hg); lanes j = 0..7 of a head cover 128 contiguous
-// bytes, the 8 head groups of a wave 8 such lines: every load and store is whole cache lines.
+// q/k of one token: thread = (chunk j of the half-row, head hg; hg + step, … where a workgroup has fewer threads than that); lanes j = 0..7 of a
+// head cover 128 contiguous bytes, the 8 heads of a wave 8 such lines: every load and store is whole cache lines.
 template <bool KV8>
 __device__ __forceinline__ void turn_heads(uint16_t* row, int pos, const float* cos_sin, int slot, void* k_cache_, int Hq, int Hkv,
-                                           float k_inv_scale_, const float* kv_scales) {
-  const int hg = threadIdx.x >> 3, j = threadIdx.x & 7;
+                                           float k_inv_scale_, const float* kv_scales, int hg, int step) {
+  const int j = threadIdx.x & 7;
   f32x4 c0, c1, s0, s1;
   if (cos_sin != nullptr) {
     const float* cs = cos_sin + (int64_t)pos * D + j * 8;
@@ -32,7 +33,7 @@ __device__ __forceinline__ void turn_heads(uint16_t* row, int pos, const float* 
     s0 = *reinterpret_cast<const f32x4*>(cs + 64);
     s1 = *reinterpret_cast<const f32x4*>(cs + 68);
   }
-  for (int head = hg; head < Hq + Hkv; head += 32) {
+  for (int head = hg; head < Hq + Hkv; head += step) {
     uint16_t* p = row + head * D + j * 8;
     bf16x8 a = *reinterpret_cast<const bf16x8*>(p);
     bf16x8 b = *reinterpret_cast<const bf16x8*>(p + 64);
@@ -102,9 +103,13 @@ __device__ __forceinline__ void put_values(const uint16_t* v, int64_t row_stride
 }
 
 // v_groups == 0 (few tokens: pure latency): workgroup t does everything of token t.  Otherwise workgroups 0 … 8·ceil(v_groups / 8) − 1
-// write the v entries of VT tokens each and the others turn one token's q and k.  Many small workgroups are what the in-place rotation
+// write the v entries of VT tokens each and the others turn the q and k of `per` tokens.  Many small workgroups are what the in-place rotation
 // needs: with four tokens and their v in one, whose loads, stores and loads again wait for each other, 4100 tokens of 32 + 8
-// heads (109 MB) took 33 µs; now 22.6 (VT = 8: 24.5, 16: 26.5), 684 tokens 7.9 → 6.3.
+// heads in five prompts (109 MB) took 33 µs; now 22 (VT = 8: 24.5, 16: 26.5), 740 tokens of twenty 9.6 → 6.6.  A workgroup has a thread for every
+// chunk of its tokens' heads (up to 1024), so that nobody has a second head to wait for and few are idle: with 256 threads for any number of
+// heads 8 + 1 heads of 4096 tokens took 7.4 µs (four tokens a workgroup 6.2; now 6.3), one token of 32 + 8 3.7 → 3.4.  Rows that arrive from memory, one prompt of
+// 4096 tokens, four tokens a workgroup / 256 threads / now: 32 + 8 heads 29.9 / 30.9 / 29.8, 64 + 8 44.3 / 44.4 / 41.9, 2047 tokens 17.0 / 18.0 / 17.4.
+// (Two or four tokens a thread: 5 and 20 % slower.)
 //   v: tokens 4k…4k+3 of a page occupy 4 ADJACENT slots of every d row (v_slot), so a prefill chunk — whose tokens sit in consecutive
 // cache slots — is written with one 8-byte store per (d row, 4 tokens) instead of four 2-byte ones.  The groups of four go by SLOTS: the second
 // prompt of a step starts at any row of the batch (groups of four batch rows left most prompts to 2-byte stores: 21 µs for 16 MB of v).  A
@@ -112,21 +117,21 @@ __device__ __forceinline__ void put_values(const uint16_t* v, int64_t row_stride
 // leaving as partial lines of eight.
 constexpr int VT = 4;
 template <bool KV8>
-__global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ qkv, int64_t row_stride,
+__global__ __launch_bounds__(1024) void rope_cache_kernel(uint16_t* __restrict__ qkv, int64_t row_stride,
                                                          const int* __restrict__ positions,
                                                          const float* __restrict__ cos_sin,  // [max_pos, D] or null
                                                          const int* __restrict__ slot_mapping,
                                                          void* __restrict__ k_cache, void* __restrict__ v_cache,
                                                          int T, int Hq, int Hkv, float k_inv_scale, float v_inv_scale,
                                                          const float* __restrict__ kv_scales,   // [k | v][Hkv] or null
-                                                         int v_groups) {
+                                                         int v_groups, int per) {
   const int v_blocks = (v_groups + 7) & ~7;
   const uint16_t* v0 = qkv + (int64_t)(Hq + Hkv) * D;
   const int vi_count = Hkv * (D / 8);
   if ((int)blockIdx.x < v_blocks) {
     const int grp = (int)(blockIdx.x & 7) * (v_blocks >> 3) + (int)(blockIdx.x >> 3);
     const int t0 = grp * VT;
-    for (int it = threadIdx.x; it < VT * vi_count; it += 256) {
+    for (int it = threadIdx.x; it < VT * vi_count; it += blockDim.x) {
       const int t = t0 + it / vi_count, vi = it % vi_count, h = vi >> 4, d0 = (vi & 15) * 8;
       if (t >= T) break;
       // one token of every run of up to four neighbouring slots inside a group writes for all of them
@@ -147,12 +152,14 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
     }
     return;
   }
-  const int t = (int)blockIdx.x - v_blocks;
-  if (t >= T) return;
+  const int heads = Hq + Hkv, hg = threadIdx.x >> 3, in = per == 1 ? 0 : hg / heads;
+  const int t = ((int)blockIdx.x - v_blocks) * per + in;
+  if (t >= T || in >= per) return;
   const int slot = slot_mapping[t];
-  turn_heads<KV8>(qkv + t * row_stride, positions[t], cos_sin, slot, k_cache, Hq, Hkv, k_inv_scale, kv_scales);
+  turn_heads<KV8>(qkv + t * row_stride, positions[t], cos_sin, slot, k_cache, Hq, Hkv, k_inv_scale, kv_scales, hg - in * heads,
+                  per == 1 ? blockDim.x >> 3 : heads);
   if (v_groups == 0 && slot >= 0)
-    for (int vi = threadIdx.x; vi < vi_count; vi += 256)
+    for (int vi = threadIdx.x; vi < vi_count; vi += blockDim.x)
       put_values<KV8, 1>(v0 + t * row_stride, row_stride, slot, vi >> 4, (vi & 15) * 8, Hkv, v_cache, v_inv_scale, kv_scales);
 }
 
@@ -161,10 +168,12 @@ void launch_rope_and_cache(void* qkv, int64_t row_stride, const int* positions, 
                            bool kv_fp8, float k_scale, float v_scale, const float* kv_scales, hipStream_t stream) {
   if (T == 0) return;
   const int v_groups = T <= 128 ? 0 : (T + VT - 1) / VT;
-  const dim3 grid((v_groups + 7) / 8 * 8 + T);
+  const int chunks = (Hq + Hkv) * 8, per = v_groups == 0 ? 1 : std::max(1, 256 / chunks);
+  const int threads = std::min(1024, (per * chunks + 63) / 64 * 64);
+  const dim3 grid((v_groups + 7) / 8 * 8 + (T + per - 1) / per);
 #define DLI_ROPE(KV8_, ks_, vs_)                                                                                        \
-  hipLaunchKernelGGL((rope_cache_kernel<KV8_>), grid, dim3(256), 0, stream, (uint16_t*)qkv, row_stride, positions, cos_sin, slot_mapping, \
-                     k_cache, v_cache, T, Hq, Hkv, ks_, vs_, kv_fp8 ? kv_scales : nullptr, v_groups)
+  hipLaunchKernelGGL((rope_cache_kernel<KV8_>), grid, dim3(threads), 0, stream, (uint16_t*)qkv, row_stride, positions, cos_sin, slot_mapping, \
+                     k_cache, v_cache, T, Hq, Hkv, ks_, vs_, kv_fp8 ? kv_scales : nullptr, v_groups, per)
   if (kv_fp8) DLI_ROPE(true, 1.f / k_scale, 1.f / v_scale);
   else DLI_ROPE(false, 1.f, 1.f);
 #undef DLI_ROPE

@@ -129,6 +129,23 @@ def test_rope_and_cache_runs_of_slots(T, kv_dtype):
         torch.testing.assert_close(kc.float(), kc_ref.float(), rtol=0.13, atol=0.02)
 
 
+@pytest.mark.parametrize("T", [5, 131])
+@pytest.mark.parametrize("Hq,Hkv", [(128, 8), (1, 1), (40, 1)])     # more heads than a workgroup has threads for, sixteen tokens a workgroup, one
+def test_rope_and_cache_of_other_head_counts(Hq, Hkv, T):
+    slots = (torch.arange(T) + 3).to(torch.int32).to(DEV)
+    qkv = _bf(T, (Hq + 2 * Hkv) * 128, seed=12)
+    pos = (torch.arange(T) * 7).to(torch.int32).to(DEV)
+    cs = ref.build_cos_sin_cache(4096, 128, 500000.0, DEV)
+    kc, vc = _caches(6, Hkv)
+    kc_ref, vc_ref = _caches(6, Hkv)
+    qkv_ref = qkv.clone()
+    ops.rope_and_cache(qkv, pos, cs, slots, kc, vc, Hq, Hkv, 128)
+    ref.rope_and_cache_ref(qkv_ref, pos, cs, slots, kc_ref, vc_ref, Hq, Hkv, 128)
+    torch.testing.assert_close(qkv.float(), qkv_ref.float(), rtol=2 ** -7, atol=2 ** -6)
+    torch.testing.assert_close(kc.float(), kc_ref.float(), rtol=2 ** -7, atol=2 ** -6)
+    assert torch.equal(vc, vc_ref)
+
+
 def test_fp8_cache_write_saturates_instead_of_nan():
     """Values past scale × 448 (activation outliers beyond the calibrated head-room) must store ±448, never the e4m3
     NaN pattern: one NaN key poisons every later softmax of its sequence (found with the 80 req/s fp8 bench)."""
