@@ -48,7 +48,7 @@ void launch_sample(const void* logits, bool logits_fp32, int64_t row_stride, int
                    const float* top_p, const int* top_k, const int64_t* seeds, const int64_t* steps, const float* noise,
                    int64_t* out, void* ws, hipStream_t stream);
 bool sample_by_slices(bool logits_fp32, const void* logits, int64_t row_stride, int B, int V);
-size_t sample_workspace_bytes(int B);
+size_t sample_workspace_bytes(int B, int V);
 
 // mixture of experts (moe.hip)
 void launch_moe_route(const void* logits, int T, int E, int K, int* ids, float* weights, hipStream_t stream);

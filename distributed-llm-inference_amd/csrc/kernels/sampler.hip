@@ -1,4 +1,4 @@
-// K6: temperature / top-k / top-p / multinomial sampling, sort-free (SURVEY.md §2.5).
+// K6: temperature / top-k / top-p / multinomial sampling, sort-free.
 //
 //   * temperature == 0          → arg-max (lowest index on ties).
 //   * top_k == 0 && top_p >= 1  → Gumbel-max draw  argmax_i(x_i / T + g_i) (shift invariant, so neither the row max nor the
@@ -6,7 +6,8 @@
 //   * otherwise                 → a cut-off on the logit instead of a sort, then the Gumbel-max draw over what reaches it.
 //
 // Serving path (bf16 rows of up to 131072 logits, 16-byte aligned): sample_cut_kernel finds the cut-off key of the rows that need
-// one, sample_draw_kernel draws with a row's slices spread over the chip.  Other rows (fp32, unaligned, longer) take
+// one, sample_draw_kernel draws with a row's slices spread over the chip; rows of up to 8192 logits are done by sample_whole_kernel alone.
+// Other rows (fp32, unaligned, longer) take
 // sample_kernel: one 1024-thread workgroup per row, cut-off by a 4-pass radix descent (8 bits per pass, 256-bin LDS histogram of
 // *counts* for top-k, of *probability mass* for top-p).
 // Gumbel noise comes from Philox4x32-10 keyed by the request seed, counter = (element/4, step), so a
@@ -405,33 +406,35 @@ __device__ __forceinline__ void count_logits(uint4 (&regs)[NCH], int nchunks, in
   }
 }
 
-template <int NCH>
-__global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
-                                                         const float* __restrict__ temperature, const float* __restrict__ top_p,
-                                                         const int* __restrict__ top_k, SampleRow* __restrict__ rows) {
-  __shared__ uint32_t counts[2 * MBINS];
-  __shared__ float sv[SNT / 64];
-  __shared__ CutScratch cs;
-  __shared__ uint32_t s_pick;
-  __shared__ float s_rem;
+struct CutShared {
+  uint32_t counts[2 * MBINS];
+  float sv[SNT / 64];
+  CutScratch cs;
+  uint32_t pick;
+  float rem;
+};
 
-  const int b = blockIdx.x;
-  const float temp = temperature[b];
-  const float p = top_p[b];
-  int k = top_k[b];
+// what a row asks for; k is set to V where there is no top-k
+__device__ __forceinline__ bool needs_cut(float temp, float p, int& k, int V) {
   if (k <= 0 || k > V) k = V;
-  if (temp <= 0.f || (k >= V && !(p < 1.f))) {              // nothing to cut
-    if (threadIdx.x == 0) rows[b] = SampleRow{0ull, 0u, 0u};
-    return;
-  }
-  const uint4* row = reinterpret_cast<const uint4*>(logits + (int64_t)b * row_stride);
-  const int nchunks = V >> 3;
-  uint4 regs[NCH];
+  return temp > 0.f && (k < V || p < 1.f);
+}
+
+template <int NCH>
+__device__ __forceinline__ void load_row(uint4 (&regs)[NCH], const uint16_t* logits, int nchunks) {
+  const uint4* row = reinterpret_cast<const uint4*>(logits);
 #pragma clang loop unroll(full)
   for (int c = 0; c < NCH; ++c) {
     const int idx = c * SNT + threadIdx.x;
     regs[c] = idx < nchunks ? row[idx] : make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);   // -inf padding
   }
+}
+
+// smallest 16-bit key that takes part
+template <int NCH>
+__device__ __forceinline__ uint32_t row_cut(uint4 (&regs)[NCH], int nchunks, int V, float temp, float p, int k, CutShared& sh) {
+  uint32_t* counts = sh.counts;
+  float* sv = sh.sv;
   for (int i = threadIdx.x; i < 2 * MBINS; i += SNT) counts[i] = 0u;
 
   const float inv_t_log2 = 1.4426950408889634f / temp;    // z = x / T in log2 units
@@ -464,7 +467,7 @@ __global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restr
     __syncthreads();
     int d = 2 * MBINS - 1;
     if (k < V) {
-      d = scan_cut<false, false>(counts, lo, inv_t_log2, zmax, (float)k, d, &cs);
+      d = scan_cut<false, false>(counts, lo, inv_t_log2, zmax, (float)k, d, &sh.cs);
       if (d < 0) {                                          // among the logits outside the bins, all of them negative: one value?
         const float far_max = block_max((float)far_any, sv), far_min = -block_max(far_any != 0u ? -(float)far_all : -32768.f, sv);
         exact = far_max == far_min;
@@ -476,7 +479,7 @@ __global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restr
       }
     }
     if (exact && p < 1.f) {
-      d = scan_cut<true, true>(counts, lo, inv_t_log2, zmax, p, d, &cs);
+      d = scan_cut<true, true>(counts, lo, inv_t_log2, zmax, p, d, &sh.cs);
       exact = d >= 0 && !(lo > 0 && (d == MBINS - 1 || d == MBINS));
       floor_key = d < MBINS ? 0x8000u | (uint32_t)(MBINS - 1 - d + lo) : 0x7FFFu - (uint32_t)(d - MBINS + lo);
     }
@@ -484,7 +487,7 @@ __global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restr
   if (!exact) {
     floor_key = 0;
     float* hist = reinterpret_cast<float*>(counts);
-    if (k < V) floor_key = radix_cut16<NCH, false>(regs, inv_t_log2, zmax, (float)k, 0u, hist, &s_pick, &s_rem);
+    if (k < V) floor_key = radix_cut16<NCH, false>(regs, inv_t_log2, zmax, (float)k, 0u, hist, &sh.pick, &sh.rem);
     if (p < 1.f) {
       float tot = 0.f;                                     // mass of what survived top-k
       opaque(regs);
@@ -503,22 +506,111 @@ __global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restr
       tot = 0.f;
       for (int w = 0; w < SNT / 64; ++w) tot += sv[w];
       __syncthreads();
-      floor_key = radix_cut16<NCH, true>(regs, inv_t_log2, zmax, p * tot, floor_key, hist, &s_pick, &s_rem);
+      floor_key = radix_cut16<NCH, true>(regs, inv_t_log2, zmax, p * tot, floor_key, hist, &sh.pick, &sh.rem);
     }
   }
-  if (threadIdx.x == 0) rows[b] = SampleRow{0ull, floor_key, 0u};
+  return floor_key;
 }
 
-// ---- draw.  Grid (slices, B): a 256-thread workgroup takes 256 · NC chunks of 8 logits.  Its best candidate goes into the row's
+// ---- draw.  The Philox counter of element i is i/4 exactly as in sample_kernel: all paths draw the same token.
+struct DrawArgs {
+  const int64_t *seeds, *steps;
+  const float* noise;
+};
+__device__ __forceinline__ ArgMax no_candidate() { return ArgMax{-3.0e38f, 0x7fffffff}; }
+__device__ __forceinline__ void greedy_chunk(const uint4& x, int chunk, ArgMax& a) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a = amax(a, ArgMax{bf2f((uint16_t)half_of(x, e)), chunk * 8 + e});
+}
+__device__ __forceinline__ void draw_chunk(const uint4& x, int chunk, float inv_t_log2, uint32_t floor_key, uint2 key, uint64_t step,
+                                           const float* noise_row, ArgMax& a) {
+  const float ln2 = 0.6931471805599453f;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    bool any = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) any = any || okey16(half_of(x, half * 4 + e)) >= floor_key;
+    if (!any) continue;                                    // behind a cut-off most groups of four draw nothing
+    const int i4 = chunk * 2 + half;
+    uint4 r = make_uint4(0, 0, 0, 0);
+    if (noise_row == nullptr) r = philox4x32_10(make_uint4((uint32_t)i4, (uint32_t)step, (uint32_t)(step >> 32), 0x5A17u), key);
+    const uint32_t rr[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t h = half_of(x, half * 4 + e);
+      if (okey16(h) >= floor_key) {
+        const float u = noise_row != nullptr ? noise_row[i4 * 4 + e] : u01(rr[e]);
+        a = amax(a, ArgMax{bf2f((uint16_t)h) * inv_t_log2 * ln2 + gumbel(u), i4 * 4 + e});
+      }
+    }
+  }
+}
+// a thread's best of chunks first, first + stride, …
+template <int NC>
+__device__ __forceinline__ ArgMax best_of(uint4 (&regs)[NC], int first, int stride, int nchunks, int V, float temp, uint32_t floor_key, int b,
+                                          const DrawArgs& draw) {
+  ArgMax a = no_candidate();
+  if (temp <= 0.f) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (first + c * stride < nchunks) greedy_chunk(regs[c], first + c * stride, a);
+    return a;
+  }
+  const uint64_t seed = (uint64_t)draw.seeds[b], step = (uint64_t)draw.steps[b];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if (first + c * stride < nchunks)
+      draw_chunk(regs[c], first + c * stride, 1.4426950408889634f / temp, floor_key, make_uint2((uint32_t)seed, (uint32_t)(seed >> 32)), step,
+                 draw.noise != nullptr ? draw.noise + (int64_t)b * V : nullptr, a);
+  }
+  return a;
+}
+// Rows of up to 8192 logits: a workgroup each, from the logits to the token in one launch.  V = 2048, one row, µs, two launches / one: greedy 6.5 / 4.6,
+// plain 8.1 / 5.7, top-p 11.2 / 8.9.  (Rows of 32000 logits would take 17 µs for a plain draw, 8.8 in slices; 512 of them 34 and 31.5.)
+__global__ __launch_bounds__(SNT) void sample_whole_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
+                                                           const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                           const int* __restrict__ top_k, DrawArgs draw, int64_t* __restrict__ out) {
+  __shared__ CutShared sh;
+  __shared__ int si[SNT / 64];
+  const int b = blockIdx.x, nchunks = V >> 3;
+  const float temp = temperature[b], p = top_p[b];
+  int k = top_k[b];
+  uint4 regs[1];
+  load_row<1>(regs, logits + (int64_t)b * row_stride, nchunks);
+  uint32_t floor_key = 0;
+  if (needs_cut(temp, p, k, V)) floor_key = row_cut<1>(regs, nchunks, V, temp, p, k, sh);
+  const ArgMax a = block_argmax(best_of<1>(regs, threadIdx.x, SNT, nchunks, V, temp, floor_key, b, draw), sh.sv, si);
+  if (threadIdx.x == 0) out[b] = valid_token(a.i, V);
+}
+
+// Longer rows take two launches, the first of which only clears the words of a row without cut-off.  (That is 1 µs of a greedy row of 32000 logits, 6.7
+// instead of the 5.7 of a workgroup a row, which takes 12.1 instead of 7.2 for 128256.  Slices of these rows in the first launch, with no
+// words to clear, have the cut-off's registers and LDS and so one workgroup a compute unit: 57 greedy rows of 128256 17 instead of 10.8.)
+template <int NCH>
+__global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
+                                                         const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                         const int* __restrict__ top_k, SampleRow* __restrict__ rows) {
+  __shared__ CutShared sh;
+  const int b = blockIdx.x, nchunks = V >> 3;
+  const float temp = temperature[b], p = top_p[b];
+  int k = top_k[b];
+  uint32_t cut = 0;
+  if (needs_cut(temp, p, k, V)) {
+    uint4 regs[NCH];
+    load_row<NCH>(regs, logits + (int64_t)b * row_stride, nchunks);
+    cut = row_cut<NCH>(regs, nchunks, V, temp, p, k, sh);
+  }
+  if (threadIdx.x == 0) rows[b] = SampleRow{0ull, cut, 0u};
+}
+
+// Grid (slices, B): a 256-thread workgroup takes 256 · NC chunks of 8 logits.  Its best candidate goes into the row's
 // 64-bit maximum (value in the order-preserving 32 bits, then the lowest index); the slice that delivers last reads the result.
-// The Philox counter of element i is i/4 exactly as in sample_kernel: both paths draw the same token.  V = 128256, a quarter of the rows
-// without cut-off: 12 µs at B = 57, 20 at 120.
+// V = 128256, a quarter of the rows without cut-off: 12 µs at B = 57, 20 at 120.
 constexpr int DNT = 256;
 template <int NC>
 __global__ __launch_bounds__(DNT) void sample_draw_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,
-                                                          const float* __restrict__ temperature, const int64_t* __restrict__ seeds,
-                                                          const int64_t* __restrict__ steps, const float* __restrict__ noise,
-                                                          SampleRow* __restrict__ rows, int64_t* __restrict__ out) {
+                                                          const float* __restrict__ temperature, DrawArgs draw, SampleRow* __restrict__ rows,
+                                                          int64_t* __restrict__ out) {
   __shared__ ArgMax sa[DNT / 64];
   const int b = blockIdx.y;
   const uint4* row = reinterpret_cast<const uint4*>(logits + (int64_t)b * row_stride);
@@ -527,48 +619,7 @@ __global__ __launch_bounds__(DNT) void sample_draw_kernel(const uint16_t* __rest
 #pragma unroll
   for (int c = 0; c < NC; ++c) regs[c] = first + c * DNT < nchunks ? row[first + c * DNT] : make_uint4(0, 0, 0, 0);
   const float temp = temperature[b];
-  ArgMax a{-3.0e38f, 0x7fffffff};
-  if (temp <= 0.f) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if (first + c * DNT < nchunks) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a = amax(a, ArgMax{bf2f((uint16_t)half_of(regs[c], e)), (first + c * DNT) * 8 + e});
-      }
-    }
-  } else {
-    const float inv_t_log2 = 1.4426950408889634f / temp;
-    const float ln2 = 0.6931471805599453f;
-    const uint32_t floor_key = rows[b].cut;
-    const uint64_t seed = (uint64_t)seeds[b];
-    const uint64_t step = (uint64_t)steps[b];
-    const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int chunk = first + c * DNT;
-      if (chunk >= nchunks) break;
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        bool any = false;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) any = any || okey16(half_of(regs[c], half * 4 + e)) >= floor_key;
-        if (!any) continue;                                // behind a cut-off most groups of four draw nothing
-        const int i4 = chunk * 2 + half;
-        uint4 r = make_uint4(0, 0, 0, 0);
-        if (noise == nullptr) r = philox4x32_10(make_uint4((uint32_t)i4, (uint32_t)step, (uint32_t)(step >> 32), 0x5A17u), key);
-        const uint32_t rr[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t h = half_of(regs[c], half * 4 + e);
-          if (okey16(h) >= floor_key) {
-            const int i = i4 * 4 + e;
-            const float u = noise != nullptr ? noise[(int64_t)b * V + i] : u01(rr[e]);
-            a = amax(a, ArgMax{bf2f((uint16_t)h) * inv_t_log2 * ln2 + gumbel(u), i});
-          }
-        }
-      }
-    }
-  }
+  ArgMax a = best_of<NC>(regs, first, DNT, nchunks, V, temp, temp <= 0.f ? 0u : rows[b].cut, b, draw);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) a = amax(a, ArgMax{__shfl_xor(a.v, o, 64), __shfl_xor(a.i, o, 64)});
   if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
@@ -597,34 +648,40 @@ bool sample_by_slices(bool logits_fp32, const void* logits, int64_t row_stride, 
          B <= 65535;
 }
 
-size_t sample_workspace_bytes(int B) { return (size_t)B * sizeof(SampleRow); }
+static bool sample_whole(int V) { return V <= SNT * 8; }
+size_t sample_workspace_bytes(int B, int V) { return sample_whole(V) ? 0 : (size_t)B * sizeof(SampleRow); }
 
-// `ws`: sample_workspace_bytes(B) where sample_by_slices says so (contents do not matter), else not read.
+// `ws`: sample_workspace_bytes where sample_by_slices says so (contents do not matter), else not read.
 void launch_sample(const void* logits, bool logits_fp32, int64_t row_stride, int B, int V, const float* temperature,
                    const float* top_p, const int* top_k, const int64_t* seeds, const int64_t* steps, const float* noise,
                    int64_t* out, void* ws, hipStream_t stream) {
   if (B == 0) return;
-  if (sample_by_slices(logits_fp32, logits, row_stride, B, V)) {
-    const uint16_t* x = (const uint16_t*)logits;
-    SampleRow* rows = (SampleRow*)ws;
-    if (V <= 4 * SNT * 8)
-      hipLaunchKernelGGL(sample_cut_kernel<4>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
+  if (!sample_by_slices(logits_fp32, logits, row_stride, B, V)) {
+    if (logits_fp32)
+      hipLaunchKernelGGL(sample_kernel<float>, dim3(B), dim3(SNT), 0, stream, (const float*)logits, row_stride, V,
+                         temperature, top_p, top_k, seeds, steps, noise, out);
     else
-      hipLaunchKernelGGL(sample_cut_kernel<16>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
-    // slices of 8192 logits where they keep all compute units busy several times over (half the atomics), of 2048 below: B = 57 18 → 16 µs
-    const int wide = (V / 8 + DNT * 4 - 1) / (DNT * 4);
-    if ((int64_t)wide * B >= 2048)
-      hipLaunchKernelGGL(sample_draw_kernel<4>, dim3(wide, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, seeds, steps, noise, rows, out);
-    else
-      hipLaunchKernelGGL(sample_draw_kernel<1>, dim3((V / 8 + DNT - 1) / DNT, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, seeds,
-                         steps, noise, rows, out);
-  } else if (logits_fp32) {
-    hipLaunchKernelGGL(sample_kernel<float>, dim3(B), dim3(SNT), 0, stream, (const float*)logits, row_stride, V,
-                       temperature, top_p, top_k, seeds, steps, noise, out);
-  } else {
-    hipLaunchKernelGGL(sample_kernel<uint16_t>, dim3(B), dim3(SNT), 0, stream, (const uint16_t*)logits, row_stride, V,
-                       temperature, top_p, top_k, seeds, steps, noise, out);
+      hipLaunchKernelGGL(sample_kernel<uint16_t>, dim3(B), dim3(SNT), 0, stream, (const uint16_t*)logits, row_stride, V,
+                         temperature, top_p, top_k, seeds, steps, noise, out);
+    return;
   }
+  const uint16_t* x = (const uint16_t*)logits;
+  const DrawArgs draw{seeds, steps, noise};
+  if (sample_whole(V)) {
+    hipLaunchKernelGGL(sample_whole_kernel, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, draw, out);
+    return;
+  }
+  SampleRow* rows = (SampleRow*)ws;
+  if (V <= 4 * SNT * 8)
+    hipLaunchKernelGGL(sample_cut_kernel<4>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
+  else
+    hipLaunchKernelGGL(sample_cut_kernel<16>, dim3(B), dim3(SNT), 0, stream, x, row_stride, V, temperature, top_p, top_k, rows);
+  // slices of 8192 logits where they keep all compute units busy several times over (half the atomics), of 2048 below: B = 57 18 → 16 µs
+  const int wide = (V / 8 + DNT * 4 - 1) / (DNT * 4);
+  if ((int64_t)wide * B >= 2048)
+    hipLaunchKernelGGL(sample_draw_kernel<4>, dim3(wide, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, draw, rows, out);
+  else
+    hipLaunchKernelGGL(sample_draw_kernel<1>, dim3((V / 8 + DNT - 1) / DNT, B), dim3(DNT), 0, stream, x, row_stride, V, temperature, draw, rows, out);
 }
 
 // Pipelined stepping: a decode row whose input id was sampled by the step still in flight reads it from the

@@ -284,7 +284,7 @@ void sample(Tensor out, const Tensor& logits, const Tensor& temperature, const T
   const bool fp32 = logits.scalar_type() == at::kFloat;
   Tensor ws;
   if (dli::sample_by_slices(fp32, logits.data_ptr(), logits.stride(0), (int)B, (int)V))
-    ws = at::empty({(int64_t)dli::sample_workspace_bytes((int)B)}, logits.options().dtype(at::kByte));
+    ws = at::empty({(int64_t)dli::sample_workspace_bytes((int)B, (int)V)}, logits.options().dtype(at::kByte));
   dli::launch_sample(logits.data_ptr(), fp32, logits.stride(0), (int)B, (int)V,
                      temperature.data_ptr<float>(), top_p.data_ptr<float>(), top_k.data_ptr<int>(), seeds.data_ptr<int64_t>(),
                      steps.data_ptr<int64_t>(), nz, out.data_ptr<int64_t>(), ws.defined() ? ws.data_ptr() : nullptr, cur_stream(logits));

@@ -446,9 +446,10 @@ def test_sampler_matches_reference_with_shared_noise(V, dtype):
     assert agree >= rounds * B - 2, f"only {agree}/{rounds * B} draws agree with the reference"
 
 
-@pytest.mark.parametrize("B,V", [(1, 8), (7, 2040), (24, 2056), (12, 32768), (12, 32776), (64, 65536), (12, 131064)])
+@pytest.mark.parametrize("B,V", [(1, 8), (7, 2040), (24, 2056), (12, 32768), (12, 32776), (64, 65536), (12, 131064),
+                                 (9, 8192), (9, 8200), (256, 8200), (257, 32768), (520, 32776)])
 def test_sampler_slices_draw_what_the_row_kernel_draws(B, V):
-    """bf16 rows (histogram cut-off, slices of a row over the chip) against the same values in fp32 (one workgroup per row, radix
+    """bf16 rows (histogram cut-off, slices of a row over the chip or a workgroup a row) against the same values in fp32 (one workgroup per row, radix
     descent): the formulas of value and noise are the same, so every id is — nothing but a nucleus boundary within rounding of ``p``
     (~1e-6 of the mass) could differ.  Rows that are hard for the histogram among them: equal logits, signed zeros, masked tokens, a
     cut-off among values 33 octaves below the largest, an infinity."""
