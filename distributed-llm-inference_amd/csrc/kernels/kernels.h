@@ -215,6 +215,7 @@ void launch_hm_softmax_route(const void* h, bool bf16, int64_t h_stride, const f
                              int W, int* ids, float* wts, bool all, hipStream_t stream);
 // gated linear recurrences and gated latent attention (recurmix.hip)
 int rm_max_taps();
+bool rm_conv_by_runs(int rows, int C);
 void launch_rm_causal_conv(const void* x, bool bf16, int64_t x_stride, const float* w, const float* bias, int taps, float* state,
                            const int* positions, const int* token_seq, const int* qsl, const int* state_slots, const int* counts,
                            int rows, int seqs, int C, void* out, bool out_bf16, bool silu, int unit_n, int unit_d, int unit_scaled,

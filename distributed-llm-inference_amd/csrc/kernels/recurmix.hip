@@ -732,6 +732,11 @@ int rm_max_taps() { return RM_MAX_TAPS; }
 
 static bool al16(const void* p) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+// One workgroup per token in small steps, where its four times as many workgroups matter more than their bytes.  4096 / 8192 channels, µs, a token /
+// a run each: 128 rows 7.1 / 6.9 and 11.0 / 7.8, 256 10.2 / 7.3 and 14.7 / 11.1, 1200 20.1 / 14.4 and 32.1 / 20.7; 17 rows 6.8 / 6.9.  Fewer channels
+// need more rows: 2304 × 200 rows 6.9 / 6.8, 1024 × 200 6.4 / 6.8, × 700 7.0 / 6.9, 256 × 700 6.3 / 6.4, × 1232 6.7 / 7.0, × 2000 7.0 / 6.6.
+bool rm_conv_by_runs(int rows, int C) { return rows >= 128 && (int64_t)rows * C >= 3 << 17; }
+
 void launch_rm_causal_conv(const void* x, bool bf16, int64_t x_stride, const float* w, const float* bias, int taps, float* state,
                            const int* positions, const int* token_seq, const int* qsl, const int* state_slots, const int* counts,
                            int rows, int seqs, int C, void* out, bool out_bf16, bool silu, int unit_n, int unit_d, int unit_scaled,
@@ -750,11 +755,9 @@ void launch_rm_causal_conv(const void* x, bool bf16, int64_t x_stride, const flo
                                                            (GateArgs<A>{gate_kind, gate_heads, (const A*)gate, gate_rate, gate_bias,  \
                                                                         decay, weight}), span)))
   const bool wide = C % 4 == 0 && nu % 4 == 0 && x_stride % 4 == 0 && al16(x) && al16(w) && al16(bias) && al16(state) && al16(out);
-  // One workgroup per token below 128 rows, where its four times as many workgroups matter more than their bytes: 4096 / 8192 channels, µs, a token /
-  // a run each: 128 rows 7.1 / 6.9 and 11.0 / 7.8, 256 10.2 / 7.3 and 14.7 / 11.1, 1200 20.1 / 14.4 and 32.1 / 20.7; 17 rows 6.8 / 6.9.  Steps of
-  // single tokens only (no chunks) read four state rows a token whatever the split.
+  // Steps of single tokens only (no chunks) read four state rows a token whatever the split.
   const bool vectors_in_lanes = nu == 0 || (unit_d >= 4 && unit_d <= 256 && (unit_d & (unit_d - 1)) == 0);
-  if (wide && taps == 4 && chunks && rows >= 128 && vectors_in_lanes)
+  if (wide && taps == 4 && chunks && rm_conv_by_runs(rows, C) && vectors_in_lanes)
     RM_BF16(bf16, A, RM_BF16(out_bf16, O, hipLaunchKernelGGL((causal_conv_run_kernel<A, O>), dim3((rows + RUN - 1) / RUN, (C + 4 * NT - 1) / (4 * NT)), dim3(NT), 0,
                                                              stream, (const A*)x, x_stride, w, bias, state, positions, token_seq, qsl,
                                                              state_slots, C, rows, (O*)out, silu ? 1 : 0, unit,

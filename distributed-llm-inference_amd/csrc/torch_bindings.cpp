@@ -786,6 +786,7 @@ TORCH_LIBRARY(dli, m) {
   m.def("paged_attention_prefill(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor seq_lens, "
         "Tensor query_start_loc, Tensor tile_seq, Tensor tile_q0, int num_tiles, int num_heads, int num_kv_heads, float scale, "
         "float k_scale, float v_scale, Tensor? kv_scales=None, Tensor? counts=None, int longest=0, int sequences=0) -> ()", &paged_attention_prefill);
+  m.def("rm_conv_by_runs(int rows, int channels) -> bool", [](int64_t rows, int64_t c) -> bool { return dli::rm_conv_by_runs((int)rows, (int)c); });
   m.def("prefill_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences) -> int",
         [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s) -> int64_t { return dli::prefill_page_groups((int)t, (int)h, (int)g, (int)l, (int)s); });
   m.def("paged_attention_decode_worklist(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "

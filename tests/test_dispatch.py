@@ -122,6 +122,13 @@ def test_prefill_page_groups(new, ctx, n, G, groups):
     assert rule(tiles, heads, G, 0, 0) == (2 if tiles * heads <= 256 else 1)        # lengths not known
 
 
+def test_convolution_runs_where_they_fill_the_chip():
+    """Sizes timed with a workgroup a token and a workgroup a run of tokens: a step of few channels needs more rows."""
+    by_runs = ops.hip().rm_conv_by_runs
+    assert all(by_runs(*size) for size in ((128, 4096), (200, 2304), (700, 1024), (2000, 256), (3162, 16384), (128, 3072)))
+    assert not any(by_runs(*size) for size in ((127, 8192), (17, 16384), (200, 1024), (1232, 256), (128, 3068)))
+
+
 def test_plain_tensors():
     import torch.autograd.forward_ad as fw
     t, seen = torch.zeros(4, 4), []

@@ -159,7 +159,9 @@ def test_scan_kernels_against_the_reference(delta, normaliser, H, G, D, Dv, dtyp
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lens,C,unit,gate", [([1, 1, 2, 3, 5, 500], 4 * 1024 + 128, (6, 128, 3, 0.5), "delta"), ([600, 1, 7, 8, 9, 1], 1020, (255, 4, 9, 2.0), "ssd"),
-                                              ([1, 700], 768, (3, 256, 1, 0.25), "beta"), ([121, 3], 64, None, None), ([122, 3], 512, (2, 128, 1, 1.0), "delta")])
+                                              ([1, 700], 768, (3, 256, 1, 0.25), "beta"), ([121, 3], 64, None, None), ([122, 3], 512, (2, 128, 1, 1.0), "delta"),
+                                              ([122, 3], 3072, (2, 128, 1, 1.0), "delta"), ([121, 3], 3072, None, None), ([122, 3], 3068, None, "ssd"),
+                                              ([3, 6138], 64, None, None)])
 def test_convolution_runs_against_the_reference(lens, C, unit, gate, dtype):
     """Four taps over sequences that begin, end and are single tokens anywhere in a run of tokens, chunks at positions 0 … 3 and later, three
     padding rows, channels past the last whole workgroup, vectors of one to 64 lanes, 127 and 128 rows.  Two steps, so that the
