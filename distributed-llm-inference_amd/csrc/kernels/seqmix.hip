@@ -1097,14 +1097,17 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
     mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
     // the maximum that a query's weights refer to moves only when a page passes it by more than 2^8 (for some query of the wave; then
     // each takes its own): fp32 sums and the weights' head and remainder hold 2^8 as well, and most pages rescale nothing
-    // (Sizes below the bounds rescale each time: with their conditions per step the branch costs registers that they do not have.)
+    // (Sizes below the bounds rescale each time, each tile in front of its products: all tiles ahead of them cost a 320-wide page the
+    // products of tiles that it does not have, 200 tokens of 8 heads 44.2 instead of 41.8 µs, and a branch registers that they do not have.)
+    float corr = 1.f;
     if (!FULL || __any(mx > m + 8.f)) {
       const float mn = fmaxf(m, mx);
-      const float corr = fast_exp2(m - (mn == -INFINITY ? 0.f : mn));
+      corr = fast_exp2(m - (mn == -INFINITY ? 0.f : mn));
       m = mn;
       l *= corr;
+      if (FULL)
 #pragma unroll
-      for (int i = 0; i < MTMAX; ++i) acc[i] *= corr;
+        for (int i = 0; i < MTMAX; ++i) acc[i] *= corr;
     }
     const float mu = m == -INFINITY ? 0.f : m;            // nothing visible yet: keep everything at zero
     bf16x8 ph, plo;
@@ -1123,7 +1126,9 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
       if (i < MT) {
         const bf16x4* vp = reinterpret_cast<const bf16x4*>(Vt + at + (16 * i + c) * VST + 8 * g4);
         const bf16x8 vf = __builtin_shufflevector(vp[0], vp[1], 0, 1, 2, 3, 4, 5, 6, 7);
-        acc[i] = mfma16(vf, plo, mfma16(vf, ph, acc[i]));
+        f32x4 a = acc[i];
+        if (!FULL) a *= corr;
+        acc[i] = mfma16(vf, plo, mfma16(vf, ph, a));
       }
     }
     if constexpr (PREF) lds_barrier();                    // everyone is done with this page and has put the next one
