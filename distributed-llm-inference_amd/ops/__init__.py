@@ -273,18 +273,33 @@ def stream_rows_ok(m: int, n: int, k: int, swiglu: bool = False) -> bool:
     * up to 6144: always (4096 × 14336 at 96 rows 63 / 34, 3072 × 12288 at 64 35 / 24), but exactly 64 MiB only past 32 rows (4096 × 8192 at
       17 rows 16.9 / 19.1, at 48 22.3 / 21.0);
     * up to 10240, in two row tiles up to 8192: from 112 MiB (8192 × 8192 at 64 rows 32.7 / 31.4, at 128 48 / 39), with less where the library needs an
-      activation pass or falls off (8192 × 4096 at 40 rows 17.8 / 19.8, with SwiGLU at 48 20.7 / 19.7, at 192 rows 34.0 / 28.8);
+      activation pass or falls off (8192 × 4096 at 40 rows 17.8 / 19.8, with SwiGLU at 48 20.7 / 19.7);
+    * two row tiles of less than 112 MiB, from 5120 columns on: the library falls off at whole 32 rows (8192 × 4096 at 192 34.4 / 30.9, 193 28.4 /
+      31.1, 208 29.7 / 31.9, 224 38.6 / 32.4, 248 31.3 / 33.6, 256 41.0 / 33.6; 6144 × 5632 at 176 35.0 / 33.5, 193 33.8 / 34.9, 224 49.0 / 37.7),
+      an activation pass decides for the tiles above 64 MiB (8192 × 4608 at 129 31.9 / 30.5; 8192 × 4096 at 129 28.4 / 29.2, 160 32.3 / 29.8);
     * up to 16384: never — two K slices or half the chip (16384 × 2048 at 128 rows 20.6 / 28.3, 12288 × 4096 31.2 / 35.0, 14336 × 4096 33.4 / 37.7);
-    * more: no slices; up to 64 rows two workgroups a unit (17408 × 4096 at 17 36.4 / 29.6, at 64 40.5 / 37.3), up to 128 where the columns fill
+    * up to 32768: no slices; up to 64 rows two workgroups a unit (17408 × 4096 at 17 36.4 / 29.6, at 64 40.5 / 37.3), up to 128 where the columns fill
       three quarters of the units (28672 × 2048 32.0 / 30.9; 20480 × 3072 34.2 / 39.1) or the library needs its activation pass (22016 × 4096
-      49.8 / 46.2); not in two row tiles (28672 × 4096 at 192 rows 66 / 77)."""
+      49.8 / 46.2); not in two row tiles (28672 × 4096 at 192 rows 66 / 77);
+    * more column tiles than units, so a last round that may be nearly empty.  Rows of a whole 4 KiB, which slow the library down: up to 64 rows (36864 × 4096
+      at 64 77.2 / 71.7), up to 128 where the rounds are two thirds full (45056 × 4096 94.1 / 93.7, 36864 × 4096 79.0 / 89.6).  Others: where they are
+      nine tenths full (36864 × 7168 at 17 107.6 / 113.3, 57344 × 7168 at 64 145 / 147), past 64 rows only from three rounds on (65536 × 5120 at 96
+      124 / 139, 98304 × 7168 265 / 251)."""
     if not (0 < m <= 256 and n % 128 == 0 and k % 64 == 0 and n * k >= 1 << 25):
         return False
+    large = n * k >= 7 << 23
     if n <= 6144:
-        return m > 32 or n * k > 1 << 25
+        return (m > 32 or n * k > 1 << 25) and (n <= 5120 or m <= 192 or swiglu or large or m % 32 == 0)
     if n <= (10240 if m <= 128 else 8192):
-        return swiglu or m >= 192 or n * k >= 7 << 23
-    return n > 16384 and (m <= 64 or (m <= 128 and (swiglu or n >= 24576)))
+        if swiglu:
+            return m <= 128 or m >= 192 or n * k > 1 << 25 or m % 32 == 0
+        return large or (m >= 192 and m % 32 == 0)
+    if n <= 32768:
+        return n > 16384 and (m <= 64 or (m <= 128 and (swiglu or n >= 24576)))
+    blocks, rounds = n // 128, (n // 128 + 255) // 256
+    if k % 2048 == 0:
+        return m <= 64 or (m <= 128 and 3 * blocks >= 512 * rounds)
+    return 10 * blocks >= 2304 * rounds and (m <= 64 or (m <= 128 and rounds > 2))
 
 
 def _plain(*tensors: torch.Tensor) -> bool:

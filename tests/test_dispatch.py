@@ -40,16 +40,29 @@ def test_expert_row_tiles_by_rows_and_by_choice(hidden):
 @pytest.mark.parametrize("n,k,plain,swiglu", [
     # rows 17, 32, 33, 64, 65, 128, 129, 192, 256, 257; 1: the streaming tiles
     (4096, 14336, "1111111110", "1111111110"), (4096, 8192, "0011111110", "0011111110"), (6144, 6144, "1111111110", "1111111110"),
-    (6144, 4096, "0000000000", "0000000000"), (8192, 4096, "0000000110", "1111111110"), (8192, 8192, "1111111110", "1111111110"),
+    (6144, 4096, "0000000000", "0000000000"), (8192, 4096, "0000000110", "1111110110"), (8192, 8192, "1111111110", "1111111110"),
     (10240, 4096, "0000000000", "1111110000"), (10240, 8192, "1111110000", "1111110000"), (12288, 4096, "0000000000", "0000000000"),
     (16384, 4096, "0000000000", "0000000000"), (16512, 4096, "1111000000", "1111110000"), (24576, 2048, "1111110000", "1111110000"),
     (128256, 4096, "1111110000", "1111110000"), (8192, 28672, "1111111110", "1111111110"), (4097, 14336, "0000000000", "0000000000"),
-    (4096, 14400, "1111111110", "1111111110"), (4096, 14337, "0000000000", "0000000000")])
+    (4096, 14400, "1111111110", "1111111110"), (4096, 14337, "0000000000", "0000000000"), (36864, 4096, "1111000000", "1111000000"),
+    (45056, 4096, "1111110000", "1111110000"), (36864, 7168, "0000000000", "0000000000"), (57344, 8192, "1111110000", "1111110000"),
+    (65536, 5120, "1111000000", "1111000000"), (73728, 7168, "0000000000", "0000000000"), (98304, 7168, "1111110000", "1111110000"),
+    (32768, 5120, "1111110000", "1111110000")])
 def test_shapes_of_the_streaming_tiles(n, k, plain, swiglu):
     rows = (17, 32, 33, 64, 65, 128, 129, 192, 256, 257)
     assert "".join(str(int(ops.stream_rows_ok(m, n, k))) for m in rows) == plain
     assert "".join(str(int(ops.stream_rows_ok(m, n, k, True))) for m in rows) == swiglu
     assert not ops.stream_rows_ok(0, n, k)
+
+
+@pytest.mark.parametrize("n,k,plain,swiglu", [
+    # rows 144, 160, 193, 208, 224, 248: two row tiles, where the library is slow at whole 32 rows
+    (8192, 4096, "000010", "011111"), (8192, 4608, "000010", "111111"), (6144, 5632, "110010", "111111"), (5120, 7168, "111111", "111111"),
+    (8192, 7168, "111111", "111111"), (6144, 16384, "111111", "111111"), (4096, 8192, "111111", "111111"), (10240, 8192, "000000", "000000")])
+def test_shapes_of_the_streaming_tiles_in_two_row_tiles(n, k, plain, swiglu):
+    rows = (144, 160, 193, 208, 224, 248)
+    assert "".join(str(int(ops.stream_rows_ok(m, n, k))) for m in rows) == plain
+    assert "".join(str(int(ops.stream_rows_ok(m, n, k, True))) for m in rows) == swiglu
 
 
 class _Recorder:
