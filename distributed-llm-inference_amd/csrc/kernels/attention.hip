@@ -399,7 +399,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens,
     const int* __restrict__ query_start_loc, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     uint16_t* __restrict__ out, int64_t out_stride, int Hq, int Hkv, int num_tiles, float scale_log2, float v_scale,
-    const float* __restrict__ kv_scales, const int* __restrict__ counts) {
+    const float* __restrict__ kv_scales, const int* __restrict__ counts, int units) {
   // inside a hipGraph the grid is an upper bound and the step's tile count lives in device memory (counts[2])
   if (counts != nullptr) num_tiles = counts[2];
   constexpr int ESZ = KV8 ? 1 : 2;
@@ -415,15 +415,19 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   // kv heads XCD x serves head x — a sequence's pages of that head are fetched into one L2 instead of eight —, with 2 or 4 every XCD
   // serves one head too, and every XCD gets the same mix of long and short tiles (a contiguous eighth of one head's tiles, longest
   // first, would leave most XCDs waiting for the first).
-  const int id = (int)blockIdx.x;
-  if (id >= num_tiles * Hkv) return;
-  const int kvh = id % Hkv, rank = id / Hkv;
   const int G = Hq / Hkv;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: LDS-DMA destinations and the wave's page bounds in SGPRs
   const int wave = wave_all & 3, grp = GROUPS == 2 ? wave_all >> 2 : 0;
   char* smem = smem_all + grp * RING;
   const int c32 = lane & 31, hi = lane >> 5;
+  // Two groups and more tiles than `units` workgroups: what is left over, the shortest tiles, goes to the second groups of the last workgroups, whose
+  // two groups then do a tile each; the longest tiles keep both.
+  const int items = num_tiles * Hkv, over = GROUPS == 2 ? max(items - units, 0) : 0;
+  if ((int)blockIdx.x >= items - over) return;
+  const bool alone = GROUPS == 2 && (int)blockIdx.x >= units - over;
+  const int id = (int)blockIdx.x + (alone ? grp * over : 0);
+  const int kvh = id % Hkv, rank = id / Hkv;
   const int tile_id = num_tiles - 1 - rank;
   if (KV8 && kv_scales != nullptr) {
     scale_log2 *= kv_scales[kvh];
@@ -456,10 +460,12 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   // A tile of a few pages is done by one group alone, the other ends here (a barrier waits for the waves that are left): meeting at the end
   // costs as much as a turn of four pages less saves (prompts of 64 tokens, µs, two groups / one / now 8.25 / 7.28 / 7.4, of 160 10.4 / 9.7 / 9.8,
   // of 256 12.0 / 12.3 / 12.2).
-  const bool both = GROUPS == 2 && nblk > 7;
-  if (GROUPS == 2 && !both && grp == 1) return;
-  const int turns = both ? (nblk + 1) >> 1 : nblk;
+  const bool both = GROUPS == 2 && !alone && nblk > 7;
+  if (GROUPS == 2 && !both && !alone && grp == 1) return;
+  int turns = both ? (nblk + 1) >> 1 : nblk;
   const int step = both ? 2 : 1, start = both ? grp : 0;
+  __shared__ int turns_of[2];
+  if (alone && lane == 0 && wave == 0) turns_of[grp] = turns;
 
   // Qᵀ fragments: k-step j covers d = 16 j + 8 hi … + 7 (fp8 pages keep d in 64-wide chunks: same d, other address)
   bf16x8 qf[8];
@@ -510,7 +516,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   const int v_off0 = c32 * 64 + ((hi ^ swz) << 4), v_off1 = c32 * 64 + (((2 + hi) ^ swz) << 4);
   const int v8_off = c32 * 32 + 8 * hi;
 
-  // group g walks pages g, g + 2, … in a ring of its own; both pass the same barriers
+  // group g walks pages g, g + 2, … (of a tile of its own: all) in a ring of its own; both pass the same barriers
   if (start < nblk) DLI_STAGE(start, 0);
   if (start + step < nblk) {
     DLI_STAGE(start + step, 1);
@@ -519,6 +525,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   __syncthreads();
+  if (alone) turns = max(turns_of[0], turns_of[1]);
   int st = 0;
   for (int t = 0; t < turns; ++t) {
     const int b = step * t + start;
@@ -707,22 +714,31 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
                        out_stride, Hq, 1, kv_fp8 ? v_scale : 1.f, kv_fp8 ? kv_scales : nullptr, Hkv, (const int4*)red, counts);
 }
 
+static constexpr int PREFILL_UNITS = 256;                      // workgroups of two groups that run at once: one a compute unit
 // Two groups where a compute unit gets one workgroup: a tile's pages are a serial chain of 0.7 µs each, and what the chip
 // has no second tile for, a second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: prompts of 1000 tokens (256
 // workgroups) 32.3 / 26.9, of 2000 with 8/1 heads (250) 57.8 / 45.7, 8 × 128 tokens behind 1000 (256) 37.9 / 34.5, 32 × 16 behind 300 15.0 / 15.3.
-// A unit holds one workgroup of two groups (100 KB of LDS), but three of one: past 256 the rest comes in a second round, whose
-// workgroups all start with 5 µs of latencies.  16 × 100 tokens (512) 12.5 / 17.2, 9 × 128 behind 1000 (288) 46.3 / 60.4, 3 × 600 (456) 25.0 /
-// 26.6.  It pays there only if the second round is made of short tiles: long prompts with little in front of them (one of 2000 (504) 62.2 / 56.1, two of
-// 600 (304) 23.7 / 19.4, one of 1300 behind 300 (328) 50.8 / 40.0).  With 5 µs + 0.0285 µs a token for one group, 5.5 + 0.0225 for two, and the
-// first tile of the second round at `second` tokens of context, that is what the last line says (fitted on 190 steps of equal prompts).
+// A unit holds one workgroup of two groups (100 KB of LDS; e4m3 68 KB, but its registers leave room for one too), and three of one.  Past 256 tiles:
+//   * the shortest share workgroups, a group each (SHARED).  Both pass the same barriers, so they wait for their loads and products at the same time
+//     and take 1.25 of what they take in workgroups of their own; the longest take 0.8.  It pays where the shared ones are the shorter ones: 2 × 600
+//     tokens (304 tiles) 24.1 / 20.7, 4 × 300 (320) 16.1 / 14.7, one of 1100 behind 500 (280) 51.0 / 39.9, but 3 × 400 behind 1000 (312) 48.6 / 55.9,
+//     2 × 1024 (512, all shared) 37.4 / 46.6.  e4m3, whose one group is slower: 2 × 600 behind 600 49.9 / 47.6, 4 × 1500 behind 500 with 8/1 heads (376)
+//     77.2 / 74.1, a mixed step of 96 rows and two chunks of up to 1024 behind up to 1024 (296) 73.8 / 62.5 (in bf16 77 / 89).
+//   * or the rest comes in a second round (ROUNDS), whose workgroups all start with 5 µs of latencies: 16 × 100 tokens (512) 12.5 / 17.2, 9 × 128 behind
+//     1000 (288) 46.3 / 60.4.  It pays only if that is made of short tiles: one prompt of 2000 (504) 63.5 / 58.1.  With 5 µs + 0.0285 µs a token for
+//     one group, 5.5 + 0.0225 for two, and the first tile of the second round at `second` tokens of context, that is what the last line says
+//     (fitted on 190 steps of equal prompts).
 // longest: tokens of context (new ones included) of the longest sequence, sequences: with new tokens; 0: not known, as for a captured launch of bounds.
-int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences) {
+int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, bool kv_fp8) {
+  constexpr int ONE = 1, ROUNDS = 2, SHARED = 3;
   const int blocks = num_tiles * Hkv, tile_tokens = 16 * (8 / G);
-  if (blocks <= 256) return longest == 0 || longest > 224 ? 2 : 1;
-  if (blocks > 512 || longest <= 0 || sequences <= 0) return 1;
+  if (blocks <= PREFILL_UNITS) return longest == 0 || longest > 224 ? ROUNDS : ONE;
+  if (blocks > 2 * PREFILL_UNITS || longest <= 224 || sequences <= 0) return ONE;
   const float mean = std::min((float)longest, (float)num_tiles * tile_tokens / sequences);
-  const float second = longest - mean + mean * (blocks - 256) / blocks;
-  return second < 0.63f * longest - 180.f ? 2 : 1;
+  const float shared = longest - mean * (2 * PREFILL_UNITS - blocks) / blocks;        // context of the longest tile that shares
+  if (shared < (kv_fp8 ? 0.75f : 0.7f) * longest) return SHARED;
+  const float second = longest - mean + mean * (blocks - PREFILL_UNITS) / blocks;
+  return second < 0.63f * longest - 180.f ? ROUNDS : ONE;
 }
 
 void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
@@ -731,15 +747,15 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
                           int Hkv, float scale, bool kv_fp8, float k_scale, float v_scale, const float* kv_scales,
                           const int* counts, int longest, int sequences, hipStream_t stream) {
   if (num_tiles == 0) return;
-  const int G = Hq / Hkv;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-  const int groups = prefill_page_groups(num_tiles, Hkv, G, longest, sequences);
-  dim3 grid((num_tiles * Hkv + 7) / 8 * 8);
+  const int form = prefill_page_groups(num_tiles, Hkv, Hq / Hkv, longest, sequences, kv_fp8), groups = form == 1 ? 1 : 2;
+  const int units = form == 3 ? PREFILL_UNITS : num_tiles * Hkv;
+  const dim3 grid(std::min(num_tiles * Hkv, units));
 #define DLI_PREFILL_GO(KV8_, G_)                                                                                              \
   hipLaunchKernelGGL((paged_prefill_kernel<KV8_, G_>), grid, dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, v_cache, \
                      block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, Hq, Hkv, num_tiles, \
-                     scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, counts)
+                     scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, counts, units)
   if (kv_fp8) { if (groups == 2) DLI_PREFILL_GO(true, 2); else DLI_PREFILL_GO(true, 1); }
   else { if (groups == 2) DLI_PREFILL_GO(false, 2); else DLI_PREFILL_GO(false, 1); }
 #undef DLI_PREFILL_GO

@@ -36,7 +36,7 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
                           const int* tile_seq, const int* tile_q0, int num_tiles, void* out, int64_t out_stride, int Hq,
                           int Hkv, float scale, bool kv_fp8, float k_scale, float v_scale, const float* kv_scales,
                           const int* counts, int longest, int sequences, hipStream_t stream);
-int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences);
+int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, bool kv_fp8);
 
 void launch_skinny_linear(void* out, int64_t out_stride, const void* x, int64_t x_stride, const void* w, const void* bias,
                           int M, int N, int K, bool swiglu, const float* w_scale, hipStream_t stream);

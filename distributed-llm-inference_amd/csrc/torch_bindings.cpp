@@ -787,8 +787,8 @@ TORCH_LIBRARY(dli, m) {
         "Tensor query_start_loc, Tensor tile_seq, Tensor tile_q0, int num_tiles, int num_heads, int num_kv_heads, float scale, "
         "float k_scale, float v_scale, Tensor? kv_scales=None, Tensor? counts=None, int longest=0, int sequences=0) -> ()", &paged_attention_prefill);
   m.def("rm_conv_by_runs(int rows, int channels) -> bool", [](int64_t rows, int64_t c) -> bool { return dli::rm_conv_by_runs((int)rows, (int)c); });
-  m.def("prefill_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences) -> int",
-        [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s) -> int64_t { return dli::prefill_page_groups((int)t, (int)h, (int)g, (int)l, (int)s); });
+  m.def("prefill_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences, bool kv_fp8=False) -> int",
+        [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s, bool f) -> int64_t { return dli::prefill_page_groups((int)t, (int)h, (int)g, (int)l, (int)s, f); });
   m.def("paged_attention_decode_worklist(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor seq_lens, Tensor work, Tensor red, Tensor counts, int items, int reds, int max_parts, int Hq, int Hkv, float scale, "
         "Tensor workspace, float k_scale, float v_scale, Tensor? kv_scales=None) -> ()", &paged_attention_decode_worklist);

@@ -119,20 +119,30 @@ def test_the_plan_goes_before_the_rule(monkeypatch):
     assert plan.load(plan.export()) is None and plan.splits_for(128, n, k, True) == gemm_plan.STREAM
 
 
-@pytest.mark.parametrize("new,ctx,n,G,groups", [
-    # 8 kv heads of 4 (32-token tiles) or one of 8 (16-token tiles); timed with one and with two page groups
-    (64, 0, 4, 4, 1), (200, 0, 4, 4, 1), (256, 0, 4, 4, 2), (16, 1000, 32, 4, 2), (128, 1000, 8, 4, 2), (1000, 0, 1, 4, 2), (2000, 0, 2, 8, 2),
-    (17, 0, 37, 4, 1), (100, 0, 16, 4, 1), (128, 1000, 9, 4, 1), (300, 0, 6, 4, 1), (400, 0, 4, 4, 1), (600, 0, 3, 4, 1), (600, 600, 2, 4, 1),
-    (1000, 1000, 2, 4, 1), (16, 1000, 300, 8, 1), (600, 0, 11, 8, 1), (400, 0, 13, 8, 1), (800, 600, 8, 8, 1), (2000, 2000, 1, 4, 1),
-    (600, 0, 2, 4, 2), (1300, 300, 1, 4, 2), (2000, 0, 1, 4, 2), (2048, 0, 1, 4, 2), (1000, 300, 5, 8, 2), (2000, 0, 3, 8, 2), (1300, 600, 4, 8, 2),
-    (2049, 0, 1, 4, 1), (100, 0, 40, 4, 1), (4000, 0, 1, 4, 1)])
-def test_prefill_page_groups(new, ctx, n, G, groups):
-    """Two groups of waves a tile where the chip takes all tiles at once, or where only short ones are left for later."""
+@pytest.mark.parametrize("new,ctx,n,G,form,e4m3", [
+    # 8 kv heads of 4 (32-token tiles) or one of 8 (16-token tiles); timed with one page group, two in rounds, two of which the last share: 1, 2, 3
+    (64, 0, 4, 4, 1, 1), (200, 0, 4, 4, 1, 1), (256, 0, 4, 4, 2, 2), (16, 1000, 32, 4, 2, 2), (128, 1000, 8, 4, 2, 2), (1000, 0, 1, 4, 2, 2),
+    (2000, 0, 2, 8, 2, 2), (17, 0, 37, 4, 1, 1), (100, 0, 16, 4, 1, 1), (128, 1000, 9, 4, 1, 1), (300, 0, 6, 4, 1, 1), (600, 0, 3, 4, 1, 1),
+    (400, 1000, 3, 4, 1, 1), (1000, 1000, 2, 4, 1, 1), (16, 1000, 300, 8, 1, 1), (600, 3000, 2, 4, 1, 1), (128, 200, 10, 4, 1, 1),
+    (300, 0, 4, 4, 3, 3), (600, 0, 2, 4, 3, 3), (600, 600, 2, 4, 3, 3), (1100, 500, 1, 4, 3, 3), (1300, 300, 1, 4, 3, 3), (2000, 0, 3, 8, 3, 3),
+    (1500, 500, 4, 8, 2, 3), (2000, 0, 1, 4, 2, 2), (2048, 0, 1, 4, 2, 2), (2000, 2000, 1, 4, 1, 1), (2049, 0, 1, 4, 1, 1), (100, 0, 40, 4, 1, 1),
+    (4000, 0, 1, 4, 1, 1)])
+def test_prefill_page_groups(new, ctx, n, G, form, e4m3):
+    """Two groups of waves a tile where the chip takes all tiles at once, or where those that share or wait are short ones."""
     heads, tile = (8, 32) if G == 4 else (1, 16)
     tiles = n * ((new + tile - 1) // tile)
     rule = ops.hip().prefill_page_groups
-    assert rule(tiles, heads, G, new + ctx, n) == groups
-    assert rule(tiles, heads, G, 0, 0) == (2 if tiles * heads <= 256 else 1)        # lengths not known
+    assert [rule(tiles, heads, G, new + ctx, n, f) for f in (False, True)] == [form, e4m3]
+    assert rule(tiles, heads, G, 0, 0, False) == (2 if tiles * heads <= 256 else 1)        # lengths not known
+
+
+def test_every_prefill_tile_is_taken_once():
+    """What a workgroup of two groups takes where the last of them share (``units`` of them), for every number of tiles."""
+    units = 256
+    for items in range(1, 2 * units + 1):
+        over = max(items - units, 0)
+        taken = [b + g * over for b in range(items - over) for g in ((0, 1) if b >= units - over else (0,))]
+        assert sorted(taken) == list(range(items))
 
 
 def test_convolution_runs_where_they_fill_the_chip():

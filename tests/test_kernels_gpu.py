@@ -370,11 +370,11 @@ def test_prefill_page_groups_at_the_dispatch_line(n, kv_dtype):
     torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -9 * 4.5)
 
 
-@pytest.mark.parametrize("new,ctx,n", [(600, 0, 2), (1300, 300, 1), (1300, 2000, 1)])      # 304 and 328 workgroups: two groups, two, one
+@pytest.mark.parametrize("new,ctx,n", [(600, 0, 2), (1300, 300, 1), (1300, 2000, 1), (2000, 0, 1)])      # 304, 328, 328, 504 tiles: shared twice, one group, rounds
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 def test_prefill_long_prompts_in_a_second_round(new, ctx, n, kv_dtype):
-    """Steps whose known lengths choose the page groups past 256 workgroups; the same bits from the form that a step of unknown lengths
-    takes where that is the same one.  Tolerances as above."""
+    """Steps whose known lengths choose the page groups past 256 workgroups; the same bits from the form that a step of unknown lengths, exact or a
+    bound, takes where that is the same one.  Tolerances as above."""
     Hq, Hkv = 32, 8
     lens = [new + ctx] * n
     kc, vc, bt = _fill_cache(Hq, Hkv, lens, kv_dtype, seed=25)
@@ -382,15 +382,39 @@ def test_prefill_long_prompts_in_a_second_round(new, ctx, n, kv_dtype):
     i32 = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int32, device=DEV)
     ts, t0 = ops.build_prefill_tiles(np.full(n, new), 0, ops.prefill_tile_tokens(Hq, Hkv), np.array(lens))
     out = []
-    for longest in (new + ctx, 0):
+    for longest, bound in ((new + ctx, 0), (0, 0), (0, 64)):
+        pad = np.zeros(max(bound - len(ts), 0), np.int32)
         meta = ops.AttnMetadata(num_decode=0, num_prefill=n, num_tokens=n * new, positions=None, slot_mapping=None, block_tables=bt, seq_lens=i32(lens),
-                                query_start_loc=i32(np.arange(n + 1) * new), max_seq_len=longest, prefill_tile_seq=i32(ts), prefill_tile_q0=i32(t0),
-                                num_prefill_tiles=len(ts))
+                                query_start_loc=i32(np.arange(n + 1) * new), max_seq_len=longest, prefill_tile_seq=i32(np.append(ts, pad)),
+                                prefill_tile_q0=i32(np.append(t0, pad)), num_prefill_tiles=bound or len(ts), counts=i32([0, 0, len(ts), n]),
+                                counts_on_device=bound > 0)
         out.append(ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088).float())
     want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(n * new, Hq, 128), kc, vc, bt, i32(lens), i32(np.arange(n + 1) * new), 0.088).float()
     for got in out:
         torch.testing.assert_close(got.view_as(want), want, rtol=2 ** -7, atol=2 ** -8 * 4.5)
-    assert torch.equal(out[0], out[1]) == (ctx == 2000)
+    assert torch.equal(out[1], out[2]) and torch.equal(out[0], out[1]) == (ctx == 2000)
+
+
+@pytest.mark.parametrize("more", [1, 5, 14, 17])                  # tiles of 8 heads past 32: 8, 40, 112, 136 of 256 workgroups are shared
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_prefill_tiles_that_share_a_workgroup(more, kv_dtype):
+    """Tiles of 1 to 20 pages with masked last pages, two of unequal length to a workgroup, others with both groups.  Tolerances as above."""
+    Hq = Hkv = 8                                                    # tiles of 128 tokens
+    n = 32 + more
+    seq_lens = [1 + (37 * i) % 640 for i in range(n)]
+    qlens = [min(L, 1 + 29 * i % 128) for i, L in enumerate(seq_lens)]
+    kc, vc, bt = _fill_cache(Hq, Hkv, seq_lens, kv_dtype, seed=27)
+    T = sum(qlens)
+    qkv = _bf(T, (Hq + 2 * Hkv) * 128, seed=28)
+    i32 = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    sl, qsl = i32(seq_lens), i32(np.concatenate([[0], np.cumsum(qlens)]))
+    ts, t0 = ops.build_prefill_tiles(np.array(qlens), 0, 128, np.array(seq_lens))
+    assert ops.hip().prefill_page_groups(n, Hkv, 1, 640, 1, kv_dtype != torch.bfloat16) == 3       # (what the rule says to one long sequence)
+    meta = ops.AttnMetadata(num_decode=0, num_prefill=1, num_tokens=T, positions=None, slot_mapping=None, block_tables=bt, seq_lens=sl,
+                            query_start_loc=qsl, max_seq_len=640, prefill_tile_seq=i32(ts), prefill_tile_q0=i32(t0), num_prefill_tiles=n)
+    got = ops.paged_attention(qkv, kc, vc, meta, Hq, Hkv, 128, 0.088).float()
+    want = ref.paged_attention_ref(qkv[:, :Hq * 128].reshape(T, Hq, 128), kc, vc, bt, sl, qsl, 0.088).float()
+    torch.testing.assert_close(got.view_as(want), want, rtol=2 ** -7, atol=2 ** -8 * 4.5)
 
 
 @pytest.mark.parametrize("n", [1, 65])                            # two page groups and one
