@@ -66,6 +66,10 @@ void launch_grouped_gemm256(int epilogue, const void* A, int64_t a_stride, const
 void launch_dense_gemm256(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M,
                           int K, int N_out, int k_splits, float* workspace, bool split_tail, hipStream_t stream);
 void dense_gemm256_tail_plan(int M, int K, int N_out, bool swiglu, int* tail_tiles, int* tail_slices);
+// W8A8 product (gemm_e4m3.hip)
+void launch_gemm_e4m3(const void* x, int64_t x_stride, const void* w, const float* x_scale, const float* w_scale, void* out,
+                      int64_t out_stride, int M, int N, int K, hipStream_t stream);
+double gemm_e4m3_fill(int64_t M, int64_t N);
 // activation rows 17 … 256: weight-streaming tiles (stream_gemm.hip)
 void launch_stream_gemm(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M, int K, int N,
                         int k_splits, hipStream_t stream);

@@ -327,6 +327,32 @@ Tensor dense_gemm256(const Tensor& x, const Tensor& w, bool swiglu, int64_t k_sp
   return out;
 }
 
+// y = (x · x_scale) · (w · w_scale)ᵀ on the e4m3 matrix cores (gemm_e4m3.hip): x [M, K], w [N, K] e4m3, scales fp32 per row, y bf16
+Tensor gemm_e4m3(const Tensor& x, const Tensor& x_scale, const Tensor& w, const Tensor& w_scale, const c10::optional<Tensor>& out_) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.get_device() == w.get_device() && x.scalar_type() == at::kFloat8_e4m3fn &&
+              w.scalar_type() == at::kFloat8_e4m3fn && x.dim() == 2 && w.dim() == 2 && w.is_contiguous() && x.size(1) == w.size(1),
+              "gemm_e4m3: x [M, K] and contiguous w [N, K] must be float8_e4m3fn on one GPU");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && K >= 256 && K % 256 == 0 && N >= 256 && N % 256 == 0, "gemm_e4m3: K % 256 == 0, N % 256 == 0; got M=", M, " N=", N, " K=", K);
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) >= K && x.stride(0) % 16 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "gemm_e4m3: rows must be 16-byte aligned");
+  TORCH_CHECK(M * x.stride(0) < (int64_t(1) << 32) && N * K < (int64_t(1) << 32) && M <= (int64_t(1) << 24), "gemm_e4m3: operand too large");
+  for (const Tensor* s : {&x_scale, &w_scale})
+    TORCH_CHECK(s->is_cuda() && s->get_device() == x.get_device() && s->scalar_type() == at::kFloat && s->is_contiguous(), "gemm_e4m3: scales must be contiguous fp32");
+  TORCH_CHECK(x_scale.numel() == M && w_scale.numel() == N && reinterpret_cast<uintptr_t>(w_scale.data_ptr()) % 16 == 0, "gemm_e4m3: one scale per row");
+  Tensor out;
+  if (out_.has_value()) {
+    out = *out_;
+    TORCH_CHECK(out.is_cuda() && out.get_device() == x.get_device() && out.scalar_type() == at::kBFloat16 && out.dim() == 2 && out.size(0) == M &&
+                out.size(1) == N && out.is_contiguous() && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "gemm_e4m3: out must be a contiguous bf16 [M, N]");
+  } else {
+    out = at::empty({M, N}, x.options().dtype(at::kBFloat16));
+  }
+  dli::launch_gemm_e4m3(x.data_ptr(), x.stride(0), w.data_ptr(), x_scale.data_ptr<float>(), w_scale.data_ptr<float>(), out.data_ptr(), out.stride(0),
+                        (int)M, (int)N, (int)K, cur_stream(x));
+  return out;
+}
+
 // y = x · Wᵀ on the weight-streaming tiles (stream_gemm.hip), swiglu as for dense_gemm256.  k_splits = 0: as many K slices as it takes
 // to give every compute unit a workgroup.
 Tensor stream_gemm(const Tensor& x, const Tensor& w, bool swiglu, int64_t k_splits, const c10::optional<Tensor>& out_) {
@@ -771,6 +797,8 @@ TORCH_LIBRARY(dli, m) {
   m.def("rms_norm_quant(Tensor x, Tensor(a!)? residual, Tensor weight, float eps) -> (Tensor, Tensor)", &rms_norm_quant);
   m.def("skinny_linear(Tensor x, Tensor w, Tensor? bias, bool swiglu=False, Tensor? out=None, Tensor? w_scale=None) -> Tensor", &skinny_linear);
   m.def("dense_gemm256(Tensor x, Tensor w, bool swiglu=False, int k_splits=1, Tensor? out=None, bool split_tail=False) -> Tensor", &dense_gemm256);
+  m.def("gemm_e4m3(Tensor x, Tensor x_scale, Tensor w, Tensor w_scale, Tensor? out=None) -> Tensor", &gemm_e4m3);
+  m.def("gemm_e4m3_fill(int m, int n) -> float", &dli::gemm_e4m3_fill);
   m.def("stream_gemm(Tensor x, Tensor w, bool swiglu=False, int k_splits=0, Tensor? out=None) -> Tensor", &stream_gemm);
   m.def("moe_tile_rows(int given, int rows, int hidden, bool fits256) -> int", &moe_tile_rows);
   m.def("ar_staging_tensor(int state, int rows, int cols, Tensor like) -> Tensor", &ar_staging_tensor);

@@ -7,6 +7,7 @@ a GPU tensor raises.
 """
 from __future__ import annotations
 
+import functools
 import os
 from dataclasses import dataclass
 from typing import Optional
@@ -407,13 +408,39 @@ def quant_weight_fp8(w: torch.Tensor):
     return (wf / scale).clamp(-FP8_MAX, FP8_MAX).to(torch.float8_e4m3fn).contiguous(), scale.t().contiguous()
 
 
+@functools.lru_cache(maxsize=4096)
+def _e4m3_tiles_fill(m: int, n: int) -> bool:
+    """Do the own e4m3 tiles (``csrc/kernels/gemm_e4m3.hip``) fill at least half of the chip while they run?  From there they beat the library
+    (ratios of the times at 28672 × 4096, 4096 × 14336, 7168 × 8192, 8192 × 3584, 6144 × 4096, 4096 × 4096 weights and 200 to 4096 rows: 0.70 to
+    0.95, once 1.05), below they leave too many compute units idle, which the library fills by cutting K (512 rows of 4096 × 14336: 90 against
+    49 µs)."""
+    return hip().gemm_e4m3_fill(m, n) >= 0.5
+
+
+def _e4m3_ok(q: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, out: Optional[torch.Tensor]) -> bool:
+    f32, e4m3 = torch.float32, torch.float8_e4m3fn
+    if not (q.dim() == 2 and wq.dim() == 2 and q.dtype == e4m3 and wq.dtype == e4m3 and xs.dtype == f32 and ws.dtype == f32
+            and _plain(q, xs, wq, ws) and (out is None or _plain(out))):
+        return False
+    (m, k), n = q.shape, wq.shape[0]
+    if not (wq.shape[1] == k and xs.shape == (m, 1) and ws.shape == (1, n) and k % 256 == 0 and n % 256 == 0 and 0 < m <= 1 << 24 and k and n
+            and _e4m3_tiles_fill(m, n)):
+        return False
+    return (wq.is_contiguous() and q.stride(1) == 1 and q.stride(0) >= k and q.stride(0) % 16 == 0 and xs.is_contiguous() and ws.is_contiguous()
+            and all(t.device == q.device for t in (wq, xs, ws)) and m * q.stride(0) < 2 ** 32 and n * k < 2 ** 32
+            and all(t.data_ptr() % 16 == 0 for t in (q, wq, ws))
+            and (out is None or (out.shape == (m, n) and out.dtype == torch.bfloat16 and out.device == q.device and out.data_ptr() % 16 == 0)))
+
+
 def linear_fp8(x: Optional[torch.Tensor], wq: torch.Tensor, w_scale: torch.Tensor, out: Optional[torch.Tensor] = None,
                xq=None) -> torch.Tensor:
     """``x @ Wᵀ`` with both operands in e4m3 and fp32 accumulation on the fp8 matrix cores; per-token × per-channel scales
-    applied by the GEMM's epilogue (hipBLASLt through ``torch._scaled_mm``), bf16 result.  ``xq``: an already quantised
-    input ``(q, scale)`` (the SwiGLU output comes out of ``quant_rows_fp8(silu=True)`` that way)."""
+    applied by the GEMM's epilogue (own tiles where they fill the chip, else hipBLASLt through ``torch._scaled_mm``), bf16 result.  ``xq``:
+    an already quantised input ``(q, scale)`` (the SwiGLU output comes out of ``quant_rows_fp8(silu=True)`` that way)."""
     q, xs = xq if xq is not None else quant_rows_fp8(x)
     if q.is_cuda:
+        if (out is None or out.is_contiguous()) and _e4m3_ok(q, xs, wq, w_scale, out):
+            return hip().gemm_e4m3(q, xs, wq, w_scale, out)
         if out is not None and out.is_contiguous():          # e.g. the all-reduce's IPC staging buffer: no copy pass
             return torch._scaled_mm(q, wq.t(), scale_a=xs, scale_b=w_scale, out_dtype=torch.bfloat16, out=out)
         y = torch._scaled_mm(q, wq.t(), scale_a=xs, scale_b=w_scale, out_dtype=torch.bfloat16)
