@@ -92,7 +92,8 @@ std::tuple<Tensor, Tensor> gm_gated_scan(const Tensor& q, const Tensor& k, const
     TORCH_CHECK(tile_seq->numel() >= num_tiles && tile_q0->numel() >= num_tiles, "tile lists shorter than num_tiles");
     tsp = tile_seq->data_ptr<int>();
     tqp = tile_q0->data_ptr<int>();
-    ws = at::empty({dli::gm_scan_ws_floats((int)T, (int)num_seqs, (int)H, delta)}, state.options());
+    ws = at::empty({delta ? dli::gm_delta_ws_floats((int)T, (int)num_seqs, (int)H, (int)D, (int)Dv) : dli::gm_scan_ws_floats((int)T, (int)num_seqs, (int)H)},
+                   state.options());
   } else {
     num_tiles = 0;
   }
@@ -138,7 +139,7 @@ Tensor gm_channel_scan(const Tensor& q, const Tensor& k, const Tensor& v, const 
     TORCH_CHECK(tile_seq->numel() >= num_tiles && tile_q0->numel() >= num_tiles, "tile lists shorter than num_tiles");
     tsp = tile_seq->data_ptr<int>();
     tqp = tile_q0->data_ptr<int>();
-    ws = at::empty({dli::gm_channel_ws_floats((int)T, (int)num_seqs, (int)H, (int)D)}, state.options());
+    ws = at::empty({dli::gm_delta_ws_floats((int)T, (int)num_seqs, (int)H, (int)D, (int)Dv)}, state.options());
   } else {
     num_tiles = 0;
   }

@@ -336,15 +336,39 @@ __global__ __launch_bounds__(NT) void scan_step_kernel(const A* __restrict__ q, 
 //   o_t = q_t · (exp(P_t) S0 + Σ_{j ≤ t} exp(P_t - P_j) k_j u_jᵀ),   S = exp(P_end) S0 + Σ_j exp(P_end - P_j) k_j u_jᵀ
 // and u = w ⊙ v, or for the delta rule the solution of u_t = w_t (v_t - exp(P_t) S0ᵀ k_t - Σ_{j < t} exp(P_t - P_j) (k_t · k_j) u_j), i.e.
 // U = (I + M)⁻¹ diag(w) (V - diag(exp P) K S0) with M strictly lower triangular.
-//   scan_block_kernel: per (block, head), all blocks side by side: A = tril(exp(P_t - P_j) q_t · k_j), (I + M)⁻¹ and the vectors
-//     exp(P), exp(P_end - P), w → workspace
+//   scan_block_kernel: per (block, head), all blocks side by side: A = tril(exp(P_t - P_j) q_t · k_j) and the vectors exp(P), exp(P_end - P),
+//     w → workspace
 //   scan_walk_kernel: per (sequence, head, 16·CT state columns) over its blocks in order, the state on the matrix cores' accumulators;
 //     everything a block reads from memory is fetched while the block before it is computed (one register set: a fragment is
 //     refilled as soon as it has been used).  The normaliser n = exp(P_end) n0 + Σ_j exp(P_end - P_j) w_j k_j and its product with q
 //     ride on the fragments of the first columns' workgroup.
 // Workspace row of a block = (first token >> 6) + batch row (unique: rows of later sequences start at later tokens): per head
-// [64][64] A | delta: [64][64] (I + M)⁻¹ | [3][64] vectors.
-template <bool DELTA> __host__ __device__ constexpr int64_t block_floats() { return (DELTA ? 2 : 1) * BT * BT + 3 * BT; }
+// [64][64] A | [3][64] vectors.  The delta rule has kernels of its own (below): of its block form only
+//   U = U0 - W S0, O = Q̃ S0 + A U, S = e^{P_end} ⊙ S0 + K̃ᵀ U  with  [W | U0] = (I + M)⁻¹ diag(w) [diag(e^P) K | V]
+// depends on the state, so W and U0 are solved for with all blocks side by side and the walk over the blocks is three products.
+constexpr int64_t scan_block_floats = BT * BT + 3 * BT;
+
+// Workspace of the delta rule per (block, head), all matrices as 16 × 16 tiles in the order in which a wave's lanes read them (1 KB each):
+// A [4][4] | e^{P_end} [DP] | Q̃ [4][DT] | W [4][DT] | K̃ᵀ [DT][4] | U0 [CV][4], DP = 16 DT, CV 16-column tiles of values
+constexpr int TILE = 256;
+struct DeltaSpace {
+  int DT, CV;
+  __host__ __device__ DeltaSpace(int D, int Dv) : DT((D + 15) >> 4), CV((Dv + 15) >> 4) {}
+  __host__ __device__ int pe() const { return 16 * TILE; }
+  __host__ __device__ int q() const { return pe() + 16 * DT; }
+  __host__ __device__ int w() const { return q() + 4 * DT * TILE; }
+  __host__ __device__ int kt() const { return w() + 4 * DT * TILE; }
+  __host__ __device__ int u() const { return kt() + 4 * DT * TILE; }
+  __host__ __device__ int64_t floats() const { return u() + (int64_t)4 * CV * TILE; }
+};
+// A tile as the A operand: lane row + 16 (k / 4) holds 4 consecutive k.  As the B operand, and as a product leaves it: lane column + 16 (row / 4)
+// holds 4 consecutive rows.  turned(): from either form to the other one, a product with the unit matrix (exact); the kernels below store
+// every tile as 1 KB in lane order (4-byte stores of the turned order: channel_block_kernel 87 → 83 µs at 51 blocks of 16 heads of 128).
+__device__ __forceinline__ f32x4 unit_tile(int lane) {
+  const int k = (lane & 15) - 4 * (lane >> 4);
+  return f32x4{k == 0 ? 1.f : 0.f, k == 1 ? 1.f : 0.f, k == 2 ? 1.f : 0.f, k == 3 ? 1.f : 0.f};
+}
+__device__ __forceinline__ f32x4 turned(f32x4 a, f32x4 unit) { return mfma_k16(a, unit, f32x4{0.f, 0.f, 0.f, 0.f}); }
 
 // 4 consecutive entries of a row of D (zero past its end)
 template <typename A> __device__ __forceinline__ f32x4 row4(const A* row, int d, int D, bool wide) {
@@ -355,22 +379,91 @@ template <typename A> __device__ __forceinline__ f32x4 row4(const A* row, int d,
   return r;
 }
 
-// one wave: column `lane` of (I + M)⁻¹ by forward substitution, rows of M [64][BS] (strictly lower part) broadcast from LDS
-__device__ __forceinline__ void unit_lower_inverse(const float* M, float* __restrict__ wi, int lane) {
-  float x[BT];
+// Mn [64][BS]: -M below the diagonal.  Wave w: (I + M)⁻¹ of its 16 × 16 diagonal tile, in place (columns by forward substitution).
+__device__ __forceinline__ void diagonal_inverse(float* Mn, int wave, int lane) {
+  const int c = lane & 15, g4 = lane >> 4;
+  float* m = Mn + 16 * wave * BS + 16 * wave;
+  float x[16];
 #pragma unroll
-  for (int t = 0; t < BT; ++t) {
-    float a0 = t == lane ? 1.f : 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+  for (int t = 0; t < 16; ++t) {
+    float a0 = t == c ? 1.f : 0.f, a1 = 0.f;
 #pragma unroll
     for (int s = 0; s < t; s += 4) {
-      const f32x4 m = *reinterpret_cast<const f32x4*>(M + t * BS + s);
-      a0 -= m[0] * x[s];
-      if (s + 1 < t) a1 -= m[1] * x[s + 1];
-      if (s + 2 < t) a2 -= m[2] * x[s + 2];
-      if (s + 3 < t) a3 -= m[3] * x[s + 3];
+      const f32x4 r = *reinterpret_cast<const f32x4*>(m + t * BS + s);
+      a0 += r[0] * x[s];
+      if (s + 1 < t) a1 += r[1] * x[s + 1];
+      if (s + 2 < t) a0 += r[2] * x[s + 2];
+      if (s + 3 < t) a1 += r[3] * x[s + 3];
     }
-    x[t] = (a0 + a1) + (a2 + a3);
-    wi[t * BT + lane] = x[t];
+    x[t] = a0 + a1;
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t)
+    if (g4 == (t & 3)) m[t * BS + c] = x[t];
+}
+// x ← (I + M)⁻¹ x for N column tiles of 16: block rows in order, a solved row's accumulators are the next ones' operands as they are
+template <int N>
+__device__ __forceinline__ void solve_tiles(const float* Mn, f32x4 (&x)[N][4], int lane) {
+  const int c = lane & 15, g4 = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x4 sum[N];
+#pragma unroll
+    for (int k = 0; k <= i; ++k) {
+      const f32x4 m = *reinterpret_cast<const f32x4*>(Mn + (16 * i + c) * BS + 16 * k + 4 * g4);
+#pragma unroll
+      for (int t = 0; t < N; ++t) {
+        if (k == i && i > 0) x[t][i] += sum[t];
+        const f32x4 p = mfma_k16(m, x[t][k], f32x4{0.f, 0.f, 0.f, 0.f});       // (sums of 16 products each: fewer roundings, and no chain)
+        if (k == i) x[t][i] = p;
+        else sum[t] = k == 0 ? p : sum[t] + p;
+      }
+    }
+  }
+}
+// The end of both block kernels: Mn complete in LDS, the W region holding diag(w e^P) K, wt the weights.  Column tiles of W, then of U0.
+template <typename A>
+__device__ __forceinline__ void solve_block(float* Mn, const float* wt, float* wa, const DeltaSpace& sp, const A* __restrict__ v,
+                                            int64_t v_stride, int n, int Dv, int wave, int lane) {
+  const int c = lane & 15, g4 = lane >> 4;
+  __syncthreads();
+  diagonal_inverse(Mn, wave, lane);
+  __syncthreads();
+  float* ww = wa + sp.w();
+  const f32x4 unit = unit_tile(lane);
+  const int tiles = sp.DT + sp.CV;
+  for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
+    f32x4 x[2][4];
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int t = min(t0 + y, tiles - 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (t < sp.DT) {
+          x[y][i] = *reinterpret_cast<const f32x4*>(ww + (i * sp.DT + t) * TILE + lane * 4);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = 16 * i + 4 * g4 + r, e = (t - sp.DT) * 16 + c;
+            x[y][i][r] = row < n && e < Dv ? wt[row] * ldf<A>(v + row * v_stride + e) : 0.f;
+          }
+        }
+      }
+    }
+    solve_tiles<2>(Mn, x, lane);
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int t = t0 + y;
+      if (t >= tiles) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (t < sp.DT) {
+          *reinterpret_cast<f32x4*>(ww + (i * sp.DT + t) * TILE + lane * 4) = turned(x[y][i], unit);
+        } else {
+          *reinterpret_cast<f32x4*>(wa + sp.u() + ((t - sp.DT) * 4 + i) * TILE + lane * 4) = x[y][i];
+        }
+      }
+    }
   }
 }
 // sum over the four lane groups l>>4 (every lane gets it)
@@ -379,7 +472,14 @@ __device__ __forceinline__ float group_sum(float v) {
   return v + __shfl_xor(v, 32, 64);
 }
 
-template <typename A, bool DELTA>
+// sums of v[0 … 3] over the four lane groups: group i gets that of v[i] (three exchanges, where group_sum takes eight)
+__device__ __forceinline__ float group_sum_each(const float* v, int g4) {
+  const bool hi = g4 & 2, odd = g4 & 1;
+  const float a = (hi ? v[2] : v[0]) + __shfl_xor(hi ? v[0] : v[2], 32, 64), b = (hi ? v[3] : v[1]) + __shfl_xor(hi ? v[1] : v[3], 32, 64);
+  return (odd ? b : a) + __shfl_xor(odd ? a : b, 16, 64);
+}
+
+template <typename A>
 __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q, int64_t q_stride, const A* __restrict__ k, int64_t k_stride,
                                                         const float* __restrict__ decay, const float* __restrict__ weight,
                                                         const int* __restrict__ qsl, const int* __restrict__ state_slots,
@@ -387,8 +487,6 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
                                                         const int* __restrict__ tile_q0, int num_tiles, int H, int G, int D, int wide,
                                                         float q_scale, float* __restrict__ ws) {
   __shared__ double P[BT];
-  __shared__ float wt[BT];
-  __shared__ __align__(16) float M[DELTA ? BT * BS : 4];
   const int tile = blockIdx.x, h = blockIdx.y;
   if (tile >= min(counts[2], num_tiles)) return;
   const int seq = tile_seq[tile];
@@ -399,9 +497,8 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
   if (n <= 0) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
   const int g = h / (H / G);
-  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * block_floats<DELTA>();
-  float* wi = wa + BT * BT;                               // delta: (I + M)⁻¹
-  float* wv = wa + (DELTA ? 2 : 1) * BT * BT;             // exp(P) | exp(P_end - P) | w
+  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * scan_block_floats;
+  float* wv = wa + BT * BT;             // exp(P) | exp(P_end - P) | w
   if (wave == 0) {
     double p = lane < n ? (double)decay[(int64_t)(t0 + lane) * H + h] : 0.0;
 #pragma unroll
@@ -412,18 +509,16 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
     const double end = __shfl(p, 63, 64);
     const float wl = lane < n ? weight[(int64_t)(t0 + lane) * H + h] : 0.f;
     P[lane] = p;
-    wt[lane] = wl;
     wv[lane] = expf((float)p);
     wv[BT + lane] = expf((float)(end - p));
     wv[2 * BT + lane] = wl;
   }
-  // rows 16·wave … of Q Kᵀ (and K Kᵀ) against the column tiles up to the diagonal; rows past the block repeat its last token
+  // rows 16·wave … of Q Kᵀ against the column tiles up to the diagonal; rows past the block repeat its last token
   auto row_of = [&](int i) { return (int64_t)(t0 + min(i, n - 1)); };
-  f32x4 qk[4], kk[4];
+  f32x4 qk[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) qk[s] = kk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < 4; ++s) qk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
   const A* qr = q + row_of(16 * wave + c) * q_stride + g * D;
-  const A* kr = k + row_of(16 * wave + c) * k_stride + g * D;
   const A* kc[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) kc[s] = k + row_of(16 * s + c) * k_stride + g * D;
@@ -431,14 +526,10 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
   for (int d0 = 0; d0 < D; d0 += 16) {
     const int d = d0 + 4 * g4;
     const f32x4 qa = row4(qr, d, D, wide);
-    f32x4 ka;
-    if (DELTA) ka = row4(kr, d, D, wide);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
       if (s <= wave) {
-        const f32x4 kb = row4(kc[s], d, D, wide);
-        qk[s] = mfma_k16(qa, kb, qk[s]);
-        if (DELTA) kk[s] = mfma_k16(ka, kb, kk[s]);
+        qk[s] = mfma_k16(qa, row4(kc[s], d, D, wide), qk[s]);
       }
   }
   __syncthreads();
@@ -450,13 +541,89 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
         const int row = 16 * wave + 4 * g4 + r, col = 16 * s + c;
         const float f = col <= row ? expf((float)(P[row] - P[col])) : 0.f;
         wa[row * BT + col] = f * q_scale * qk[s][r];
-        if (DELTA) M[row * BS + col] = col < row ? f * wt[row] * kk[s][r] : 0.f;
       }
     }
-  if (!DELTA) return;
+}
+
+// the same for the delta rule: A, M = strictly lower exp(P_t - P_j) w_t k_t · k_j, and the solve
+template <typename A>
+__global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict__ q, int64_t q_stride, const A* __restrict__ k, int64_t k_stride,
+                                                         const A* __restrict__ v, int64_t v_stride, const float* __restrict__ decay,
+                                                         const float* __restrict__ weight, const int* __restrict__ qsl,
+                                                         const int* __restrict__ state_slots, const int* __restrict__ counts,
+                                                         const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int num_tiles, int H,
+                                                         int G, int D, int Dv, int wide, float q_scale, float* __restrict__ ws) {
+  __shared__ double P[BT];
+  __shared__ float wt[BT];
+  __shared__ __align__(16) float M[BT * BS];
+  const int tile = blockIdx.x, h = blockIdx.y;
+  if (tile >= min(counts[2], num_tiles)) return;
+  const int seq = tile_seq[tile];
+  const int s0 = qsl[seq], s1 = qsl[seq + 1];
+  if (s1 - s0 < 2 || state_slots[seq] < 0) return;        // single tokens belong to the step kernel
+  const int t0 = s0 + tile_q0[tile];
+  const int n = min(BT, s1 - t0);
+  if (n <= 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
+  const int g = h / (H / G);
+  const DeltaSpace sp(D, Dv);
+  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * sp.floats();
+  if (wave == 0) {
+    double p = lane < n ? (double)decay[(int64_t)(t0 + lane) * H + h] : 0.0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double x = __shfl_up(p, o, 64);
+      if (lane >= o) p += x;
+    }
+    P[lane] = p;
+    wt[lane] = lane < n ? weight[(int64_t)(t0 + lane) * H + h] : 0.f;
+  }
   __syncthreads();
-  if (wave != 0) return;
-  unit_lower_inverse(M, wi, lane);
+  const int row = 16 * wave + c;
+  const double end = P[BT - 1];
+  const f32x4 unit = unit_tile(lane);
+  const float ep = expf((float)P[row]), er = expf((float)(end - P[row])), eq = ep * q_scale, ew = ep * wt[row];
+  for (int d = threadIdx.x; d < 16 * sp.DT; d += NT) wa[sp.pe() + d] = expf((float)end);
+  // rows 16·wave … of Q Kᵀ and K Kᵀ against the column tiles up to the diagonal; rows past the block repeat its last token
+  auto row_of = [&](int i) { return (int64_t)(t0 + min(i, n - 1)); };
+  f32x4 qk[4], kk[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) qk[s] = kk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const A* qr = q + row_of(row) * q_stride + g * D;
+  const A* kr = k + row_of(row) * k_stride + g * D;
+  const A* kc[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) kc[s] = k + row_of(16 * s + c) * k_stride + g * D;
+#pragma unroll 2
+  for (int it = 0; it < sp.DT; ++it) {
+    const int d = 16 * it + 4 * g4;
+    const f32x4 qa = row4(qr, d, D, wide), ka = row4(kr, d, D, wide);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s <= wave) {
+        const f32x4 kb = row4(kc[s], d, D, wide);
+        qk[s] = mfma_k16(qa, kb, qk[s]);
+        kk[s] = mfma_k16(ka, kb, kk[s]);
+      }
+    const int at = (wave * sp.DT + it) * TILE + lane * 4;
+    *reinterpret_cast<f32x4*>(wa + sp.q() + at) = f32x4{qa[0] * eq, qa[1] * eq, qa[2] * eq, qa[3] * eq};
+    *reinterpret_cast<f32x4*>(wa + sp.w() + at) = turned(f32x4{ka[0] * ew, ka[1] * ew, ka[2] * ew, ka[3] * ew}, unit);
+    *reinterpret_cast<f32x4*>(wa + sp.kt() + (it * 4 + wave) * TILE + lane * 4) = turned(f32x4{ka[0] * er, ka[1] * er, ka[2] * er, ka[3] * er}, unit);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    if (s <= wave) {
+      f32x4 a;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * wave + 4 * g4 + r, col = 16 * s + c;
+        const float f = col <= i ? expf((float)(P[i] - P[col])) : 0.f;
+        a[r] = f * q_scale * qk[s][r];
+        M[i * BS + col] = col < i ? -(f * wt[i] * kk[s][r]) : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(wa + (wave * 4 + s) * TILE + lane * 4) = turned(a, unit);
+    }
+  solve_block<A>(M, wt, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
 }
 
 // Channel decays.  With P_t[d] the log decays summed to token t inside the block, the same block form reads
@@ -466,9 +633,7 @@ __global__ __launch_bounds__(NT) void scan_block_kernel(const A* __restrict__ q,
 // through the lane's own, R = product from the next token to the sub-block's end, both prefix products over 16 lanes.  A sub-block
 // of rows meets an earlier sub-block of columns as (q ⊙ L) · (k ⊙ R ⊙ totals of the sub-blocks between)ᵀ on the fp32 matrix cores;
 // inside a sub-block, pairs at distance s use the running product of the s decays between them (lane rotations, no exponential).
-// Workspace per (block, head): A [64][64] | (I + M)⁻¹ [64][64] | weights [64] | e^{P_end} [DP] | q ⊙ e^{P} [64][DP] |
-// k ⊙ e^{P} [64][DP] | (k ⊙ e^{P_end - P})ᵀ [DP][64], DP = D rounded up to 16.
-__host__ __device__ constexpr int64_t channel_block_floats(int DP) { return 2 * BT * BT + BT + DP + 3 * (int64_t)BT * DP; }
+// Q̃ = q ⊙ e^{P}, K̃ᵀ = (k ⊙ e^{P_end - P})ᵀ.
 
 // value of the lane N below (ror: rotated within 16 lanes; shr / shl: `fill` where there is none)
 template <int N> __device__ __forceinline__ float row_ror(float v) {
@@ -500,139 +665,6 @@ __device__ __forceinline__ void all_near_pairs(std::integer_sequence<int, S...>,
   (near_pairs<S + 1>(q, k, g, e, aq, ak), ...);
 }
 
-template <typename Z>
-__global__ __launch_bounds__(NT) void channel_block_kernel(const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k,
-                                                           int64_t k_stride, ChannelArgs<Z> ch, const float* __restrict__ weight,
-                                                           const int* __restrict__ qsl, const int* __restrict__ state_slots,
-                                                           const int* __restrict__ counts, const int* __restrict__ tile_seq,
-                                                           const int* __restrict__ tile_q0, int num_tiles, int H, int G, int D, int wide,
-                                                           float* __restrict__ ws) {
-  __shared__ float wt[BT];
-  __shared__ __align__(16) float M[BT * BS];
-  __shared__ __align__(16) float KR[2][BT][20], EM[2][4][16];
-  const int tile = blockIdx.x, h = blockIdx.y;
-  if (tile >= min(counts[2], num_tiles)) return;
-  const int seq = tile_seq[tile];
-  const int s0 = qsl[seq], s1 = qsl[seq + 1];
-  if (s1 - s0 < 2 || state_slots[seq] < 0) return;        // single tokens belong to the step kernel
-  const int t0 = s0 + tile_q0[tile];
-  const int n = min(BT, s1 - t0);
-  if (n <= 0) return;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
-  const int g = h / (H / G), DP = (D + 15) & ~15;
-  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * channel_block_floats(DP);
-  float* wi = wa + BT * BT;
-  float* we = wi + BT * BT + BT;                          // e^{P_end}
-  float* wq = we + DP;
-  float* wk = wq + BT * DP;
-  float* wkt = wk + BT * DP;
-  if (wave == 0) wt[lane] = wi[BT * BT + lane] = lane < n ? weight[(int64_t)(t0 + lane) * H + h] : 0.f;
-  const int row = 16 * wave + c;
-  const bool live = row < n;
-  const int64_t tok = t0 + min(row, n - 1);               // rows past the block repeat its last token, with decay 1
-  const float* qr = q + tok * q_stride + g * D;
-  const float* kr = k + tok * k_stride + g * D;
-  const Z* zr = ch.z + tok * ch.stride + (int64_t)h * D;
-  const float* br = ch.bias + (int64_t)h * D;
-  const float rate = ch.rate[h];
-  f32x4 qk[3], kk[3];
-#pragma unroll
-  for (int s = 0; s < 3; ++s) qk[s] = kk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float aq[16], ak[16];
-#pragma unroll
-  for (int s = 0; s < 16; ++s) aq[s] = ak[s] = 0.f;
-  f32x4 qn = row4(qr, 4 * g4, D, wide), kn = row4(kr, 4 * g4, D, wide), zn = row4(zr, 4 * g4, D, wide), bn = row4(br, 4 * g4, D, wide);
-  for (int d0 = 0, it = 0; d0 < D; d0 += 16, ++it) {
-    const int d = d0 + 4 * g4, buf = it & 1;
-    const f32x4 qc = qn, kc = kn, zc = zn, bc = bn;
-    if (d0 + 16 < D) {                                    // the next channels are fetched while these are computed
-      qn = row4(qr, d + 16, D, wide);
-      kn = row4(kr, d + 16, D, wide);
-      zn = row4(zr, d + 16, D, wide);
-      bn = row4(br, d + 16, D, wide);
-    }
-    f32x4 gd, L, R, ql, kl, kR;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      gd[j] = live && d + j < D ? channel_decay<Z>(zc[j] + bc[j], rate) : 1.f;
-      float p = gd[j];
-      p *= row_shr<1>(p, 1.f);
-      p *= row_shr<2>(p, 1.f);
-      p *= row_shr<4>(p, 1.f);
-      p *= row_shr<8>(p, 1.f);
-      L[j] = p;
-      float r = row_shl<1>(gd[j], 1.f);
-      r *= row_shl<1>(r, 1.f);
-      r *= row_shl<2>(r, 1.f);
-      r *= row_shl<4>(r, 1.f);
-      r *= row_shl<8>(r, 1.f);
-      R[j] = r;
-      ql[j] = qc[j] * p;
-      kl[j] = kc[j] * p;
-      kR[j] = kc[j] * r;
-    }
-    *reinterpret_cast<f32x4*>(&KR[buf][row][4 * g4]) = kR;
-    if (c == 15) *reinterpret_cast<f32x4*>(&EM[buf][wave][4 * g4]) = L;
-    __syncthreads();                                      // (the other buffer's readers are past the barrier before this one)
-    f32x4 before = {1.f, 1.f, 1.f, 1.f}, behind = before;
-#pragma unroll
-    for (int b = 2; b >= 0; --b)
-      if (b < wave) {                                     // `before`: totals of the sub-blocks between b and this one
-        const f32x4 kb = *reinterpret_cast<const f32x4*>(&KR[buf][16 * b + c][4 * g4]);
-        const f32x4 f = {kb[0] * before[0], kb[1] * before[1], kb[2] * before[2], kb[3] * before[3]};
-        qk[b] = mfma_k16(ql, f, qk[b]);
-        kk[b] = mfma_k16(kl, f, kk[b]);
-        const f32x4 m = *reinterpret_cast<const f32x4*>(&EM[buf][b][4 * g4]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) before[j] *= m[j];
-      }
-#pragma unroll
-    for (int b = 1; b < 4; ++b)
-      if (b > wave) {
-        const f32x4 m = *reinterpret_cast<const f32x4*>(&EM[buf][b][4 * g4]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) behind[j] *= m[j];
-      }
-    f32x4 oq, ok;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      oq[j] = ql[j] * before[j];
-      ok[j] = kl[j] * before[j];
-      wkt[(int64_t)(d + j) * BT + row] = kR[j] * behind[j];
-      aq[0] += qc[j] * kc[j];
-    }
-    *reinterpret_cast<f32x4*>(wq + (int64_t)row * DP + d) = oq;
-    *reinterpret_cast<f32x4*>(wk + (int64_t)row * DP + d) = ok;
-    if (wave == 3 && c == 15)
-      *reinterpret_cast<f32x4*>(we + d) = f32x4{L[0] * before[0], L[1] * before[1], L[2] * before[2], L[3] * before[3]};
-    all_near_pairs(std::make_integer_sequence<int, 15>{}, qc, kc, gd, aq, ak);
-  }
-  // off-diagonal tiles
-#pragma unroll
-  for (int b = 0; b < 3; ++b)
-    if (b < wave) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = 16 * wave + 4 * g4 + r, col = 16 * b + c;
-        wa[i * BT + col] = qk[b][r];
-        M[i * BS + col] = wt[i] * kk[b][r];
-      }
-    }
-  // the diagonal tile: lane c's entry at distance s; the lanes that wrapped around hold nothing and clear the upper triangle
-  const float wr = wt[row];
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const float x = group_sum(aq[s]), y = group_sum(ak[s]);
-    if (g4 == (s & 3)) {
-      const int col = 16 * wave + ((c - s) & 15);
-      wa[row * BT + col] = c >= s ? x : 0.f;
-      M[row * BS + col] = s > 0 && c >= s ? wr * y : 0.f;
-    }
-  }
-  __syncthreads();
-  if (wave == 0) unit_lower_inverse(M, wi, lane);
-}
-
 // fragments as they come from memory (converted where they are used, so that a fetch ahead does not wait for its data)
 template <typename A> struct Raw;
 template <> struct Raw<float> {
@@ -657,9 +689,292 @@ template <typename A> __device__ __forceinline__ typename Raw<A>::v4 raw4(const 
   for (int j = 0; j < 4; ++j) r[j] = d + j < D ? row[d + j] : A(0);
   return r;
 }
-// CHAN (delta rule, A = float): q, k and kᵀ come from the workspace with their channel decays in them (channel_block_kernel).
+// WIDE: D a multiple of 16, all rows 16-byte aligned: the next channels' fetches have no condition, so the compiler can count them and the
+// current channels' arithmetic does not wait for them.
+template <typename Z, bool WIDE>
+__global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k,
+                                                           int64_t k_stride, const float* __restrict__ v, int64_t v_stride,
+                                                           ChannelArgs<Z> ch, const float* __restrict__ weight,
+                                                           const int* __restrict__ qsl, const int* __restrict__ state_slots,
+                                                           const int* __restrict__ counts, const int* __restrict__ tile_seq,
+                                                           const int* __restrict__ tile_q0, int num_tiles, int H, int G, int D, int Dv, int wide,
+                                                           float* __restrict__ ws) {
+  __shared__ float wt[BT];
+  __shared__ __align__(16) float M[BT * BS];
+  __shared__ __align__(16) float KR[2][BT][20], EM[2][4][16];
+  const int tile = blockIdx.x, h = blockIdx.y;
+  if (tile >= min(counts[2], num_tiles)) return;
+  const int seq = tile_seq[tile];
+  const int s0 = qsl[seq], s1 = qsl[seq + 1];
+  if (s1 - s0 < 2 || state_slots[seq] < 0) return;        // single tokens belong to the step kernel
+  const int t0 = s0 + tile_q0[tile];
+  const int n = min(BT, s1 - t0);
+  if (n <= 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
+  const int g = h / (H / G);
+  const DeltaSpace sp(D, Dv);
+  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * sp.floats();
+  if (wave == 0) wt[lane] = lane < n ? weight[(int64_t)(t0 + lane) * H + h] : 0.f;
+  const int row = 16 * wave + c;
+  const float wl = row < n ? weight[(int64_t)(t0 + row) * H + h] : 0.f;
+  const bool live = row < n;
+  const int64_t tok = t0 + min(row, n - 1);               // rows past the block repeat its last token, with decay 1
+  const float* qr = q + tok * q_stride + g * D;
+  const float* kr = k + tok * k_stride + g * D;
+  const Z* zr = ch.z + tok * ch.stride + (int64_t)h * D;
+  const float* br = ch.bias + (int64_t)h * D;
+  const float rate = ch.rate[h];
+  f32x4 qk[3], kk[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) qk[s] = kk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float aq[16], ak[16];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) aq[s] = ak[s] = 0.f;
+  const f32x4 unit = unit_tile(lane);
+  f32x4 qn, kn, bn;
+  typename Raw<Z>::v4 zn;
+  auto fetch = [&](int d) {
+    if constexpr (WIDE) {
+      qn = *reinterpret_cast<const f32x4*>(qr + d);
+      kn = *reinterpret_cast<const f32x4*>(kr + d);
+      zn = *reinterpret_cast<const typename Raw<Z>::v4*>(zr + d);
+      bn = *reinterpret_cast<const f32x4*>(br + d);
+    } else {
+      qn = row4(qr, d, D, wide);
+      kn = row4(kr, d, D, wide);
+      zn = raw4<Z>(zr, d, D, wide);
+      bn = row4(br, d, D, wide);
+    }
+  };
+  fetch(4 * g4);
+  for (int d0 = 0, it = 0; d0 < D; d0 += 16, ++it) {
+    const int d = d0 + 4 * g4, buf = it & 1;
+    const f32x4 qc = qn, kc = kn, zc = Raw<Z>::cvt(zn), bc = bn;
+    if (WIDE) fetch(min(d + 16, D - 16 + 4 * g4));        // the next channels are fetched while these are computed
+    else if (d0 + 16 < D) fetch(d + 16);
+    f32x4 gd, L, R, ql, kl, kR;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      gd[j] = live && d + j < D ? channel_decay<Z>(zc[j] + bc[j], rate) : 1.f;
+      float p = gd[j];
+      p *= row_shr<1>(p, 1.f);
+      p *= row_shr<2>(p, 1.f);
+      p *= row_shr<4>(p, 1.f);
+      p *= row_shr<8>(p, 1.f);
+      L[j] = p;
+      float r = row_shl<1>(gd[j], 1.f);
+      r *= row_shl<1>(r, 1.f);
+      r *= row_shl<2>(r, 1.f);
+      r *= row_shl<4>(r, 1.f);
+      r *= row_shl<8>(r, 1.f);
+      R[j] = r;
+      ql[j] = qc[j] * p;
+      kl[j] = kc[j] * p;
+      kR[j] = kc[j] * r;
+    }
+    *reinterpret_cast<f32x4*>(&KR[buf][row][4 * g4]) = kR;
+    if (c == 15) *reinterpret_cast<f32x4*>(&EM[buf][wave][4 * g4]) = L;
+    lds_barrier();                                        // (the other buffer's readers are past the barrier before this one)
+    f32x4 before = {1.f, 1.f, 1.f, 1.f}, behind = before;
+#pragma unroll
+    for (int b = 2; b >= 0; --b)
+      if (b < wave) {                                     // `before`: totals of the sub-blocks between b and this one
+        const f32x4 kb = *reinterpret_cast<const f32x4*>(&KR[buf][16 * b + c][4 * g4]);
+        const f32x4 f = {kb[0] * before[0], kb[1] * before[1], kb[2] * before[2], kb[3] * before[3]};
+        qk[b] = mfma_k16(ql, f, qk[b]);
+        kk[b] = mfma_k16(kl, f, kk[b]);
+        const f32x4 m = *reinterpret_cast<const f32x4*>(&EM[buf][b][4 * g4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) before[j] *= m[j];
+      }
+#pragma unroll
+    for (int b = 1; b < 4; ++b)
+      if (b > wave) {
+        const f32x4 m = *reinterpret_cast<const f32x4*>(&EM[buf][b][4 * g4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) behind[j] *= m[j];
+      }
+    f32x4 oq, ok, ot;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      oq[j] = ql[j] * before[j];
+      ok[j] = wl * (kl[j] * before[j]);
+      ot[j] = kR[j] * behind[j];
+      aq[0] += qc[j] * kc[j];
+    }
+    const int at = (wave * sp.DT + it) * TILE + lane * 4;
+    *reinterpret_cast<f32x4*>(wa + sp.q() + at) = oq;
+    *reinterpret_cast<f32x4*>(wa + sp.w() + at) = turned(ok, unit);
+    *reinterpret_cast<f32x4*>(wa + sp.kt() + (it * 4 + wave) * TILE + lane * 4) = turned(ot, unit);
+    if (wave == 3 && c == 15)
+      *reinterpret_cast<f32x4*>(wa + sp.pe() + d) = f32x4{L[0] * before[0], L[1] * before[1], L[2] * before[2], L[3] * before[3]};
+    all_near_pairs(std::make_integer_sequence<int, 15>{}, qc, kc, gd, aq, ak);
+  }
+  // off-diagonal tiles
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
+    if (b < wave) {
+      *reinterpret_cast<f32x4*>(wa + (wave * 4 + b) * TILE + lane * 4) = turned(qk[b], unit);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * wave + 4 * g4 + r, col = 16 * b + c;
+        M[i * BS + col] = -(wt[i] * kk[b][r]);
+      }
+    }
+  // the diagonal tile: lane c's entry at distance s; the lanes that wrapped around hold nothing and clear the upper triangle
+  const float wr = wt[row];
+#pragma unroll
+  for (int s4 = 0; s4 < 16; s4 += 4) {
+    const float x = group_sum_each(aq + s4, g4), y = group_sum_each(ak + s4, g4);
+    const int s = s4 + g4, col = (c - s) & 15;
+    wa[(wave * 4 + wave) * TILE + (c + 16 * (col >> 2)) * 4 + (col & 3)] = c >= s ? x : 0.f;
+    M[row * BS + 16 * wave + col] = s > 0 && c >= s ? -(wr * y) : 0.f;
+  }
+  solve_block<float>(M, wt, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
+}
+
+// The walk of the delta rule: per (sequence, head, 16·CT state columns) over its blocks in order, the state on the accumulators.  A block is
+//   [o | x] = [Q̃ | W] S, u = U0 - x → LDS → o += A u, S = e^{P_end} ⊙ S + K̃ᵀ u → LDS,
+// two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 85 µs (36 of them fp32 matrix instructions, were they spread
+// evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83.  The next block's tiles are fetched as soon as
+// their registers are free and without a condition (the last block fetches itself again): behind a condition the compiler has to wait for
+// everything that is in flight.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
+// below that of the walk before (2.7e-7 against 2.9e-7 of its norm).
+template <int DTMAX, int CT, bool FULL>
+__global__ __launch_bounds__(NT) void delta_walk_kernel(float* __restrict__ state, const int* __restrict__ positions,
+                                                        const int* __restrict__ qsl, const int* __restrict__ state_slots,
+                                                        const int* __restrict__ counts, int H, int D, int Dv, const float* __restrict__ ws,
+                                                        float* __restrict__ out) {
+  constexpr int DW = (DTMAX + 3) / 4;                     // state row tiles per wave: wave, wave + 4, …
+  __shared__ __align__(16) float St[DTMAX * CT * TILE], Ut[4 * CT * TILE];
+  const int h = blockIdx.x, seq = blockIdx.z;             // a head's column slices share an XCD (its tiles stay in one L2)
+  if (seq >= counts[3]) return;
+  const int s0 = qsl[seq], n = qsl[seq + 1] - s0;
+  const int slot = state_slots[seq];
+  if (slot < 0 || n < 2) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
+  const DeltaSpace sp(D, Dv);
+  const int DT = FULL ? DTMAX : sp.DT, ct0 = blockIdx.y * CT;
+  float* head = state + ((int64_t)slot * H + h) * D * Dv;
+  const bool carry = positions[s0] > 0;
+  const int blocks = (n + BT - 1) / BT;
+
+  f32x4 qf[DTMAX], wf[DTMAX], kt[DW][4], aa[4], u0[CT], pe[DW];
+  auto base_of = [&](int b) { return ws + ((int64_t)(((s0 + BT * b) >> 6) + seq) * H + h) * sp.floats(); };
+  auto fetch_rows = [&](const float* wb) {
+#pragma unroll
+    for (int i = 0; i < DTMAX; ++i)
+      if (i < DT) {
+        qf[i] = ld4<float>(wb + sp.q() + (wave * DT + i) * TILE + lane * 4);
+        wf[i] = ld4<float>(wb + sp.w() + (wave * DT + i) * TILE + lane * 4);
+      }
+  };
+  auto fetch_values = [&](const float* wb) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) u0[ct] = ld4<float>(wb + sp.u() + (min(ct0 + ct, sp.CV - 1) * 4 + wave) * TILE + lane * 4);
+  };
+  auto fetch_rest = [&](const float* wb) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) aa[s] = ld4<float>(wb + (wave * 4 + s) * TILE + lane * 4);     // (above the diagonal: never used)
+#pragma unroll
+    for (int i = 0; i < DW; ++i) {
+      const int dt = FULL ? wave + 4 * i : min(wave + 4 * i, DT - 1);
+      pe[i] = ld4<float>(wb + sp.pe() + 16 * dt + 4 * g4);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) kt[i][s] = ld4<float>(wb + sp.kt() + (dt * 4 + s) * TILE + lane * 4);
+    }
+  };
+  fetch_rows(base_of(0));
+  fetch_values(base_of(0));
+  fetch_rest(base_of(0));
+
+  f32x4 S[DW][CT];
+#pragma unroll
+  for (int i = 0; i < DW; ++i)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (wave + 4 * i) + 4 * g4 + r, e = (ct0 + ct) * 16 + c;
+        S[i][ct][r] = (carry && d < D && e < Dv) ? head[(int64_t)d * Dv + e] : 0.f;
+      }
+
+  for (int b = 0; b < blocks; ++b) {
+    const int t0 = s0 + BT * b, nn = min(BT, n - BT * b);
+    const float* next = base_of(min(b + 1, blocks - 1));
+#pragma unroll
+    for (int i = 0; i < DW; ++i)
+      if (FULL || wave + 4 * i < DT)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<f32x4*>(St + ((wave + 4 * i) * CT + ct) * TILE + lane * 4) = S[i][ct];
+    lds_barrier();                                        // (the readers of Ut are past the block before)
+    __builtin_amdgcn_sched_barrier(0);                    // (what needs the block's last fetches stays behind its first products)
+    f32x4 x[4][CT], o[CT];                                // x: four sums over every fourth tile: fewer roundings, shorter chains
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) x[0][ct] = x[1][ct] = x[2][ct] = x[3][ct] = o[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < DTMAX; ++i)
+      if (i < DT) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          const f32x4 sb = *reinterpret_cast<const f32x4*>(St + (i * CT + ct) * TILE + lane * 4);
+          x[i & 3][ct] = mfma_k16(wf[i], sb, x[i & 3][ct]);
+          o[ct] = mfma_k16(qf[i], sb, o[ct]);
+        }
+      }
+    fetch_rows(next);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<f32x4*>(Ut + (wave * CT + ct) * TILE + lane * 4) = u0[ct] - ((x[0][ct] + x[1][ct]) + (x[2][ct] + x[3][ct]));
+    fetch_values(next);
+    lds_barrier();                                        // (the readers of St are past it)
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 ub[4][CT], add[DW][2][CT];                         // (summed by itself: the state is rounded once a block)
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) ub[s][ct] = *reinterpret_cast<const f32x4*>(Ut + (s * CT + ct) * TILE + lane * 4);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int i = 0; i < DW; ++i) add[i][s & 1][ct] = mfma_k16(kt[i][s], ub[s][ct], s < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : add[i][s & 1][ct]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s <= wave) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) o[ct] = mfma_k16(aa[s], ub[s][ct], o[ct]);
+      }
+#pragma unroll
+    for (int i = 0; i < DW; ++i)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][ct][r] = pe[i][r] * S[i][ct][r] + (add[i][0][ct][r] + add[i][1][ct][r]);
+    fetch_rest(next);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int e = (ct0 + ct) * 16 + c;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * wave + 4 * g4 + r;
+        if (i < nn && e < Dv) out[((int64_t)(t0 + i) * H + h) * Dv + e] = o[ct][r];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < DW; ++i)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (wave + 4 * i) + 4 * g4 + r, e = (ct0 + ct) * 16 + c;
+        if (d < D && e < Dv) head[(int64_t)d * Dv + e] = S[i][ct][r];
+      }
+}
+
 // FULL: D fills the DTMAX tiles, and no step of the loops over them has a condition in front of its reads.
-template <typename A, bool DELTA, int DTMAX, int CT, bool CHAN, bool FULL>
+template <typename A, int DTMAX, int CT, bool FULL>
 __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, int64_t q_stride, const A* __restrict__ k, int64_t k_stride,
                                                        const A* __restrict__ v, int64_t v_stride, float* __restrict__ state,
                                                        const int* __restrict__ positions, const int* __restrict__ qsl,
@@ -678,44 +993,26 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
   const int DT = FULL ? DTMAX : (D + 15) >> 4, DS = DT * 16 + 4;
   constexpr int DW = (DTMAX + 3) / 4;                     // state row tiles per wave: wave, wave + 4, …
   float* St = sh;                                         // [16·CT columns][DS]: the state at the block's start
-  float* Rt = St + 16 * CT * DS;                          // [columns][BS]: right-hand sides of the delta rule
-  float* Ut = Rt + (DELTA ? 16 * CT * BS : 0);            // [columns][BS]: u
-  float* Us = CHAN ? Ut : Ut + 16 * CT * BS;              // [columns][BS]: exp(P_end - P) u
+  float* Ut = St + 16 * CT * DS;                          // [columns][BS]: u
+  float* Us = Ut + 16 * CT * BS;                          // [columns][BS]: exp(P_end - P) u
   const int e0 = blockIdx.y * 16 * CT;
-  const bool norm = !DELTA && nq != nullptr && blockIdx.y == 0;
+  const bool norm = nq != nullptr && blockIdx.y == 0;
   float* head = state + ((int64_t)slot * H + h) * D * (Dv + (nq != nullptr ? 1 : 0));
   const bool carry = positions[s0] > 0;
   const int blocks = (n + BT - 1) / BT;
 
   using R4 = typename Raw<A>::v4;
-  R4 qf[DTMAX], kf[DELTA ? DTMAX : 1], kt[DW][4];
+  R4 qf[DTMAX], kt[DW][4];
   A vf[CT][4];
-  f32x4 ia[DELTA ? 4 : 1], aa[4], ep, er, wt;
-  f32x4 pe4[CHAN ? DW : 1];                               // decay of this wave's state rows over the block
+  f32x4 aa[4], ep, er, wt;
   float pend = 0.f, wl = 0.f, el = 0.f, epc = 0.f;
-  const int DP = DT * 16;
-  const int64_t bf = CHAN ? channel_block_floats(DP) : block_floats<DELTA>();
-  auto base_of = [&](int b) { return ws + ((int64_t)(((s0 + BT * b) >> 6) + seq) * H + h) * bf; };
-  auto fetch_rows = [&](int b) {                          // q (and k) rows 16·wave + c; rows past the chunk repeat its last token
-    if constexpr (CHAN) {
-      const float* wq = base_of(b) + 2 * BT * BT + BT + DP + (int64_t)(16 * wave + c) * DP + 4 * g4;
-#pragma unroll
-      for (int i = 0; i < DTMAX; ++i)
-        if (i < DT) {
-          qf[i] = ld4<float>(wq + 16 * i);
-          kf[i] = ld4<float>(wq + (int64_t)BT * DP + 16 * i);
-        }
-      return;
-    }
+  auto base_of = [&](int b) { return ws + ((int64_t)(((s0 + BT * b) >> 6) + seq) * H + h) * scan_block_floats; };
+  auto fetch_rows = [&](int b) {                          // q rows 16·wave + c; rows past the chunk repeat its last token
     const int64_t tr = s0 + min(BT * b + 16 * wave + c, n - 1);
     const A* qr = q + tr * q_stride + g * D;
-    const A* kr = k + tr * k_stride + g * D;
 #pragma unroll
     for (int i = 0; i < DTMAX; ++i)
-      if (i < DT) {
-        qf[i] = raw4<A>(qr, 16 * i + 4 * g4, D, wide);
-        if (DELTA) kf[i] = raw4<A>(kr, 16 * i + 4 * g4, D, wide);
-      }
+      if (i < DT) qf[i] = raw4<A>(qr, 16 * i + 4 * g4, D, wide);
   };
   auto fetch_values = [&](int b) {
 #pragma unroll
@@ -727,15 +1024,7 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
     }
   };
   auto fetch_vectors = [&](int b) {
-    if constexpr (CHAN) {
-      const float* wv = base_of(b) + 2 * BT * BT;
-      wt = ld4<float>(wv + 16 * wave + 4 * g4);
-#pragma unroll
-      for (int i = 0; i < DW; ++i)
-        if (wave + 4 * i < DT) pe4[i] = ld4<float>(wv + BT + 16 * (wave + 4 * i) + 4 * g4);
-      return;
-    }
-    const float* wv = base_of(b) + (DELTA ? 2 : 1) * BT * BT;
+    const float* wv = base_of(b) + BT * BT;
     ep = ld4<float>(wv + 16 * wave + 4 * g4);
     er = ld4<float>(wv + BT + 16 * wave + 4 * g4);
     wt = ld4<float>(wv + 2 * BT + 16 * wave + 4 * g4);
@@ -746,12 +1035,6 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
       epc = wv[16 * wave + c];
     }
   };
-  auto fetch_inverse = [&](int b) {
-    const float* wi = base_of(b) + BT * BT;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (DELTA && s <= wave) ia[s] = ld4<float>(wi + (16 * wave + c) * BT + 16 * s + 4 * g4);
-  };
   auto fetch_scores = [&](int b) {
     const float* wa = base_of(b);
 #pragma unroll
@@ -759,16 +1042,6 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
       if (s <= wave) aa[s] = ld4<float>(wa + (16 * wave + c) * BT + 16 * s + 4 * g4);
   };
   auto fetch_columns = [&](int b) {                       // kᵀ of this wave's state row tiles
-    if constexpr (CHAN) {
-      const float* wkt = base_of(b) + 2 * BT * BT + BT + DP + 2 * (int64_t)BT * DP + (int64_t)c * BT + 4 * g4;
-#pragma unroll
-      for (int i = 0; i < DW; ++i)
-        if (wave + 4 * i < DT) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) kt[i][s] = ld4<float>(wkt + (int64_t)16 * (wave + 4 * i) * BT + 16 * s);
-        }
-      return;
-    }
 #pragma unroll
     for (int i = 0; i < DW; ++i)
       if (wave + 4 * i < DT) {
@@ -782,7 +1055,6 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
   fetch_rows(0);
   fetch_vectors(0);
   fetch_values(0);
-  fetch_inverse(0);
   fetch_scores(0);
   fetch_columns(0);
 
@@ -812,23 +1084,20 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
       ews[b & 1][lane] = wl * el;
     }
     lds_barrier();
-    // rows 16·wave … of K S0 and Q S0
-    f32x4 ks[CT], o[CT];
+    // rows 16·wave … of Q S0
+    f32x4 o[CT];
     float pn = 0.f;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) ks[ct] = o[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < CT; ++ct) o[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < DTMAX; ++i)
       if (i < DT) {
         const int d = 16 * i + 4 * g4;
         const f32x4 qa = Raw<A>::cvt(qf[i]);
-        f32x4 ka;
-        if (DELTA) ka = Raw<A>::cvt(kf[i]);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
           const f32x4 sb = *reinterpret_cast<const f32x4*>(St + (16 * ct + c) * DS + d);
           o[ct] = mfma_k16(qa, sb, o[ct]);
-          if (DELTA) ks[ct] = mfma_k16(ka, sb, ks[ct]);
         }
         if (norm) pn += (qa[0] * ns[d] + qa[1] * ns[d + 1]) + (qa[2] * ns[d + 2] + qa[3] * ns[d + 3]);
       }
@@ -838,35 +1107,16 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
     for (int ct = 0; ct < CT; ++ct) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float x = ldf<A>(&vf[ct][r]);
-        if (CHAN) x -= ks[ct][r];
-        else if (DELTA) x -= ep[r] * ks[ct][r];
-        u[ct][r] = 16 * wave + 4 * g4 + r < nn ? wt[r] * x : 0.f;
-        if (!CHAN) o[ct][r] *= ep[r] * q_scale;
+        u[ct][r] = 16 * wave + 4 * g4 + r < nn ? wt[r] * ldf<A>(&vf[ct][r]) : 0.f;
+        o[ct][r] *= ep[r] * q_scale;
       }
     }
     if (more) fetch_values(b + 1);
-    if (DELTA) {
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        *reinterpret_cast<f32x4*>(Rt + (16 * ct + c) * BS + 16 * wave + 4 * g4) = u[ct];
-        u[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      lds_barrier();
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        if (s <= wave) {
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-            u[ct] = mfma_k16(ia[s], *reinterpret_cast<const f32x4*>(Rt + (16 * ct + c) * BS + 16 * s + 4 * g4), u[ct]);
-        }
-      if (more) fetch_inverse(b + 1);
-    }
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       float* p = Ut + (16 * ct + c) * BS + 16 * wave + 4 * g4;
       *reinterpret_cast<f32x4*>(p) = u[ct];
-      if (!CHAN) *reinterpret_cast<f32x4*>(p + (Us - Ut)) = f32x4{u[ct][0] * er[0], u[ct][1] * er[1], u[ct][2] * er[2], u[ct][3] * er[3]};
+      *reinterpret_cast<f32x4*>(p + (Us - Ut)) = f32x4{u[ct][0] * er[0], u[ct][1] * er[1], u[ct][2] * er[2], u[ct][3] * er[3]};
     }
     lds_barrier();
     float rs = 0.f;
@@ -886,14 +1136,6 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
       if (g4 == 0 && 16 * wave + c < nn) nq[(int64_t)(t0 + 16 * wave + c) * H + h] = x;
     }
     const float pe = pend;
-    if (CHAN)                                             // (before the next block's decays arrive)
-#pragma unroll
-      for (int i = 0; i < DW; ++i)
-        if (wave + 4 * i < DT)
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[i][ct][r] *= pe4[CHAN ? i : 0][r];
     if (more) {
       fetch_scores(b + 1);
       fetch_vectors(b + 1);
@@ -916,8 +1158,7 @@ __global__ __launch_bounds__(NT) void scan_walk_kernel(const A* __restrict__ q, 
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (!CHAN) S[i][ct][r] *= pe;
+          for (int r = 0; r < 4; ++r) S[i][ct][r] *= pe;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           f32x4 ka = Raw<A>::cvt(kt[i][s]);
@@ -1011,8 +1252,27 @@ void launch_gm_max_gates(const void* g, bool bf16, int64_t g_stride, const float
 
 int gm_step_max_dim() { return GM_STEP_MAX_D; }
 int gm_block_max_dim() { return GM_BLOCK_MAX_D; }
-int64_t gm_scan_ws_floats(int rows, int seqs, int H, bool delta) {
-  return (int64_t)((rows >> 6) + seqs + 1) * H * (delta ? block_floats<true>() : block_floats<false>());
+int64_t gm_scan_ws_floats(int rows, int seqs, int H) { return (int64_t)((rows >> 6) + seqs + 1) * H * scan_block_floats; }
+int64_t gm_delta_ws_floats(int rows, int seqs, int H, int D, int Dv) { return (int64_t)((rows >> 6) + seqs + 1) * H * DeltaSpace(D, Dv).floats(); }
+
+static void delta_walk(float* state, const int* positions, const int* qsl, const int* state_slots, const int* counts, int seqs, int H, int D, int Dv,
+                       const float* ws, float* out, hipStream_t stream) {
+  const int ct = H * ((Dv + 31) / 32) >= 128 ? 2 : 1;   // 32 state columns per workgroup where that still leaves enough of them
+  const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
+#define GM_WALK(DT, CTV, FULLV)                                                                                                               \
+  hipLaunchKernelGGL((delta_walk_kernel<DT, CTV, FULLV>), grid, dim3(NT), 0, stream, state, positions, qsl, state_slots, counts, H, D, Dv, ws, out)
+#define GM_WALK_D(DT)                                             \
+  do {                                                            \
+    if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
+    else if (ct == 2) GM_WALK(DT, 2, false);                      \
+    else if (D > 16 * DT - 16) GM_WALK(DT, 1, true);              \
+    else GM_WALK(DT, 1, false);                                   \
+  } while (0)
+  if (D <= 64) GM_WALK_D(4);
+  else if (D <= 128) GM_WALK_D(8);
+  else GM_WALK_D(16);
+#undef GM_WALK_D
+#undef GM_WALK
 }
 
 template <typename A, bool DELTA>
@@ -1034,14 +1294,20 @@ static void gated_scan(const A* q, int64_t q_stride, const A* k, int64_t k_strid
 #undef GM_STEP
   if (!blocks) return;
   const int wide = D % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && al16(q) && al16(k);     // 4 entries at a time
-  hipLaunchKernelGGL((scan_block_kernel<A, DELTA>), dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, decay, weight, qsl,
+  if constexpr (DELTA) {
+    hipLaunchKernelGGL(delta_block_kernel<A>, dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride, decay, weight, qsl,
+                       state_slots, counts, tile_seq, tile_q0, num_tiles, H, G, D, Dv, wide, q_scale, ws);
+    delta_walk(state, positions, qsl, state_slots, counts, seqs, H, D, Dv, ws, out, stream);
+    return;
+  }
+  hipLaunchKernelGGL(scan_block_kernel<A>, dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, decay, weight, qsl,
                      state_slots, counts, tile_seq, tile_q0, num_tiles, H, G, D, wide, q_scale, ws);
   const int ct = H * ((Dv + 31) / 32) >= 128 ? 2 : 1;   // 32 state columns per workgroup where that still leaves enough of them
   const int DS = ((D + 15) / 16) * 16 + 4;
-  const size_t lds = (size_t)16 * ct * (DS + (DELTA ? 3 : 2) * BS) * sizeof(float);
+  const size_t lds = (size_t)16 * ct * (DS + 2 * BS) * sizeof(float);
   const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
 #define GM_WALK(DT, CTV, FULLV)                                                                                                               \
-  hipLaunchKernelGGL((scan_walk_kernel<A, DELTA, DT, CTV, false, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state,  \
+  hipLaunchKernelGGL((scan_walk_kernel<A, DT, CTV, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state,  \
                      positions, qsl, state_slots, counts, H, G, D, Dv, wide, q_scale, ws, out, nq)
   // D that fills its bound, two column tiles: 32 heads of 128, whole scans, µs, with / without conditions: 799 rows, channel decays 117.8 / 110.1,
   // 2048 rows 329.9 / 305.9.  One column tile has half the products a read and is no faster without (16 heads, 3162 rows: 213.8 / 220.2, 201.7 / 202.2).
@@ -1074,10 +1340,6 @@ void launch_gm_gated_scan(const void* q, int64_t q_stride, const void* k, int64_
 #undef GM_SCAN
 }
 
-int64_t gm_channel_ws_floats(int rows, int seqs, int H, int D) {
-  return (int64_t)((rows >> 6) + seqs + 1) * H * channel_block_floats((D + 15) & ~15);
-}
-
 void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v, int64_t v_stride,
                             const void* z, bool z_bf16, int64_t z_stride, const float* rate, const float* bias, const float* weight,
                             float* state, const int* positions, const int* qsl, const int* state_slots, const int* counts, int seqs,
@@ -1099,27 +1361,10 @@ void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, in
 #undef GM_STEP
   if (!blocks) return;
   const int wide = D % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && z_stride % 4 == 0 && al16(q) && al16(k) && al16(z) && al16(bias);
-  GM_BF16(z_bf16, Z, hipLaunchKernelGGL(channel_block_kernel<Z>, dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride,
+  GM_BF16(z_bf16, Z, hipLaunchKernelGGL((wide && D % 16 == 0 ? channel_block_kernel<Z, true> : channel_block_kernel<Z, false>), dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride,
                                         (ChannelArgs<Z>{(const Z*)z, z_stride, rate, bias}), weight, qsl, state_slots, counts, tile_seq,
-                                        tile_q0, num_tiles, H, G, D, wide, ws));
-  const int ct = H * ((Dv + 31) / 32) >= 128 ? 2 : 1;   // 32 state columns per workgroup where that still leaves enough of them
-  const int DS = ((D + 15) / 16) * 16 + 4;
-  const size_t lds = (size_t)16 * ct * (DS + 2 * BS) * sizeof(float);
-  const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
-#define GM_WALK(DT, CTV, FULLV)                                                                                                                \
-  hipLaunchKernelGGL((scan_walk_kernel<float, true, DT, CTV, true, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state, \
-                     positions, qsl, state_slots, counts, H, G, D, Dv, wide, 1.f, ws, out, (float*)nullptr)
-#define GM_WALK_D(DT)                                             \
-  do {                                                            \
-    if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
-    else if (ct == 2) GM_WALK(DT, 2, false);                      \
-    else GM_WALK(DT, 1, false);                                   \
-  } while (0)
-  if (D <= 64) GM_WALK_D(4);
-  else if (D <= 128) GM_WALK_D(8);
-  else GM_WALK_D(16);
-#undef GM_WALK_D
-#undef GM_WALK
+                                        tile_q0, num_tiles, H, G, D, Dv, wide, ws));
+  delta_walk(state, positions, qsl, state_slots, counts, seqs, H, D, Dv, ws, out, stream);
 }
 
 }  // namespace dli
