@@ -24,6 +24,8 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -343,14 +345,20 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
 //
 // Staging.  Unlike decode, all four waves of a tile walk the SAME pages, so K and V pages go through LDS: the block
 // copies each 32-token page (K + V, 16 KB bf16 / 8 KB fp8) once by LDS-DMA (global_load_lds, 16 bytes per lane, no
-// VGPRs) into a ring of three stages, two pages ahead of the math (one barrier per page, counted vmcnt), and every
-// wave reads its fragments with ds_read_b128.  The page keeps its global layout in LDS except that the four 16-byte
+// VGPRs) into a ring, and every wave reads its fragments with ds_read_b128.  A turn (one barrier) is one page of three stages, two pages ahead of
+// the math, or with two groups, whose one workgroup a compute unit has the registers for it, two pages of two stages: two score
+// chains side by side, one maximum and one rescale of the accumulators for both.  The page keeps its global layout in LDS except that the four 16-byte
 // slots of every 64-byte row are permuted by the row (slot ^ h[(row >> 2) & 3], h = {0,2,3,1}; the DMA's LDS image is
 // lane-linear, so the permutation sits on the SOURCE address): the 16 lanes the hardware serves together for a
 // ds_read_b128 — {0–3, 12–15, 20–27} etc. — then touch 16 different slots of the 256-byte bank row.
 //
-// GROUPS = 2 (few tiles): a workgroup has two such sets of four waves; group g takes pages g, g + 2, … in a ring of its own, and at the end the
+// GROUPS = 2 (few tiles): a workgroup has two such sets of four waves; group g takes turns g, g + 2, … in a ring of its own, and at the end the
 // groups' maxima, sums and accumulators meet in LDS.
+// Two pages a turn: e4m3 with two groups.  µs, one page / two: 2 × 1024 behind 1024 41.7 / 36.5, one of 2048 behind 1500 with 8/1 heads 92.2 / 78.1, 64 behind
+// 1900 54.7 / 46.5 (with 16-byte reads of the pages, which alone give 0.95: 8-byte ones of rows of 32 bytes met in 4 of 16 bank groups).  One group,
+// where three workgroups share a compute unit, keeps one page (two leave two of them: e4m3, five prompts of up to 1333, 55.0 / 56.5; with 8-byte
+// reads 61.4).  bf16 keeps one too: with two groups two pages are 4 % faster, but the maximum of two pages rounds more weights
+// (error against 64 bits 0.00290 → 0.00291; e4m3, where the stored values' own error is four times that, 0.01118 either way).
 //
 // Math on v_mfma_f32_32x32x16_bf16: a wave's 32 query columns are ONE MFMA column set.  Lane (c = lane & 31,
 // hi = lane >> 5) owns column c:
@@ -393,7 +401,7 @@ __device__ __forceinline__ float page_weights32(const f32x16& s, int tok0, int l
   return ps;
 }
 
-template <bool KV8, int GROUPS>
+template <bool KV8, int GROUPS, int NPG>
 __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens,
@@ -405,9 +413,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   constexpr int ESZ = KV8 ? 1 : 2;
   constexpr int PAGE_BYTES = PAGE_ELEMS * ESZ;
   constexpr int NCH = PAGE_BYTES / (16 * 256);
-  constexpr int NSTAGE = 3;
-  constexpr int NDMA = 2 * NCH;
-  constexpr int RING = NSTAGE * 2 * PAGE_BYTES;
+  constexpr int STAGE = NPG * 2 * PAGE_BYTES;               // K and V of a turn's pages
+  constexpr int NSTAGE = NPG == 1 ? 3 : 2;
+  constexpr int FLIGHT = 2 * NCH;                           // (three stages) DMA instructions of a wave for a turn
+  constexpr int RING = NSTAGE * STAGE;
   constexpr int SWAP = GROUPS == 2 ? 4 * 2 * 8192 : 0;      // what two groups exchange at the end
   __shared__ __attribute__((aligned(16))) char smem_all[GROUPS * RING > SWAP ? GROUPS * RING : SWAP];
 
@@ -462,17 +471,18 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   // of 256 12.0 / 12.3 / 12.2).
   const bool both = GROUPS == 2 && !alone && nblk > 7;
   if (GROUPS == 2 && !both && !alone && grp == 1) return;
-  int turns = both ? (nblk + 1) >> 1 : nblk;
+  const int nturn = (nblk + NPG - 1) / NPG;
+  int turns = both ? (nturn + 1) >> 1 : nturn;
   const int step = both ? 2 : 1, start = both ? grp : 0;
   __shared__ int turns_of[2];
   if (alone && lane == 0 && wave == 0) turns_of[grp] = turns;
 
-  // Qᵀ fragments: k-step j covers d = 16 j + 8 hi … + 7 (fp8 pages keep d in 64-wide chunks: same d, other address)
+  // Qᵀ fragments: k-step j covers d = 16 j + 8 hi … + 7; with e4m3 pages, whose 16-byte slots hold two k-steps, d = 32 (j / 2) + 16 hi + 8 (j % 2) … + 7
   bf16x8 qf[8];
   {
-    const uint16_t* qp = q + (int64_t)(qs + min(qtok, n_new - 1)) * q_stride + (kvh * G + head) * HD + 8 * hi;
+    const uint16_t* qp = q + (int64_t)(qs + min(qtok, n_new - 1)) * q_stride + (kvh * G + head) * HD;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) qf[j] = *reinterpret_cast<const bf16x8*>(qp + 16 * j);
+    for (int j = 0; j < 8; ++j) qf[j] = *reinterpret_cast<const bf16x8*>(qp + (KV8 ? 32 * (j >> 1) + 16 * hi + 8 * (j & 1) : 16 * j + 8 * hi));
   }
 
   f32x16 o[4];
@@ -495,32 +505,121 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   }
   using gptr_t = const __attribute__((address_space(1))) void*;
   using lptr_t = __attribute__((address_space(3))) void*;
-#define DLI_STAGE(b_, buf_)                                                                                        \
-  {                                                                                                                \
-    const int64_t page_ = ((int64_t)bt[b_] * Hkv + kvh) * PAGE_BYTES;                                             \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i) {                                                              \
-      char* dst_ = smem + (buf_) * 2 * PAGE_BYTES + (wave + 4 * i) * 1024;                                         \
-      __builtin_amdgcn_global_load_lds((gptr_t)(kc + page_ + src_k[i]), (lptr_t)dst_, 16, 0, 0);                   \
-      __builtin_amdgcn_global_load_lds((gptr_t)(vc + page_ + src_v[i]), (lptr_t)(dst_ + PAGE_BYTES), 16, 0, 0);    \
-    }                                                                                                              \
-  }
+  auto stage_page = [&](int b, char* to) {
+    const int64_t page = ((int64_t)bt[b] * Hkv + kvh) * PAGE_BYTES;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      char* dst = to + (wave + 4 * i) * 1024;
+      __builtin_amdgcn_global_load_lds((gptr_t)(kc + page + src_k[i]), (lptr_t)dst, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_t)(vc + page + src_v[i]), (lptr_t)(dst + PAGE_BYTES), 16, 0, 0);
+    }
+  };
+  auto stage = [&](int turn, int at) {
+#pragma unroll
+    for (int p = 0; p < NPG; ++p)
+      if (p == 0 || NPG * turn + p < nblk) stage_page(NPG * turn + p, smem + at * STAGE + p * 2 * PAGE_BYTES);
+  };
   // Lane offsets inside a staged page.  Rows of 64 bytes (K: token rows of a d chunk; bf16 V: d rows) carry the slot
   // swizzle of their row; it depends on (row >> 2) & 3 only, and every row this lane reads is c32 + a multiple of 32.
   const int swz = slot_swizzle(c32);
-  int k_off[2];                                   // bf16: logical slot 2 (j & 1) + hi;  fp8: slot j & 3, byte 8 hi inside
+  int k_off[2];                                   // logical slot 2 p + hi
 #pragma unroll
   for (int p = 0; p < 2; ++p) k_off[p] = c32 * 64 + (((2 * p + hi) ^ swz) << 4);
-  int k8_off[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) k8_off[p] = c32 * 64 + ((p ^ swz) << 4) + 8 * hi;
   const int v_off0 = c32 * 64 + ((hi ^ swz) << 4), v_off1 = c32 * 64 + (((2 + hi) ^ swz) << 4);
-  const int v8_off = c32 * 32 + 8 * hi;
+  const int v8_off = c32 * 32 + 16 * hi;
 
-  // group g walks pages g, g + 2, … (of a tile of its own: all) in a ring of its own; both pass the same barriers
-  if (start < nblk) DLI_STAGE(start, 0);
-  if (start + step < nblk) {
-    DLI_STAGE(start + step, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+  // NP pages from b on, staged at `kb`: scores, one running maximum, weights, P·V
+  auto pages = [&](auto np, int b, const char* kb) __attribute__((always_inline)) {
+    constexpr int NP = decltype(np)::value;
+    f32x16 s[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[p][r] = 0.f;
+    if constexpr (!KV8) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+          s[p] = mfma32(*reinterpret_cast<const bf16x8*>(kb + p * 2 * PAGE_BYTES + (j >> 1) * 2048 + k_off[j & 1]), qf[j], s[p]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const u32x4 raw = *reinterpret_cast<const u32x4*>(kb + p * 2 * PAGE_BYTES + (j >> 1) * 2048 + k_off[j & 1]);
+          bf16x8 k0, k1;
+          fp8x4_to_bf16(raw[0], k0, 0);
+          fp8x4_to_bf16(raw[1], k0, 4);
+          fp8x4_to_bf16(raw[2], k1, 0);
+          fp8x4_to_bf16(raw[3], k1, 4);
+          s[p] = mfma32(k0, qf[2 * j], s[p]);
+          s[p] = mfma32(k1, qf[2 * j + 1], s[p]);
+        }
+    }
+    const int tok0 = b * 32 + 4 * hi;
+    const bool edge = b * 32 + 32 * NP - 1 > first_tok;
+    float mx = edge ? page_max32<true>(s[0], tok0, qpos) : page_max32<false>(s[0], tok0, qpos);
+#pragma unroll
+    for (int p = 1; p < NP; ++p) mx = fmaxf(mx, edge ? page_max32<true>(s[p], tok0 + 32 * p, qpos) : page_max32<false>(s[p], tok0 + 32 * p, qpos));
+    mx *= scale_log2;
+    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    // The maximum moves with every turn that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
+    // 2^8 saves these 64 products on most pages, 3 – 10 % of a launch, but rounds the largest weight like all others: relative error
+    // against 64 bits 0.00266 → 0.00272, e4m3 pages 0.00731 → 0.00734.)
+    if (__any(mx > m)) {
+      asm volatile("" ::: "memory");
+      const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
+      m = mn;
+      lsum *= alpha;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) o[n] *= alpha;
+    }
+    bf16x8 pb[NP][2];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      lsum += edge ? page_weights32<true>(s[p], tok0 + 32 * p, qpos, scale_log2, m, pb[p]) : page_weights32<false>(s[p], tok0 + 32 * p, qpos, scale_log2, m, pb[p]);
+      if constexpr (KV8) {
+        // 16 bytes of an e4m3 V row are slots 2 hi and 2 hi + 1, not hi and 2 + hi: the weights of slots 1 and 2 change places
+        u32x4 w0 = __builtin_bit_cast(u32x4, pb[p][0]), w1 = __builtin_bit_cast(u32x4, pb[p][1]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          auto x = __builtin_amdgcn_permlane32_swap(w0[e], w1[e], false, false);
+          w0[e] = x[0];
+          w1[e] = x[1];
+        }
+        pb[p][0] = __builtin_bit_cast(bf16x8, w0);
+        pb[p][1] = __builtin_bit_cast(bf16x8, w1);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const char* vb = kb + p * 2 * PAGE_BYTES + PAGE_BYTES;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        bf16x8 v0, v1;                           // row d = 32 n + c32: the A fragments of the two k-steps
+        if constexpr (!KV8) {
+          v0 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off0);
+          v1 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off1);
+        } else {
+          const u32x4 raw = *reinterpret_cast<const u32x4*>(vb + n * 1024 + v8_off);
+          fp8x4_to_bf16(raw[0], v0, 0);
+          fp8x4_to_bf16(raw[1], v0, 4);
+          fp8x4_to_bf16(raw[2], v1, 0);
+          fp8x4_to_bf16(raw[3], v1, 4);
+        }
+        o[n] = mfma32(v0, pb[p][0], o[n]);
+        o[n] = mfma32(v1, pb[p][1], o[n]);
+      }
+    }
+  };
+
+  // group g takes turns g, g + 2, … (of a tile of its own: all) in a ring of its own; both pass the same barriers
+  if (start < nturn) stage(start, 0);
+  if (NSTAGE == 3 && start + step < nturn) {
+    stage(start + step, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLIGHT) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
@@ -528,65 +627,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   if (alone) turns = max(turns_of[0], turns_of[1]);
   int st = 0;
   for (int t = 0; t < turns; ++t) {
-    const int b = step * t + start;
-    const bool ahead = b + 2 * step < nblk;
-    const int st2 = st == 0 ? NSTAGE - 1 : st - 1;
-    if (ahead) DLI_STAGE(b + 2 * step, st2);
-    if (b < my_nblk) {
-      const char* kb = smem + st * 2 * PAGE_BYTES;
-      const char* vb = kb + PAGE_BYTES;
-      f32x16 s;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        bf16x8 kf;
-        if constexpr (!KV8) {
-          kf = *reinterpret_cast<const bf16x8*>(kb + (j >> 1) * 2048 + k_off[j & 1]);
-        } else {
-          const uint2 raw = *reinterpret_cast<const uint2*>(kb + (j >> 2) * 2048 + k8_off[j & 3]);
-          fp8x4_to_bf16(raw.x, kf, 0);
-          fp8x4_to_bf16(raw.y, kf, 4);
-        }
-        s = mfma32(kf, qf[j], s);
-      }
-      bf16x8 pb[2];
-      const int tok0 = b * 32 + 4 * hi;
-      const bool edge = b * 32 + 31 > first_tok;
-      float mx = (edge ? page_max32<true>(s, tok0, qpos) : page_max32<false>(s, tok0, qpos)) * scale_log2;
-      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      // The maximum moves with every page that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
-      // 2^8 saves these 64 products on most pages, 3 – 10 % of a launch, but rounds the largest weight like all others: relative error
-      // against 64 bits 0.00266 → 0.00272, e4m3 pages 0.00731 → 0.00734.)
-      if (__any(mx > m)) {
-        asm volatile("" ::: "memory");
-        const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
-        m = mn;
-        lsum *= alpha;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) o[n] *= alpha;
-      }
-      lsum += edge ? page_weights32<true>(s, tok0, qpos, scale_log2, m, pb) : page_weights32<false>(s, tok0, qpos, scale_log2, m, pb);
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        bf16x8 v0, v1;                           // slots hi and 2 + hi of row d = 32 n + c32: the A fragments of the two k-steps
-        if constexpr (!KV8) {
-          v0 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off0);
-          v1 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off1);
-        } else {
-          const uint2 r0 = *reinterpret_cast<const uint2*>(vb + n * 1024 + v8_off);
-          const uint2 r1 = *reinterpret_cast<const uint2*>(vb + n * 1024 + v8_off + 16);
-          fp8x4_to_bf16(r0.x, v0, 0);
-          fp8x4_to_bf16(r0.y, v0, 4);
-          fp8x4_to_bf16(r1.x, v1, 0);
-          fp8x4_to_bf16(r1.y, v1, 4);
-        }
-        o[n] = mfma32(v0, pb[0], o[n]);
-        o[n] = mfma32(v1, pb[1], o[n]);
-      }
-    }
-    if (ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+    const int turn = step * t + start;
+    const bool ahead = turn + (NSTAGE - 1) * step < nturn;
+    if (ahead) stage(turn + (NSTAGE - 1) * step, st == 0 ? NSTAGE - 1 : st - 1);
+    const char* kb = smem + st * STAGE;
+    if (NPG == 2 && 2 * turn + 1 < my_nblk) pages(std::integral_constant<int, 2>{}, 2 * turn, kb);
+    else if (NPG * turn < my_nblk) pages(std::integral_constant<int, 1>{}, NPG * turn, kb);
+    if (NSTAGE == 3 && ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLIGHT) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     st = st == NSTAGE - 1 ? 0 : st + 1;
@@ -645,7 +692,6 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
         }
     }
   }
-#undef DLI_STAGE
 }
 
 // ---- launchers -------------------------------------------------------------------------------------
@@ -752,12 +798,12 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
   const int form = prefill_page_groups(num_tiles, Hkv, Hq / Hkv, longest, sequences, kv_fp8), groups = form == 1 ? 1 : 2;
   const int units = form == 3 ? PREFILL_UNITS : num_tiles * Hkv;
   const dim3 grid(std::min(num_tiles * Hkv, units));
-#define DLI_PREFILL_GO(KV8_, G_)                                                                                              \
-  hipLaunchKernelGGL((paged_prefill_kernel<KV8_, G_>), grid, dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, v_cache, \
+#define DLI_PREFILL_GO(KV8_, G_, N_)                                                                                              \
+  hipLaunchKernelGGL((paged_prefill_kernel<KV8_, G_, N_>), grid, dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, v_cache, \
                      block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, Hq, Hkv, num_tiles, \
                      scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, counts, units)
-  if (kv_fp8) { if (groups == 2) DLI_PREFILL_GO(true, 2); else DLI_PREFILL_GO(true, 1); }
-  else { if (groups == 2) DLI_PREFILL_GO(false, 2); else DLI_PREFILL_GO(false, 1); }
+  if (kv_fp8) { if (groups == 2) DLI_PREFILL_GO(true, 2, 2); else DLI_PREFILL_GO(true, 1, 1); }
+  else { if (groups == 2) DLI_PREFILL_GO(false, 2, 1); else DLI_PREFILL_GO(false, 1, 1); }
 #undef DLI_PREFILL_GO
 }
 
