@@ -309,12 +309,19 @@ __device__ __forceinline__ uint32_t radix_cut16(uint4 (&regs)[NCH], float inv_t_
 // fixed order.  The logits of the shared bin count as ± its bound there: at most 2^-32 of max(|zmax|, 128 − zmax), i.e. a relative error of
 // 1e-7 where their weights are not zero beside the largest.  A cut-off inside the shared bin, or a row with +inf or NaN, is left to
 // radix_cut16; one outside the bins too, unless all logits there are equal.  The atomics and the row's
-// arrival at one compute unit bound it: 23 µs a launch at V = 128256 up to 256 filtered rows (radix descents of the whole row: 235).
+// arrival at one compute unit bound it: 20 µs a launch at V = 128256 up to 256 filtered rows (radix descents of the whole row: 235).
 // Position d runs from the largest value down: positive magnitude index c at MBINS − 1 − c, negative at MBINS + c.
 constexpr int MBINS = 4096;
 constexpr int BINS_PER_THREAD = 2 * MBINS / SNT;
-// LDS word of position d: thread t scans positions 8 t … 8 t + 7, rotated so that the lanes of a read fall on different banks
-__device__ __forceinline__ int bin_word(int d) { return (d & ~7) | ((d + (d >> 3)) & 7); }
+static_assert(BINS_PER_THREAD == 8, "scan_cut reads a thread's bins as two 16-byte words");
+// position of the logit in half `odd` of a word: MBINS + i for a negative one, MBINS - 1 - i = MBINS + ~i for another, i = max(magnitude - lo, 0).  Five
+// instructions a logit with the address; rotated positions and maxima of values, one logit at a time, took twice as many (V = 128256: a launch 22.5 → 20 µs).
+template <int ODD> __device__ __forceinline__ int bin_of(uint32_t word, int lo) {
+  const uint32_t mag = __builtin_amdgcn_ubfe(word, 16 * ODD, 15);
+  const int i = (int)__builtin_elementwise_sub_sat(mag, (uint32_t)lo);
+  const int neg = __builtin_amdgcn_sbfe((int)word, 16 * ODD + 15, 1);                // -1: negative
+  return MBINS + ~(i ^ neg);
+}
 
 struct CutScratch {
   float wave_tot[SNT / 64];
@@ -329,10 +336,12 @@ __device__ __forceinline__ int scan_cut(const uint32_t* counts, int lo, float in
                                         CutScratch* s) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   float w[BINS_PER_THREAD], local = 0.f;
+  const uint4 c0 = reinterpret_cast<const uint4*>(counts)[2 * t], c1 = reinterpret_cast<const uint4*>(counts)[2 * t + 1];
+  const uint32_t cnt[BINS_PER_THREAD] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
 #pragma unroll
   for (int j = 0; j < BINS_PER_THREAD; ++j) {
     const int d = t * BINS_PER_THREAD + j;
-    const uint32_t n = d <= d_last ? counts[bin_word(d)] : 0u;
+    const uint32_t n = d <= d_last ? cnt[j] : 0u;
     const int c = d < MBINS ? MBINS - 1 - d : d - MBINS;
     const float x = bf2f((uint16_t)(c + lo)) * (d < MBINS ? inv_t_log2 : -inv_t_log2);
     w[j] = n == 0u ? 0.f : MASS ? (float)n * fast_exp2(x - zmax) : (float)n;
@@ -390,16 +399,20 @@ __device__ __forceinline__ void count_logits(uint4 (&regs)[NCH], int nchunks, in
 #pragma clang loop unroll(full)
   for (int c = 0; c < NCH; ++c) {
     if (c * SNT + (int)threadIdx.x < nchunks) {
+      const uint32_t words[4] = {regs[c].x, regs[c].y, regs[c].z, regs[c].w};
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint32_t h = half_of(regs[c], e);
-        const int m = (int)(h & 0x7FFFu), i = max(m - lo, 0);
-        if (!FAR || m <= top) {
-          atomicAdd(&counts[bin_word((h & 0x8000u) ? MBINS + i : MBINS - 1 - i)], 1u);
-        } else {
-          far_any |= (uint32_t)m;
-          far_all &= (uint32_t)m;
+        const uint32_t word = words[e >> 1];
+        const int d = e & 1 ? bin_of<1>(word, lo) : bin_of<0>(word, lo);
+        if (FAR) {
+          const int m = (int)((e & 1 ? word >> 16 : word) & 0x7FFFu);
+          if (m > top) {
+            far_any |= (uint32_t)m;
+            far_all &= (uint32_t)m;
+            continue;
+          }
         }
+        atomicAdd(&counts[d], 1u);
       }
     }
     __builtin_amdgcn_sched_barrier(0);        // one chunk at a time: keeps the row registers the only long-lived ones
@@ -438,20 +451,38 @@ __device__ __forceinline__ uint32_t row_cut(uint4 (&regs)[NCH], int nchunks, int
   for (int i = threadIdx.x; i < 2 * MBINS; i += SNT) counts[i] = 0u;
 
   const float inv_t_log2 = 1.4426950408889634f / temp;    // z = x / T in log2 units
-  float vmax = -3.0e38f;
-  uint32_t mag_max = 0;
+  // Largest value and largest magnitude, two logits an instruction: as signed 16-bit numbers positive logits are in order and above all negative
+  // ones, and negative ones are in reverse order.
+  typedef short s16x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  s16x2 hi2 = {-32768, -32768}, lo2 = {32767, 32767};
+  u16x2 mag2 = {0, 0};
 #pragma clang loop unroll(full)
   for (int c = 0; c < NCH; ++c) {
-    const bool in = c * SNT + (int)threadIdx.x < nchunks;
+    if (c * SNT + (int)threadIdx.x < nchunks) {
+      const uint32_t words[4] = {regs[c].x, regs[c].y, regs[c].z, regs[c].w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t h = half_of(regs[c], e);
-      vmax = fmaxf(vmax, bf2f((uint16_t)h));
-      mag_max = max(mag_max, in ? h & 0x7FFFu : 0u);
+      for (int e = 0; e < 4; ++e) {
+        const s16x2 w = __builtin_bit_cast(s16x2, words[e]);
+        hi2 = __builtin_elementwise_max(hi2, w);
+        lo2 = __builtin_elementwise_min(lo2, w);
+        mag2 = __builtin_elementwise_max(mag2, __builtin_bit_cast(u16x2, words[e] & 0x7FFF7FFFu));
+      }
     }
   }
-  vmax = block_max(vmax, sv);
-  const int mag = (int)block_max((float)mag_max, sv);       // (a 15-bit whole number is exact in fp32)
+  const int hi = (int)block_max((float)max(hi2[0], hi2[1]), sv), low = -(int)block_max(-(float)min(lo2[0], lo2[1]), sv);
+  const int mag = (int)block_max((float)max(mag2[0], mag2[1]), sv);         // (whole numbers of 16 bits are exact in fp32)
+  float vmax = bf2f((uint16_t)(hi >= 0 ? hi : low));
+  if (mag > 0x7F80) {                                       // NaN among them: the largest of the others
+    vmax = -3.0e38f;
+#pragma clang loop unroll(full)
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vmax = fmaxf(vmax, bf2f((uint16_t)half_of(regs[c], e)));
+    }
+    vmax = block_max(vmax, sv);
+  }
+  vmax = fmaxf(vmax, -3.0e38f);
   const float zmax = vmax * inv_t_log2;
   uint32_t floor_key = 0;                                   // 16-bit key of the raw bf16 logit (x → x/T is monotone)
   bool exact = mag <= 0x7F80 && vmax > -3.0e38f && vmax < 3.4e38f;      // no NaN; a finite maximum
