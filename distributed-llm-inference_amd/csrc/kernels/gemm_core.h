@@ -1,11 +1,12 @@
-// K loop of the large matrix products: a workgroup of four waves multiplies a 256 × 256 (or 128 × 256) tile, each wave 128 × 128 (64 × 128)
-// of it, C[rows, n] = A[rows, :] · W[n, :]ᵀ, operands of two bytes (bf16) or one (e4m3), sums in fp32.
+// K loop of the large e4m3 products: a workgroup of four waves multiplies a 256 × 256 (or 128 × 256) tile, each wave 128 × 128 (64 × 128)
+// of it, C[rows, n] = A[rows, :] · W[n, :]ᵀ, sums in fp32.  (The same loop on bf16 operands, twice the instructions of half the length,
+// took 312 µs for 4096 × 4096 × 14336 where the eight-wave tile of gemm256.hip takes 305: both run at the clock that the card's power allows.)
 //
-//   * A K-step is 128 bytes of every row: 64 bf16 or 128 e4m3.  Both run the matrix cores for 2048 cycles per step of a 256² tile.
+//   * A K-step is 128 bytes of every row, 2048 cycles of the matrix cores for a 256² tile.
 //   * One wave per SIMD and the largest wave tile its registers hold (256 accumulators + 128 fragment registers of 512): a step reads
 //     128 KB of fragments from LDS, where eight waves of 128 × 64 read 192 KB — beside the 64 KB the DMA writes, that alone fills the LDS
 //     port for as long as the matrix cores need.
-//   * Matrix instructions are issued in program order and take 16 (bf16) or 32 (e4m3) cycles each; what else the wave has to issue
+//   * Matrix instructions are issued in program order and take 32 cycles each; what else the wave has to issue
 //     (fragment reads of the NEXT quadrant, LDS-DMA of the step after next) stands between them, one at a time, so nothing waits.
 //   * Both operands go global → LDS by LDS-DMA, two step buffers.  The LDS image is lane-linear: slot p of row r holds 16-byte chunk
 //     p ^ (r & 7), applied on the source address and on the read; ds_read_b128 then has no bank conflicts.
@@ -40,16 +41,11 @@ __device__ __forceinline__ int b_piece_row(int h, int piece) { return (piece >> 
 // and target apart, and with 256 + 128 registers taken the allocator then moved accumulators about in the loop and spilled 70.  The
 // compiler does not see a matrix instruction here, so the waits are ours: two cycles behind a write of an operand by a vector instruction
 // (the s_nop; the matrix pipe is busy longer), and before anything but another product reads a sum (behind the K loop).
-// e4m3: 16 × 16 × 128, a lane's 32 bytes are chunks g and 4 + g of its row (both operands alike: any order of k will do).
-template <bool E4M3>
-__device__ __forceinline__ void mma(const u32x4 (&w)[2], const u32x4 (&a)[2], int ks, f32x4& c) {
-  if constexpr (E4M3) {
-    const i32x8 wv = __builtin_bit_cast(i32x8, __builtin_shufflevector(w[0], w[1], 0, 1, 2, 3, 4, 5, 6, 7));
-    const i32x8 av = __builtin_bit_cast(i32x8, __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7));
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(wv), "v"(av));
-  } else {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w[ks]), "v"(a[ks]));
-  }
+// A lane's 32 bytes are chunks g and 4 + g of its row (both operands alike: any order of k will do).
+__device__ __forceinline__ void mma(const u32x4 (&w)[2], const u32x4 (&a)[2], f32x4& c) {
+  const i32x8 wv = __builtin_bit_cast(i32x8, __builtin_shufflevector(w[0], w[1], 0, 1, 2, 3, 4, 5, 6, 7));
+  const i32x8 av = __builtin_bit_cast(i32x8, __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7));
+  asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(wv), "v"(av));
 }
 
 // Runs `tiles.count` tiles of nk K-steps each (an even number: the buffers change places), one stream of steps: behind a tile's last step the DMA goes on with the next tile's
@@ -58,12 +54,11 @@ __device__ __forceinline__ void mma(const u32x4 (&w)[2], const u32x4 (&a)[2], in
 //     DMA piece wave · (pieces per wave) + j of half h; may fetch into LDS what store(i) needs (landed by then, ring of four tiles)
 //   tiles.store(i, lane, wave, acc): acc[m][n]: rows wr·16·MB + m·16 + (lane & 15), columns wc·128 + n·16 + 4 (lane >> 4) + r;
 //     true: it issued exactly MB · 4 vector memory instructions (whole tiles), else any number
-template <bool E4M3, int MB, class Tiles>
+template <int MB, class Tiles>
 __device__ __forceinline__ void stream_tiles(char* lds, Tiles& tiles, int nk) {
   constexpr int A_TILE = tile_rows<MB> * STEP_BYTES, W_TILE = TN * STEP_BYTES;
   constexpr int HB = MB / 2;                                 // row blocks of a quadrant
-  constexpr int KS = E4M3 ? 1 : 2;                           // matrix instructions per block and step
-  constexpr int NMMA = HB * 4 * KS;                          // of a quadrant
+  constexpr int NMMA = HB * 4;                               // matrix instructions of a quadrant
   constexpr int FLIGHT = MB + 8;                             // DMA instructions of a wave in a step
   constexpr int STORES = MB * 4;
   if (tiles.count <= 0) return;
@@ -116,8 +111,8 @@ __device__ __forceinline__ void stream_tiles(char* lds, Tiles& tiles, int nk) {
   // instruction (n_dma, evenly over the quadrant's second half)
 #define GC_QUAD(MH, NH, n_rd, RD, n_dma, DMA)                                                                      \
   _Pragma("unroll") for (int i = 0; i < NMMA; ++i) {                                                               \
-    const int ks = i / (HB * 4), b = i % (HB * 4), m = b >> 2, n = b & 3;                                          \
-    mma<E4M3>(fw[NH][n], fa[MH][m], ks, acc[(MH) * HB + m][(NH) * 4 + n]);                                         \
+    const int m = i >> 2, n = i & 3;                                                                               \
+    mma(fw[NH][n], fa[MH][m], acc[(MH) * HB + m][(NH) * 4 + n]);                                                   \
     constexpr int first = NMMA / 2, rd_gap = first / (n_rd) > 0 ? first / (n_rd) : 1, dma_gap = first / (n_dma);   \
     if (i % rd_gap == 0 && i / rd_gap < (n_rd)) { const int x = i / rd_gap; RD; }                                  \
     if (i >= first && (i - first) % dma_gap == 0 && (i - first) / dma_gap < (n_dma)) { const int x = (i - first) / dma_gap; DMA; } \

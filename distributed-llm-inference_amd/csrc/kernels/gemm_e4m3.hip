@@ -121,9 +121,9 @@ struct Tiles {
 __global__ __launch_bounds__(256, 1) void gemm_e4m3_kernel(Args p) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   Tiles<8> whole(p, lds);
-  stream_tiles<true, 8>(lds, whole, p.K / STEP_BYTES);
+  stream_tiles<8>(lds, whole, p.K / STEP_BYTES);
   Tiles<4> halves(p, lds);
-  stream_tiles<true, 4>(lds, halves, p.K / STEP_BYTES);
+  stream_tiles<4>(lds, halves, p.K / STEP_BYTES);
 }
 
 }  // namespace ge4
