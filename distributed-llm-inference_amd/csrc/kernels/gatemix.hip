@@ -835,7 +835,7 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
 
 // The walk of the delta rule: per (sequence, head, 16·CT state columns) over its blocks in order, the state on the accumulators.  A block is
 //   [o | x] = [Q̃ | W] S, u = U0 - x → LDS → o += A u, S = e^{P_end} ⊙ S + K̃ᵀ u → LDS,
-// two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 85 µs (36 of them fp32 matrix instructions, were they spread
+// two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 75 µs (36 of them fp32 matrix instructions, were they spread
 // evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83.  The next block's tiles are fetched as soon as
 // their registers are free and without a condition (the last block fetches itself again): behind a condition the compiler has to wait for
 // everything that is in flight.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
@@ -843,16 +843,30 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
 template <int DTMAX, int CT, bool FULL>
 __global__ __launch_bounds__(NT) void delta_walk_kernel(float* __restrict__ state, const int* __restrict__ positions,
                                                         const int* __restrict__ qsl, const int* __restrict__ state_slots,
-                                                        const int* __restrict__ counts, int H, int D, int Dv, const float* __restrict__ ws,
-                                                        float* __restrict__ out) {
+                                                        const int* __restrict__ counts, int H, int D, int Dv, int by_length,
+                                                        const float* __restrict__ ws, float* __restrict__ out) {
   constexpr int DW = (DTMAX + 3) / 4;                     // state row tiles per wave: wave, wave + 4, …
   __shared__ __align__(16) float St[DTMAX * CT * TILE], Ut[4 * CT * TILE];
-  const int h = blockIdx.x, seq = blockIdx.z;             // a head's column slices share an XCD (its tiles stay in one L2)
-  if (seq >= counts[3]) return;
+  const int h = blockIdx.x, seqs = counts[3];             // a head's column slices share an XCD (its tiles stay in one L2)
+  int seq = blockIdx.z;
+  if (seq >= seqs) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
+  if (by_length && seqs <= 64) {
+    // Longest first, every second round of one workgroup a compute unit in reverse, so that the long chains share theirs with the short ones (four
+    // sequences of 512 to 1069 tokens, 16 heads of 128, 85 → 75 µs).
+    const int len = lane < seqs ? qsl[lane + 1] - qsl[lane] : -1;
+    int rank = 0;
+    for (int j = 0; j < seqs; ++j) {
+      const int other = __builtin_amdgcn_readlane(len, j);
+      rank += other > len || (other == len && j < lane) ? 1 : 0;
+    }
+    const int per = max(1, 256 / (int)(gridDim.x * gridDim.y)), round = seq / per, in = seq - round * per, last = min(per, seqs - round * per) - 1;
+    const int want = round * per + (round & 1 ? last - in : in);
+    seq = __ffsll((long long)__ballot(lane < seqs && rank == want)) - 1;
+  }
   const int s0 = qsl[seq], n = qsl[seq + 1] - s0;
   const int slot = state_slots[seq];
   if (slot < 0 || n < 2) return;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
   const DeltaSpace sp(D, Dv);
   const int DT = FULL ? DTMAX : sp.DT, ct0 = blockIdx.y * CT;
   float* head = state + ((int64_t)slot * H + h) * D * Dv;
@@ -1262,8 +1276,11 @@ static void delta_walk(float* state, const int* positions, const int* qsl, const
   // one a tile; single tokens beside them end at once.)
   const int ct = (int64_t)H * ((Dv + 15) / 16) * std::min(seqs, num_tiles) > 512 ? 2 : 1;
   const dim3 grid(H, (Dv + 16 * ct - 1) / (16 * ct), seqs);
+  // sequences in order of their length where they have more than two blocks on average: finding the order takes a workgroup 0.5 µs (15 of up to 69 tokens,
+  // 32 heads: 111.1 µs a layer without, 113.4 with)
+  const int by_length = seqs > 1 && num_tiles > 2 * seqs;
 #define GM_WALK(DT, CTV, FULLV)                                                                                                               \
-  hipLaunchKernelGGL((delta_walk_kernel<DT, CTV, FULLV>), grid, dim3(NT), 0, stream, state, positions, qsl, state_slots, counts, H, D, Dv, ws, out)
+  hipLaunchKernelGGL((delta_walk_kernel<DT, CTV, FULLV>), grid, dim3(NT), 0, stream, state, positions, qsl, state_slots, counts, H, D, Dv, by_length, ws, out)
 #define GM_WALK_D(DT)                                             \
   do {                                                            \
     if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
