@@ -420,12 +420,13 @@ __device__ __forceinline__ void count_logits(uint4 (&regs)[NCH], int nchunks, in
 }
 
 struct CutShared {
-  uint32_t counts[2 * MBINS];
+  alignas(16) uint32_t counts[2 * MBINS];
   float sv[SNT / 64];
   CutScratch cs;
   uint32_t pick;
   float rem;
 };
+static_assert(alignof(CutShared) % 16 == 0, "scan_cut reads the counts 16 bytes at a time");
 
 // what a row asks for; k is set to V where there is no top-k
 __device__ __forceinline__ bool needs_cut(float temp, float p, int& k, int V) {
