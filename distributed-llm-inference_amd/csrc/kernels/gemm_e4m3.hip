@@ -23,6 +23,11 @@ constexpr int TURN = stage_bytes<8>;                         // LDS behind the s
 constexpr int SCALES = TURN + 4 * 4096;                      // [4 tiles][256 row scales, 256 column scales]
 constexpr int LDS_BYTES = SCALES + 4 * 2048;
 
+// byte offset, inside the operand that starts at it, of lane `lane`'s 16 bytes of row r (swizzled as the LDS image is).  Rows of a weight
+// tile lie up to 255 · K bytes apart, K up to 2^24: beyond the signed range.
+constexpr __host__ __device__ uint32_t chunk_offset(int r, int K, int lane) { return (uint32_t)r * (uint32_t)K + (uint32_t)(((lane & 7) ^ (r & 7)) << 4); }
+static_assert(chunk_offset(255, (1 << 24) - 256, 0) == 255u * ((1u << 24) - 256u) + 112u, "the last row of a tile at the largest K");
+
 struct Args {
   const uint8_t* X;
   int64_t x_stride;
@@ -76,7 +81,7 @@ struct Tiles {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int r = b_piece_row(h, wave * 4 + j) + (lane >> 3);
-        w_src[h][j] = (uint32_t)(r * p.K + (((lane & 7) ^ (r & 7)) << 4));
+        w_src[h][j] = chunk_offset(r, p.K, lane);
       }
     }
     char* s = lds + SCALES + (i & 3) * 2048;
