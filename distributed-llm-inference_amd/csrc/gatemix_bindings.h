@@ -59,6 +59,13 @@ std::tuple<Tensor, Tensor, Tensor> gm_max_gates(const Tensor& g, const Tensor& b
   return {keep, write, floor_};
 }
 
+// bytes that a step of these extents takes beside its results (num_tiles: of 64 tokens), for whoever sizes a cache
+int64_t gm_scan_workspace_bytes(int64_t rows, int64_t num_seqs, int64_t num_tiles, int64_t H, int64_t D, int64_t Dv, bool delta) {
+  if (num_tiles <= 0 || D > dli::gm_block_max_dim()) return 0;
+  return 4 * (delta ? dli::gm_delta_ws_floats((int)num_seqs, (int)num_tiles, (int)H, (int)D, (int)Dv)
+                    : dli::gm_scan_ws_floats((int)rows, (int)num_seqs, (int)H));
+}
+
 // the recurrence with a gated matrix state (see ops/seqmix.py: gated_scan) → (o fp32 [T, H·Dv], n · q fp32 [T, H] or empty)
 std::tuple<Tensor, Tensor> gm_gated_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& decay, const Tensor& weight,
                                          Tensor state, const Tensor& positions, const Tensor& qsl, const Tensor& state_slots,
@@ -92,7 +99,7 @@ std::tuple<Tensor, Tensor> gm_gated_scan(const Tensor& q, const Tensor& k, const
     TORCH_CHECK(tile_seq->numel() >= num_tiles && tile_q0->numel() >= num_tiles, "tile lists shorter than num_tiles");
     tsp = tile_seq->data_ptr<int>();
     tqp = tile_q0->data_ptr<int>();
-    ws = at::empty({delta ? dli::gm_delta_ws_floats((int)T, (int)num_seqs, (int)H, (int)D, (int)Dv) : dli::gm_scan_ws_floats((int)T, (int)num_seqs, (int)H)},
+    ws = at::empty({delta ? dli::gm_delta_ws_floats((int)num_seqs, (int)num_tiles, (int)H, (int)D, (int)Dv) : dli::gm_scan_ws_floats((int)T, (int)num_seqs, (int)H)},
                    state.options());
   } else {
     num_tiles = 0;
@@ -139,7 +146,7 @@ Tensor gm_channel_scan(const Tensor& q, const Tensor& k, const Tensor& v, const 
     TORCH_CHECK(tile_seq->numel() >= num_tiles && tile_q0->numel() >= num_tiles, "tile lists shorter than num_tiles");
     tsp = tile_seq->data_ptr<int>();
     tqp = tile_q0->data_ptr<int>();
-    ws = at::empty({dli::gm_delta_ws_floats((int)T, (int)num_seqs, (int)H, (int)D, (int)Dv)}, state.options());
+    ws = at::empty({dli::gm_delta_ws_floats((int)num_seqs, (int)num_tiles, (int)H, (int)D, (int)Dv)}, state.options());
   } else {
     num_tiles = 0;
   }

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(NTH) void max_gates_kernel(const A* __restrict__ g,
 
 // Token by token: one workgroup per (sequence, head, 64 state columns); wave v keeps rows v·DR … of its lane's column in registers,
 // the workgroup of the first columns also the normaliser.  Serves single tokens (and, with single_only = 0, whole chunks: sizes
-// the block path does not take).
+// the block path does not take).  For the delta rule's block path it also notes where a chunk's workspace rows begin (first_row).
 //
 // Channel decays (Z, the type of z, not void; delta rule): g[d] = exp(-rate[h] · softplus(z[t, h, d] + bias[h, d])) instead of exp(decay).
 template <typename Z> struct ChannelArgs {
@@ -250,13 +250,26 @@ __global__ __launch_bounds__(NT) void scan_step_kernel(const A* __restrict__ q, 
                                                        const int* __restrict__ positions, const int* __restrict__ qsl,
                                                        const int* __restrict__ state_slots, const int* __restrict__ counts, int H, int G,
                                                        int D, int Dv, float q_scale, float* __restrict__ out, float* __restrict__ nq,
-                                                       int single_only, ChannelArgs<Z> ch) {
+                                                       int single_only, int* __restrict__ first_row, ChannelArgs<Z> ch) {
   constexpr bool CHAN = !std::is_void_v<Z>;
   __shared__ float qs[DRMAX * 4], ks[DRMAX * 4], gs[CHAN ? DRMAX * 4 : 1], red[4][64], red2[4][64], sred[NT / 64];
   const int h = blockIdx.x, seq = blockIdx.z;
   if (seq >= counts[3]) return;
   const int t0 = qsl[seq], t1 = qsl[seq + 1];
   const int slot = state_slots[seq];
+  if (DELTA && first_row != nullptr && t1 - t0 > 1 && slot >= 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+    __shared__ int blocks_of[NT / 64];
+    int before = 0;                                       // blocks of the chunks of earlier batch rows
+    for (int j = threadIdx.x; j < seq; j += NT) {
+      const int n = qsl[j + 1] - qsl[j];
+      before += n > 1 && state_slots[j] >= 0 ? (n + BT - 1) / BT : 0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if ((threadIdx.x & 63) == 0) blocks_of[threadIdx.x >> 6] = before;
+    __syncthreads();
+    if (threadIdx.x == 0) first_row[seq] = (blocks_of[0] + blocks_of[1]) + (blocks_of[2] + blocks_of[3]);
+  }
   if (slot < 0 || t1 <= t0 || (single_only && t1 - t0 != 1)) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int e = blockIdx.y * 64 + lane;
@@ -343,13 +356,15 @@ __global__ __launch_bounds__(NT) void scan_step_kernel(const A* __restrict__ q, 
 //     refilled as soon as it has been used).  The normaliser n = exp(P_end) n0 + Σ_j exp(P_end - P_j) w_j k_j and its product with q
 //     ride on the fragments of the first columns' workgroup.
 // Workspace row of a block = (first token >> 6) + batch row (unique: rows of later sequences start at later tokens): per head
-// [64][64] A | [3][64] vectors.  The delta rule has kernels of its own (below): of its block form only
+// [64][64] A | [3][64] vectors, 34 KB.  The delta rule has kernels of its own (below): of its block form only
 //   U = U0 - W S0, O = Q̃ S0 + A U, S = e^{P_end} ⊙ S0 + K̃ᵀ U  with  [W | U0] = (I + M)⁻¹ diag(w) [diag(e^P) K | V]
 // depends on the state, so W and U0 are solved for with all blocks side by side and the walk over the blocks is three products.
 constexpr int64_t scan_block_floats = BT * BT + 3 * BT;
 
-// Workspace of the delta rule per (block, head), all matrices as 16 × 16 tiles in the order in which a wave's lanes read them (1 KB each):
-// A [4][4] | e^{P_end} [DP] | Q̃ [4][DT] | W [4][DT] | K̃ᵀ [DT][4] | U0 [CV][4], DP = 16 DT, CV 16-column tiles of values
+// Workspace of the delta rule: a row per (block, head), all matrices as 16 × 16 tiles in the order in which a wave's lanes read them (1 KB each):
+// A [4][4] | e^{P_end} [DP] | Q̃ [4][DT] | W [4][DT] | K̃ᵀ [DT][4] | U0 [CV][4], DP = 16 DT, CV 16-column tiles of values; 148 KB at 128 × 128, so
+// single tokens take none: chunks have theirs one behind the other, as many as the step has tiles, and behind them a table of the first one of
+// each.  (By (first token >> 6) + batch row a step of 8192 tokens and 512 sequences took 2.8 GB for 32 heads.)
 constexpr int TILE = 256;
 struct DeltaSpace {
   int DT, CV;
@@ -361,6 +376,8 @@ struct DeltaSpace {
   __host__ __device__ int u() const { return kt() + 4 * DT * TILE; }
   __host__ __device__ int64_t floats() const { return u() + (int64_t)4 * CV * TILE; }
 };
+// workspace row of block b of a chunk (of a chunk that the tile list lacks: some row, never one past them)
+__device__ __forceinline__ int64_t block_row(int first, int b, int num_tiles) { return min((unsigned)(first + b), (unsigned)(num_tiles - 1)); }
 // A tile as the A operand: lane row + 16 (k / 4) holds 4 consecutive k.  As the B operand, and as a product leaves it: lane column + 16 (row / 4)
 // holds 4 consecutive rows.  turned(): from either form to the other one, a product with the unit matrix (exact); the kernels below store
 // every tile as 1 KB in lane order (4-byte stores of the turned order: channel_block_kernel 87 → 83 µs at 51 blocks of 16 heads of 128).
@@ -552,7 +569,8 @@ __global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict_
                                                          const float* __restrict__ weight, const int* __restrict__ qsl,
                                                          const int* __restrict__ state_slots, const int* __restrict__ counts,
                                                          const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int num_tiles, int H,
-                                                         int G, int D, int Dv, int wide, float q_scale, float* __restrict__ ws) {
+                                                         int G, int D, int Dv, int wide, float q_scale, const int* __restrict__ first_row,
+                                                         float* __restrict__ ws) {
   __shared__ double P[BT];
   __shared__ float wt[BT];
   __shared__ __align__(16) float M[BT * BS];
@@ -567,7 +585,7 @@ __global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict_
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
   const int g = h / (H / G);
   const DeltaSpace sp(D, Dv);
-  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * sp.floats();
+  float* wa = ws + (block_row(first_row[seq], (t0 - s0) / BT, num_tiles) * H + h) * sp.floats();
   if (wave == 0) {
     double p = lane < n ? (double)decay[(int64_t)(t0 + lane) * H + h] : 0.0;
 #pragma unroll
@@ -698,7 +716,7 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
                                                            const int* __restrict__ qsl, const int* __restrict__ state_slots,
                                                            const int* __restrict__ counts, const int* __restrict__ tile_seq,
                                                            const int* __restrict__ tile_q0, int num_tiles, int H, int G, int D, int Dv, int wide,
-                                                           float* __restrict__ ws) {
+                                                           const int* __restrict__ first_row, float* __restrict__ ws) {
   __shared__ float wt[BT];
   __shared__ __align__(16) float M[BT * BS];
   __shared__ __align__(16) float KR[2][BT][20], EM[2][4][16];
@@ -713,7 +731,7 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g4 = lane >> 4, c = lane & 15;
   const int g = h / (H / G);
   const DeltaSpace sp(D, Dv);
-  float* wa = ws + ((int64_t)((t0 >> 6) + seq) * H + h) * sp.floats();
+  float* wa = ws + (block_row(first_row[seq], (t0 - s0) / BT, num_tiles) * H + h) * sp.floats();
   if (wave == 0) wt[lane] = lane < n ? weight[(int64_t)(t0 + lane) * H + h] : 0.f;
   const int row = 16 * wave + c;
   const float wl = row < n ? weight[(int64_t)(t0 + row) * H + h] : 0.f;
@@ -843,8 +861,9 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
 template <int DTMAX, int CT, bool FULL>
 __global__ __launch_bounds__(NT) void delta_walk_kernel(float* __restrict__ state, const int* __restrict__ positions,
                                                         const int* __restrict__ qsl, const int* __restrict__ state_slots,
-                                                        const int* __restrict__ counts, int H, int D, int Dv, int by_length,
-                                                        const float* __restrict__ ws, float* __restrict__ out) {
+                                                        const int* __restrict__ counts, int H, int D, int Dv, int by_length, int num_tiles,
+                                                        const int* __restrict__ first_row, const float* __restrict__ ws,
+                                                        float* __restrict__ out) {
   constexpr int DW = (DTMAX + 3) / 4;                     // state row tiles per wave: wave, wave + 4, …
   __shared__ __align__(16) float St[DTMAX * CT * TILE], Ut[4 * CT * TILE];
   const int h = blockIdx.x, seqs = counts[3];             // a head's column slices share an XCD (its tiles stay in one L2)
@@ -874,7 +893,8 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(float* __restrict__ stat
   const int blocks = (n + BT - 1) / BT;
 
   f32x4 qf[DTMAX], wf[DTMAX], kt[DW][4], aa[4], u0[CT], pe[DW];
-  auto base_of = [&](int b) { return ws + ((int64_t)(((s0 + BT * b) >> 6) + seq) * H + h) * sp.floats(); };
+  const int row0 = first_row[seq];
+  auto base_of = [&](int b) { return ws + (block_row(row0, b, num_tiles) * H + h) * sp.floats(); };
   auto fetch_rows = [&](const float* wb) {
 #pragma unroll
     for (int i = 0; i < DTMAX; ++i)
@@ -1267,10 +1287,11 @@ void launch_gm_max_gates(const void* g, bool bf16, int64_t g_stride, const float
 int gm_step_max_dim() { return GM_STEP_MAX_D; }
 int gm_block_max_dim() { return GM_BLOCK_MAX_D; }
 int64_t gm_scan_ws_floats(int rows, int seqs, int H) { return (int64_t)((rows >> 6) + seqs + 1) * H * scan_block_floats; }
-int64_t gm_delta_ws_floats(int rows, int seqs, int H, int D, int Dv) { return (int64_t)((rows >> 6) + seqs + 1) * H * DeltaSpace(D, Dv).floats(); }
+int64_t gm_delta_ws_floats(int seqs, int tiles, int H, int D, int Dv) { return (int64_t)tiles * H * DeltaSpace(D, Dv).floats() + seqs; }
+static int* delta_first_rows(float* ws, int tiles, int H, int D, int Dv) { return reinterpret_cast<int*>(ws + gm_delta_ws_floats(0, tiles, H, D, Dv)); }
 
 static void delta_walk(float* state, const int* positions, const int* qsl, const int* state_slots, const int* counts, int seqs, int num_tiles, int H,
-                       int D, int Dv, const float* ws, float* out, hipStream_t stream) {
+                       int D, int Dv, const int* first_row, const float* ws, float* out, hipStream_t stream) {
   // 32 state columns per workgroup (half the fetches) where workgroups of 16 would be more than two a compute unit; up to there a chain of blocks takes
   // 3 µs a block with 16 columns, 5 with 32: one sequence of 1069 tokens, 32 heads of 128, 84.7 → 55.6 µs.  (Sequences with a chunk: at most
   // one a tile; single tokens beside them end at once.)
@@ -1280,7 +1301,8 @@ static void delta_walk(float* state, const int* positions, const int* qsl, const
   // 32 heads: 111.1 µs a layer without, 113.4 with)
   const int by_length = seqs > 1 && num_tiles > 2 * seqs;
 #define GM_WALK(DT, CTV, FULLV)                                                                                                               \
-  hipLaunchKernelGGL((delta_walk_kernel<DT, CTV, FULLV>), grid, dim3(NT), 0, stream, state, positions, qsl, state_slots, counts, H, D, Dv, by_length, ws, out)
+  hipLaunchKernelGGL((delta_walk_kernel<DT, CTV, FULLV>), grid, dim3(NT), 0, stream, state, positions, qsl, state_slots, counts, H, D, Dv, by_length, num_tiles, \
+                     first_row, ws, out)
 #define GM_WALK_D(DT)                                             \
   do {                                                            \
     if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \
@@ -1301,10 +1323,11 @@ static void gated_scan(const A* q, int64_t q_stride, const A* k, int64_t k_strid
                        const int* counts, int seqs, int H, int G, int D, int Dv, float q_scale, float* out, float* nq,
                        const int* tile_seq, const int* tile_q0, int num_tiles, float* ws, hipStream_t stream) {
   const bool blocks = num_tiles > 0 && ws != nullptr && D <= GM_BLOCK_MAX_D;
+  int* first_row = DELTA && blocks ? delta_first_rows(ws, num_tiles, H, D, Dv) : nullptr;
 #define GM_STEP(DR)                                                                                                                   \
   hipLaunchKernelGGL((scan_step_kernel<A, DR, DELTA, void>), dim3(H, (Dv + 63) / 64, seqs), dim3(NT), 0, stream, q, q_stride, k, k_stride, \
                      v, v_stride, decay, weight, state, positions, qsl, state_slots, counts, H, G, D, Dv, q_scale, out, nq,           \
-                     blocks ? 1 : 0, ChannelArgs<void>{})
+                     blocks ? 1 : 0, first_row, ChannelArgs<void>{})
   const int dr = (D + 3) / 4;
   if (dr <= 8) GM_STEP(8);
   else if (dr <= 16) GM_STEP(16);
@@ -1316,8 +1339,8 @@ static void gated_scan(const A* q, int64_t q_stride, const A* k, int64_t k_strid
   const int wide = D % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && al16(q) && al16(k);     // 4 entries at a time
   if constexpr (DELTA) {
     hipLaunchKernelGGL(delta_block_kernel<A>, dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride, decay, weight, qsl,
-                       state_slots, counts, tile_seq, tile_q0, num_tiles, H, G, D, Dv, wide, q_scale, ws);
-    delta_walk(state, positions, qsl, state_slots, counts, seqs, num_tiles, H, D, Dv, ws, out, stream);
+                       state_slots, counts, tile_seq, tile_q0, num_tiles, H, G, D, Dv, wide, q_scale, first_row, ws);
+    delta_walk(state, positions, qsl, state_slots, counts, seqs, num_tiles, H, D, Dv, first_row, ws, out, stream);
     return;
   }
   hipLaunchKernelGGL(scan_block_kernel<A>, dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, decay, weight, qsl,
@@ -1367,10 +1390,11 @@ void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, in
                             hipStream_t stream) {
   if (seqs == 0) return;
   const bool blocks = num_tiles > 0 && ws != nullptr && D <= GM_BLOCK_MAX_D;
+  int* first_row = blocks ? delta_first_rows(ws, num_tiles, H, D, Dv) : nullptr;
 #define GM_STEP(DR)                                                                                                                    \
   GM_BF16(z_bf16, Z, hipLaunchKernelGGL((scan_step_kernel<float, DR, true, Z>), dim3(H, (Dv + 63) / 64, seqs), dim3(NT), 0, stream, q, q_stride, \
                                         k, k_stride, v, v_stride, (const float*)nullptr, weight, state, positions, qsl, state_slots,   \
-                                        counts, H, G, D, Dv, 1.f, out, (float*)nullptr, blocks ? 1 : 0,                                \
+                                        counts, H, G, D, Dv, 1.f, out, (float*)nullptr, blocks ? 1 : 0, first_row,                     \
                                         (ChannelArgs<Z>{(const Z*)z, z_stride, rate, bias})))
   const int dr = (D + 3) / 4;
   if (dr <= 8) GM_STEP(8);
@@ -1383,8 +1407,8 @@ void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, in
   const int wide = D % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && z_stride % 4 == 0 && al16(q) && al16(k) && al16(z) && al16(bias);
   GM_BF16(z_bf16, Z, hipLaunchKernelGGL((wide && D % 16 == 0 ? channel_block_kernel<Z, true> : channel_block_kernel<Z, false>), dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride,
                                         (ChannelArgs<Z>{(const Z*)z, z_stride, rate, bias}), weight, qsl, state_slots, counts, tile_seq,
-                                        tile_q0, num_tiles, H, G, D, Dv, wide, ws));
-  delta_walk(state, positions, qsl, state_slots, counts, seqs, num_tiles, H, D, Dv, ws, out, stream);
+                                        tile_q0, num_tiles, H, G, D, Dv, wide, first_row, ws));
+  delta_walk(state, positions, qsl, state_slots, counts, seqs, num_tiles, H, D, Dv, first_row, ws, out, stream);
 }
 
 }  // namespace dli

@@ -259,7 +259,7 @@ void launch_gm_max_gates(const void* g, bool bf16, int64_t g_stride, const float
 int gm_step_max_dim();
 int gm_block_max_dim();
 int64_t gm_scan_ws_floats(int rows, int seqs, int H);
-int64_t gm_delta_ws_floats(int rows, int seqs, int H, int D, int Dv);
+int64_t gm_delta_ws_floats(int seqs, int tiles, int H, int D, int Dv);
 void launch_gm_gated_scan(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride, bool bf16,
                           const float* decay, const float* weight, float* state, const int* positions, const int* qsl,
                           const int* state_slots, const int* counts, int seqs, int H, int G, int D, int Dv, bool delta, float q_scale,

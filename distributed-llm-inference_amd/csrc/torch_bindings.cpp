@@ -754,6 +754,7 @@ TORCH_LIBRARY(dli, m) {
   m.def("gm_gelu_rows(Tensor x, Tensor(a!)? out) -> Tensor", &gm_gelu_rows);
   m.def("gm_max_gates(Tensor g, Tensor bias, float cap, Tensor(a!) state, Tensor positions, Tensor qsl, Tensor state_slots, Tensor counts, "
         "int num_seqs, bool chunks) -> (Tensor, Tensor, Tensor)", &gm_max_gates);
+  m.def("gm_scan_workspace_bytes(int rows, int num_seqs, int num_tiles, int H, int D, int Dv, bool delta) -> int", &gm_scan_workspace_bytes);
   m.def("gm_gated_scan(Tensor q, Tensor k, Tensor v, Tensor decay, Tensor weight, Tensor(a!) state, Tensor positions, Tensor qsl, "
         "Tensor state_slots, Tensor counts, int num_seqs, int H, int G, int D, int Dv, bool delta, float q_scale, bool normaliser, "
         "Tensor? tile_seq, Tensor? tile_q0, int num_tiles) -> (Tensor, Tensor)", &gm_gated_scan);
