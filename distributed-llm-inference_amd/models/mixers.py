@@ -789,6 +789,15 @@ class MaskedAttention(nn.Module):
         seqmix.map_attention(out, q, cache.k, cache.v, meta, G, Dv, s.scale, s.window, self._lam, self.eps, (1.0 - s.map_diff) * self.out_scale)
 
 
+def scan_workspace_bytes(specs, rows: int, seqs: int) -> int:
+    """The largest workspace that a matrix-state scan of the layers ``specs`` takes on the GPU in a step of up to ``rows`` tokens of ``seqs``
+    sequences: one row per 64-token tile, and every sequence can end in a tile that is not full."""
+    delta_rule = {"delta": True, "channel_delta": True, "mlstm": False, "ssd": False}
+    tiles = rows // seqmix.PREFILL_TILE_TOKENS + min(seqs, rows)
+    return max((ops.hip().gm_scan_workspace_bytes(rows, seqs, tiles, p.heads, p.dim, p.vdim, delta_rule[p.kind])
+                for s in specs for p in (s, *s.parts) if p.kind in delta_rule), default=0)
+
+
 class ChannelDelta(nn.Module):
     """Per head: ``S ← g ⊙ S`` (a decay per row, i.e. key channel), ``u = β (v - Sᵀ k)``, ``S ← S + k uᵀ``, ``o = Sᵀ q``; each head's ``o`` divided by its
     root mean square, times a weight shared by the heads, times ``sigmoid(W_g2 W_g1 h)``.  ``g = exp(-exp(A) softplus(W_a2 W_a1 h + bias))``.

@@ -27,6 +27,7 @@ import torch
 from .. import ops
 from ..config import EngineConfig, KV_BLOCK_SIZE
 from ..models import build_model, torch_dtype
+from ..models.mixers import scan_workspace_bytes
 from ..ops import AttnMetadata
 from ..ops.kv_layout import allocate_kv_cache, bytes_per_block
 from ..parallel.state import SINGLE, ParallelContext, drain_collectives
@@ -109,12 +110,7 @@ class ModelRunner:
             return 2048
         torch.cuda.synchronize()
         free, total = torch.cuda.mem_get_info(self.device)
-        T = c.sched.max_num_batched_tokens
-        tp = self.ctx.tp_size
-        act = T * 2 * (4 * m.hidden_size + (m.num_heads + 2 * m.num_kv_heads) * m.head_dim // tp * 2
-                       + 3 * m.intermediate_size // tp * max(m.top_k_experts, 1))
-        logits = c.sched.max_num_seqs * m.vocab_size * 8
-        reserve = max(3 * (act + logits), 4 << 30) + (2 << 30)       # + graph pools
+        reserve = self._step_reserve()
         budget = free - (total * (1.0 - c.cache.gpu_memory_utilization)) - reserve
         n_dev = max(torch.cuda.device_count(), 1)
         # rehearsal mode: several ranks (of a TP group, or data-parallel replicas of a job started with DLI_SHARE_GPU=1) live
@@ -135,6 +131,17 @@ class ModelRunner:
         if n < self.max_blocks_per_seq:
             raise RuntimeError(f"not enough HBM for the KV cache: {budget / 2**30:.1f} GiB left after weights")
         return n
+
+    def _step_reserve(self) -> int:
+        """Bytes left beside weights and cache for what a step allocates."""
+        m, sched, tp = self.cfg.model, self.cfg.sched, self.ctx.tp_size
+        T = sched.max_num_batched_tokens
+        act = T * 2 * (4 * m.hidden_size + (m.num_heads + 2 * m.num_kv_heads) * m.head_dim // tp * 2
+                       + 3 * m.intermediate_size // tp * max(m.top_k_experts, 1))
+        logits = sched.max_num_seqs * m.vocab_size * 8
+        scan = scan_workspace_bytes(m.layer_specs, T, sched.max_num_seqs) if self.stateful else 0
+        # + graph pools; the scans' workspace once for eager steps and once in the captured ones' pool
+        return max(3 * (act + logits), 4 << 30) + (2 << 30) + 2 * scan
 
     @property
     def kv_cache_tokens(self) -> int:
