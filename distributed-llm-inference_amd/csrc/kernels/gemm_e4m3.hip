@@ -136,37 +136,48 @@ __global__ __launch_bounds__(256, 1) void gemm_e4m3_kernel(Args p) {
 // Of the 256-row tiles, those beyond the last whole round of one per compute unit are cut in two where that is shorter.  A 128-row tile takes
 // 0.58 of a 256-row one (4096 × 4096 × 14336 as one round of the latter 150 µs, 2000 rows as one round of the former 87).
 constexpr int NUM_CU = 256;
-static void plan(int M, int col_blocks, int* whole, int* halves, double* rounds) {
-  constexpr double HALF = 0.58;
-  const int units = (M + 127) / 128, odd = (units & 1) * col_blocks, total = units / 2 * col_blocks;
-  const int full = total / NUM_CU, rest = total % NUM_CU;
-  auto up = [](int a, int b) { return (a + b - 1) / b; };
-  const double keep = full + (rest ? std::max(1.0, HALF * up(odd, NUM_CU - rest)) : HALF * up(odd, NUM_CU));
-  const double cut = full + HALF * up(2 * rest + odd, NUM_CU);
-  *whole = keep <= cut ? total : full * NUM_CU;
-  *halves = 2 * (total - *whole) + odd;
-  *rounds = std::min(keep, cut);
+constexpr double HALF = 0.58;
+struct Plan {
+  int whole, halves, grid;
+  double rounds;                                             // of the workgroup that has most, in 256-row tiles
+  Plan(int whole_, int halves_) : whole(whole_), halves(halves_), rounds(0) {
+    grid = std::min(NUM_CU, (whole + 7) / 8 * 8 + (halves + 7) / 8 * 8);         // enough of them on every XCD
+    // As gcore::Places deals them: an XCD's 256-row tiles in turn from its first workgroup on, its 128-row tiles from the last one back.  What the
+    // turns leave over meets in one workgroup where there is more of it than workgroups.
+    const int groups = grid >> 3;
+    for (int x = 0; x < 8 && groups > 0; ++x) {
+      auto mine = [&](int total) { const int per = (total + 7) >> 3; return std::max(0, std::min(per, total - x * per)); };
+      const int w = mine(whole), h = mine(halves), w_over = w % groups, h_over = h % groups;
+      const double over = w_over + h_over > groups ? 1 + HALF : w_over ? 1 : h_over ? HALF : 0;
+      rounds = std::max(rounds, w / groups + HALF * (h / groups) + over);
+    }
+  }
+};
+static Plan plan(int M, int col_blocks) {
+  const int units = (M + 127) / 128, odd = (units & 1) * col_blocks, total = units / 2 * col_blocks, rest = total % NUM_CU;
+  const Plan keep(total, odd), cut(total - rest, 2 * rest + odd);
+  return keep.rounds <= cut.rounds ? keep : cut;
 }
 
 // multiplied part of what the chip could multiply in the time that launch_gemm_e4m3 takes by its plan
 double gemm_e4m3_fill(int64_t M, int64_t N) {
-  int whole, halves;
-  double rounds;
-  plan((int)M, (int)(N / gcore::TN), &whole, &halves, &rounds);
-  return (double)M * N / (256.0 * gcore::TN * NUM_CU * rounds);
+  return (double)M * N / (256.0 * gcore::TN * NUM_CU * plan((int)M, (int)(N / gcore::TN)).rounds);
+}
+
+// (256-row tiles, 128-row tiles, workgroups, rounds)
+std::tuple<int64_t, int64_t, int64_t, double> gemm_e4m3_plan(int64_t M, int64_t N) {
+  const Plan p = plan((int)M, (int)(N / gcore::TN));
+  return {p.whole, p.halves, p.grid, p.rounds};
 }
 
 // x [M, K] (rows 16-byte aligned), w [N, K] contiguous, K % 256 == 0, N % 256 == 0, both operands below 4 GiB
 void launch_gemm_e4m3(const void* x, int64_t x_stride, const void* w, const float* x_scale, const float* w_scale, void* out,
                       int64_t out_stride, int M, int N, int K, hipStream_t stream) {
   const int col_blocks = N / gcore::TN, units = (M + 127) / 128, pairs = units / 2;
-  int whole, halves;
-  double rounds;
-  plan(M, col_blocks, &whole, &halves, &rounds);
-  const int grid = std::min(NUM_CU, (whole + 7) / 8 * 8 + (halves + 7) / 8 * 8);   // enough of them on every XCD
-  hipLaunchKernelGGL(ge4::gemm_e4m3_kernel, dim3(grid), dim3(256), 0, stream,
+  const Plan p = plan(M, col_blocks);
+  hipLaunchKernelGGL(ge4::gemm_e4m3_kernel, dim3(p.grid), dim3(256), 0, stream,
                      ge4::Args{(const uint8_t*)x, x_stride, (const uint8_t*)w, x_scale, w_scale, (uint16_t*)out, out_stride, M, K,
-                               col_blocks, pairs, whole, halves});
+                               col_blocks, pairs, p.whole, p.halves});
 }
 
 }  // namespace dli

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <tuple>
+
 namespace dli {
 
 void launch_rms_norm(void* out, const void* x, const void* w, float eps, int rows, int H, int64_t x_stride,
@@ -70,6 +72,7 @@ void dense_gemm256_tail_plan(int M, int K, int N_out, bool swiglu, int* tail_til
 void launch_gemm_e4m3(const void* x, int64_t x_stride, const void* w, const float* x_scale, const float* w_scale, void* out,
                       int64_t out_stride, int M, int N, int K, hipStream_t stream);
 double gemm_e4m3_fill(int64_t M, int64_t N);
+std::tuple<int64_t, int64_t, int64_t, double> gemm_e4m3_plan(int64_t M, int64_t N);
 // activation rows 17 … 256: weight-streaming tiles (stream_gemm.hip)
 void launch_stream_gemm(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M, int K, int N,
                         int k_splits, hipStream_t stream);

@@ -800,6 +800,7 @@ TORCH_LIBRARY(dli, m) {
   m.def("dense_gemm256(Tensor x, Tensor w, bool swiglu=False, int k_splits=1, Tensor? out=None, bool split_tail=False) -> Tensor", &dense_gemm256);
   m.def("gemm_e4m3(Tensor x, Tensor x_scale, Tensor w, Tensor w_scale, Tensor? out=None) -> Tensor", &gemm_e4m3);
   m.def("gemm_e4m3_fill(int m, int n) -> float", &dli::gemm_e4m3_fill);
+  m.def("gemm_e4m3_plan(int m, int n) -> (int, int, int, float)", &dli::gemm_e4m3_plan);
   m.def("stream_gemm(Tensor x, Tensor w, bool swiglu=False, int k_splits=0, Tensor? out=None) -> Tensor", &stream_gemm);
   m.def("moe_tile_rows(int given, int rows, int hidden, bool fits256) -> int", &moe_tile_rows);
   m.def("ar_staging_tensor(int state, int rows, int cols, Tensor like) -> Tensor", &ar_staging_tensor);

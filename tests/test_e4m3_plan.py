@@ -1,0 +1,41 @@
+"""How the e4m3 tiles are dealt to workgroups (``csrc/kernels/gemm_e4m3.hip``): every tile once, and the cost that the plan names is that of the
+workgroup with most to do.  Arithmetic only: no GPU."""
+import pytest
+
+from dli_amd import ops
+
+HALF, CUS = 0.58, 256
+
+
+def _places(total, grid, back):
+    """``gcore::Places``: the places of every workgroup's tiles."""
+    per, groups, out = -(-total // 8), grid // 8, []
+    for block in range(grid):
+        x, i = block & 7, block >> 3
+        i = groups - 1 - i if back else i
+        mine = min(per, total - x * per) - i
+        out.append([x * per + i + j * groups for j in range(-(-mine // groups) if mine > 0 else 0)])
+    return out
+
+
+def _rounds(whole, halves):
+    grid = min(CUS, -(-whole // 8) * 8 + -(-halves // 8) * 8)
+    a, b = _places(whole, grid, False), _places(halves, grid, True)
+    assert sorted(sum(a, [])) == list(range(whole)) and sorted(sum(b, [])) == list(range(halves))
+    return max(len(p) + HALF * len(q) for p, q in zip(a, b)), grid
+
+
+SIZES = [(m, n) for n in (256, 2304, 4096, 6144, 8192, 10240, 14336, 28672) for m in (1, 128, 129, 256, 385, 513, 640, 1025, 1152, 1300, 1664, 2000, 2688, 3200, 3456, 4096)]
+
+
+@pytest.mark.parametrize("m,n", SIZES)
+def test_plan_costs_what_its_workgroups_do(m, n):
+    whole, halves, grid, rounds = ops.hip().gemm_e4m3_plan(m, n)
+    units, cols = -(-m // 128), n // 256
+    total, odd = units // 2 * cols, units % 2 * cols
+    assert 2 * whole + halves == units * cols
+    assert (rounds, grid) == (pytest.approx(_rounds(whole, halves)[0]), _rounds(whole, halves)[1])
+    # never the slower of the two forms: all 256-row tiles kept, or those beyond the last whole round cut in two
+    rest = total % CUS
+    assert rounds == pytest.approx(min(_rounds(total, odd)[0], _rounds(total - rest, 2 * rest + odd)[0]))
+    assert ops.hip().gemm_e4m3_fill(m, n) == pytest.approx(m * n / (256 * 256 * CUS * rounds))
