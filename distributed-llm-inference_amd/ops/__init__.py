@@ -409,12 +409,14 @@ def quant_weight_fp8(w: torch.Tensor):
 
 
 @functools.lru_cache(maxsize=4096)
-def _e4m3_tiles_fill(m: int, n: int) -> bool:
-    """Do the own e4m3 tiles (``csrc/kernels/gemm_e4m3.hip``) fill at least half of the chip while they run?  From there they beat the library
-    (ratios of the times at 28672 × 4096, 4096 × 14336, 7168 × 8192, 8192 × 3584, 6144 × 4096, 4096 × 4096 weights and 200 to 4096 rows: 0.70 to
-    0.95, once 1.05), below they leave too many compute units idle, which the library fills by cutting K (512 rows of 4096 × 14336: 90 against
-    49 µs)."""
-    return hip().gemm_e4m3_fill(m, n) >= 0.5
+def _e4m3_tiles_pay(m: int, n: int, k: int) -> bool:
+    """Do the own e4m3 tiles (``csrc/kernels/gemm_e4m3.hip``) beat the library?  They do where they fill at least half of the chip while they run
+    (nine weights from 4096 × 4096 to 28672 × 4096 and 10240 × 8192, 128 to 4096 rows: 0.59 to 1.02 of the library's time in 214 products), below
+    they leave too many compute units idle, which the library fills by cutting K (512 rows of 4096 × 14336: 90 against 49 µs).  Where one round
+    of 128-row tiles is all there is, K beyond 4096 gives the library long enough slices up to a fill of 0.66 (K of 5120 to 14336: of 85 products
+    with 0.5 to 0.66 55 were slower on own tiles, up to 1.15; from 0.66 on 0.81 to 1.01.  K up to 4096: 0.63 to 1.03 from 0.5 on)."""
+    short = hip().gemm_e4m3_plan(m, n)[3] < 1.0
+    return hip().gemm_e4m3_fill(m, n) >= (0.66 if short and k > 4096 else 0.5)
 
 
 def _e4m3_ok(q: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, out: Optional[torch.Tensor]) -> bool:
@@ -424,7 +426,7 @@ def _e4m3_ok(q: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tens
         return False
     (m, k), n = q.shape, wq.shape[0]
     if not (wq.shape[1] == k and xs.shape == (m, 1) and ws.shape == (1, n) and k % 256 == 0 and n % 256 == 0 and 0 < m <= 1 << 24 and k and n
-            and _e4m3_tiles_fill(m, n)):
+            and _e4m3_tiles_pay(m, n, k)):
         return False
     return (wq.is_contiguous() and q.stride(1) == 1 and q.stride(0) >= k and q.stride(0) % 16 == 0 and xs.is_contiguous() and ws.is_contiguous()
             and all(t.device == q.device for t in (wq, xs, ws)) and m * q.stride(0) < 2 ** 32 and n * k < 2 ** 32

@@ -39,3 +39,11 @@ def test_plan_costs_what_its_workgroups_do(m, n):
     rest = total % CUS
     assert rounds == pytest.approx(min(_rounds(total, odd)[0], _rounds(total - rest, 2 * rest + odd)[0]))
     assert ops.hip().gemm_e4m3_fill(m, n) == pytest.approx(m * n / (256 * 256 * CUS * rounds))
+
+
+# the longest K at which half of the chip is enough, and the fills around the two lines (the last three: more than one round)
+@pytest.mark.parametrize("m,n,k,own", [(1280, 4096, 4096, True), (1152, 4096, 4096, False), (1280, 4096, 4352, False), (1408, 4096, 14336, False), (1536, 4096, 14336, False),
+                                       (1600, 4096, 14336, True), (768, 8192, 8192, False), (512, 10240, 8192, False), (640, 10240, 8192, True),
+                                       (2176, 4096, 14336, True), (1025, 8192, 8192, True), (640, 28672, 4096, True)])
+def test_half_filled_rounds_go_where_they_are_faster(m, n, k, own):
+    assert ops._e4m3_tiles_pay(m, n, k) == own
