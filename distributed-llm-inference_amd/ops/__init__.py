@@ -420,13 +420,16 @@ def _e4m3_tiles_pay(m: int, n: int, k: int) -> bool:
 
 
 def _e4m3_ok(q: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, out: Optional[torch.Tensor]) -> bool:
-    f32, e4m3 = torch.float32, torch.float8_e4m3fn
-    if not (q.dim() == 2 and wq.dim() == 2 and q.dtype == e4m3 and wq.dtype == e4m3 and xs.dtype == f32 and ws.dtype == f32
-            and _plain(q, xs, wq, ws) and (out is None or _plain(out))):
+    # sizes first: small calls, whose launches the host can hardly keep up with, end here (1.2 µs; all checks take 8, the types alone 3)
+    if torch.compiler.is_compiling() or q.dim() != 2 or wq.dim() != 2:
         return False
     (m, k), n = q.shape, wq.shape[0]
-    if not (wq.shape[1] == k and xs.shape == (m, 1) and ws.shape == (1, n) and k % 256 == 0 and n % 256 == 0 and 0 < m <= 1 << 24 and k and n
+    if not (type(m) is int and type(k) is int and type(n) is int and 0 < m <= 1 << 24 and k and n and k % 256 == 0 and n % 256 == 0
             and _e4m3_tiles_pay(m, n, k)):
+        return False
+    f32, e4m3 = torch.float32, torch.float8_e4m3fn
+    if not (q.dtype == e4m3 and wq.dtype == e4m3 and xs.dtype == f32 and ws.dtype == f32 and _plain(q, xs, wq, ws)
+            and (out is None or _plain(out)) and wq.shape[1] == k and xs.shape == (m, 1) and ws.shape == (1, n)):
         return False
     return (wq.is_contiguous() and q.stride(1) == 1 and q.stride(0) >= k and q.stride(0) % 16 == 0 and xs.is_contiguous() and ws.is_contiguous()
             and all(t.device == q.device for t in (wq, xs, ws)) and m * q.stride(0) < 2 ** 32 and n * k < 2 ** 32

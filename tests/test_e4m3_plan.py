@@ -1,6 +1,7 @@
 """How the e4m3 tiles are dealt to workgroups (``csrc/kernels/gemm_e4m3.hip``): every tile once, and the cost that the plan names is that of the
 workgroup with most to do.  Arithmetic only: no GPU."""
 import pytest
+import torch
 
 from dli_amd import ops
 
@@ -47,3 +48,28 @@ def test_plan_costs_what_its_workgroups_do(m, n):
                                        (2176, 4096, 14336, True), (1025, 8192, 8192, True), (640, 28672, 4096, True)])
 def test_half_filled_rounds_go_where_they_are_faster(m, n, k, own):
     assert ops._e4m3_tiles_pay(m, n, k) == own
+
+
+def test_only_plain_tensors_and_whole_numbers_reach_the_rule():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    m, n, k = 2000, 4096, 256
+    q, wq = torch.zeros(m, k).to(torch.float8_e4m3fn), torch.zeros(n, k).to(torch.float8_e4m3fn)
+    xs, ws = torch.ones(m, 1), torch.ones(1, n)
+    assert ops._e4m3_ok(q, xs, wq, ws, None)
+    assert ops._e4m3_ok(q, xs, torch.nn.Parameter(wq, requires_grad=False), ws, torch.empty(m, n, dtype=torch.bfloat16))
+    said = []
+
+    def ask(q, xs):
+        said.append(ops._e4m3_ok(q, xs, wq, ws, None))
+        return xs * 2
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        ask(mode.from_tensor(q), mode.from_tensor(xs))
+    make_fx(ask)(q, xs)
+    make_fx(ask, tracing_mode="symbolic")(q, xs)
+    torch.jit.trace(ask, (q, xs), check_trace=False)
+    torch.vmap(ask, in_dims=(None, 0))(q, xs.unsqueeze(0))
+    assert said and not any(said)
+    for bad in (q[:0], q[:, :128], q.t(), q[0], q.float(), q[::2, :]):
+        assert not ops._e4m3_ok(bad, xs[:len(bad)], wq, ws, None)
+    assert not ops._e4m3_ok(q, xs.t(), wq, ws, None) and not ops._e4m3_ok(q, xs, wq[:, :128], ws, None) and not ops._e4m3_ok(q, xs, wq, ws.double(), None)
