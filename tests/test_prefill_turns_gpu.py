@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 def test_page_counts_of_a_turn(kv_dtype, copies):
     """1 to 12 pages, the last of 1 and of 32 tokens (the chunk crosses a page's end), 3 new tokens each.  Weights and results are rounded to bf16
-    (2^-9 each, |v| ≤ 4.5 here); e4m3 keys and values enter as they are stored."""
+    (half an ulp each: 2^-8 of the value at most, half of that on average; |v| ≤ 4.5 here); e4m3 keys and values enter as they are stored."""
     Hq, Hkv = 16, 4
     seq_lens = [32 * p + e for p in range(12) for e in (4, 32)] * copies
     n = len(seq_lens)
