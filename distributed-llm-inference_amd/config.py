@@ -874,9 +874,9 @@ class EngineConfig:
     tune_gemms: bool = True
     weights_path: Optional[str] = None      # safetensors dir/file; None → random init
     # "fp8": W8A8 dense projections — weights quantised once to OCP e4m3 with one scale per output channel, activations per
-    # token on the fly (csrc/kernels/quant.hip), GEMMs on the fp8 matrix cores (hipBLASLt through torch._scaled_mm) for
-    # steps of more than 64 rows; decode-sized steps keep the bf16 weight-streaming kernels (both copies stay resident:
-    # 288 GB).  None: bf16 throughout (the default, and what every headline number is measured with).
+    # token on the fly (csrc/kernels/quant.hip), GEMMs on the fp8 matrix cores for steps of 17 rows and more (own tiles where they
+    # beat the library, csrc/kernels/gemm_e4m3.hip, else hipBLASLt); smaller steps stream the e4m3 weights against bf16 activations (the bf16
+    # weights stay resident: 288 GB).  None: bf16 throughout (the default, and what every headline number is measured with).
     quantization: Optional[str] = None
     # Path of a PyTorch TunableOp results file: the vendor-library GEMMs (hipBLASLt / rocBLAS behind torch) are tuned per
     # shape during warm-up (seconds per shape on the first start; the file is written and simply loaded by later starts),

@@ -768,8 +768,9 @@ static constexpr int PREFILL_UNITS = 256;                      // workgroups of 
 //   * the shortest share workgroups, a group each (SHARED).  Both pass the same barriers, so they wait for their loads and products at the same time
 //     and take 1.25 of what they take in workgroups of their own; the longest take 0.8.  It pays where the shared ones are the shorter ones: 2 × 600
 //     tokens (304 tiles) 24.1 / 20.7, 4 × 300 (320) 16.1 / 14.7, one of 1100 behind 500 (280) 51.0 / 39.9, but 3 × 400 behind 1000 (312) 48.6 / 55.9,
-//     2 × 1024 (512, all shared) 37.4 / 46.6.  e4m3, whose one group is slower: 2 × 600 behind 600 49.9 / 47.6, 4 × 1500 behind 500 with 8/1 heads (376)
-//     77.2 / 74.1, a mixed step of 96 rows and two chunks of up to 1024 behind up to 1024 (296) 73.8 / 62.5 (in bf16 77 / 89).
+//     2 × 1024 (512, all shared) 37.4 / 46.6.  e4m3, whose two groups take two pages a turn: 2 × 600 behind 600 42.2 / 41.5, 1100 behind 2000 (280) 100.0 /
+//     96.2, 4 × 1500 behind 500 with 8/1 heads (376) 63.1 / 61.8, a mixed step of 96 rows and two chunks of up to 1024 behind up to 1024 (296), called
+//     eagerly and with the decode rows, 89.2 / 75.6 (in bf16 94 / 99).
 //   * or the rest comes in a second round (ROUNDS), whose workgroups all start with 5 µs of latencies: 16 × 100 tokens (512) 12.5 / 17.2, 9 × 128 behind
 //     1000 (288) 46.3 / 60.4.  It pays only if that is made of short tiles: one prompt of 2000 (504) 63.5 / 58.1.  With 5 µs + 0.0285 µs a token for
 //     one group, 5.5 + 0.0225 for two, and the first tile of the second round at `second` tokens of context, that is what the last line says

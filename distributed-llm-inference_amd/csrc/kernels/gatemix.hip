@@ -379,8 +379,9 @@ struct DeltaSpace {
 // workspace row of block b of a chunk (of a chunk that the tile list lacks: some row, never one past them)
 __device__ __forceinline__ int64_t block_row(int first, int b, int num_tiles) { return min((unsigned)(first + b), (unsigned)(num_tiles - 1)); }
 // A tile as the A operand: lane row + 16 (k / 4) holds 4 consecutive k.  As the B operand, and as a product leaves it: lane column + 16 (row / 4)
-// holds 4 consecutive rows.  turned(): from either form to the other one, a product with the unit matrix (exact); the kernels below store
-// every tile as 1 KB in lane order (4-byte stores of the turned order: channel_block_kernel 87 → 83 µs at 51 blocks of 16 heads of 128).
+// holds 4 consecutive rows.  turned(): from either form to the other one, a product with the unit matrix: exact for finite values, an infinity
+// becomes NaN in its row's 16 entries (rows of W, K̃ and A that hold one make what they are multiplied into infinite or NaN in either form).
+// The kernels below store every tile as 1 KB in lane order (4-byte stores of the turned order: channel_block_kernel 87 → 83 µs at 51 blocks of 16 heads of 128).
 __device__ __forceinline__ f32x4 unit_tile(int lane) {
   const int k = (lane & 15) - 4 * (lane >> 4);
   return f32x4{k == 0 ? 1.f : 0.f, k == 1 ? 1.f : 0.f, k == 2 ? 1.f : 0.f, k == 3 ? 1.f : 0.f};
@@ -855,8 +856,8 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
 //   [o | x] = [Q̃ | W] S, u = U0 - x → LDS → o += A u, S = e^{P_end} ⊙ S + K̃ᵀ u → LDS,
 // two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 75 µs (36 of them fp32 matrix instructions, were they spread
 // evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83.  The next block's tiles are fetched as soon as
-// their registers are free and without a condition (the last block fetches itself again): behind a condition the compiler has to wait for
-// everything that is in flight.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
+// their registers are free and without a condition (the last block fetches itself again), so they land during the products; the compiler
+// still waits for all of them at the end of a block, where some change registers.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
 // below that of the walk before (2.7e-7 against 2.9e-7 of its norm).
 template <int DTMAX, int CT, bool FULL>
 __global__ __launch_bounds__(NT) void delta_walk_kernel(float* __restrict__ state, const int* __restrict__ positions,
@@ -1352,8 +1353,9 @@ static void gated_scan(const A* q, int64_t q_stride, const A* k, int64_t k_strid
 #define GM_WALK(DT, CTV, FULLV)                                                                                                               \
   hipLaunchKernelGGL((scan_walk_kernel<A, DT, CTV, FULLV>), grid, dim3(NT), lds, stream, q, q_stride, k, k_stride, v, v_stride, state,  \
                      positions, qsl, state_slots, counts, H, G, D, Dv, wide, q_scale, ws, out, nq)
-  // D that fills its bound, two column tiles: 32 heads of 128, whole scans, µs, with / without conditions: 799 rows, channel decays 117.8 / 110.1,
-  // 2048 rows 329.9 / 305.9.  One column tile has half the products a read and is no faster without (16 heads, 3162 rows: 213.8 / 220.2, 201.7 / 202.2).
+  // D that fills its bound, two column tiles: whole scans in bf16, µs, with / without conditions: 32 heads of 128, 799 rows 103.4 / 99.2, 2048 rows 223.4 /
+  // 212.3 (with the normaliser 238.8 / 223.8), 64 heads of 64, 2048 rows 146.7 / 142.0, 32 heads of 256, 1024 rows 220.3 / 204.6.  One column tile has
+  // half the products a read (16 heads of 128, 3162 rows, as one or four prompts: 213.8 / 220.2, 201.7 / 202.2).
 #define GM_WALK_D(DT)                                             \
   do {                                                            \
     if (ct == 2 && D > 16 * DT - 16) GM_WALK(DT, 2, true);        \

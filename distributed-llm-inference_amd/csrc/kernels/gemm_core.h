@@ -49,7 +49,8 @@ __device__ __forceinline__ void mma(const u32x4 (&w)[2], const u32x4 (&a)[2], f3
 }
 
 // Runs `tiles.count` tiles of nk K-steps each (an even number: the buffers change places), one stream of steps: behind a tile's last step the DMA goes on with the next tile's
-// first, so only the first tile of a workgroup waits for memory, and a tile's results are stored while the next one's steps land.
+// first, so only the first tile of a workgroup waits for memory; a tile's results are stored with the next one's steps on their way, and their
+// instructions are counted in its first waits (a store() that waits for memory itself drains these steps: its loss, not an error).
 //   tiles.sources(i, lane, wave, A, W, a_src, w_src): bases of tile i's operands (wave-uniform) and this lane's byte offsets at k = 0 for
 //     DMA piece wave · (pieces per wave) + j of half h; may fetch into LDS what store(i) needs (landed by then, ring of four tiles)
 //   tiles.store(i, lane, wave, acc): acc[m][n]: rows wr·16·MB + m·16 + (lane & 15), columns wc·128 + n·16 + 4 (lane >> 4) + r;

@@ -1,12 +1,13 @@
 // W8A8 product on the e4m3 matrix cores: y[m, n] = bf16(Σ_k x[m, k] · w[n, k] · x_scale[m] · w_scale[n]).
 //
 // The K loop is gemm_core.h's; at most one workgroup per compute unit runs 256 × 256 tiles, then 128 × 256 ones.  What bounds it: the matrix
-// cores at the clock that the card holds under them.  Results leave through LDS, 256 contiguous bytes of a row at a time, while the
-// next tile's steps are fetched (one tile per workgroup, 8-byte stores from the accumulators: 191 µs instead of 173 for the first line).
+// cores at the clock that the card holds under them.  Results leave through LDS, 256 contiguous bytes of a row at a time, with the next tile's
+// first steps already on their way (one tile per workgroup, 8-byte stores from the accumulators: 191 µs instead of 173 for the first line's 2000
+// rows).  The kernel takes all 512 registers and spills four 8-byte row offsets; store() reloads each and waits for everything in flight with it.
 // Measured (µs; library product in brackets):
-//   28672 × 4096 weights   M = 512 51 (56)   1024 93 (113)   2000 173 (225)   4096 325 (366, 2.96 against 2.63 PFLOP/s)
-//   4096 × 14336           M = 1300 84 (91)   2000 87 (104)   4096 150 (168, 3.2 against 2.86 PFLOP/s)
-//   8192 × 3584            M = 700 29 (30)   1024 31 (37)   2000 45 (53)   4096 86 (99)
+//   28672 × 4096 weights   M = 512 50 (63)   1024 94 (118)   2000 173 (230)   4096 329 (402, 2.92 against 2.40 PFLOP/s)
+//   4096 × 14336           M = 1600 89 (94)   2000 95 (110)   4096 151 (178, 3.18 against 2.71 PFLOP/s)
+//   8192 × 3584            M = 700 28 (30)   1024 31 (37)   2000 47 (57)   4096 89 (105)
 #include <algorithm>
 
 #include "common.h"

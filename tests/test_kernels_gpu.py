@@ -908,7 +908,7 @@ def test_skinny_linear_w8_matches_the_dequantised_product(M, N, K, swiglu):
 
 @pytest.mark.parametrize("M,N,K", [(2304, 6144, 4096), (70, 4096, 14336), (300, 28672, 4096)])
 def test_linear_fp8_tracks_fp32_reference(M, N, K):
-    """W8A8 GEMM (per-token × per-channel scales, fp8 matrix cores through torch._scaled_mm) against the fp32 product of the
+    """W8A8 GEMM (per-token × per-channel scales, fp8 matrix cores: own tiles, and torch._scaled_mm for the 70 rows) against the fp32 product of the
     bf16 operands, and against the fp32 product of the SAME quantised operands (that one tightly: the GEMM itself is exact
     up to accumulation order)."""
     x = _bf(M, K, seed=83)
