@@ -347,18 +347,18 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
 // copies each 32-token page (K + V, 16 KB bf16 / 8 KB fp8) once by LDS-DMA (global_load_lds, 16 bytes per lane, no
 // VGPRs) into a ring, and every wave reads its fragments with ds_read_b128.  A turn (one barrier) is one page of three stages, two pages ahead of
 // the math, or with two groups, whose one workgroup a compute unit has the registers for it, two pages of two stages: two score
-// chains side by side, one maximum and one rescale of the accumulators for both.  The page keeps its global layout in LDS except that the four 16-byte
+// chains side by side, and one question for both whether a maximum rises.  The page keeps its global layout in LDS except that the four 16-byte
 // slots of every 64-byte row are permuted by the row (slot ^ h[(row >> 2) & 3], h = {0,2,3,1}; the DMA's LDS image is
 // lane-linear, so the permutation sits on the SOURCE address): the 16 lanes the hardware serves together for a
 // ds_read_b128 — {0–3, 12–15, 20–27} etc. — then touch 16 different slots of the 256-byte bank row.
 //
 // GROUPS = 2 (few tiles): a workgroup has two such sets of four waves; group g takes turns g, g + 2, … in a ring of its own, and at the end the
 // groups' maxima, sums and accumulators meet in LDS.
-// Two pages a turn: e4m3 with two groups.  µs, one page / two: 2 × 1024 behind 1024 41.7 / 36.5, one of 2048 behind 1500 with 8/1 heads 92.2 / 78.1, 64 behind
-// 1900 54.7 / 46.5 (with 16-byte reads of the pages, which alone give 0.95: 8-byte ones of rows of 32 bytes met in 4 of 16 bank groups).  One group,
+// Two pages a turn: e4m3 with two groups.  µs, one page / two: 2 × 1024 behind 1024 41.7 / 35.5, one of 2048 behind 1500 with 8/1 heads 92.2 / 75.7, 64 behind
+// 1900 54.7 / 45.8 (with 16-byte reads of the pages, which alone give 0.95: 8-byte ones of rows of 32 bytes met in 4 of 16 bank groups).  One group,
 // where three workgroups share a compute unit, keeps one page (two leave two of them: e4m3, five prompts of up to 1333, 55.0 / 56.5; with 8-byte
-// reads 61.4).  bf16 keeps one too: with two groups two pages are 4 % faster, but the maximum of two pages rounds more weights
-// (error against 64 bits 0.00290 → 0.00291; e4m3, where the stored values' own error is four times that, 0.01118 either way).
+// reads 61.4).  bf16 keeps one too: with two groups and one maximum for both, two pages are 4 % faster but round more weights (error against 64
+// bits 0.00290 → 0.00291); with a maximum each they are not measured.
 //
 // Math on v_mfma_f32_32x32x16_bf16: a wave's 32 query columns are ONE MFMA column set.  Lane (c = lane & 31,
 // hi = lane >> 5) owns column c:
@@ -399,6 +399,34 @@ __device__ __forceinline__ float page_weights32(const f32x16& s, int tok0, int l
     pb[(r >> 2) & 1][(r & 3) + 4 * (r >> 3)] = (short)f2bf(p);
   }
   return ps;
+}
+
+// 16 bytes of an e4m3 V row are slots 2 hi and 2 hi + 1, not hi and 2 + hi: the weights of slots 1 and 2 change places
+__device__ __forceinline__ void swap_slots(bf16x8 (&w)[2]) {
+  u32x4 w0 = __builtin_bit_cast(u32x4, w[0]), w1 = __builtin_bit_cast(u32x4, w[1]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    auto x = __builtin_amdgcn_permlane32_swap(w0[e], w1[e], false, false);
+    w0[e] = x[0];
+    w1[e] = x[1];
+  }
+  w[0] = __builtin_bit_cast(bf16x8, w0);
+  w[1] = __builtin_bit_cast(bf16x8, w1);
+}
+
+// row d = 32 n + c32 of a staged V page: the A fragments of the two k-steps (off0, off1: this lane's offsets in n = 0; e4m3: one)
+template <bool KV8>
+__device__ __forceinline__ void value_fragments(const char* vb, int n, int off0, int off1, bf16x8& v0, bf16x8& v1) {
+  if constexpr (!KV8) {
+    v0 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + off0);
+    v1 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + off1);
+  } else {
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(vb + n * 1024 + off0);
+    fp8x4_to_bf16(raw[0], v0, 0);
+    fp8x4_to_bf16(raw[1], v0, 4);
+    fp8x4_to_bf16(raw[2], v1, 0);
+    fp8x4_to_bf16(raw[3], v1, 4);
+  }
 }
 
 template <bool KV8, int GROUPS, int NPG>
@@ -528,7 +556,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   const int v_off0 = c32 * 64 + ((hi ^ swz) << 4), v_off1 = c32 * 64 + (((2 + hi) ^ swz) << 4);
   const int v8_off = c32 * 32 + 16 * hi;
 
-  // NP pages from b on, staged at `kb`: scores, one running maximum, weights, P·V
+  // NP pages from b on, staged at `kb`: scores, maxima, weights, P·V
   auto pages = [&](auto np, int b, const char* kb) __attribute__((always_inline)) {
     constexpr int NP = decltype(np)::value;
     f32x16 s[NP];
@@ -558,60 +586,81 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
         }
     }
     const int tok0 = b * 32 + 4 * hi;
-    const bool edge = b * 32 + 32 * NP - 1 > first_tok;
-    float mx = edge ? page_max32<true>(s[0], tok0, qpos) : page_max32<false>(s[0], tok0, qpos);
-#pragma unroll
-    for (int p = 1; p < NP; ++p) mx = fmaxf(mx, edge ? page_max32<true>(s[p], tok0 + 32 * p, qpos) : page_max32<false>(s[p], tok0 + 32 * p, qpos));
-    mx *= scale_log2;
-    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    // The maximum moves with every turn that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
+    // The maximum moves with every page that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
     // 2^8 saves these 64 products on most pages, 3 – 10 % of a launch, but rounds the largest weight like all others: relative error
     // against 64 bits 0.00266 → 0.00272, e4m3 pages 0.00731 → 0.00734.)
-    if (__any(mx > m)) {
-      asm volatile("" ::: "memory");
-      const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
-      m = mn;
-      lsum *= alpha;
+    if constexpr (NP == 1) {
+      const bool edge = b * 32 + 31 > first_tok;
+      float mx = edge ? page_max32<true>(s[0], tok0, qpos) : page_max32<false>(s[0], tok0, qpos);
+      mx *= scale_log2;
+      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      if (__any(mx > m)) {
+        asm volatile("" ::: "memory");
+        const float mn = fmaxf(m, mx), alpha = fast_exp2(m - mn);
+        m = mn;
+        lsum *= alpha;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) o[n] *= alpha;
-    }
-    bf16x8 pb[NP][2];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      lsum += edge ? page_weights32<true>(s[p], tok0 + 32 * p, qpos, scale_log2, m, pb[p]) : page_weights32<false>(s[p], tok0 + 32 * p, qpos, scale_log2, m, pb[p]);
-      if constexpr (KV8) {
-        // 16 bytes of an e4m3 V row are slots 2 hi and 2 hi + 1, not hi and 2 + hi: the weights of slots 1 and 2 change places
-        u32x4 w0 = __builtin_bit_cast(u32x4, pb[p][0]), w1 = __builtin_bit_cast(u32x4, pb[p][1]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          auto x = __builtin_amdgcn_permlane32_swap(w0[e], w1[e], false, false);
-          w0[e] = x[0];
-          w1[e] = x[1];
-        }
-        pb[p][0] = __builtin_bit_cast(bf16x8, w0);
-        pb[p][1] = __builtin_bit_cast(bf16x8, w1);
+        for (int n = 0; n < 4; ++n) o[n] *= alpha;
       }
-    }
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const char* vb = kb + p * 2 * PAGE_BYTES + PAGE_BYTES;
+      bf16x8 pb[2];
+      lsum += edge ? page_weights32<true>(s[0], tok0, qpos, scale_log2, m, pb) : page_weights32<false>(s[0], tok0, qpos, scale_log2, m, pb);
+      if constexpr (KV8) swap_slots(pb);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
-        bf16x8 v0, v1;                           // row d = 32 n + c32: the A fragments of the two k-steps
-        if constexpr (!KV8) {
-          v0 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off0);
-          v1 = *reinterpret_cast<const bf16x8*>(vb + n * 2048 + v_off1);
-        } else {
-          const u32x4 raw = *reinterpret_cast<const u32x4*>(vb + n * 1024 + v8_off);
-          fp8x4_to_bf16(raw[0], v0, 0);
-          fp8x4_to_bf16(raw[1], v0, 4);
-          fp8x4_to_bf16(raw[2], v1, 0);
-          fp8x4_to_bf16(raw[3], v1, 4);
-        }
-        o[n] = mfma32(v0, pb[p][0], o[n]);
-        o[n] = mfma32(v1, pb[p][1], o[n]);
+        bf16x8 v0, v1;
+        value_fragments<KV8>(kb + PAGE_BYTES, n, KV8 ? v8_off : v_off0, v_off1, v0, v1);
+        o[n] = mfma32(v0, pb[0], o[n]);
+        o[n] = mfma32(v1, pb[1], o[n]);
       }
+    } else {
+      // both maxima, then both pages' weights, each to its own maximum; only where one of them rises are the accumulators asked twice.  (One
+      // maximum for both rounds the first page's largest weights: 0.007210 → 0.007213 for a mixed step, larger in 43 of 48 calls, and takes 1.00 to 1.03 of the time.)
+      bool edge[2];
+      float mx[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        edge[p] = (b + p) * 32 + 31 > first_tok;
+        const float x = (edge[p] ? page_max32<true>(s[p], tok0 + 32 * p, qpos) : page_max32<false>(s[p], tok0 + 32 * p, qpos)) * scale_log2;
+        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        mx[p] = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      }
+      bf16x8 pb[2][2];
+      auto weights = [&](int p, float top) __attribute__((always_inline)) {
+        const float ps = edge[p] ? page_weights32<true>(s[p], tok0 + 32 * p, qpos, scale_log2, top, pb[p]) : page_weights32<false>(s[p], tok0 + 32 * p, qpos, scale_log2, top, pb[p]);
+        if constexpr (KV8) swap_slots(pb[p]);
+        return ps;
+      };
+      auto rescale = [&](float alpha) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        lsum *= alpha;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) o[n] *= alpha;
+      };
+      auto add_values = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          bf16x8 v0, v1;
+          value_fragments<KV8>(kb + p * 2 * PAGE_BYTES + PAGE_BYTES, n, KV8 ? v8_off : v_off0, v_off1, v0, v1);
+          o[n] = mfma32(v0, pb[p][0], o[n]);
+          o[n] = mfma32(v1, pb[p][1], o[n]);
+        }
+      };
+      const float m0 = fmaxf(m, mx[0]), m1 = fmaxf(m0, mx[1]);
+      const float ps0 = weights(0, m0), ps1 = weights(1, m1);
+      if (__any(m1 > m)) {
+        rescale(fast_exp2(m - m0));
+        lsum += ps0;
+        add_values(0);
+        rescale(fast_exp2(m0 - m1));
+        add_values(1);
+      } else {
+        lsum += ps0;
+        add_values(0);
+        add_values(1);
+      }
+      lsum += ps1;
+      m = m1;
     }
   };
 
