@@ -550,29 +550,50 @@ struct DrawArgs {
   const float* noise;
 };
 __device__ __forceinline__ ArgMax no_candidate() { return ArgMax{-3.0e38f, 0x7fffffff}; }
+// a thread meets its logits in order of index, so an equal one never wins
+__device__ __forceinline__ void take(ArgMax& a, float v, int i) {
+  if (v > a.v) a = ArgMax{v, i};
+}
 __device__ __forceinline__ void greedy_chunk(const uint4& x, int chunk, ArgMax& a) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) a = amax(a, ArgMax{bf2f((uint16_t)half_of(x, e)), chunk * 8 + e});
+  for (int e = 0; e < 8; ++e) take(a, bf2f((uint16_t)half_of(x, e)), chunk * 8 + e);
 }
+// __logf of a normal number with a finite logarithm, the same bits in six instructions (__logf also scales subnormal numbers and lets infinities by: 14)
+__device__ __forceinline__ float log_normal(float x) {
+  const float hi = __uint_as_float(0x3F317217u), lo = __uint_as_float(0x3377D1CFu), y = __builtin_amdgcn_logf(x);
+  return __builtin_fmaf(y, hi, __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -(y * hi))));
+}
+// gumbel(u01(r)): u01 gives 2^-25 … 1, so -log(u) is 0 or at least 2^-24
+__device__ __forceinline__ float gumbel_of(uint32_t r) {
+  const float t = -log_normal(u01(r));
+  return t == 0.f ? __builtin_inff() : -log_normal(t);
+}
+// Groups of four logits, a Philox block each.  CUT: only what reaches floor_key draws.
+template <bool CUT>
 __device__ __forceinline__ void draw_chunk(const uint4& x, int chunk, float inv_t_log2, uint32_t floor_key, uint2 key, uint64_t step,
                                            const float* noise_row, ArgMax& a) {
   const float ln2 = 0.6931471805599453f;
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
-    bool any = false;
+    if (CUT) {
+      bool any = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) any = any || okey16(half_of(x, half * 4 + e)) >= floor_key;
-    if (!any) continue;                                    // behind a cut-off most groups of four draw nothing
+      for (int e = 0; e < 4; ++e) any = any || okey16(half_of(x, half * 4 + e)) >= floor_key;
+      if (!any) continue;                                  // behind a cut-off most groups of four draw nothing
+    }
     const int i4 = chunk * 2 + half;
     uint4 r = make_uint4(0, 0, 0, 0);
-    if (noise_row == nullptr) r = philox4x32_10(make_uint4((uint32_t)i4, (uint32_t)step, (uint32_t)(step >> 32), 0x5A17u), key);
+    if (!CUT || noise_row == nullptr) r = philox4x32_10(make_uint4((uint32_t)i4, (uint32_t)step, (uint32_t)(step >> 32), 0x5A17u), key);
     const uint32_t rr[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const uint32_t h = half_of(x, half * 4 + e);
-      if (okey16(h) >= floor_key) {
+      const float z = bf2f((uint16_t)h) * inv_t_log2 * ln2;
+      if (!CUT) {
+        take(a, z + gumbel_of(rr[e]), i4 * 4 + e);
+      } else if (okey16(h) >= floor_key) {
         const float u = noise_row != nullptr ? noise_row[i4 * 4 + e] : u01(rr[e]);
-        a = amax(a, ArgMax{bf2f((uint16_t)h) * inv_t_log2 * ln2 + gumbel(u), i4 * 4 + e});
+        take(a, z + gumbel(u), i4 * 4 + e);
       }
     }
   }
@@ -589,12 +610,20 @@ __device__ __forceinline__ ArgMax best_of(uint4 (&regs)[NC], int first, int stri
     return a;
   }
   const uint64_t seed = (uint64_t)draw.seeds[b], step = (uint64_t)draw.steps[b];
+  const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
+  const float inv_t_log2 = 1.4426950408889634f / temp;
+  const float* noise_row = draw.noise != nullptr ? draw.noise + (int64_t)b * V : nullptr;
+  if (floor_key == 0 && noise_row == nullptr) {
+    // Every logit draws: no keys and short logarithms (bound by the vector instructions: µs a call, before → now: rows of 128256 1 8.5 → 7.6,
+    // 57 18.9 → 15.2, 256 54.9 → 41.5; of 32000 100 12.3 → 10.3).  Behind a cut-off few do: __logf in a branch of its own (without branches 57 rows 30 → 33).
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    if (first + c * stride < nchunks)
-      draw_chunk(regs[c], first + c * stride, 1.4426950408889634f / temp, floor_key, make_uint2((uint32_t)seed, (uint32_t)(seed >> 32)), step,
-                 draw.noise != nullptr ? draw.noise + (int64_t)b * V : nullptr, a);
+    for (int c = 0; c < NC; ++c)
+      if (first + c * stride < nchunks) draw_chunk<false>(regs[c], first + c * stride, inv_t_log2, 0u, key, step, nullptr, a);
+    return a;
   }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (first + c * stride < nchunks) draw_chunk<true>(regs[c], first + c * stride, inv_t_log2, floor_key, key, step, noise_row, a);
   return a;
 }
 // Rows of up to 8192 logits: a workgroup each, from the logits to the token in one launch.  V = 2048, one row, µs, two launches / one: greedy 6.5 / 4.6,
@@ -637,7 +666,8 @@ __global__ __launch_bounds__(SNT) void sample_cut_kernel(const uint16_t* __restr
 
 // Grid (slices, B): a 256-thread workgroup takes 256 · NC chunks of 8 logits.  Its best candidate goes into the row's
 // 64-bit maximum (value in the order-preserving 32 bits, then the lowest index); the slice that delivers last reads the result.
-// V = 128256, a quarter of the rows without cut-off: 12 µs at B = 57, 20 at 120.
+// V = 128256, a quarter of the rows without cut-off: 10.5 µs at B = 57.  (Slices of 4096 logits from 2048 workgroups on: greedy rows 57 9.6 → 7.9, but
+// rows behind a cut-off 80 33 → 38, whose Philox blocks then follow one another.)
 constexpr int DNT = 256;
 template <int NC>
 __global__ __launch_bounds__(DNT) void sample_draw_kernel(const uint16_t* __restrict__ logits, int64_t row_stride, int V,

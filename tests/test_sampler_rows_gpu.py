@@ -62,3 +62,18 @@ def test_cut_off_rows(v):
         score[z < cut] = -_INF
         best = score.max()
         assert score[got[i]] >= best - 1e-5 * max(1.0, abs(best.item())), (kinds[i // 3], i % 3)
+
+
+# rows that every logit draws in: one launch, slices of one and of four chunks a thread; −0, masks and equal logits among them
+@pytest.mark.parametrize("b,v", [(3, 8), (5, 8192), (7, 8200), (40, 131072), (520, 32776)])
+def test_plain_draws_are_the_row_kernels(b, v):
+    """The draw of rows without cut-off takes its logarithms in fewer instructions; the fp32 rows' kernel takes ``__logf``: same ids."""
+    g = torch.Generator().manual_seed(v)
+    x = (torch.randn(b, v, generator=g) * torch.tensor([0.0, 0.5, 4.0])[torch.arange(b) % 3, None]).bfloat16()
+    x[1, ::2], x[2, v // 2:] = -0.0, -_INF
+    i = torch.arange(b)
+    temp, ones, none = (0.3 + 0.35 * (i % 5)).cuda(), torch.ones(b).cuda(), torch.zeros(b, dtype=torch.int32).cuda()
+    x = x.cuda()
+    for r in range(3):
+        seeds, steps = (i * 104729 + r).cuda(), (i * 17 + r).cuda()
+        assert torch.equal(ops.sample(x, temp, ones, none, seeds, steps), ops.sample(x.float(), temp, ones, none, seeds, steps))
