@@ -127,10 +127,16 @@ def decode_chunk_pages(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int =
     5.73 TB/s, 32-page ranges 5.64, 16-page 5.40, 8-page 5.11 — per-workgroup fixed cost and the extra reduce pass
     outweigh the better balance; row order, longest first, is what recovers the tail), so big batches get ONE range per
     row.  Smaller batches cut the longest row into as many ranges as it takes to reach that fill (whole multiples of 4
-    pages: one per wave and iteration of an e4m3 workgroup's four; of a bf16 workgroup's eight half may have none, which costs nothing) — each row by its own length, a short row stays one range.  ``cap_items``:
+    pages: one per wave and iteration of an e4m3 workgroup's four; of a bf16 workgroup's eight half may have none, which costs nothing) — each row by its own length, a short row stays one range.  Short rows stay whole in any batch: the launch that adds up
+    ranges costs 3 µs, a range's pages come at what one compute unit reads (a page of eight waves' first round 0.2 µs), and the more
+    workgroups there are the less a cut spreads.  Whole against cut, 32/8 and 64/8 heads, both page types: one row of 8 pages 0.79–0.84,
+    of 12 0.85–0.91, of 16 0.95–1.05, of 20 1.0–1.06; 16 rows of 16 pages 0.89–0.95, of 25 1.0–1.07; 32 of 25 0.83–0.97, of 50 0.9–1.09;
+    60 of 31 0.88–0.94.  ``cap_items``:
     ranges are doubled until the list fits (the fixed grid of a hipGraph)."""
     pages = (np.asarray(seq_lens, dtype=np.int64) + 31) >> 5
     n, maxp = len(pages), max(int(pages.max()) if len(pages) else 1, 1)
+    if maxp <= 12 + n * num_kv_heads // 20:
+        return (maxp + 3) // 4 * 4
     want = (2 * num_cus + n * num_kv_heads - 1) // max(n * num_kv_heads, 1)      # ranges the longest row should give
     if want <= 1:
         return (maxp + 3) // 4 * 4

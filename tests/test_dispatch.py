@@ -3,6 +3,7 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 import torch
 
@@ -168,3 +169,10 @@ def test_plain_tensors():
         look(fw.make_dual(t, t))
     torch.jit.trace(look, (t,), check_trace=False)
     assert seen == [False] * 5 and ops._plain(t)
+
+
+def test_short_decode_rows_stay_whole():
+    """Sizes timed with rows cut into ranges and whole: (rows, heads, pages of the longest) on both sides of the line."""
+    cut = lambda n, heads, pages: len(ops.build_decode_work(np.full(n, 32 * pages), heads)[1]) > 0
+    assert not any(cut(*size) for size in ((1, 8, 12), (1, 1, 12), (16, 8, 18), (32, 8, 24), (60, 8, 36), (250, 1, 24), (64, 8, 64)))
+    assert all(cut(*size) for size in ((1, 8, 13), (1, 1, 20), (8, 8, 20), (16, 8, 25), (32, 8, 50), (60, 8, 48)))
