@@ -517,7 +517,7 @@ def rope_and_cache(qkv: torch.Tensor, positions: torch.Tensor, cos_sin: Optional
                                head_dim, k_scale, v_scale)
 
 
-# Mixed steps: prefill tiles next to the decode rows on a side stream (same-box serving A/B: TPOT p50 39.4 → 38.4 ms,
+# Captured mixed steps: prefill tiles next to the decode rows on a side stream (same-box serving A/B: TPOT p50 39.4 → 38.4 ms,
 # profiles/bench_r3aj_concurrent_attention_{0,1}.json).  DLI_CONCURRENT_ATTN=0: one after the other.
 CONCURRENT_ATTN = os.environ.get("DLI_CONCURRENT_ATTN", "1") != "0"
 _ATTN_STREAMS: dict = {}
@@ -528,6 +528,23 @@ def _attn_stream(device):
     if key not in _ATTN_STREAMS:
         _ATTN_STREAMS[key] = torch.cuda.Stream(device=device)
     return _ATTN_STREAMS[key]
+
+
+def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page_element_bytes: int) -> bool:
+    """Does an eager mixed step pay for a second stream?  Its events cost 30 to 55 µs of host time and, where the host keeps up, 10 of the GPU's; a captured
+    graph's branches cost neither.  And the two launches only run beside each other where their registers fit a compute unit together: prompts of one
+    page group, not of two.  Then it pays from about 0.7 GB of cache pages on (rows × longest context), in bf16 from half of that where up to two
+    prompt workgroups a unit leave room.  µs, beside / one after the other, 32/8 heads: 2 rows of up to 400 tokens and a prompt of 40 42.4 / 19.9; e4m3
+    96 of up to 1500 and two chunks of 1024 behind 1024 86.5 / 83.0 (bf16, one group, 0.59 GB 111 / 116), 400 of up to 1500 and three of 1000 behind 500 165.6 / 188.8, with 200 of up to 1000 124 / 109; bf16 64 rows of up to 1000 and three of
+    1000 behind 500 105 / 94, 200 140 / 150; two groups, 160 of up to 2000 and one of 800 behind 300 159 / 165, 300 of up to 1500 and one of 200 behind
+    500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97.  Captured: 0.65 to 0.95 of the
+    time one after the other for a prompt of 40 tokens, 0.87 to 1.04 for 4 × 300, 1.0 to 1.39 for longer ones, so branches there."""
+    longest = meta.max_seq_len or 1024                       # (0: not known)
+    room = page_element_bytes == 2 and meta.num_prefill_tiles * num_kv_heads <= 512
+    if meta.num_decode * longest * num_kv_heads * 256 * page_element_bytes < (350_000_000 if room else 700_000_000):
+        return False
+    return hip().prefill_page_groups(meta.num_prefill_tiles, num_kv_heads, num_heads // num_kv_heads, meta.max_seq_len, meta.num_prefill,
+                                     page_element_bytes == 1) == 1
 
 
 def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, meta: AttnMetadata,
@@ -546,7 +563,9 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         lib = hip()
         side = None
         known = (0, 0) if meta.counts_on_device else (meta.max_seq_len, meta.num_prefill)    # a captured launch has bounds only
-        if CONCURRENT_ATTN and meta.num_prefill_tiles > 0 and (meta.decode_items > 0 or meta.num_decode > 0):
+        if (CONCURRENT_ATTN and meta.num_prefill_tiles > 0 and (meta.decode_items > 0 or meta.num_decode > 0)
+                and (torch.cuda.is_current_stream_capturing()
+                     or attention_beside(meta, num_heads, num_kv_heads, k_cache.element_size()))):
             # mixed step: the prefill tiles (MFMA / VALU-bound, a few hundred workgroups) run on a side stream next to the
             # decode rows (HBM-bound) — disjoint rows of `out`; inside a capture the side stream forks from and joins the
             # capturing stream, so the step's graph gets two parallel branches per layer

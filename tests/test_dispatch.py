@@ -176,3 +176,14 @@ def test_short_decode_rows_stay_whole():
     cut = lambda n, heads, pages: len(ops.build_decode_work(np.full(n, 32 * pages), heads)[1]) > 0
     assert not any(cut(*size) for size in ((1, 8, 12), (1, 1, 12), (16, 8, 18), (32, 8, 24), (60, 8, 36), (250, 1, 24), (64, 8, 64)))
     assert all(cut(*size) for size in ((1, 8, 13), (1, 1, 20), (8, 8, 20), (16, 8, 25), (32, 8, 50), (60, 8, 48)))
+
+
+def test_mixed_attention_takes_a_second_stream_where_it_pays():
+    """Sizes timed both ways: (decode rows, longest context, prefill tiles, prompts, heads, kv heads, bytes of a page element)."""
+    def beside(rows, longest, tiles, prompts, heads, kv_heads, size):
+        meta = ops.AttnMetadata(rows, prompts, 0, None, None, None, None, None, max_seq_len=longest, num_prefill_tiles=tiles)
+        return ops.attention_beside(meta, heads, kv_heads, size)
+    assert all(beside(*size) for size in ((400, 1500, 66, 3, 32, 8, 1), (200, 1500, 66, 3, 32, 8, 2), (400, 1500, 94, 1, 64, 8, 2),
+                                          (96, 1490, 37, 2, 32, 8, 2), (60, 1490, 43, 2, 64, 8, 2), (400, 0, 94, 3, 32, 8, 2)))
+    assert not any(beside(*size) for size in ((2, 400, 2, 1, 32, 8, 1), (96, 1490, 37, 2, 32, 8, 1), (200, 1500, 66, 3, 32, 8, 1),
+                                              (64, 1318, 65, 3, 32, 8, 2), (64, 994, 76, 4, 32, 8, 2), (200, 999, 51, 4, 64, 8, 1), (400, 1500, 47, 1, 32, 8, 2), (400, 1500, 94, 1, 8, 1, 2), (1, 0, 2, 1, 32, 8, 2)))
