@@ -452,21 +452,33 @@ __device__ __forceinline__ void solve_block(float* Mn, const float* wt, float* w
   const int tiles = sp.DT + sp.CV;
   for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
     f32x4 x[2][4];
+    // All loads in flight together, the values' at clamped places: a branch around each of them made every one of 32 wait for itself.
+    A raw[2][4][4];
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
-      const int t = min(t0 + y, tiles - 1);
+      const int t = min(t0 + y, tiles - 1), e = (t - sp.DT) * 16 + c;
+      if (t < sp.DT) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (t < sp.DT) {
-          x[y][i] = *reinterpret_cast<const f32x4*>(ww + (i * sp.DT + t) * TILE + lane * 4);
-        } else {
+        for (int i = 0; i < 4; ++i) x[y][i] = *reinterpret_cast<const f32x4*>(ww + (i * sp.DT + t) * TILE + lane * 4);
+      } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int row = 16 * i + 4 * g4 + r, e = (t - sp.DT) * 16 + c;
-            x[y][i][r] = row < n && e < Dv ? wt[row] * ldf<A>(v + row * v_stride + e) : 0.f;
-          }
-        }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) raw[y][i][r] = v[min(16 * i + 4 * g4 + r, n - 1) * v_stride + min(e, Dv - 1)];
       }
+    }
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int t = min(t0 + y, tiles - 1), e = (t - sp.DT) * 16 + c;
+      if (t < sp.DT) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * i + 4 * g4 + r;
+          const float u = wt[row] * ldf<A>(&raw[y][i][r]);
+          x[y][i][r] = row < n && e < Dv ? u : 0.f;
+        }
     }
     solve_tiles<2>(Mn, x, lane);
 #pragma unroll
@@ -613,22 +625,35 @@ __global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict_
   const A* kc[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) kc[s] = k + row_of(16 * s + c) * k_stride + g * D;
+  // (the kind of reads is asked for once, and a turn's six come together: behind conditions each of them was waited for by itself)
+  auto products = [&](auto wide_rows) __attribute__((always_inline)) {
+    constexpr bool WIDE = decltype(wide_rows)::value;
+    auto read = [&](const A* r, int d) __attribute__((always_inline)) {
+      if constexpr (!WIDE) return row4(r, d, D, false);
+      const f32x4 x = ld4<A>(r + min(d, D - 4));
+      return d < D ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
 #pragma unroll 2
-  for (int it = 0; it < sp.DT; ++it) {
-    const int d = 16 * it + 4 * g4;
-    const f32x4 qa = row4(qr, d, D, wide), ka = row4(kr, d, D, wide);
+    for (int it = 0; it < sp.DT; ++it) {
+      const int d = 16 * it + 4 * g4;
+      const f32x4 qa = read(qr, d), ka = read(kr, d);
+      f32x4 kb[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (s <= wave) {
-        const f32x4 kb = row4(kc[s], d, D, wide);
-        qk[s] = mfma_k16(qa, kb, qk[s]);
-        kk[s] = mfma_k16(ka, kb, kk[s]);
-      }
-    const int at = (wave * sp.DT + it) * TILE + lane * 4;
-    *reinterpret_cast<f32x4*>(wa + sp.q() + at) = f32x4{qa[0] * eq, qa[1] * eq, qa[2] * eq, qa[3] * eq};
-    *reinterpret_cast<f32x4*>(wa + sp.w() + at) = turned(f32x4{ka[0] * ew, ka[1] * ew, ka[2] * ew, ka[3] * ew}, unit);
-    *reinterpret_cast<f32x4*>(wa + sp.kt() + (it * 4 + wave) * TILE + lane * 4) = turned(f32x4{ka[0] * er, ka[1] * er, ka[2] * er, ka[3] * er}, unit);
-  }
+      for (int s = 0; s < 4; ++s) kb[s] = read(kc[s], d);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s <= wave) {
+          qk[s] = mfma_k16(qa, kb[s], qk[s]);
+          kk[s] = mfma_k16(ka, kb[s], kk[s]);
+        }
+      const int at = (wave * sp.DT + it) * TILE + lane * 4;
+      *reinterpret_cast<f32x4*>(wa + sp.q() + at) = f32x4{qa[0] * eq, qa[1] * eq, qa[2] * eq, qa[3] * eq};
+      *reinterpret_cast<f32x4*>(wa + sp.w() + at) = turned(f32x4{ka[0] * ew, ka[1] * ew, ka[2] * ew, ka[3] * ew}, unit);
+      *reinterpret_cast<f32x4*>(wa + sp.kt() + (it * 4 + wave) * TILE + lane * 4) = turned(f32x4{ka[0] * er, ka[1] * er, ka[2] * er, ka[3] * er}, unit);
+    }
+  };
+  if (wide) products(std::true_type{});
+  else products(std::false_type{});
 #pragma unroll
   for (int s = 0; s < 4; ++s)
     if (s <= wave) {
