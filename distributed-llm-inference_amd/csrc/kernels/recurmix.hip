@@ -236,6 +236,11 @@ __global__ __launch_bounds__(NT) void causal_conv_run_kernel(const A* __restrict
   Vec<A, 4> in[RUN];
 #pragma unroll
   for (int i = 0; i < RUN; ++i) in[i].load(x + (int64_t)(t0 + min(i, n - 1)) * x_stride + c);
+  // The rows in front of the run, before it is known whose they are: a run inside a chunk (most are) waits for memory once, not for its sequence's
+  // number, its bounds and then for its rows.
+  Vec<A, 4> front[3];
+#pragma unroll
+  for (int d = 1; d <= 3; ++d) front[d - 1].load(x + (int64_t)max(t0 - d, 0) * x_stride + c);
   Vec<float, 4> wt[4], b, h1, h2, h3;                            // h_d: the input d tokens back
 #pragma unroll
   for (int j = 0; j < 4; ++j) wt[j].load(w + (int64_t)j * C + c);
@@ -265,7 +270,8 @@ __global__ __launch_bounds__(NT) void causal_conv_run_kernel(const A* __restrict
           Vec<float, 4> v;
           if (d <= back) {
             Vec<A, 4> xv;
-            xv.load(xr - (int64_t)d * x_stride);
+            if (i == 0) xv = front[d - 1];
+            else xv.load(xr - (int64_t)d * x_stride);
 #pragma unroll
             for (int k = 0; k < 4; ++k) v.v[k] = xv.v[k];
           } else {
