@@ -787,7 +787,9 @@ __global__ __launch_bounds__(NT) void token_attention_kernel(
   }
 }
 
-// combine the nsplit (≤ 16) partial results of a (token, head): part [T][H][nsplit][2 + Dv] = (max, sum, unnormalised output)
+// Combine the nsplit (≤ 8) partial results of a (token, head): part [T][H][nsplit][2 + Dv] = (max, sum, unnormalised output).  Bound by the loads'
+// latency, so all of them are asked for at once, from places that exist: a split's numbers by a lane each, its first outputs by all.
+constexpr int SPLITS = 8;
 template <typename A>
 __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restrict__ out, int64_t o_ts, int64_t o_hs,
                                                                     const float* __restrict__ part,
@@ -796,28 +798,38 @@ __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restric
                                                                     AttnOpts opt) {
   const int64_t t = blockIdx.x;
   const int h = blockIdx.y;
+  const int ps = Dv + 2;
+  const float* pr = part + (t * H + h) * nsplit * (int64_t)ps;
+  const float* mine = pr + min((int)threadIdx.x & (SPLITS - 1), nsplit - 1) * ps;
+  const float mz = mine[0], lz = mine[1];
+  float v[SPLITS];
+  auto fetch = [&](int e) {
+#pragma unroll
+    for (int z = 0; z < SPLITS; ++z) v[z] = pr[min(z, nsplit - 1) * ps + 2 + min(e, Dv - 1)];
+  };
+  fetch(threadIdx.x);
+  float gv = gate != nullptr ? ldf<A>(gate + t * g_ts + h) : 0.f;
   if (token_seq[t] < 0) {
     for (int e = threadIdx.x; e < Dv; e += 128) store_out(out, opt, t * o_ts + h * o_hs + e, 0.f);
     return;
   }
-  const float* pr = part + (t * H + h) * nsplit * (int64_t)(Dv + 2);
-  float M = -INFINITY;
-  for (int z = 0; z < nsplit; ++z) M = fmaxf(M, pr[z * (Dv + 2)]);
-  float f[16];
-  float L = 0.f;
+  const float M = wave_max(mz);                           // (lanes past the last split repeat it)
+  const float fz = mz == -INFINITY ? 0.f : expf(mz - M);
+  float f[SPLITS], L = 0.f;
 #pragma unroll
-  for (int z = 0; z < 16; ++z) {
-    const float mz = z < nsplit ? pr[z * (Dv + 2)] : -INFINITY;
-    f[z] = mz == -INFINITY ? 0.f : expf(mz - M);
-    if (z < nsplit) L += f[z] * pr[z * (Dv + 2) + 1];
+  for (int z = 0; z < SPLITS; ++z) {
+    f[z] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fz), z));
+    const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lz), z));
+    if (z < nsplit) L += f[z] * l;
   }
   if (sink != nullptr) L += expf(sink[h] - M);
-  const float rl = (gate != nullptr ? 1.f / (1.f + expf(-ldf<A>(gate + t * g_ts + h))) : 1.f) / L * opt.out_scale;
+  const float rl = (gate != nullptr ? 1.f / (1.f + expf(-gv)) : 1.f) / L * opt.out_scale;
   for (int e = threadIdx.x; e < Dv; e += 128) {
+    if (e != (int)threadIdx.x) fetch(e);
     float o = 0.f;
 #pragma unroll
-    for (int z = 0; z < 16; ++z)
-      if (z < nsplit) o += f[z] * pr[z * (Dv + 2) + 2 + e];
+    for (int z = 0; z < SPLITS; ++z)
+      if (z < nsplit) o += f[z] * v[z];
     store_out(out, opt, t * o_ts + h * o_hs + e, o * rl);
   }
 }
@@ -837,27 +849,37 @@ __global__ __launch_bounds__(128) void map_merge_kernel(A* __restrict__ out, int
   }
   const int64_t ps = Dv + 2;
   const float* pr[2];
-  float f[2][16];
+  float f[2][SPLITS], mz[2], lz[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {                           // a lane a split, as above
+    pr[m] = part + (t * H2 + (head / per * 2 + m) * per + head % per) * nsplit * ps;
+    const float* mine = pr[m] + min((int)threadIdx.x & (SPLITS - 1), nsplit - 1) * ps;
+    mz[m] = mine[0];
+    lz[m] = mine[1];
+  }
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
-    pr[m] = part + (t * H2 + (head / per * 2 + m) * per + head % per) * nsplit * ps;
-    float M = -INFINITY, L = 0.f;
-    for (int z = 0; z < nsplit; ++z) M = fmaxf(M, pr[m][z * ps]);
+    const float M = wave_max(mz[m]), fz = mz[m] == -INFINITY ? 0.f : expf(mz[m] - M);
+    float L = 0.f;
 #pragma unroll
-    for (int z = 0; z < 16; ++z) {
-      const float mz = z < nsplit ? pr[m][z * ps] : -INFINITY;
-      f[m][z] = mz == -INFINITY ? 0.f : expf(mz - M);
-      if (z < nsplit) L += f[m][z] * pr[m][z * ps + 1];
+    for (int z = 0; z < SPLITS; ++z) {
+      f[m][z] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fz), z));
+      const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lz[m]), z));
+      if (z < nsplit) L += f[m][z] * l;
     }
     const float r = (m == 0 ? 1.f : -opt.lam[0]) / L;
 #pragma unroll
-    for (int z = 0; z < 16; ++z) f[m][z] *= r;
+    for (int z = 0; z < SPLITS; ++z) f[m][z] *= r;
   }
   auto value = [&](int e) {
-    float d = 0.f;
+    float d = 0.f, v[2][SPLITS];
 #pragma unroll
-    for (int z = 0; z < 16; ++z)
-      if (z < nsplit) d += f[0][z] * pr[0][z * ps + 2 + e] + f[1][z] * pr[1][z * ps + 2 + e];
+    for (int z = 0; z < SPLITS; ++z)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) v[m][z] = pr[m][min(z, nsplit - 1) * ps + 2 + min(e, Dv - 1)];
+#pragma unroll
+    for (int z = 0; z < SPLITS; ++z)
+      if (z < nsplit) d += f[0][z] * v[0][z] + f[1][z] * v[1][z];
     return d;
   };
   float d[4], ss = 0.f;                                   // Dv ≤ 512
@@ -1207,8 +1229,12 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 // (K rows, V transposed into the MFMA slot order); all four waves compute the same Sᵀ = K·Qᵀ tile and online softmax, and
 // each accumulates its own quarter of the value columns, so nothing is merged inside the workgroup.  gridDim.z slices of
 // the key range leave (max, sum, unnormalised output) in `part` for token_attention_merge_kernel.
-template <int KSMAX, int MTQ>
-__global__ __launch_bounds__(NT) void head_decode_attention_kernel(
+// Few rows are bound by the chain through a slice's pages, many by the LDS (every wave reads all of a page's keys).  A page is therefore
+// asked for, whole, while the one before it is computed, and goes from registers to both of its places (VK: values that lead the key row
+// are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed → now:
+// 1 row of 200 24.5 → 13.4, of 2000 58.7 → 37.3, 32 of 1500 64.7 → 41.7, 256 of 2000 504 → 257.
+template <int KSMAX, int MTQ, bool VK>
+__global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
     const uint16_t* __restrict__ q2, int64_t q2_ts, int64_t q2_hs, int D2, const uint16_t* __restrict__ kc, int rowk,
     const uint16_t* __restrict__ vc, int rowv, int vhead, int Dv, const int* __restrict__ block_tables, int max_blocks,
@@ -1233,7 +1259,7 @@ __global__ __launch_bounds__(NT) void head_decode_attention_kernel(
   const int KS = (Dk + 31) >> 5, MT = Dv >> 4;
   const int MTW = (MT + 3) >> 2;                         // value tiles per wave
   const int KST = KS * 32 + 8;
-  constexpr int VST = 40;
+  constexpr int VST = 36;                                 // as in the tile kernel
   uint16_t* Ks = tl;
   uint16_t* Vt = tl + 32 * KST;
   for (int i = threadIdx.x; i < 32 * (KS * 32 - Dk); i += NT) {
@@ -1269,26 +1295,69 @@ __global__ __launch_bounds__(NT) void head_decode_attention_kernel(
 #pragma unroll
   for (int i = 0; i < MTQ; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int kchunks = Dk >> 3, vchunks = Dv >> 3;
-  const bool vfromk = vc == kc && rowv == rowk && vhead == Dk;     // latent attention: one row is key and value
+  // a thread's share of a page: pieces of 4 rows × 8 columns, whose slots are neighbours in Vt (VK: the value columns lead the key row, and
+  // a piece fetched once is put in both places)
+  constexpr int NK = (KSMAX + 7) / 8, NV = VK ? 1 : (MTQ + 3) / 4;
+  bf16x8 kr[NK][4], vr[NV][4];
+  auto fetch = [&](int it) {
+    const int64_t page_row = (int64_t)bt[it < kb_lo ? it - it_lo : it] * kBlockTokens;
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+      const int i = min((int)threadIdx.x + u * NT, 8 * kchunks - 1);
+      const uint16_t* p4 = kc + (page_row + 4 * (i & 7)) * rowk + g * Dk + 8 * (i >> 3);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) kr[u][r] = *reinterpret_cast<const bf16x8*>(p4 + (int64_t)r * rowk);
+    }
+    if constexpr (!VK) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int i = min((int)threadIdx.x + u * NT, 8 * vchunks - 1);
+        const uint16_t* p4 = vc + (page_row + 4 * (i & 7)) * rowv + gv * vhead + 8 * (i >> 3);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vr[u][r] = *reinterpret_cast<const bf16x8*>(p4 + (int64_t)r * rowv);
+      }
+    }
+  };
+  auto put_values = [&](int i, bf16x8 v0, bf16x8 v1, bf16x8 v2, bf16x8 v3) {
+    uint16_t* dst = Vt + (i >> 3) * 8 * VST + (i & 3) * 8 + ((i & 7) >> 2) * 4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<bf16x4*>(dst + j * VST) = bf16x4{v0[j], v1[j], v2[j], v3[j]};
+  };
+  if (it_begin <= it_end) fetch(it_begin);
+  // the queries have arrived here (otherwise they, and the page on its way with them, are waited for in front of every page's first product)
+#pragma unroll
+  for (int s = 0; s < KSMAX; ++s) asm volatile("" : "+v"(qf[s]));
   for (int it = it_begin; it <= it_end; ++it) {
     const int kb = it < kb_lo ? it - it_lo : it;
-    __syncthreads();
-    const int64_t page_row = (int64_t)bt[kb] * kBlockTokens;
-    for (int i = threadIdx.x; i < 32 * kchunks; i += NT) {
-      const int row = i / kchunks, ch = i - row * kchunks;
-      *reinterpret_cast<bf16x8*>(Ks + row * KST + 8 * ch) =
-          *reinterpret_cast<const bf16x8*>(kc + (page_row + row) * rowk + g * Dk + 8 * ch);
-    }
-    if (vfromk) __syncthreads();                          // values = leading columns of the key rows just staged
-    for (int i = threadIdx.x; i < 32 * vchunks; i += NT) {
-      const int row = i & 31, ch = i >> 5;
-      const bf16x8 v = vfromk ? *reinterpret_cast<const bf16x8*>(Ks + row * KST + 8 * ch)
-                              : *reinterpret_cast<const bf16x8*>(vc + (page_row + row) * rowv + gv * vhead + 8 * ch);
-      const int slot = ((row & 15) >> 2) * 8 + (row >> 4) * 4 + (row & 3);
+    lds_barrier();                                        // everyone is done with the page before
 #pragma unroll
-      for (int j = 0; j < 8; ++j) Vt[(8 * ch + j) * VST + slot] = (uint16_t)v[j];
+    for (int u = 0; u < NK; ++u) {
+      const int i = (int)threadIdx.x + u * NT;
+      if (i < 8 * kchunks) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) *reinterpret_cast<bf16x8*>(Ks + (4 * (i & 7) + r) * KST + 8 * (i >> 3)) = kr[u][r];
+        if (VK && i < 8 * vchunks) put_values(i, kr[u][0], kr[u][1], kr[u][2], kr[u][3]);
+      }
     }
-    __syncthreads();
+    if constexpr (!VK) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int i = (int)threadIdx.x + u * NT;
+        if (i < 8 * vchunks) put_values(i, vr[u][0], vr[u][1], vr[u][2], vr[u][3]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NK; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(kr[u][r]));
+    if constexpr (!VK) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(vr[u][r]));
+    }
+    if (it < it_end) fetch(it + 1);
+    lds_barrier();
     f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KSMAX; ++s) {
@@ -1332,7 +1401,8 @@ __global__ __launch_bounds__(NT) void head_decode_attention_kernel(
     for (int ii = 0; ii < MTQ; ++ii) {
       const int i = wave * MTW + ii;
       if (ii < MTW && i < MT) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(Vt + (16 * i + c) * VST + 8 * g4);
+        const bf16x4* vp = reinterpret_cast<const bf16x4*>(Vt + (16 * i + c) * VST + 8 * g4);   // (rows of Vt are 8-byte aligned)
+        const bf16x8 vf = __builtin_shufflevector(vp[0], vp[1], 0, 1, 2, 3, 4, 5, 6, 7);
         f32x4 a = acc[ii];
         a[0] *= corr; a[1] *= corr; a[2] *= corr; a[3] *= corr;
         a = mfma16(vf, ph, a);
@@ -1683,7 +1753,7 @@ int sm_token_attention_splits(int rows, int H, int G) {
   const int per = H / G;
   const int hg = per % 4 == 0 ? 4 : (per % 2 == 0 ? 2 : 1);
   const int wgs = std::max(rows * (H / hg), 1);
-  return std::max(1, std::min(8, 1024 / wgs));
+  return std::max(1, std::min(SPLITS, 1024 / wgs));
 }
 
 // prefill tiles on the matrix cores (bf16; see tile_attention_kernel).  Returns false when the shapes do not fit its
@@ -1763,26 +1833,29 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
                   o_hs % 4 == 0 && al(out, 8) && al(opt.out_f32, 16) && al(q1, 16) && al(q2, 16) && al(kc, 16) && al(vc, 16);
   if (!ok) return false;
   if (rows == 0) return true;
-  const size_t lds = (size_t)(32 * (KS * 32 + 8) + Dv * 40) * sizeof(uint16_t);
+  const size_t lds = (size_t)(32 * (KS * 32 + 8) + Dv * 36) * sizeof(uint16_t);
   const int groups = (per + 15) / 16;
+  const bool vfromk = vc == kc && rowv == rowk && vhead == Dk && Dv <= Dk;   // latent attention: one row is key and value
   const dim3 grid(rows, G * groups, nsplit);
-#define SM_HD(KSM, MTQV)                                                                                                         \
+#define SM_HD2(KSM, MTQV, VKV)                                                                                                      \
   do {                                                                                                                           \
     static bool big = false;                                                                                                     \
     if (lds > 48 * 1024 && !big) {                                                                                               \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&head_decode_attention_kernel<KSM, MTQV>),                         \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&head_decode_attention_kernel<KSM, MTQV, VKV>),                         \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 100 * 1024);                                         \
       big = true;                                                                                                                \
     }                                                                                                                            \
-    hipLaunchKernelGGL((head_decode_attention_kernel<KSM, MTQV>), grid, dim3(NT), lds, stream, (uint16_t*)out, o_ts, o_hs,       \
+    hipLaunchKernelGGL((head_decode_attention_kernel<KSM, MTQV, VKV>), grid, dim3(NT), lds, stream, (uint16_t*)out, o_ts, o_hs,       \
                        (const uint16_t*)q1, q1_ts, q1_hs, D1, (const uint16_t*)q2, q2_ts, q2_hs, D2, (const uint16_t*)kc, rowk,  \
                        (const uint16_t*)vc, rowv, vhead, Dv, block_tables, max_blocks, positions, token_seq, H, G, groups, scale,\
                        window, temp, r1, r2, nsplit, part, (const uint16_t*)gate, g_ts, sink, opt);                                         \
   } while (0)
+#define SM_HD(KSM, MTQV) do { if (vfromk) SM_HD2(KSM, MTQV, true); else SM_HD2(KSM, MTQV, false); } while (0)
   if (KS <= 4 && MT <= 8) SM_HD(4, 2);
   else if (KS <= 8 && MT <= 16) SM_HD(8, 4);
   else SM_HD(18, 8);
 #undef SM_HD
+#undef SM_HD2
   if (opt.lam != nullptr)
     hipLaunchKernelGGL(map_merge_kernel<uint16_t>, dim3(rows, H / 2), dim3(128), 0, stream, (uint16_t*)out, o_ts, o_hs, (const float*)part,
                        token_seq, per, Dv, nsplit, opt);
@@ -1796,7 +1869,7 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
 int sm_head_decode_splits(int rows, int H, int G) {
   const int per = H / G;
   const int wgs = std::max(rows * G * ((per + 15) / 16), 1);
-  return std::max(1, std::min(8, 512 / wgs));
+  return std::max(1, std::min(SPLITS, 512 / wgs));
 }
 
 // rows of the state one wave keeps: D is cut into parts so that a wave's per-token loop is short and more waves share the work

@@ -1,0 +1,60 @@
+"""Decode rows over token-major pages: whole and split key ranges, page remainders, one row as key and value, shared heads."""
+import pytest
+import torch
+
+from dli_amd.ops import AttnMetadata, seqmix
+
+pytestmark = pytest.mark.gpu
+PAGE = 32
+
+
+def _rows(lens, seed):
+    """Pages of the rows in a shuffled order; the last row is padding."""
+    n = [-(-x // PAGE) for x in lens]
+    order = (torch.randperm(sum(n), generator=torch.Generator().manual_seed(seed)) + 1).int()
+    tables = torch.zeros(len(lens) + 1, max(n), dtype=torch.int32)
+    at = 0
+    for i, k in enumerate(n):
+        tables[i, :k] = order[at:at + k]
+        at += k
+    return tables, sum(n) + 1
+
+
+def _exact(q, k, v, tables, lens, G, scale, window, cap):
+    out = torch.zeros(len(lens) + 1, q.shape[1], v.shape[-1], dtype=torch.float64)
+    per = q.shape[1] // G
+    for i, x in enumerate(lens):
+        j = torch.arange(max(0, x - window) if window else 0, x)
+        at = tables[i, j // PAGE].long() * PAGE + j % PAGE
+        for h in range(q.shape[1]):
+            s = k[at, h // per].double() @ q[i, h].double() * scale
+            s = cap * torch.tanh(s / cap) if cap else s
+            out[i, h] = torch.softmax(s, 0) @ v[at, h // per].double()
+    return out
+
+
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33, 65], [700], [257] * 70])
+@pytest.mark.parametrize("H,G,Dk,Dv,shared", [(8, 1, 24, 16, False), (16, 2, 128, 128, False), (20, 1, 72, 80, False), (32, 1, 576, 512, True),
+                                              (8, 1, 320, 512, False), (24, 2, 192, 64, True), (6, 2, 20, 33, False)])
+def test_decode_rows(H, G, Dk, Dv, shared, lens):
+    g = torch.Generator().manual_seed(H * Dk + len(lens))
+    tables, pages = _rows(lens, Dk)
+    T = len(lens) + 1
+    q = torch.randn(T, H, Dk, generator=g).bfloat16()
+    k = torch.randn(pages * PAGE, G, Dk, generator=g).bfloat16()
+    v = k[..., :Dv] if shared else torch.randn(pages * PAGE, G, Dv, generator=g).bfloat16()
+    scale = Dk ** -0.5
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    meta = AttnMetadata(num_decode=T, num_prefill=0, num_tokens=T, positions=ints([x - 1 for x in lens] + [0]), slot_mapping=ints([-1] * T),
+                        block_tables=tables.cuda(), seq_lens=ints(lens + [0]), query_start_loc=ints(range(T + 1)), token_seq=ints([*range(T - 1), -1]))
+    for window, cap in ((0, 0.0), (40, 5.0)):
+        want = _exact(q, k, v, tables, lens, G, scale, window, cap)
+        for dtype in (torch.bfloat16, torch.float32):
+            out = torch.full((T, H, Dv), float("nan"), dtype=dtype, device="cuda")
+            seqmix.token_attention(out, q.cuda(), None, k.cuda().view(pages, PAGE, -1), None if shared else v.cuda().view(pages, PAGE, -1), meta, G, Dv,
+                                   scale, window, cap=cap)
+            got = out.double().cpu()
+            # weights of 16 bits at least and scores to some 2^-20, times the largest value; bf16 results are rounded once more
+            bound = float(v.abs().max()) * 2.0 ** -15 + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
+            assert ((got - want).abs() <= bound).all(), (window, cap, dtype, (got - want).abs().max())
+            assert not got[-1].any()
