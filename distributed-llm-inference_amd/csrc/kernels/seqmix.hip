@@ -787,9 +787,9 @@ __global__ __launch_bounds__(NT) void token_attention_kernel(
   }
 }
 
-// Combine the nsplit (≤ 8) partial results of a (token, head): part [T][H][nsplit][2 + Dv] = (max, sum, unnormalised output).  Bound by the loads'
+// Combine the nsplit (≤ 16) partial results of a (token, head): part [T][H][nsplit][2 + Dv] = (max, sum, unnormalised output).  Bound by the loads'
 // latency, so all of them are asked for at once, from places that exist: a split's numbers by a lane each, its first outputs by all.
-constexpr int SPLITS = 8;
+constexpr int SPLITS = 16;
 template <typename A>
 __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restrict__ out, int64_t o_ts, int64_t o_hs,
                                                                     const float* __restrict__ part,
@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 }
 
 // ------------------------------------------------------------------------------------------------ attention, decode rows, heads as columns
-// bf16 only; for mixers whose query heads share a key / value head in groups of 8 or more (latent attention: all of them).
+// bf16 only; for mixers whose query heads share a key / value head in groups of 4 or more (latent attention: all of them).
 // One workgroup per (token, group of up to 16 heads, slice of the key range): the 16 MFMA columns are the HEADS of one
 // token, so a key row fetched once meets every head on the matrix cores.  Pages are staged as in tile_attention_kernel
 // (K rows, V transposed into the MFMA slot order); all four waves compute the same Sᵀ = K·Qᵀ tile and online softmax, and
@@ -1232,8 +1232,9 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 // Few rows are bound by the chain through a slice's pages, many by the LDS (every wave reads all of a page's keys).  A page is therefore
 // asked for, whole, while the one before it is computed, and goes from registers to both of its places (VK: values that lead the key row
 // are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed → now:
-// 1 row of 200 24.5 → 13.4, of 2000 58.7 → 37.3, 32 of 1500 64.7 → 41.7, 256 of 2000 504 → 257.
-template <int KSMAX, int MTQ, bool VK>
+// 1 row of 200 24.5 → 14.3, of 2000 58.7 → 24.6, 32 of 1500 64.7 → 42, 256 of 2000 504 → 258.
+// FINE: the weights enter P·V in three bf16 parts instead of two.
+template <int KSMAX, int MTQ, bool VK, bool FINE>
 __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
     const uint16_t* __restrict__ q2, int64_t q2_ts, int64_t q2_hs, int D2, const uint16_t* __restrict__ kc, int rowk,
@@ -1299,8 +1300,9 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
   // a piece fetched once is put in both places)
   constexpr int NK = (KSMAX + 7) / 8, NV = VK ? 1 : (MTQ + 3) / 4;
   bf16x8 kr[NK][4], vr[NV][4];
-  auto fetch = [&](int it) {
-    const int64_t page_row = (int64_t)bt[it < kb_lo ? it - it_lo : it] * kBlockTokens;
+  auto page_of = [&](int it) { return bt[it < kb_lo ? it - it_lo : it]; };
+  auto fetch = [&](int page) {
+    const int64_t page_row = (int64_t)page * kBlockTokens;
 #pragma unroll
     for (int u = 0; u < NK; ++u) {
       const int i = min((int)threadIdx.x + u * NT, 8 * kchunks - 1);
@@ -1323,7 +1325,11 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) *reinterpret_cast<bf16x4*>(dst + j * VST) = bf16x4{v0[j], v1[j], v2[j], v3[j]};
   };
-  if (it_begin <= it_end) fetch(it_begin);
+  int next = 0;                                           // the page to fetch next: its number is known a turn before it is used
+  if (it_begin <= it_end) {
+    fetch(page_of(it_begin));
+    next = page_of(min(it_begin + 1, it_end));
+  }
   // the queries have arrived here (otherwise they, and the page on its way with them, are waited for in front of every page's first product)
 #pragma unroll
   for (int s = 0; s < KSMAX; ++s) asm volatile("" : "+v"(qf[s]));
@@ -1356,7 +1362,10 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(vr[u][r]));
     }
-    if (it < it_end) fetch(it + 1);
+    if (it < it_end) {
+      fetch(next);
+      next = page_of(min(it + 2, it_end));
+    }
     lds_barrier();
     f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1386,7 +1395,7 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     const float mu = mn == -INFINITY ? 0.f : mn;
     const float corr = fast_exp2(m - mu);
     m = mn;
-    bf16x8 ph, plo;
+    bf16x8 ph, plo, pl2;
     float ps = 0.f;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
@@ -1394,7 +1403,10 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
       ps += pv;
       const uint16_t hi = f2bf(pv);
       ph[r] = (short)hi;
-      plo[r] = (short)f2bf(pv - bf2f(hi));
+      const float rest = pv - bf2f(hi);
+      const uint16_t lo = f2bf(rest);
+      plo[r] = (short)lo;
+      if constexpr (FINE) pl2[r] = (short)f2bf(rest - bf2f(lo));
     }
     l = l * corr + ps;
 #pragma unroll
@@ -1406,7 +1418,9 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
         f32x4 a = acc[ii];
         a[0] *= corr; a[1] *= corr; a[2] *= corr; a[3] *= corr;
         a = mfma16(vf, ph, a);
-        acc[ii] = mfma16(vf, plo, a);
+        a = mfma16(vf, plo, a);
+        if constexpr (FINE) a = mfma16(vf, pl2, a);
+        acc[ii] = a;
       }
     }
   }
@@ -1753,7 +1767,7 @@ int sm_token_attention_splits(int rows, int H, int G) {
   const int per = H / G;
   const int hg = per % 4 == 0 ? 4 : (per % 2 == 0 ? 2 : 1);
   const int wgs = std::max(rows * (H / hg), 1);
-  return std::max(1, std::min(SPLITS, 1024 / wgs));
+  return std::max(1, std::min(8, 1024 / wgs));
 }
 
 // prefill tiles on the matrix cores (bf16; see tile_attention_kernel).  Returns false when the shapes do not fit its
@@ -1828,7 +1842,12 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
                                      AttnOpts opt, hipStream_t stream) {
   const int Dk = D1 + D2, KS = (Dk + 31) / 32, MT = Dv / 16, per = H / G;
   auto al = [](const void* p, int64_t a) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % a == 0; };
-  const bool ok = per >= 8 && D1 % 8 == 0 && D2 % 8 == 0 && Dv % 16 == 0 && KS <= 18 && MT <= 32 && rowk % 8 == 0 && rowv % 8 == 0 &&
+  // Groups of 4 … 7 heads leave columns idle, and still beat a lane per key (token_attention_kernel) by far: 32 heads on 8 of 128, in a graph, µs:
+  // 1 row of 200 16.7 → 8.1, 8 of 700 21.6 → 13.4, 128 of 1500 129 → 103, 256 of 2000 241 → 195.  (Groups of 2: 8 of 300 11.8 → 10.0, but 256 of
+  // 100 with heads of 64 22.3 → 27.3.)  That kernel's weights are fp32 values, so these take them in three bf16 parts, 24 bits; what shows
+  // more than the rounding of a bf16 result (fp32 results, the difference of two maps) and a soft cap's logistic form stay there.
+  const bool fine = per < 8;
+  const bool ok = (!fine || (per >= 4 && KS <= 8 && MT <= 16 && opt.out_f32 == nullptr && opt.cap == 0.f && opt.lam == nullptr)) && D1 % 8 == 0 && D2 % 8 == 0 && Dv % 16 == 0 && KS <= 18 && MT <= 32 && rowk % 8 == 0 && rowv % 8 == 0 &&
                   vhead % 8 == 0 && q1_ts % 8 == 0 && q1_hs % 8 == 0 && q2_ts % 8 == 0 && q2_hs % 8 == 0 && o_ts % 4 == 0 &&
                   o_hs % 4 == 0 && al(out, 8) && al(opt.out_f32, 16) && al(q1, 16) && al(q2, 16) && al(kc, 16) && al(vc, 16);
   if (!ok) return false;
@@ -1837,23 +1856,30 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
   const int groups = (per + 15) / 16;
   const bool vfromk = vc == kc && rowv == rowk && vhead == Dk && Dv <= Dk;   // latent attention: one row is key and value
   const dim3 grid(rows, G * groups, nsplit);
-#define SM_HD2(KSM, MTQV, VKV)                                                                                                      \
+#define SM_HD2(KSM, MTQV, ...)                                                                                                      \
   do {                                                                                                                           \
     static bool big = false;                                                                                                     \
     if (lds > 48 * 1024 && !big) {                                                                                               \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&head_decode_attention_kernel<KSM, MTQV, VKV>),                         \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&head_decode_attention_kernel<KSM, MTQV, __VA_ARGS__>),                         \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 100 * 1024);                                         \
       big = true;                                                                                                                \
     }                                                                                                                            \
-    hipLaunchKernelGGL((head_decode_attention_kernel<KSM, MTQV, VKV>), grid, dim3(NT), lds, stream, (uint16_t*)out, o_ts, o_hs,       \
+    hipLaunchKernelGGL((head_decode_attention_kernel<KSM, MTQV, __VA_ARGS__>), grid, dim3(NT), lds, stream, (uint16_t*)out, o_ts, o_hs,       \
                        (const uint16_t*)q1, q1_ts, q1_hs, D1, (const uint16_t*)q2, q2_ts, q2_hs, D2, (const uint16_t*)kc, rowk,  \
                        (const uint16_t*)vc, rowv, vhead, Dv, block_tables, max_blocks, positions, token_seq, H, G, groups, scale,\
                        window, temp, r1, r2, nsplit, part, (const uint16_t*)gate, g_ts, sink, opt);                                         \
   } while (0)
-#define SM_HD(KSM, MTQV) do { if (vfromk) SM_HD2(KSM, MTQV, true); else SM_HD2(KSM, MTQV, false); } while (0)
+#define SM_HD(KSM, MTQV)                                                                                                         \
+  do {                                                                                                                           \
+    if (vfromk && fine) SM_HD2(KSM, MTQV, true, true);                                                                           \
+    else if (vfromk) SM_HD2(KSM, MTQV, true, false);                                                                             \
+    else if (fine) SM_HD2(KSM, MTQV, false, true);                                                                               \
+    else SM_HD2(KSM, MTQV, false, false);                                                                                        \
+  } while (0)
   if (KS <= 4 && MT <= 8) SM_HD(4, 2);
   else if (KS <= 8 && MT <= 16) SM_HD(8, 4);
-  else SM_HD(18, 8);
+  else if (vfromk) SM_HD2(18, 8, true, false);
+  else SM_HD2(18, 8, false, false);
 #undef SM_HD
 #undef SM_HD2
   if (opt.lam != nullptr)
@@ -1865,11 +1891,14 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
   return true;
 }
 
-// slices of the key range for that kernel: about 512 workgroups
-int sm_head_decode_splits(int rows, int H, int G) {
+// Slices of the key range for that kernel: about 512 workgroups, more of them where three or four fit a compute unit: keys of up to 256, and
+// twice as many for groups below 8, which had less to do and more to wait for.  (40 rows of 1000 with 8 key heads 59 µs whole, 47 in two slices, 42
+// in three; but 256 of 100 with 2 key heads and groups of 8 12.7 whole, 18.5 in two.)
+int sm_head_decode_splits(int rows, int H, int G, int Dk) {
   const int per = H / G;
   const int wgs = std::max(rows * G * ((per + 15) / 16), 1);
-  return std::max(1, std::min(SPLITS, 512 / wgs));
+  const int slices = per < 8 && Dk <= 128 ? 1024 / wgs : (512 + (Dk <= 256 ? wgs - 1 : 0)) / wgs;
+  return std::max(1, std::min(SPLITS, slices));
 }
 
 // rows of the state one wave keeps: D is cut into parts so that a wave's per-token loop is short and more waves share the work

@@ -295,7 +295,7 @@ void sm_token_attention(Tensor out, const Tensor& q1, const c10::optional<Tensor
                                  part.defined() ? part.data_ptr<float>() : nullptr, gp, g_ts, opt_f32(sink, "sink", H), opt, cur_stream(q1));
 }
 
-// Decode rows (the first `rows` tokens) of a mixer whose heads share key / value heads in groups of 8 or more, heads as the
+// Decode rows (the first `rows` tokens) of a mixer whose heads share key / value heads in groups of 4 or more, heads as the
 // MFMA columns; bf16 only.  False: shapes that kernel does not take — nothing was launched.
 bool sm_head_decode_attention(Tensor out, const Tensor& q1, const c10::optional<Tensor>& q2, const Tensor& k_cache,
                               const c10::optional<Tensor>& v_cache, const Tensor& block_tables, const Tensor& positions,
@@ -336,7 +336,7 @@ bool sm_head_decode_attention(Tensor out, const Tensor& q1, const c10::optional<
   if (lam.has_value()) TORCH_CHECK(!gate.has_value() && !sink.has_value() && Dv <= 512, "two maps: plain softmaxes, values up to 512");
   int64_t g_ts = 0;
   const void* gp = head_gate(gate, q1, T, H, &g_ts);
-  const int nsplit = dli::sm_head_decode_splits((int)rows, (int)H, (int)G);
+  const int nsplit = dli::sm_head_decode_splits((int)rows, (int)H, (int)G, (int)Dk);
   Tensor part;
   if (nsplit > 1 || lam.has_value()) part = at::empty({std::max<int64_t>(rows, 1), H, nsplit, Dv + 2}, q1.options().dtype(at::kFloat));
   return dli::launch_sm_head_decode_attention(out.data_ptr(), out.stride(0), out.stride(1), q1.data_ptr(), q1.stride(0), q1.stride(1),

@@ -35,7 +35,8 @@ def _exact(q, k, v, tables, lens, G, scale, window, cap):
 
 @pytest.mark.parametrize("lens", [[1], [31, 32, 33, 65], [700], [257] * 70])
 @pytest.mark.parametrize("H,G,Dk,Dv,shared", [(8, 1, 24, 16, False), (16, 2, 128, 128, False), (20, 1, 72, 80, False), (32, 1, 576, 512, True),
-                                              (8, 1, 320, 512, False), (24, 2, 192, 64, True), (6, 2, 20, 33, False)])
+                                              (8, 1, 320, 512, False), (24, 2, 192, 64, True), (6, 2, 20, 33, False),
+                                              (32, 8, 128, 128, False), (14, 2, 200, 176, False), (10, 2, 8, 16, False), (4, 1, 96, 96, True)])
 def test_decode_rows(H, G, Dk, Dv, shared, lens):
     g = torch.Generator().manual_seed(H * Dk + len(lens))
     tables, pages = _rows(lens, Dk)
@@ -58,3 +59,29 @@ def test_decode_rows(H, G, Dk, Dv, shared, lens):
             bound = float(v.abs().max()) * 2.0 ** -15 + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
             assert ((got - want).abs() <= bound).all(), (window, cap, dtype, (got - want).abs().max())
             assert not got[-1].any()
+
+
+@pytest.mark.parametrize("options", ["window penalties", "chunk sink", "gate kept"])
+@pytest.mark.parametrize("H,G,D,rows", [(4, 1, 24, 1), (12, 2, 128, 70), (20, 4, 208, 3)])
+def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch):
+    """Groups of 4 to 7 heads on the matrix cores against the kernel that takes a lane per key, whose weights are fp32 values."""
+    g = torch.Generator().manual_seed(H + D)
+    lens = [(37 * i) % 300 + 1 for i in range(rows)]
+    tables, pages = _rows(lens, D)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
+    q, k, v = rand(rows, H, 2 * D)[..., D:], rand(pages, PAGE, G * D), rand(pages, PAGE, G * D)      # (queries with gaps between them)
+    pos = lambda: torch.rand(H, generator=g).cuda()
+    kw = {"window penalties": dict(window=50, temp=pos() + 0.5, r1=pos(), r2=pos()), "chunk sink": dict(chunk=64, sink=pos()),
+          "gate kept": dict(window=33, keep_first=40, gate=rand(rows, 3 * H)[:, H:2 * H], out_scale=1.5)}[options]
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    meta = AttnMetadata(num_decode=rows, num_prefill=0, num_tokens=rows, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * rows),
+                        block_tables=tables.cuda(), seq_lens=ints(lens), query_start_loc=ints(range(rows + 1)), token_seq=ints(range(rows)))
+    got = []
+    for on in (True, False):
+        monkeypatch.setattr(seqmix, "HEAD_DECODE", on)
+        out = torch.empty(H, rows, D, dtype=torch.bfloat16, device="cuda").transpose(0, 1)
+        seqmix.token_attention(out, q, None, k, v, meta, G, D, D ** -0.5, **kw)
+        got.append(out.float())
+    # each result is rounded to bf16 from fp32 sums that differ by some 2^-20 of the largest value: one step apart at most
+    assert ((got[0] - got[1]).abs() <= 2.0 ** -7 * got[1].abs() + 2.0 ** -18 * float(v.abs().max()) * 1.5).all()
+    assert (got[0] != got[1]).float().mean() < 0.02
