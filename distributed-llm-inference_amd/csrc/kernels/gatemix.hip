@@ -880,7 +880,7 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
 // The walk of the delta rule: per (sequence, head, 16·CT state columns) over its blocks in order, the state on the accumulators.  A block is
 //   [o | x] = [Q̃ | W] S, u = U0 - x → LDS → o += A u, S = e^{P_end} ⊙ S + K̃ᵀ u → LDS,
 // two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 75 µs (36 of them fp32 matrix instructions, were they spread
-// evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83.  The next block's tiles are fetched as soon as
+// evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83 (79 now that its loads are asked for at once).  The next block's tiles are fetched as soon as
 // their registers are free and without a condition (the last block fetches itself again), so they land during the products; the compiler
 // still waits for all of them at the end of a block, where some change registers.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
 // below that of the walk before (2.7e-7 against 2.9e-7 of its norm).
