@@ -1335,6 +1335,23 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
   for (int s = 0; s < KSMAX; ++s) asm volatile("" : "+v"(qf[s]));
   for (int it = it_begin; it <= it_end; ++it) {
     const int kb = it < kb_lo ? it - it_lo : it;
+    // A value meets every weight of its page on the matrix cores, a masked key's 0 too, and 0 · inf is NaN: what lies in slots that the row does not see
+    // goes to LDS as zeros.  (A piece's row is the thread's: NT is a multiple of 8.)
+    if (32 * kb + 31 > p || (32 * kb < lo && 32 * kb + 31 >= opt.keep)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = 32 * kb + 4 * ((int)threadIdx.x & 7) + r;
+        if (j <= p && (j >= lo || j < opt.keep)) continue;
+        const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        if constexpr (VK) {
+#pragma unroll
+          for (int u = 0; u < NK; ++u) kr[u][r] = zero;
+        } else {
+#pragma unroll
+          for (int u = 0; u < NV; ++u) vr[u][r] = zero;
+        }
+      }
+    }
     lds_barrier();                                        // everyone is done with the page before
 #pragma unroll
     for (int u = 0; u < NK; ++u) {

@@ -6,6 +6,7 @@ from dli_amd.ops import AttnMetadata, seqmix
 
 pytestmark = pytest.mark.gpu
 PAGE = 32
+_INF = float("inf")
 
 
 def _rows(lens, seed):
@@ -85,3 +86,32 @@ def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch
     # each result is rounded to bf16 from fp32 sums that differ by some 2^-20 of the largest value: one step apart at most
     assert ((got[0] - got[1]).abs() <= 2.0 ** -7 * got[1].abs() + 2.0 ** -18 * float(v.abs().max()) * 1.5).all()
     assert (got[0] != got[1]).float().mean() < 0.02
+
+
+@pytest.mark.parametrize("options", [dict(), dict(window=40), dict(chunk=48), dict(window=40, keep_first=37)])
+@pytest.mark.parametrize("H,G,Dk,Dv,shared", [(8, 2, 128, 128, False), (14, 2, 200, 176, False), (5, 1, 96, 96, True), (8, 1, 64, 64, False),
+                                              (32, 1, 576, 512, True), (8, 1, 320, 512, False), (4, 2, 64, 64, False)])
+def test_slots_that_a_row_does_not_see(H, G, Dk, Dv, shared, options):
+    """Infinities and NaN past a row's position, before its window or chunk, and in its pages' other slots change nothing."""
+    g = torch.Generator().manual_seed(Dk + H)
+    lens = [1, 31, 33, 64, 100, 257]
+    tables, pages = _rows(lens, Dk)
+    T = len(lens)
+    q = torch.randn(T, H, Dk, generator=g).bfloat16().cuda()
+    k = torch.randn(pages, PAGE, G, Dk, generator=g).bfloat16()
+    v = k[..., :Dv] if shared else torch.randn(pages, PAGE, G, Dv, generator=g).bfloat16()
+    seen = torch.zeros(pages, PAGE, dtype=torch.bool)
+    for i, x in enumerate(lens):
+        p = x - 1
+        low = max(0, p - options["window"] + 1) if "window" in options else p - p % options["chunk"] if "chunk" in options else 0
+        for j in [*range(min(options.get("keep_first", 0), low)), *range(low, x)]:
+            seen[tables[i, j // PAGE], j % PAGE] = True
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    meta = AttnMetadata(num_decode=T, num_prefill=0, num_tokens=T, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * T),
+                        block_tables=tables[:T].cuda(), seq_lens=ints(lens), query_start_loc=ints(range(T + 1)), token_seq=ints(range(T)))
+    out = []
+    for other in (0.0, _INF, -_INF, float("nan")):
+        k2, v2 = (torch.where(seen[..., None, None], x, torch.full_like(x, other)).cuda() for x in (k, v))
+        out.append(torch.empty(T, H, Dv, dtype=torch.bfloat16, device="cuda"))
+        seqmix.token_attention(out[-1], q, None, k2.view(pages, PAGE, -1), None if shared else v2.view(pages, PAGE, -1), meta, G, Dv, Dk ** -0.5, **options)
+    assert bool(torch.isfinite(out[0].float()).all()) and all(torch.equal(o, out[0]) for o in out[1:])
