@@ -1233,7 +1233,7 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 // asked for, whole, while the one before it is computed, and goes from registers to both of its places (VK: values that lead the key row
 // are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed → now:
 // 1 row of 200 24.5 → 14.3, of 2000 58.7 → 24.6, 32 of 1500 64.7 → 42, 256 of 2000 504 → 258.
-// FINE: the weights enter P·V in three bf16 parts instead of two.
+// FINE: the weights enter P·V in three bf16 parts, 24 bits, instead of two.
 template <int KSMAX, int MTQ, bool VK, bool FINE>
 __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
@@ -1414,16 +1414,24 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     m = mn;
     bf16x8 ph, plo, pl2;
     float ps = 0.f;
+    // FINE: a weight's three parts are its upper, middle and lower 8 bits as they are, 24 in all.  None is below 2^-100: a visible infinity times a part
+    // that is 0, or negative after rounding, would make NaN of the infinity that it is with fp32 weights.
+    auto upper = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+    constexpr float least = 0x1p-100f;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const float pv = fast_exp2(sv[r] - mu);
       ps += pv;
-      const uint16_t hi = f2bf(pv);
-      ph[r] = (short)hi;
-      const float rest = pv - bf2f(hi);
-      const uint16_t lo = f2bf(rest);
-      plo[r] = (short)lo;
-      if constexpr (FINE) pl2[r] = (short)f2bf(rest - bf2f(lo));
+      if constexpr (FINE) {
+        const float lo = fmaxf(pv - upper(pv), least), lo2 = fmaxf(lo - upper(lo), least);
+        ph[r] = (short)(__float_as_uint(pv) >> 16);
+        plo[r] = (short)(__float_as_uint(lo) >> 16);
+        pl2[r] = (short)(__float_as_uint(lo2) >> 16);
+      } else {
+        const uint16_t hi = f2bf(pv);
+        ph[r] = (short)hi;
+        plo[r] = (short)f2bf(pv - bf2f(hi));
+      }
     }
     l = l * corr + ps;
 #pragma unroll

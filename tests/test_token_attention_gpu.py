@@ -115,3 +115,29 @@ def test_slots_that_a_row_does_not_see(H, G, Dk, Dv, shared, options):
         out.append(torch.empty(T, H, Dv, dtype=torch.bfloat16, device="cuda"))
         seqmix.token_attention(out[-1], q, None, k2.view(pages, PAGE, -1), None if shared else v2.view(pages, PAGE, -1), meta, G, Dv, Dk ** -0.5, **options)
     assert bool(torch.isfinite(out[0].float()).all()) and all(torch.equal(o, out[0]) for o in out[1:])
+
+
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (14, 2, 208), (5, 1, 96)])
+def test_infinite_values_that_small_groups_see(H, G, D, monkeypatch):
+    """An infinite value is infinite in every head that sees it, as with the weights in fp32, and only there."""
+    g = torch.Generator().manual_seed(D)
+    lens = [1, 20, 33, 200]
+    tables, pages = _rows(lens, D)
+    T = len(lens)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v = rand(T, H, D).cuda(), rand(pages, PAGE, G * D).cuda(), rand(pages, PAGE, G * D)
+    finite = v.clone()
+    for i, x in enumerate(lens):                               # the last token of a row and its first: columns 3 and 16
+        v[tables[i, (x - 1) // PAGE], (x - 1) % PAGE, 3::D] = _INF
+        v[tables[i, 0], 0, 16::D] = -_INF
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    meta = AttnMetadata(num_decode=T, num_prefill=0, num_tokens=T, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * T),
+                        block_tables=tables[:T].cuda(), seq_lens=ints(lens), query_start_loc=ints(range(T + 1)), token_seq=ints(range(T)))
+    def run(values, on):
+        monkeypatch.setattr(seqmix, "HEAD_DECODE", on)
+        out = torch.empty(T, H, D, dtype=torch.bfloat16, device="cuda")
+        return seqmix.token_attention(out, q, None, k, values.cuda(), meta, G, D, D ** -0.5).float()
+    want = run(finite, True)
+    want[..., 3], want[..., 16] = _INF, -_INF
+    assert torch.equal(run(v, True), want)
+    assert torch.equal(run(v, False).isinf(), want.isinf())    # (a lane per key)
