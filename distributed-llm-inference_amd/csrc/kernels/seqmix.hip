@@ -36,6 +36,13 @@ template <> __device__ __forceinline__ float silu_act<uint16_t>(float x) {
   return x * fast_rcp(1.f + fast_exp2(-1.4426950408889634f * x));
 }
 
+// log2(1 + x) with the digits that 1 + x drops from a small x: to first order, what u lacks over u.  (x finite, so that nothing is subtracted from infinity)
+__device__ __forceinline__ float log2_1p(float x) {
+  x = fminf(x, 0x1p126f);
+  const float u = 1.f + x;
+  return __builtin_fmaf((x - (u - 1.f)) * fast_rcp(u), 1.4426950408889634f, __builtin_amdgcn_logf(u));
+}
+
 // 4 consecutive row elements ↔ fp32 (16-byte / 8-byte accesses; the callers check divisibility and alignment)
 template <typename A> __device__ __forceinline__ f32x4 ld4(const A* p);
 template <> __device__ __forceinline__ f32x4 ld4<float>(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
@@ -789,8 +796,9 @@ __global__ __launch_bounds__(NT) void token_attention_kernel(
 
 // Combine the nsplit (≤ 16) partial results of a (token, head): part [T][H][nsplit][2 + Dv] = (max, sum, unnormalised output).  Bound by the loads'
 // latency, so all of them are asked for at once, from places that exist: a split's numbers by a lane each, its first outputs by all.
+// LOG2: the maxima are exponents of 2 (turned into natural ones their rounding alone would be 2^-24 of a maximum of 16).
 constexpr int SPLITS = 16;
-template <typename A>
+template <typename A, bool LOG2 = false>
 __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restrict__ out, int64_t o_ts, int64_t o_hs,
                                                                     const float* __restrict__ part,
                                                                     const int* __restrict__ token_seq, int H, int Dv,
@@ -814,7 +822,7 @@ __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restric
     return;
   }
   const float M = wave_max(mz);                           // (lanes past the last split repeat it)
-  const float fz = mz == -INFINITY ? 0.f : expf(mz - M);
+  const float fz = mz == -INFINITY ? 0.f : (LOG2 ? fast_exp2(mz - M) : expf(mz - M));
   float f[SPLITS], L = 0.f;
 #pragma unroll
   for (int z = 0; z < SPLITS; ++z) {
@@ -822,7 +830,7 @@ __global__ __launch_bounds__(128) void token_attention_merge_kernel(A* __restric
     const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lz), z));
     if (z < nsplit) L += f[z] * l;
   }
-  if (sink != nullptr) L += expf(sink[h] - M);
+  if (sink != nullptr) L += LOG2 ? fast_exp2(__builtin_fmaf(sink[h], 1.4426950408889634f, -M)) : expf(sink[h] - M);
   const float rl = (gate != nullptr ? 1.f / (1.f + expf(-gv)) : 1.f) / L * opt.out_scale;
   for (int e = threadIdx.x; e < Dv; e += 128) {
     if (e != (int)threadIdx.x) fetch(e);
@@ -1233,9 +1241,11 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 // asked for, whole, while the one before it is computed, and goes from registers to both of its places (VK: values that lead the key row
 // are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed → now:
 // 1 row of 200 24.5 → 14.3, of 2000 58.7 → 24.6, 32 of 1500 64.7 → 42, 256 of 2000 504 → 258.
-// FINE: the weights enter P·V in three bf16 parts, 24 bits, instead of two.
+// FINE (groups of 4 to 7, which were fp32 work before): the weights enter P·V in three bf16 parts, 24 bits, instead of two; scores, penalties and exponents keep
+// fp32's digits.  Sums before their rounding to bf16, of 64 bits: 0.71 … 0.93 of the lane kernel's error (some 3e-7), up to 1.23 of its 9e-8 under
+// penalties that leave a handful of keys; without that care 0.87 … 1.31.  It takes no time: masks are asked for on the pages that have any.
 template <int KSMAX, int MTQ, bool VK, bool FINE>
-__global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
+__global__ __launch_bounds__(NT, KSMAX <= 4 ? 4 : 2) void head_decode_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
     const uint16_t* __restrict__ q2, int64_t q2_ts, int64_t q2_hs, int D2, const uint16_t* __restrict__ kc, int rowk,
     const uint16_t* __restrict__ vc, int rowv, int vhead, int Dv, const int* __restrict__ block_tables, int max_blocks,
@@ -1281,6 +1291,12 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
   const bool capped = opt.cap > 0.f;
   const float capl = opt.cap * 1.4426950408889634f;
   const float qmul = scale * (temp != nullptr ? temp[h] : 1.f) * 1.4426950408889634f * (capped ? 2.f / opt.cap : 1.f);
+  // FINE: the factor's rounding is the same in every score, and scores of some 20 would carry it into their weights: what it leaves out
+  float qlo = 0.f;
+  if constexpr (FINE) {
+    const float st = scale * (temp != nullptr ? temp[h] : 1.f), st_lo = temp != nullptr ? __builtin_fmaf(scale, temp[h], -st) : 0.f;
+    qlo = __builtin_fmaf(st, 1.4426950408889634f, -qmul) + __builtin_fmaf(st, 1.9259629911266175e-8f, st_lo * 1.4426950408889634f);
+  }
   const float r1h = r1 != nullptr ? r1[h] : 0.f, r2h = r1 != nullptr ? r2[h] : 0.f;
   const bool pen = r1 != nullptr;
   const int p = positions[t];
@@ -1337,7 +1353,8 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     const int kb = it < kb_lo ? it - it_lo : it;
     // A value meets every weight of its page on the matrix cores, a masked key's 0 too, and 0 · inf is NaN: what lies in slots that the row does not see
     // goes to LDS as zeros.  (A piece's row is the thread's: NT is a multiple of 8.)
-    if (32 * kb + 31 > p || (32 * kb < lo && 32 * kb + 31 >= opt.keep)) {
+    const bool edge = 32 * kb + 31 > p || (32 * kb < lo && 32 * kb + 31 >= opt.keep);
+    if (edge) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = 32 * kb + 4 * ((int)threadIdx.x & 7) + r;
@@ -1384,27 +1401,55 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
       next = page_of(min(it + 2, it_end));
     }
     lds_barrier();
-    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f}, sa2 = sa, sb2 = sb;
 #pragma unroll
     for (int s = 0; s < KSMAX; ++s) {
       if (s < KS) {
         const bf16x8 ka = *reinterpret_cast<const bf16x8*>(Ks + c * KST + 32 * s + 8 * g4);
         const bf16x8 kb2 = *reinterpret_cast<const bf16x8*>(Ks + (16 + c) * KST + 32 * s + 8 * g4);
-        sa = mfma16(ka, qf[s], sa);
-        sb = mfma16(kb2, qf[s], sb);
+        f32x4 &ua = FINE && s & 1 ? sa2 : sa, &ub = FINE && s & 1 ? sb2 : sb;      // (two shorter sums round less)
+        ua = mfma16(ka, qf[s], ua);
+        ub = mfma16(kb2, qf[s], ub);
       }
+    }
+    if constexpr (FINE) {
+      sa += sa2;
+      sb += sb2;
     }
     float sv[8];
     float mx = -INFINITY;
+    const float ahead = (float)(p - 32 * kb - 4 * g4);    // FINE: the distance of the lane's first key
+    auto key = [](int r) { return r < 4 ? r : 12 + r; };
+    auto seen = [&](int r) {
+      const int j = 32 * kb + 4 * g4 + key(r);
+      return j <= p && (j >= lo || j < opt.keep);
+    };
+    float w[8];                                           // FINE: scores, then weights; the products and sv, log2(1 + r2 · distance), are kept between the two
+    if constexpr (FINE) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int j = 32 * kb + (r < 4 ? 4 * g4 + r : 16 + 4 * g4 + (r - 4));
-      float v = (r < 4 ? sa[r] : sb[r - 4]) * qmul;
-      if (pen) v -= r1h * __builtin_amdgcn_logf(1.f + r2h * (float)max(p - j, 0));
-      if (capped) v = capl - 2.f * capl * fast_rcp(fast_exp2(v) + 1.f);
-      v = (j <= p && (j >= lo || j < opt.keep)) ? v : -INFINITY;
-      sv[r] = v;
-      mx = fmaxf(mx, v);
+      for (int r = 0; r < 8; ++r) w[r] = (r < 4 ? sa[r] : sb[r - 4]) * qmul;
+      if (pen) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          sv[r] = log2_1p(r2h * (ahead - (float)key(r)));
+          w[r] -= r1h * sv[r];
+        }
+      }
+      if (edge)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) w[r] = seen(r) ? w[r] : -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) mx = fmaxf(mx, w[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        float v = (r < 4 ? sa[r] : sb[r - 4]) * qmul;
+        if (pen) v -= r1h * __builtin_amdgcn_logf(1.f + r2h * (float)max(p - (32 * kb + 4 * g4 + key(r)), 0));
+        if (capped) v = capl - 2.f * capl * fast_rcp(fast_exp2(v) + 1.f);
+        v = seen(r) ? v : -INFINITY;
+        sv[r] = v;
+        mx = fmaxf(mx, v);
+      }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -1418,9 +1463,21 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
     // that is 0, or negative after rounding, would make NaN of the infinity that it is with fp32 weights.
     auto upper = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
     constexpr float least = 0x1p-100f;
+    if constexpr (FINE) {                                 // exponents from the products again: rounded where they are small, not where the scores are large
+#pragma unroll
+      for (int r = 0; r < 8; ++r) w[r] = __builtin_fmaf(r < 4 ? sa[r] : sb[r - 4], qlo, -mu);
+      if (pen)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) w[r] = __builtin_fmaf(-r1h, sv[r], w[r]);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) w[r] = fast_exp2(__builtin_fmaf(r < 4 ? sa[r] : sb[r - 4], qmul, w[r]));
+      if (edge)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) w[r] = seen(r) ? w[r] : 0.f;
+    }
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const float pv = fast_exp2(sv[r] - mu);
+      const float pv = FINE ? w[r] : fast_exp2(sv[r] - mu);
       ps += pv;
       if constexpr (FINE) {
         const float lo = fmaxf(pv - upper(pv), least), lo2 = fmaxf(lo - upper(lo), least);
@@ -1466,10 +1523,10 @@ __global__ __launch_bounds__(NT, 2) void head_decode_attention_kernel(
       }
     }
   } else {
-    // the merge kernel works with natural exponentials: hand it the maximum in that domain
+    // FINE: the maximum as it is; otherwise for natural exponentials, which the merge of two maps and that of the lane kernel's parts take
     float* pr = part + ((t * H + h) * nsplit + blockIdx.z) * (int64_t)(Dv + 2);
     if (wave == 0 && g4 == 0) {
-      pr[0] = m * 0.6931471805599453f;
+      pr[0] = FINE ? m : m * 0.6931471805599453f;
       pr[1] = l;
     }
 #pragma unroll
@@ -1910,6 +1967,9 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
   if (opt.lam != nullptr)
     hipLaunchKernelGGL(map_merge_kernel<uint16_t>, dim3(rows, H / 2), dim3(128), 0, stream, (uint16_t*)out, o_ts, o_hs, (const float*)part,
                        token_seq, per, Dv, nsplit, opt);
+  else if (nsplit > 1 && fine)
+    hipLaunchKernelGGL((token_attention_merge_kernel<uint16_t, true>), dim3(rows, H), dim3(128), 0, stream, (uint16_t*)out, o_ts, o_hs,
+                       (const float*)part, token_seq, H, Dv, nsplit, (const uint16_t*)gate, g_ts, sink, opt);
   else if (nsplit > 1)
     hipLaunchKernelGGL(token_attention_merge_kernel<uint16_t>, dim3(rows, H), dim3(128), 0, stream, (uint16_t*)out, o_ts, o_hs,
                        (const float*)part, token_seq, H, Dv, nsplit, (const uint16_t*)gate, g_ts, sink, opt);

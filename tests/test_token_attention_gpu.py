@@ -62,7 +62,7 @@ def test_decode_rows(H, G, Dk, Dv, shared, lens):
             assert not got[-1].any()
 
 
-@pytest.mark.parametrize("options", ["window penalties", "chunk sink", "gate kept"])
+@pytest.mark.parametrize("options", ["window penalties", "steep penalties", "chunk sink", "gate kept"])
 @pytest.mark.parametrize("H,G,D,rows", [(4, 1, 24, 1), (12, 2, 128, 70), (20, 4, 208, 3)])
 def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch):
     """Groups of 4 to 7 heads on the matrix cores against the kernel that takes a lane per key, whose weights are fp32 values."""
@@ -72,7 +72,8 @@ def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch
     rand = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
     q, k, v = rand(rows, H, 2 * D)[..., D:], rand(pages, PAGE, G * D), rand(pages, PAGE, G * D)      # (queries with gaps between them)
     pos = lambda: torch.rand(H, generator=g).cuda()
-    kw = {"window penalties": dict(window=50, temp=pos() + 0.5, r1=pos(), r2=pos()), "chunk sink": dict(chunk=64, sink=pos()),
+    kw = {"window penalties": dict(window=50, temp=pos() + 0.5, r1=pos(), r2=pos()), "steep penalties": dict(r1=1e6 * (pos() + 0.5), r2=1e-6 * (pos() + 0.5)),   # (1 + r2 · distance has lost them)
+          "chunk sink": dict(chunk=64, sink=pos()),
           "gate kept": dict(window=33, keep_first=40, gate=rand(rows, 3 * H)[:, H:2 * H], out_scale=1.5)}[options]
     ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
     meta = AttnMetadata(num_decode=rows, num_prefill=0, num_tokens=rows, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * rows),
