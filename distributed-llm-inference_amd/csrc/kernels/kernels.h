@@ -129,7 +129,7 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
                                      const int* token_seq, int rows, int H, int G, float scale, int window, const float* temp,
                                      const float* r1, const float* r2, int nsplit, float* part, const void* gate, int64_t g_ts, const float* sink,
                                      AttnOpts opt, hipStream_t stream);
-int sm_head_decode_splits(int rows, int H, int G, int Dk);
+int sm_head_decode_splits(int rows, int H, int G, int Dk, int pages);
 bool launch_sm_tile_attention(void* out, int64_t o_ts, int64_t o_hs, const void* q1, int64_t q1_ts, int64_t q1_hs, int D1,
                               const void* q2, int64_t q2_ts, int64_t q2_hs, int D2, const void* kc, int rowk, const void* vc,
                               int rowv, int vhead, int Dv, const int* block_tables, int max_blocks, const int* seq_lens,

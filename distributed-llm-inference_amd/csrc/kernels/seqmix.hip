@@ -1976,14 +1976,22 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
   return true;
 }
 
-// Slices of the key range for that kernel: about 512 workgroups, more of them where three or four fit a compute unit: keys of up to 256, and
-// twice as many for groups below 8, which had less to do and more to wait for.  (40 rows of 1000 with 8 key heads 59 µs whole, 47 in two slices, 42
-// in three; but 256 of 100 with 2 key heads and groups of 8 12.7 whole, 18.5 in two.)
-int sm_head_decode_splits(int rows, int H, int G, int Dk) {
+// Slices of the key range for that kernel, of rows with `pages` at most as far as the host knows: never more than pages, one page alone stays whole
+// (1 row of 33 tokens, 32 heads on 8, µs, 7.5 in 16 slices, 6.4 whole; latent, 1 of 200 13.6 in 16, 13.1 in 7).
+// Up to 256 workgroups (1 row of 2000 whole 47, in 16 slices 10; latent 217 → 24): 512 of them, 1024 for groups below 8 and keys of up to 128.
+// Past 256 a cut pays where rows are long and several workgroups fit a compute unit.  Whole / cut, keys of up to 128, 280 and 340 workgroups in three
+// slices: 100 tokens 10.4 / 13.0, 200 15.9 / 16.9, 300 21.3 / 20.0, 1000 55 / 37, 2000 104 / 64; 420 and 500 in two: 100 10.9 / 16.5, 400 27.5 / 28.7,
+// 700 39.9 / 38.6, 2000 107 / 101.  Keys of 256 in two, 280: 300 28.2 / 30.2, 700 53 / 49, 2000 144 / 133; 340: 500 41 / 43, 1000 76 / 72; 420 of 1000 80 / 99.
+// Where the length is not known, rows of up to 384 workgroups are cut, for a loss of 2 to 3 µs if they turn out short.  (Slices of at least 8
+// pages, the rest of them empty, lose more: 14.8 for 100 tokens in place of 13.0.)
+int sm_head_decode_splits(int rows, int H, int G, int Dk, int pages) {
   const int per = H / G;
   const int wgs = std::max(rows * G * ((per + 15) / 16), 1);
-  const int slices = per < 8 && Dk <= 128 ? 1024 / wgs : (512 + (Dk <= 256 ? wgs - 1 : 0)) / wgs;
-  return std::max(1, std::min(SPLITS, slices));
+  int slices = (512 + (Dk <= 256 ? wgs - 1 : 0)) / wgs;
+  if (wgs > 256 && Dk <= 128) slices = wgs < 512 && pages > (wgs <= 384 ? 8 : 16) ? 1024 / wgs : 1;
+  else if (wgs > 256) slices = Dk <= 256 && wgs <= 340 && pages > 20 ? 2 : 1;
+  else if (per < 8 && Dk <= 128) slices = 1024 / wgs;
+  return std::max(1, std::min(std::min(SPLITS, pages), slices));
 }
 
 // rows of the state one wave keeps: D is cut into parts so that a wave's per-token loop is short and more waves share the work

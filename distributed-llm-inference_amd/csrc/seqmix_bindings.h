@@ -296,12 +296,12 @@ void sm_token_attention(Tensor out, const Tensor& q1, const c10::optional<Tensor
 }
 
 // Decode rows (the first `rows` tokens) of a mixer whose heads share key / value heads in groups of 4 or more, heads as the
-// MFMA columns; bf16 only.  False: shapes that kernel does not take — nothing was launched.
+// MFMA columns; bf16 only.  `longest`: the longest context (0: not known).  False: shapes that kernel does not take — nothing was launched.
 bool sm_head_decode_attention(Tensor out, const Tensor& q1, const c10::optional<Tensor>& q2, const Tensor& k_cache,
                               const c10::optional<Tensor>& v_cache, const Tensor& block_tables, const Tensor& positions,
                               const Tensor& token_seq, int64_t G, int64_t Dv, double scale, int64_t window,
                               const c10::optional<Tensor>& temp, const c10::optional<Tensor>& r1, const c10::optional<Tensor>& r2,
-                              int64_t rows, const c10::optional<Tensor>& gate, const c10::optional<Tensor>& sink, int64_t chunk, int64_t keep, double cap,
+                              int64_t rows, int64_t longest, const c10::optional<Tensor>& gate, const c10::optional<Tensor>& sink, int64_t chunk, int64_t keep, double cap,
                         int64_t Gv, double out_scale, const c10::optional<Tensor>& lam, double eps) {
   TORCH_CHECK(q1.is_cuda() && q1.scalar_type() == at::kBFloat16 && q1.dim() == 3 && q1.stride(2) == 1, "q1 must be bfloat16 [T, H, D1]");
   const int64_t T = q1.size(0), H = q1.size(1), D1 = q1.size(2);
@@ -336,7 +336,12 @@ bool sm_head_decode_attention(Tensor out, const Tensor& q1, const c10::optional<
   if (lam.has_value()) TORCH_CHECK(!gate.has_value() && !sink.has_value() && Dv <= 512, "two maps: plain softmaxes, values up to 512");
   int64_t g_ts = 0;
   const void* gp = head_gate(gate, q1, T, H, &g_ts);
-  const int nsplit = dli::sm_head_decode_splits((int)rows, (int)H, (int)G, (int)Dk);
+  // Pages of a row's range at most: those of the longest context, where the caller knows it, of a window or a chunk.  A captured step knows none, and its table
+  // is as wide as any context may be: 16 pages, for which rows are cut where long ones gain most (sm_head_decode_splits).
+  int64_t pages = std::min(block_tables.size(1), longest > 0 ? (longest + kSmPageTokens - 1) / kSmPageTokens : (int64_t)16);
+  if (window > 0) pages = std::min(pages, (window + 2 * kSmPageTokens - 2) / kSmPageTokens + (keep + kSmPageTokens - 1) / kSmPageTokens);
+  if (chunk > 0) pages = std::min(pages, (chunk + 2 * kSmPageTokens - 2) / kSmPageTokens);
+  const int nsplit = dli::sm_head_decode_splits((int)rows, (int)H, (int)G, (int)Dk, (int)pages);
   Tensor part;
   if (nsplit > 1 || lam.has_value()) part = at::empty({std::max<int64_t>(rows, 1), H, nsplit, Dv + 2}, q1.options().dtype(at::kFloat));
   return dli::launch_sm_head_decode_attention(out.data_ptr(), out.stride(0), out.stride(1), q1.data_ptr(), q1.stride(0), q1.stride(1),

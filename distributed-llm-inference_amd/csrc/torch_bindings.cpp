@@ -697,10 +697,12 @@ TORCH_LIBRARY(dli, m) {
         "Tensor? lam=None, float eps=0.0) -> ()",
         &sm_token_attention);
   m.def("sm_head_decode_attention(Tensor(a!) out, Tensor q1, Tensor? q2, Tensor k_cache, Tensor? v_cache, Tensor block_tables, "
-        "Tensor positions, Tensor token_seq, int G, int Dv, float scale, int window, Tensor? temp, Tensor? r1, Tensor? r2, int rows, "
+        "Tensor positions, Tensor token_seq, int G, int Dv, float scale, int window, Tensor? temp, Tensor? r1, Tensor? r2, int rows, int longest, "
         "Tensor? gate, Tensor? sink, int chunk, int keep, float cap, int Gv, float out_scale, "
         "Tensor? lam=None, float eps=0.0) -> bool",
         &sm_head_decode_attention);
+  m.def("sm_head_decode_splits(int rows, int H, int G, int Dk, int pages) -> int",
+        [](int64_t r, int64_t h, int64_t g, int64_t d, int64_t p) -> int64_t { return dli::sm_head_decode_splits((int)r, (int)h, (int)g, (int)d, (int)p); });
   m.def("sm_tile_attention(Tensor(a!) out, Tensor q1, Tensor? q2, Tensor k_cache, Tensor? v_cache, Tensor block_tables, Tensor seq_lens, "
         "Tensor qsl, Tensor tile_seq, Tensor tile_q0, int num_tiles, Tensor? counts, int G, int Dv, float scale, int window, "
         "Tensor? temp, Tensor? r1, Tensor? r2, Tensor? gate, Tensor? sink, int chunk, int keep, float cap, int Gv, float out_scale, "

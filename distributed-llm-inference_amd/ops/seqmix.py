@@ -215,9 +215,10 @@ def _attend_rows(lib, out, q1, q2, k_cache, v_cache, meta, rows, args, opts) -> 
     """The first ``rows`` tokens (< 0: all of them, no tile kernel ran) on the kernels that take one token per workgroup."""
     T, H = q1.shape[0], q1.shape[1]
     todo = T if rows < 0 else rows                           # tokens the tile kernel left (all of them in a pure decode step)
+    longest = 0 if getattr(meta, "counts_on_device", False) else getattr(meta, "max_seq_len", 0)       # (a captured launch has bounds only)
     if (HEAD_DECODE and todo > 0 and q1.dtype == torch.bfloat16 and H // args[0] >= 4 and (rows >= 0 or meta.num_prefill_tiles == 0)
             and lib.sm_head_decode_attention(out, q1, q2, k_cache, v_cache, meta.block_tables, meta.positions, meta.token_seq, *args, todo,
-                                             *opts)):
+                                             longest, *opts)):
         rows = 0                                             # done with the heads as matrix-core columns
     if rows != 0:
         lib.sm_token_attention(out, q1, q2, k_cache, v_cache, meta.block_tables, meta.positions, meta.token_seq, *args, rows, *opts)

@@ -187,3 +187,15 @@ def test_mixed_attention_takes_a_second_stream_where_it_pays():
                                           (96, 1490, 37, 2, 32, 8, 2), (60, 1490, 43, 2, 64, 8, 2), (400, 0, 94, 3, 32, 8, 2)))
     assert not any(beside(*size) for size in ((2, 400, 2, 1, 32, 8, 1), (96, 1490, 37, 2, 32, 8, 1), (200, 1500, 66, 3, 32, 8, 1),
                                               (64, 1318, 65, 3, 32, 8, 2), (64, 994, 76, 4, 32, 8, 2), (200, 999, 51, 4, 64, 8, 1), (400, 1500, 47, 1, 32, 8, 2), (400, 1500, 94, 1, 8, 1, 2), (1, 0, 2, 1, 32, 8, 2)))
+
+
+def test_slices_of_decode_rows_by_length():
+    """Sizes timed whole and cut: (rows, heads, key heads, key width, pages) and the slices that were no slower than another number."""
+    slices = lambda *size: ops.hip().sm_head_decode_splits(*size)
+    # short rows of 257 … 511 workgroups stay whole whatever the group, and any that has a page alone
+    assert [slices(r, h, g, 128, 4) for r, h, g in ((250, 16, 2), (256, 16, 2), (300, 8, 1), (511, 8, 1), (50, 64, 8), (63, 32, 8), (500, 16, 2))] == [1] * 7
+    assert [slices(*s) for s in ((250, 16, 2, 128, 13), (250, 32, 2, 256, 64), (120, 16, 4, 256, 64), (128, 32, 8, 128, 64), (1, 32, 8, 128, 1))] == [1] * 5
+    # long ones are cut
+    assert [slices(*s) for s in ((140, 16, 2, 128, 16), (300, 8, 1, 128, 32), (40, 32, 8, 128, 32), (250, 16, 2, 128, 32), (511, 8, 1, 128, 63), (140, 32, 2, 256, 32))] == [3, 3, 3, 2, 2, 2]
+    # no more slices than pages
+    assert [slices(1, 32, 1, 576, p) for p in (7, 13, 63)] == [7, 13, 16] and slices(8, 32, 8, 128, 22) == 16
