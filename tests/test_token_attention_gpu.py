@@ -63,11 +63,11 @@ def test_decode_rows(H, G, Dk, Dv, shared, lens):
 
 
 @pytest.mark.parametrize("options", ["window penalties", "steep penalties", "chunk sink", "gate kept"])
-@pytest.mark.parametrize("H,G,D,rows", [(4, 1, 24, 1), (12, 2, 128, 70), (20, 4, 208, 3)])
+@pytest.mark.parametrize("H,G,D,rows", [(4, 1, 48, 1), (4, 1, 16, 1), (12, 2, 128, 70), (20, 4, 208, 3)])
 def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch):
     """Groups of 4 to 7 heads on the matrix cores against the kernel that takes a lane per key, whose weights are fp32 values."""
     g = torch.Generator().manual_seed(H + D)
-    lens = [(37 * i) % 300 + 1 for i in range(rows)]
+    lens = [(37 * i + 260) % 300 + 1 for i in range(rows)]     # (one row: several pages, most slices empty)
     tables, pages = _rows(lens, D)
     rand = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
     q, k, v = rand(rows, H, 2 * D)[..., D:], rand(pages, PAGE, G * D), rand(pages, PAGE, G * D)      # (queries with gaps between them)
@@ -78,12 +78,18 @@ def test_small_groups_as_a_lane_per_key_does(H, G, D, rows, options, monkeypatch
     ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
     meta = AttnMetadata(num_decode=rows, num_prefill=0, num_tokens=rows, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * rows),
                         block_tables=tables.cuda(), seq_lens=ints(lens), query_start_loc=ints(range(rows + 1)), token_seq=ints(range(rows)))
-    got = []
+    got, taken, lib = [], [], seqmix._hip()
+    class Watched:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            return (lambda *a: taken.append(f(*a)) or taken[-1]) if name == "sm_head_decode_attention" else f
+    monkeypatch.setattr(seqmix, "_hip", Watched)
     for on in (True, False):
         monkeypatch.setattr(seqmix, "HEAD_DECODE", on)
         out = torch.empty(H, rows, D, dtype=torch.bfloat16, device="cuda").transpose(0, 1)
         seqmix.token_attention(out, q, None, k, v, meta, G, D, D ** -0.5, **kw)
         got.append(out.float())
+    assert taken == [True]                                     # the matrix cores took the first call
     # each result is rounded to bf16 from fp32 sums that differ by some 2^-20 of the largest value: one step apart at most
     assert ((got[0] - got[1]).abs() <= 2.0 ** -7 * got[1].abs() + 2.0 ** -18 * float(v.abs().max()) * 1.5).all()
     assert (got[0] != got[1]).float().mean() < 0.02
