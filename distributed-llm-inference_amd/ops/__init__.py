@@ -131,7 +131,8 @@ def decode_chunk_pages(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int =
     ranges costs 3 µs, a range's pages come at what one compute unit reads (a page of eight waves' first round 0.2 µs), and the more
     workgroups there are the less a cut spreads.  Whole against cut, 32/8 and 64/8 heads, both page types: one row of 8 pages 0.79–0.84,
     of 12 0.85–0.91, of 16 0.95–1.05, of 20 1.0–1.06; 16 rows of 16 pages 0.89–0.95, of 25 1.0–1.07; 32 of 25 0.83–0.97, of 50 0.9–1.09;
-    60 of 31 0.88–0.94.  ``cap_items``:
+    60 of 31 0.88–0.94.  One key head (``profiles/decode_rows_whole_or_cut.txt``), 8 heads: one row of 12 pages 0.79–0.87, of 20 0.97–1.03; 64 of 15
+    0.95–1.01; 250 of 24 0.83–0.85; 4 and 16 heads the same but for 64 rows of 15 (1.05–1.07 and, 16 heads in bf16, 1.14).  ``cap_items``:
     ranges are doubled until the list fits (the fixed grid of a hipGraph)."""
     pages = (np.asarray(seq_lens, dtype=np.int64) + 31) >> 5
     n, maxp = len(pages), max(int(pages.max()) if len(pages) else 1, 1)
