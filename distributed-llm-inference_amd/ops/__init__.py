@@ -538,8 +538,9 @@ def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page
     prompt workgroups a unit leave room.  µs, beside / one after the other, 32/8 heads: 2 rows of up to 400 tokens and a prompt of 40 42.4 / 19.9; e4m3
     96 of up to 1500 and two chunks of 1024 behind 1024 86.5 / 83.0 (bf16, one group, 0.59 GB 111 / 116), 400 of up to 1500 and three of 1000 behind 500 165.6 / 188.8, with 200 of up to 1000 124 / 109; bf16 64 rows of up to 1000 and three of
     1000 behind 500 105 / 94, 200 140 / 150; two groups, 160 of up to 2000 and one of 800 behind 300 159 / 165, 300 of up to 1500 and one of 200 behind
-    500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97.  Captured: 0.65 to 0.95 of the
-    time one after the other for a prompt of 40 tokens, 0.87 to 1.04 for 4 × 300, 1.0 to 1.39 for longer ones, so branches there."""
+    500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97.  Captured
+    steps, with the launch extents that the runner captures (``profiles/mixed_steps_captured.txt``, 88 sizes): branches take 0.95 of the time one after the
+    other on average, 0.74 to 1.12 but for 256 tokens of four fresh prompts (1.07 to 1.24), so all of them have branches."""
     longest = meta.max_seq_len or 1024                       # (0: not known)
     room = page_element_bytes == 2 and meta.num_prefill_tiles * num_kv_heads <= 512
     if meta.num_decode * longest * num_kv_heads * 256 * page_element_bytes < (350_000_000 if room else 700_000_000):
