@@ -45,7 +45,22 @@ __device__ __forceinline__ uint4 philox4x32_10(uint4 ctr, uint2 key) {
   return ctr;
 }
 __device__ __forceinline__ float u01(uint32_t r) { return ((r >> 8) + 0.5f) * (1.0f / 16777216.0f); }   // (0,1)
-__device__ __forceinline__ float gumbel(float u) { return -__logf(-__logf(u)); }
+// Logarithm of a normal number whose logarithm is finite.  It gives the bits of __logf, which also scales subnormal numbers and lets infinities by: 6
+// instructions, not 14.  ln 2 in two floats, and the order of the products, are those that this compiler emits for __logf (read from this file's
+// assembly): y·hi + (y·lo + what y·hi lost), the first product unrounded as well, so that its rounding counts twice there and here.  -log(-log(u)) of all
+// 2^24 numbers that u01 gives has the same bits either way.
+__device__ __forceinline__ float log_normal(float x) {
+  const float hi = __uint_as_float(0x3F317217u), lo = __uint_as_float(0x3377D1CFu), y = __builtin_amdgcn_logf(x);
+  return __builtin_fmaf(y, hi, __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -(y * hi))));
+}
+// Gumbel noise of 32 random bits, for every kernel here: paths that pick the same token need the same bits.  u01 gives 2^-25 … 1, so -log(u) is 0 or at
+// least 2^-24.
+__device__ __forceinline__ float gumbel_of(uint32_t r) {
+  const float t = -log_normal(u01(r));
+  return t == 0.f ? __builtin_inff() : -log_normal(t);
+}
+// of a caller's number, which may be any
+__device__ __forceinline__ float gumbel_at(float u) { return -__logf(-__logf(u)); }
 
 struct ArgMax {
   float v;
@@ -193,8 +208,7 @@ __global__ __launch_bounds__(SNT) void sample_kernel(const T* __restrict__ logit
       if (i < V) {
         const float z = ld<T>(row, i) * inv_t_log2;
         if (okey(z) >= floor_key) {
-          const float u = noise != nullptr ? noise[(int64_t)b * V + i] : u01(rr[e]);
-          a = amax(a, ArgMax{z * ln2 + gumbel(u), i});
+          a = amax(a, ArgMax{z * ln2 + (noise != nullptr ? gumbel_at(noise[(int64_t)b * V + i]) : gumbel_of(rr[e])), i});
         }
       }
     }
@@ -558,16 +572,6 @@ __device__ __forceinline__ void greedy_chunk(const uint4& x, int chunk, ArgMax& 
 #pragma unroll
   for (int e = 0; e < 8; ++e) take(a, bf2f((uint16_t)half_of(x, e)), chunk * 8 + e);
 }
-// __logf of a normal number with a finite logarithm, the same bits in six instructions (__logf also scales subnormal numbers and lets infinities by: 14)
-__device__ __forceinline__ float log_normal(float x) {
-  const float hi = __uint_as_float(0x3F317217u), lo = __uint_as_float(0x3377D1CFu), y = __builtin_amdgcn_logf(x);
-  return __builtin_fmaf(y, hi, __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -(y * hi))));
-}
-// gumbel(u01(r)): u01 gives 2^-25 … 1, so -log(u) is 0 or at least 2^-24
-__device__ __forceinline__ float gumbel_of(uint32_t r) {
-  const float t = -log_normal(u01(r));
-  return t == 0.f ? __builtin_inff() : -log_normal(t);
-}
 // Groups of four logits, a Philox block each.  CUT: only what reaches floor_key draws.
 template <bool CUT>
 __device__ __forceinline__ void draw_chunk(const uint4& x, int chunk, float inv_t_log2, uint32_t floor_key, uint2 key, uint64_t step,
@@ -592,8 +596,7 @@ __device__ __forceinline__ void draw_chunk(const uint4& x, int chunk, float inv_
       if (!CUT) {
         take(a, z + gumbel_of(rr[e]), i4 * 4 + e);
       } else if (okey16(h) >= floor_key) {
-        const float u = noise_row != nullptr ? noise_row[i4 * 4 + e] : u01(rr[e]);
-        take(a, z + gumbel(u), i4 * 4 + e);
+        take(a, z + (noise_row != nullptr ? gumbel_at(noise_row[i4 * 4 + e]) : gumbel_of(rr[e])), i4 * 4 + e);
       }
     }
   }

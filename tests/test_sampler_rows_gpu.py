@@ -67,7 +67,7 @@ def test_cut_off_rows(v):
 # rows that every logit draws in: one launch, slices of one and of four chunks a thread; −0, masks and equal logits among them
 @pytest.mark.parametrize("b,v", [(3, 8), (5, 8192), (7, 8200), (40, 131072), (520, 32776)])
 def test_plain_draws_are_the_row_kernels(b, v):
-    """The draw of rows without cut-off takes its logarithms in fewer instructions; the fp32 rows' kernel takes ``__logf``: same ids."""
+    """Rows without cut-off draw in a loop of their own, without keys; the fp32 rows' kernel draws each logit that passes its cut-off: same ids."""
     g = torch.Generator().manual_seed(v)
     x = (torch.randn(b, v, generator=g) * torch.tensor([0.0, 0.5, 4.0])[torch.arange(b) % 3, None]).bfloat16()
     x[1, ::2], x[2, v // 2:] = -0.0, -_INF
