@@ -148,3 +148,23 @@ def test_infinite_values_that_small_groups_see(H, G, D, monkeypatch):
     want[..., 3], want[..., 16] = _INF, -_INF
     assert torch.equal(run(v, True), want)
     assert torch.equal(run(v, False).isinf(), want.isinf())    # (a lane per key)
+
+
+@pytest.mark.parametrize("H,G,D", [(16, 2, 128), (8, 2, 128), (8, 1, 320)])
+def test_slices_chosen_for_another_length(H, G, D):
+    """The host's longest context chooses slices only: a step captured for short rows and replayed with longer ones is right too."""
+    g = torch.Generator().manual_seed(D)
+    lens = [40 + 13 * i for i in range(70)]
+    tables, pages = _rows(lens, D)
+    T = len(lens)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v = rand(T, H, D), rand(pages * PAGE, G, D), rand(pages * PAGE, G, D)
+    want = _exact(q, k, v, tables, lens, G, D ** -0.5, 0, 0.0)[:T]
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    bound = float(v.abs().max()) * 2.0 ** -15 + 2.0 ** -8 * want.abs()     # as in test_decode_rows
+    for longest in (0, 1, 300, max(lens)):
+        meta = AttnMetadata(num_decode=T, num_prefill=0, num_tokens=T, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * T), max_seq_len=longest,
+                            block_tables=tables[:T].cuda(), seq_lens=ints(lens), query_start_loc=ints(range(T + 1)), token_seq=ints(range(T)))
+        out = torch.empty(T, H, D, dtype=torch.bfloat16, device="cuda")
+        seqmix.token_attention(out, q.cuda(), None, k.cuda().view(pages, PAGE, -1), v.cuda().view(pages, PAGE, -1), meta, G, D, D ** -0.5)
+        assert ((out.double().cpu() - want).abs() <= bound).all(), longest
