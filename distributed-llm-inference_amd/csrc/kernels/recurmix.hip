@@ -216,8 +216,8 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(const A* __restrict__ x
 // Four taps, RUN tokens of a step and 4 · NT channels per workgroup: a thread keeps its channels' four weights and the last three inputs in
 // registers, so a token costs its own row read and its result written instead of four rows of weights and four of inputs.  A sequence
 // that begins inside a run takes its inputs from its chunk or its state rows.  Vectors lie in d / 4 neighbouring lanes.  4096 channels, 3162
-// rows, state rows included: 39.2 → 20.0 µs (3.9 TB/s of the input and the result; bound by them and by how few workgroups a short step has;
-// runs of 8 tokens 23.8, of 16 41.1).
+// rows, state rows included: 39.2 → 20 to 22 µs (3.5 to 3.9 TB/s of the input and the result; bound by them and by how few workgroups a short step has;
+// beside 21.9 with runs of 4, runs of 8 tokens take 21.1, of 16 45.0).
 constexpr int RUN = 4;
 template <typename A, typename O>
 __global__ __launch_bounds__(NT) void causal_conv_run_kernel(const A* __restrict__ x, int64_t x_stride, const float* __restrict__ w,

@@ -1239,11 +1239,12 @@ __global__ __launch_bounds__(NT * HW, KSMAX <= 4 ? 4 : (KSMAX <= 8 ? 2 : 1)) voi
 // the key range leave (max, sum, unnormalised output) in `part` for token_attention_merge_kernel.
 // Few rows are bound by the chain through a slice's pages, many by the LDS (every wave reads all of a page's keys).  A page is therefore
 // asked for, whole, while the one before it is computed, and goes from registers to both of its places (VK: values that lead the key row
-// are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed → now:
-// 1 row of 200 24.5 → 14.3, of 2000 58.7 → 24.6, 32 of 1500 64.7 → 42, 256 of 2000 504 → 258.
+// are not read again).  Rows of 576 / 512 shared by 32 heads, merge included, µs, pages fetched piece by piece when needed (and the merge of that time) → now:
+// 1 row of 200 23.5 → 13.2, of 2000 57.8 → 24.3, 32 of 1500 63.9 → 42.3, 256 of 2000 509 → 261.
 // FINE (groups of 4 to 7, which were fp32 work before): the weights enter P·V in three bf16 parts, 24 bits, instead of two; scores, penalties and exponents keep
 // fp32's digits.  Sums before their rounding to bf16, of 64 bits: 0.71 … 0.93 of the lane kernel's error (some 3e-7), up to 1.23 of its 9e-8 under
-// penalties that leave a handful of keys; without that care 0.87 … 1.31.  It takes no time: masks are asked for on the pages that have any.
+// penalties that leave a handful of keys; without that care 0.87 … 1.31.  One row of 200 with penalties takes 7.9 µs so, 7.5 without the care; 128 of 1500 the
+// same 115, since masks are asked for only on the pages that have any.
 template <int KSMAX, int MTQ, bool VK, bool FINE>
 __global__ __launch_bounds__(NT, KSMAX <= 4 ? 4 : 2) void head_decode_attention_kernel(
     uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const uint16_t* __restrict__ q1, int64_t q1_ts, int64_t q1_hs, int D1,
@@ -1924,10 +1925,11 @@ bool launch_sm_head_decode_attention(void* out, int64_t o_ts, int64_t o_hs, cons
                                      AttnOpts opt, hipStream_t stream) {
   const int Dk = D1 + D2, KS = (Dk + 31) / 32, MT = Dv / 16, per = H / G;
   auto al = [](const void* p, int64_t a) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % a == 0; };
-  // Groups of 4 … 7 heads leave columns idle, and still beat a lane per key (token_attention_kernel) by far: 32 heads on 8 of 128, in a graph, µs:
-  // 1 row of 200 16.7 → 8.1, 8 of 700 21.6 → 13.4, 128 of 1500 129 → 103, 256 of 2000 241 → 195.  (Groups of 2: 8 of 300 11.8 → 10.0, but 256 of
-  // 100 with heads of 64 22.3 → 27.3.)  That kernel's weights are fp32 values, so these take them in three bf16 parts, 24 bits; what shows
-  // more than the rounding of a bf16 result (fp32 results, the difference of two maps) and a soft cap's logistic form stay there.
+  // Groups of 4 … 7 heads leave columns idle, and still beat a lane per key (token_attention_kernel) by far: 32 heads on 8 of 128, window with penalties, in
+  // a graph, µs, that kernel with the present merge / this one: 1 row of 200 16.2 / 7.9, 8 of 700 20.2 / 12.9, 128 of 1500 140 / 112, 256 of 2000 254 / 212.
+  // (Groups of 2: 8 of 300 11.8 / 10.0, but 256 of 100 with heads of 64 22.3 / 27.3.)  That kernel's weights are fp32 values, so these take them in three
+  // bf16 parts, 24 bits, and what goes into their exponents with fp32's digits; fp32 results, the difference of two maps and a soft cap's logistic form
+  // stay there.
   const bool fine = per < 8;
   const bool ok = (!fine || (per >= 4 && KS <= 8 && MT <= 16 && opt.out_f32 == nullptr && opt.cap == 0.f && opt.lam == nullptr)) && D1 % 8 == 0 && D2 % 8 == 0 && Dv % 16 == 0 && KS <= 18 && MT <= 32 && rowk % 8 == 0 && rowv % 8 == 0 &&
                   vhead % 8 == 0 && q1_ts % 8 == 0 && q1_hs % 8 == 0 && q2_ts % 8 == 0 && q2_hs % 8 == 0 && o_ts % 4 == 0 &&

@@ -129,9 +129,10 @@ def decode_chunk_pages(seq_lens: np.ndarray, num_kv_heads: int, cap_items: int =
     row.  Smaller batches cut the longest row into as many ranges as it takes to reach that fill (whole multiples of 4
     pages: one per wave and iteration of an e4m3 workgroup's four; of a bf16 workgroup's eight half may have none, which costs nothing) — each row by its own length, a short row stays one range.  Short rows stay whole in any batch: the launch that adds up
     ranges costs 3 µs, a range's pages come at what one compute unit reads (a page of eight waves' first round 0.2 µs), and the more
-    workgroups there are the less a cut spreads.  Whole against cut, 32/8 and 64/8 heads, both page types: one row of 8 pages 0.79–0.84,
+    workgroups there are the less a cut spreads.  Whole against cut (``profiles/decode_rows_whole_or_cut.txt``),
+    32/8 and 64/8 heads, both page types: one row of 8 pages 0.79–0.84,
     of 12 0.85–0.91, of 16 0.95–1.05, of 20 1.0–1.06; 16 rows of 16 pages 0.89–0.95, of 25 1.0–1.07; 32 of 25 0.83–0.97, of 50 0.9–1.09;
-    60 of 31 0.88–0.94.  One key head (``profiles/decode_rows_whole_or_cut.txt``), 8 heads: one row of 12 pages 0.79–0.87, of 20 0.97–1.03; 64 of 15
+    60 of 31 0.88–0.94.  8 of 15 0.98–1.07.  One key head, 8 heads: one row of 12 pages 0.79–0.87, of 20 0.97–1.03; 64 of 15
     0.95–1.01; 250 of 24 0.83–0.85; 4 and 16 heads the same but for 64 rows of 15 (1.05–1.07 and, 16 heads in bf16, 1.14).  ``cap_items``:
     ranges are doubled until the list fits (the fixed grid of a hipGraph)."""
     pages = (np.asarray(seq_lens, dtype=np.int64) + 31) >> 5
@@ -538,7 +539,8 @@ def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page
     prompt workgroups a unit leave room.  µs, beside / one after the other, 32/8 heads: 2 rows of up to 400 tokens and a prompt of 40 42.4 / 19.9; e4m3
     96 of up to 1500 and two chunks of 1024 behind 1024 86.5 / 83.0 (bf16, one group, 0.59 GB 111 / 116), 400 of up to 1500 and three of 1000 behind 500 165.6 / 188.8, with 200 of up to 1000 124 / 109; bf16 64 rows of up to 1000 and three of
     1000 behind 500 105 / 94, 200 140 / 150; two groups, 160 of up to 2000 and one of 800 behind 300 159 / 165, 300 of up to 1500 and one of 200 behind
-    500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97.  Captured
+    500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97, but for 400 rows
+    of up to 1500 with one prompt of 1500 in bf16, 81.9 after and 74.1 beside (more sizes: ``profiles/mixed_steps_eager.txt``).  Captured
     steps, with the launch extents that the runner captures (``profiles/mixed_steps_captured.txt``, 88 sizes): branches take 0.95 of the time one after the
     other on average, 0.74 to 1.12 but for 256 tokens of four fresh prompts (1.07 to 1.24), so all of them have branches."""
     longest = meta.max_seq_len or 1024                       # (0: not known)
