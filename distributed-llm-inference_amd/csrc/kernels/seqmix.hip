@@ -36,11 +36,10 @@ template <> __device__ __forceinline__ float silu_act<uint16_t>(float x) {
   return x * fast_rcp(1.f + fast_exp2(-1.4426950408889634f * x));
 }
 
-// log2(1 + x) with the digits that 1 + x drops from a small x: to first order, what u lacks over u.  (x finite, so that nothing is subtracted from infinity)
+// log2(1 + x) with the digits that 1 + x drops from a small x: to first order, what u lacks over u.  (A large x drops none; infinity and NaN stay what they are.)
 __device__ __forceinline__ float log2_1p(float x) {
-  x = fminf(x, 0x1p126f);
-  const float u = 1.f + x;
-  return __builtin_fmaf((x - (u - 1.f)) * fast_rcp(u), 1.4426950408889634f, __builtin_amdgcn_logf(u));
+  const float u = 1.f + x, l = __builtin_amdgcn_logf(u);
+  return x < 0x1p24f ? __builtin_fmaf((x - (u - 1.f)) * fast_rcp(u), 1.4426950408889634f, l) : l;
 }
 
 // 4 consecutive row elements ↔ fp32 (16-byte / 8-byte accesses; the callers check divisibility and alignment)

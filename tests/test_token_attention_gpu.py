@@ -168,3 +168,26 @@ def test_slices_chosen_for_another_length(H, G, D):
         out = torch.empty(T, H, D, dtype=torch.bfloat16, device="cuda")
         seqmix.token_attention(out, q.cuda(), None, k.cuda().view(pages, PAGE, -1), v.cuda().view(pages, PAGE, -1), meta, G, D, D ** -0.5)
         assert ((out.double().cpu() - want).abs() <= bound).all(), longest
+
+
+def test_penalties_past_the_usual_range(monkeypatch):
+    """r2 · distance of 0 to 1e38, and an r2 that is NaN, which makes its head NaN: on the matrix cores as with a lane per key."""
+    g = torch.Generator().manual_seed(3)
+    H, G, D, lens = 8, 2, 64, [1, 40, 200]
+    tables, pages = _rows(lens, 5)
+    T = len(lens)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
+    q, k, v = rand(T, H, D), rand(pages, PAGE, G * D), rand(pages, PAGE, G * D)
+    r1 = torch.full((H,), 2.0, device="cuda")
+    r2 = torch.tensor([5e35, 1e30, 0.0, float("nan"), 1e-30, 1.0, 2.0 ** 24, 2.0 ** 17], device="cuda")
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    meta = AttnMetadata(num_decode=T, num_prefill=0, num_tokens=T, positions=ints([x - 1 for x in lens]), slot_mapping=ints([-1] * T),
+                        block_tables=tables[:T].cuda(), seq_lens=ints(lens), query_start_loc=ints(range(T + 1)), token_seq=ints(range(T)))
+    got = []
+    for on in (True, False):
+        monkeypatch.setattr(seqmix, "HEAD_DECODE", on)
+        out = torch.empty(T, H, D, dtype=torch.bfloat16, device="cuda")
+        got.append(seqmix.token_attention(out, q, None, k, v, meta, G, D, D ** -0.5, r1=r1, r2=r2).float())
+    assert torch.equal(got[0].isnan(), got[1].isnan()) and got[0][:, 3].isnan().all() and got[0][:, 4:].isfinite().all()
+    # one bf16 step, as in test_small_groups_as_a_lane_per_key_does
+    assert torch.allclose(got[0], got[1], rtol=2.0 ** -7, atol=2.0 ** -18 * float(v.abs().max()) * 1.5, equal_nan=True)
