@@ -170,37 +170,36 @@ __device__ __forceinline__ bf16x8 softmax_step(f32x4 (&s)[2], int tok0, int limi
 // Partial results: `part_o[(p·Hq + head)·128 + d]`, `part_ml[(p·Hq + head)·2 + {m, l}]` with p = slot (WL) or
 // seq·num_splits + split; decode_reduce_kernel combines them per sequence.
 // ==================================================================================================
-template <bool KV8, bool WL, int NW, bool NT = false>
-__global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
-    const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
-    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, uint16_t* __restrict__ out,
-    int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_splits,
-    float scale_log2, float v_scale, const float* __restrict__ kv_scales, const int4* __restrict__ work,
-    const int* __restrict__ counts) {
-  extern __shared__ __attribute__((aligned(16))) float smem[];
-  const int kvh = blockIdx.x;
+// item `item` of key head kvh (WL = false: sequence `item`, split `split`) by the NW waves whose threads are tid = 0 …; smem: decode_lds(NW, G) bytes of theirs.
+// All waves of the workgroup pass its one barrier (or have ended).
+template <bool KV8, bool WL, int NW, bool NT>
+__device__ __forceinline__ void decode_item(
+    int tid, int kvh, int item, int split, float* smem, const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache,
+    const void* __restrict__ v_cache, const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens,
+    uint16_t* __restrict__ out, int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_splits,
+    float scale_log2, float v_scale, const float* __restrict__ kv_scales, const int4* __restrict__ work, const int* __restrict__ counts) {
   int seq, b_begin, b_end, part;                           // part < 0: write `out` directly
   if constexpr (WL) {
-    if ((int)blockIdx.y >= counts[0]) return;
-    const int4 w = work[blockIdx.y];
+    if (item >= counts[0]) return;
+    const int4 w = work[item];
     seq = w.x, b_begin = w.y, b_end = w.z, part = w.w;
   } else {
-    seq = blockIdx.y;
-    part = num_splits == 1 ? -1 : seq * num_splits + (int)blockIdx.z;
+    seq = item;
+    part = num_splits == 1 ? -1 : seq * num_splits + split;
   }
   if (KV8 && kv_scales != nullptr) {                       // calibrated per-(layer, kv head) fp8 scales: [k | v][Hkv]
     scale_log2 *= kv_scales[kvh];
     v_scale = kv_scales[Hkv + kvh];
   }
   const int G = Hq / Hkv;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // scalar: page loop, block-table reads and page bases in SGPRs
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: page loop, block-table reads and page bases in SGPRs
   const int col = lane & 15, g = lane >> 4;
   const int L = seq_lens[seq];
   const int nblk = (L + 31) >> 5;
   if constexpr (!WL) {
     const int per = (nblk + num_splits - 1) / num_splits;
-    b_begin = (int)blockIdx.z * per;
+    b_begin = split * per;
     b_end = min(nblk, b_begin + per);
   } else {
     b_end = min(b_end, nblk);
@@ -274,7 +273,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     if (g == 0) { sm_m[wave * G + col] = m; sm_l[wave * G + col] = lsum; }
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < G * HD; idx += NW * 64) {
+  for (int idx = tid; idx < G * HD; idx += NW * 64) {
     const int head = idx >> 7, d = idx & 127;
     float M = NEG_BIG;
 #pragma unroll
@@ -296,6 +295,18 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
       if (d == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = den; }
     }
   }
+}
+
+template <bool KV8, bool WL, int NW, bool NT = false>
+__global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
+    const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, uint16_t* __restrict__ out,
+    int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_splits,
+    float scale_log2, float v_scale, const float* __restrict__ kv_scales, const int4* __restrict__ work,
+    const int* __restrict__ counts) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  decode_item<KV8, WL, NW, NT>(threadIdx.x, blockIdx.x, blockIdx.y, blockIdx.z, smem, q, q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, out,
+                               out_stride, part_o, part_ml, Hq, Hkv, num_splits, scale_log2, v_scale, kv_scales, work, counts);
 }
 
 // Combine the partials of one (sequence, query head): 128 threads, one per d.  Uniform splits: grid (num_seqs, Hq),
@@ -429,24 +440,26 @@ __device__ __forceinline__ void value_fragments(const char* vb, int n, int off0,
   }
 }
 
+template <bool KV8, int GROUPS, int NPG> struct PrefillShape {
+  static constexpr int PAGE_BYTES = PAGE_ELEMS * (KV8 ? 1 : 2);
+  static constexpr int STAGE = NPG * 2 * PAGE_BYTES;        // K and V of a turn's pages
+  static constexpr int NSTAGE = NPG == 1 ? 3 : 2;
+  static constexpr int RING = NSTAGE * STAGE;
+  static constexpr int SWAP = GROUPS == 2 ? 4 * 2 * 8192 : 0;      // what two groups exchange at the end
+  static constexpr int LDS = GROUPS * RING > SWAP ? GROUPS * RING : SWAP;
+};
+// workgroup `block` of a launch over num_tiles · Hkv tiles; smem_all: PrefillShape::LDS bytes
 template <bool KV8, int GROUPS, int NPG>
-__global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
-    const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+__device__ __forceinline__ void prefill_tile(
+    int block, char* smem_all, const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens,
     const int* __restrict__ query_start_loc, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     uint16_t* __restrict__ out, int64_t out_stride, int Hq, int Hkv, int num_tiles, float scale_log2, float v_scale,
-    const float* __restrict__ kv_scales, const int* __restrict__ counts, int units) {
-  // inside a hipGraph the grid is an upper bound and the step's tile count lives in device memory (counts[2])
-  if (counts != nullptr) num_tiles = counts[2];
-  constexpr int ESZ = KV8 ? 1 : 2;
-  constexpr int PAGE_BYTES = PAGE_ELEMS * ESZ;
+    const float* __restrict__ kv_scales, int units) {
+  using Shape = PrefillShape<KV8, GROUPS, NPG>;
+  constexpr int PAGE_BYTES = Shape::PAGE_BYTES, STAGE = Shape::STAGE, NSTAGE = Shape::NSTAGE, RING = Shape::RING;
   constexpr int NCH = PAGE_BYTES / (16 * 256);
-  constexpr int STAGE = NPG * 2 * PAGE_BYTES;               // K and V of a turn's pages
-  constexpr int NSTAGE = NPG == 1 ? 3 : 2;
   constexpr int FLIGHT = 2 * NCH;                           // (three stages) DMA instructions of a wave for a turn
-  constexpr int RING = NSTAGE * STAGE;
-  constexpr int SWAP = GROUPS == 2 ? 4 * 2 * 8192 : 0;      // what two groups exchange at the end
-  __shared__ __attribute__((aligned(16))) char smem_all[GROUPS * RING > SWAP ? GROUPS * RING : SWAP];
 
   // Block → (kv head, tile): the kv head is the fastest index.  Workgroups are dealt round-robin over the 8 XCDs (private L2s), so with 8
   // kv heads XCD x serves head x — a sequence's pages of that head are fetched into one L2 instead of eight —, with 2 or 4 every XCD
@@ -461,9 +474,9 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   // Two groups and more tiles than `units` workgroups: what is left over, the shortest tiles, goes to the second groups of the last workgroups, whose
   // two groups then do a tile each; the longest tiles keep both.
   const int items = num_tiles * Hkv, over = GROUPS == 2 ? max(items - units, 0) : 0;
-  if ((int)blockIdx.x >= items - over) return;
-  const bool alone = GROUPS == 2 && (int)blockIdx.x >= units - over;
-  const int id = (int)blockIdx.x + (alone ? grp * over : 0);
+  if (block >= items - over) return;
+  const bool alone = GROUPS == 2 && block >= units - over;
+  const int id = block + (alone ? grp * over : 0);
   const int kvh = id % Hkv, rank = id / Hkv;
   const int tile_id = num_tiles - 1 - rank;
   if (KV8 && kv_scales != nullptr) {
@@ -743,6 +756,68 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
   }
 }
 
+template <bool KV8, int GROUPS, int NPG>
+__global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
+    const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens,
+    const int* __restrict__ query_start_loc, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
+    uint16_t* __restrict__ out, int64_t out_stride, int Hq, int Hkv, int num_tiles, float scale_log2, float v_scale,
+    const float* __restrict__ kv_scales, const int* __restrict__ counts, int units) {
+  __shared__ __attribute__((aligned(16))) char smem[PrefillShape<KV8, GROUPS, NPG>::LDS];
+  // inside a hipGraph the grid is an upper bound and the step's tile count lives in device memory (counts[2])
+  if (counts != nullptr) num_tiles = counts[2];
+  prefill_tile<KV8, GROUPS, NPG>(blockIdx.x, smem, q, q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq,
+                                 tile_q0, out, out_stride, Hq, Hkv, num_tiles, scale_log2, v_scale, kv_scales, units);
+}
+
+// Mixed steps: decode rows and prompt tiles in one launch, workgroups of four waves each.  Prompt tiles are bound by their chain of pages and the vector
+// instructions, decode rows by the cache's bytes, so a compute unit that holds both does one while the other waits; one after the other, 96 e4m3 rows of
+// up to 1500 tokens and two chunks of up to 1024 behind up to 1024 (32/8 heads) take 67 µs, here 49, and in bf16 99 → 65.  (Two streams or two branches of a
+// graph reach part of it: their launches compete for the units as they come, a captured branch costs 5 µs where the step is small, an event on an eager
+// stream 10 and 30 to 55 of the host.  In 88 captured steps this launch takes 0.86 of the branches' time on average, 0.60 to 1.04.)
+// Three workgroups share a unit (145 registers, 48 KB of LDS).  Octets of workgroups, one for each XCD so that a head's pages stay in one L2:
+//   * `period` = 3: every third octet is one of decode rows, as long as there are both, then what is left.  For many tiles, which would fill all units and
+//     leave the decode rows for the end (96 bf16 rows, one fresh prompt of 3500 tokens, 880 tiles: prompts first 152 µs, every second 185, every third 138,
+//     every fourth 152; e4m3 rows, four of 1000 behind 500, 672 tiles 68 / 78 / 58 / 65);
+//   * 0: all prompts first, whose longest chain the launch has to wait for anyway, where they leave a third of the units' room (e4m3, 504 tiles: 85 / 115 /
+//     94 / 91; 200 tiles 50 / 47 / 49 / 48).
+// GROUPS = 2: tiles by two page groups and decode items by as many waves as in their own launch
+// (both give the same bits), a workgroup a compute unit.
+template <bool KV8, bool WL, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void paged_mixed_kernel(
+    const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ query_start_loc,
+    const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, uint16_t* __restrict__ out, int64_t out_stride,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_tiles, int items, int num_splits, float scale_log2, float v_scale,
+    const float* __restrict__ kv_scales, const int4* __restrict__ work, const int* __restrict__ counts, int tiles_on_device, int period) {
+  constexpr int NPG = GROUPS == 2 && KV8 ? 2 : 1, NW = GROUPS == 2 && !KV8 ? 8 : 4, IPW = 4 * GROUPS / NW;      // IPW: decode items a workgroup
+  __shared__ __attribute__((aligned(16))) char smem[PrefillShape<KV8, GROUPS, NPG>::LDS];      // (a decode item of up to 8 heads a group takes 17 KB of it, 34 by eight waves)
+  const int octets = (num_tiles * Hkv + 7) >> 3, rows = ((items + IPW - 1) / IPW * Hkv + 7) >> 3;
+  const int octet = (int)blockIdx.x >> 3, in = (int)blockIdx.x & 7;
+  const int turns = period > 1 ? min(rows, octets / (period - 1)) : 0;
+  int tile = octet - turns, row = -1;                       // behind the turns: the other tiles, then the other rows
+  if (octet < turns * period) {
+    const int turn = octet / period, at = octet - turn * period;
+    if (at == period - 1) row = turn;
+    else tile = octet - turn;
+  } else if (tile >= octets) {
+    row = octet - octets;
+  }
+  if (row < 0) {
+    if (tiles_on_device) num_tiles = counts[2];             // (the launched number is a bound)
+    prefill_tile<KV8, GROUPS, NPG>(8 * tile + in, smem, q, q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq,
+                                   tile_q0, out, out_stride, Hq, Hkv, num_tiles, scale_log2, v_scale, kv_scales, 0x7fffffff);
+    return;
+  }
+  const int sub = IPW == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  const int id = 8 * row + in, group = id / Hkv, kvh = id - group * Hkv, item = group * IPW + sub;
+  if (item >= items) return;                                // the last octet, the last item's neighbour
+  const int seq = WL ? item : item / num_splits, split = WL ? 0 : item - seq * num_splits;
+  decode_item<KV8, WL, NW, true>((int)threadIdx.x - 256 * sub, kvh, seq, split, reinterpret_cast<float*>(smem + sub * (int)(sizeof(smem) / 2)), q, q_stride,
+                                 k_cache, v_cache, block_tables, max_blocks, seq_lens, out, out_stride, part_o, part_ml, Hq, Hkv, num_splits,
+                                 scale_log2, v_scale, kv_scales, work, counts);
+}
+
 // ---- launchers -------------------------------------------------------------------------------------
 // Decode reads every K/V byte exactly once per step: the loads are NON-TEMPORAL (streaming cache policy), so the pages do not
 // displace what the GEMMs keep in L2 / the infinity cache and are themselves not written into them: 5.95 → 6.60 TB/s on the
@@ -855,6 +930,61 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
   if (kv_fp8) { if (groups == 2) DLI_PREFILL_GO(true, 2, 2); else DLI_PREFILL_GO(true, 1, 1); }
   else { if (groups == 2) DLI_PREFILL_GO(false, 2, 1); else DLI_PREFILL_GO(false, 1, 1); }
 #undef DLI_PREFILL_GO
+}
+
+// Page groups of a mixed step's tiles (paged_mixed_kernel), 0: launches of their own.  rows: decode rows; longest, sequences as in prefill_page_groups.
+// µs of the longest tile's chain with one and two groups as there (one group on e4m3 pages 4 more); decode rows by themselves take 5 µs and their pages' bytes
+// at 5.5 TB/s (half the longest context each), a unit without a tile reads at 2.2 of its share.  One launch of one group then takes its chain and 0.4 of
+// the rows' time, or what the rows take; one of two groups its chain, 0.15 of the rows' time, and what the units without a tile leave, or 1.15 of the rows' time.  Measured, after each other / one
+// group / two — 8/1 heads, 16 bf16 rows of up to 1500 and one of 2000 behind 500 (125 tiles) 66.5 / 74.4 / 61.2, e4m3 65.2 / 80.4 / 61.6, 400 bf16 rows 94.8 /
+// 86.8 / 67.5; 64/8 heads and one of 500 behind 1500 (256), bf16, 16 rows 71.8 / 68.9 / 61.5, 96 107.7 / 83.8 / 106.5; of 400 behind 500 (200), e4m3, 48 48.9 /
+// 40.1 / 38.4, 96 58.1 / 40.0 / 48.9.  Past 256 tiles, where their own launch has two groups, one launch pays if it hides
+// rows of some length: 32/8 heads, e4m3, two of up to 1024 behind
+// up to 1024 (296), 16 rows 49.4 / 50.0, 96 67.2 / 49.4.  (More: profiles/mixed_steps_one_launch.txt.)
+int mixed_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, int rows, bool kv_fp8) {
+  const int blocks = num_tiles * Hkv;
+  const bool two = prefill_page_groups(num_tiles, Hkv, G, longest, sequences, kv_fp8) != 1;
+  if (longest == 0) return two ? 2 : 1;                       // (up to 256 tiles: at most 1.05 of launches of their own)
+  const float one_us = 5.f + 0.0285f * longest + (kv_fp8 ? 4.f : 0.f);
+  const float two_us = longest > 224 ? 5.5f + 0.0225f * longest : one_us;      // short tiles are done by one group in either form
+  const float rows_us = 5.f + (float)rows * longest * Hkv * (kv_fp8 ? 128.f : 256.f) / 5.5e6f;
+  if (blocks > PREFILL_UNITS) return two && rows_us < one_us / 2.2f ? 0 : 1;
+  const float idle = (float)(PREFILL_UNITS - blocks) / PREFILL_UNITS;
+  const float with_two = std::max(two_us + 0.15f * rows_us + std::max(0.f, rows_us - 2.2f * idle * two_us), 1.15f * rows_us);
+  return with_two < std::max(one_us + 0.4f * rows_us, rows_us + 4.f) ? 2 : 1;
+}
+
+// Decode rows as launch_paged_decode_worklist (work != nullptr: `items`, `reds`) or as launch_paged_decode (`num_seqs`, `num_splits`) takes them, prompt
+// tiles as launch_paged_prefill does.
+void launch_paged_mixed(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache, const int* block_tables, int max_blocks,
+                        const int* seq_lens, const int* query_start_loc, const int* tile_seq, const int* tile_q0, int num_tiles, void* out,
+                        int64_t out_stride, float* part_o, float* part_ml, const int* work, const int* red, const int* counts, int items, int reds,
+                        int num_seqs, int num_splits, int Hq, int Hkv, float scale, bool kv_fp8, float k_scale, float v_scale, const float* kv_scales,
+                        bool tiles_on_device, int longest, int sequences, hipStream_t stream) {
+  const bool wl = work != nullptr;
+  if (!wl) items = num_seqs * num_splits;
+  int groups = std::max(1, mixed_page_groups(num_tiles, Hkv, Hq / Hkv, longest, sequences, num_seqs, kv_fp8));
+  if (groups == 2 && !kv_fp8 && decode_waves(false, Hq / Hkv, (int64_t)Hkv * items) != 8) groups = 1;
+  const int rows = groups == 2 && kv_fp8 ? (items + 1) / 2 : items;
+  const int64_t octets = ((int64_t)num_tiles * Hkv + 7) / 8 + ((int64_t)rows * Hkv + 7) / 8;
+  if (octets == 0) return;
+  if (kv_scales != nullptr) k_scale = v_scale = 1.f;
+  const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
+  const int period = (int64_t)num_tiles * Hkv > 2 * PREFILL_UNITS ? 3 : 0;
+#define DLI_MIXED_GO(KV8_, WL_, G_)                                                                                                      \
+  hipLaunchKernelGGL((paged_mixed_kernel<KV8_, WL_, G_>), dim3((unsigned)(8 * octets)), dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, \
+                     v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, part_o, part_ml, \
+                     Hq, Hkv, num_tiles, items, wl ? 1 : num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work,  \
+                     counts, tiles_on_device ? 1 : 0, period)
+#define DLI_MIXED_WL(KV8_, G_) do { if (wl) DLI_MIXED_GO(KV8_, true, G_); else DLI_MIXED_GO(KV8_, false, G_); } while (0)
+  if (groups == 2) { if (kv_fp8) DLI_MIXED_WL(true, 2); else DLI_MIXED_WL(false, 2); }
+  else { if (kv_fp8) DLI_MIXED_WL(true, 1); else DLI_MIXED_WL(false, 1); }
+#undef DLI_MIXED_WL
+#undef DLI_MIXED_GO
+  if (wl ? reds > 0 : num_splits > 1)
+    hipLaunchKernelGGL(decode_reduce_kernel, dim3(wl ? reds : num_seqs, Hq), dim3(128), 0, stream, part_o, part_ml, (uint16_t*)out,
+                       out_stride, Hq, wl ? 1 : num_splits, kv_fp8 ? v_scale : 1.f, kv_fp8 ? kv_scales : nullptr, Hkv,
+                       wl ? (const int4*)red : nullptr, wl ? counts : nullptr);
 }
 
 }  // namespace dli

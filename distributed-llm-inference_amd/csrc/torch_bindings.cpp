@@ -175,11 +175,12 @@ void copy_pages(Tensor cache, const Tensor& pairs) {
   dli::launch_copy_pages(cache.data_ptr(), pairs.data_ptr<int>(), (int)pairs.size(0), page_bytes, cur_stream(cache));
 }
 
-// q: [T, Hq*128] view (row stride arbitrary); the first num_seqs rows are the decode queries.
-void paged_attention_decode(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
-                            const Tensor& seq_lens, int64_t num_seqs, int64_t Hq, int64_t Hkv, double scale, int64_t num_splits,
-                            const c10::optional<Tensor>& workspace, double k_scale, double v_scale,
-                            const c10::optional<Tensor>& kv_scales) {
+struct DecodeParts {
+  float *o, *ml;
+};
+static DecodeParts check_decode(const Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                                const Tensor& seq_lens, int64_t num_seqs, int64_t Hq, int64_t Hkv, int64_t num_splits,
+                                const c10::optional<Tensor>& workspace) {
   check_bf16_rows(q, "q");
   check_bf16_rows(out, "out");
   check_i32(block_tables, "block_tables");
@@ -189,17 +190,22 @@ void paged_attention_decode(Tensor out, const Tensor& q, const Tensor& k_cache, 
   TORCH_CHECK(q.size(0) >= num_seqs && out.size(0) >= num_seqs && q.size(1) == Hq * 128 && out.size(1) == Hq * 128);
   TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= num_seqs && seq_lens.numel() >= num_seqs);
   TORCH_CHECK(num_splits >= 1 && num_splits <= 64);
-  float* part_o = nullptr;
-  float* part_ml = nullptr;
-  if (num_splits > 1) {
-    TORCH_CHECK(workspace.has_value() && workspace->is_cuda() && workspace->scalar_type() == at::kFloat && workspace->is_contiguous());
-    const int64_t need = num_seqs * Hq * num_splits * (128 + 2);
-    TORCH_CHECK(workspace->numel() >= need, "decode workspace too small: need ", need, " floats");
-    part_o = workspace->data_ptr<float>();
-    part_ml = part_o + num_seqs * Hq * num_splits * 128;
-  }
+  if (num_splits == 1) return {nullptr, nullptr};
+  TORCH_CHECK(workspace.has_value() && workspace->is_cuda() && workspace->scalar_type() == at::kFloat && workspace->is_contiguous());
+  const int64_t need = num_seqs * Hq * num_splits * (128 + 2);
+  TORCH_CHECK(workspace->numel() >= need, "decode workspace too small: need ", need, " floats");
+  float* part_o = workspace->data_ptr<float>();
+  return {part_o, part_o + num_seqs * Hq * num_splits * 128};
+}
+
+// q: [T, Hq*128] view (row stride arbitrary); the first num_seqs rows are the decode queries.
+void paged_attention_decode(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                            const Tensor& seq_lens, int64_t num_seqs, int64_t Hq, int64_t Hkv, double scale, int64_t num_splits,
+                            const c10::optional<Tensor>& workspace, double k_scale, double v_scale,
+                            const c10::optional<Tensor>& kv_scales) {
+  const DecodeParts parts = check_decode(out, q, k_cache, v_cache, block_tables, seq_lens, num_seqs, Hq, Hkv, num_splits, workspace);
   dli::launch_paged_decode(q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr<int>(),
-                           (int)block_tables.size(1), seq_lens.data_ptr<int>(), out.data_ptr(), out.stride(0), part_o, part_ml,
+                           (int)block_tables.size(1), seq_lens.data_ptr<int>(), out.data_ptr(), out.stride(0), parts.o, parts.ml,
                            (int)num_seqs, (int)Hq, (int)Hkv, (int)num_splits, (float)scale, is_fp8(k_cache), (float)k_scale,
                            (float)v_scale, scales_ptr(kv_scales, Hkv), cur_stream(q));
 }
@@ -207,11 +213,9 @@ void paged_attention_decode(Tensor out, const Tensor& q, const Tensor& k_cache, 
 // Work-list decode (ops.build_decode_work): `work` int32 [≥ items, 4] = {sequence, first page, end page, partial slot},
 // `red` int32 [≥ reds, 4] = {sequence, first partial, partials, 0}, `counts` int32 [≥ 4] ON THE DEVICE = {valid items,
 // valid reduce entries, prefill tiles, -}.  `items` / `reds` are the launched grid extents (≥ the valid counts).
-void paged_attention_decode_worklist(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
-                                     const Tensor& block_tables, const Tensor& seq_lens, const Tensor& work, const Tensor& red,
-                                     const Tensor& counts, int64_t items, int64_t reds, int64_t max_parts, int64_t Hq, int64_t Hkv,
-                                     double scale, const Tensor& workspace, double k_scale, double v_scale,
-                                     const c10::optional<Tensor>& kv_scales) {
+static DecodeParts check_decode_worklist(const Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                                         const Tensor& seq_lens, const Tensor& work, const Tensor& red, const Tensor& counts, int64_t items,
+                                         int64_t reds, int64_t max_parts, int64_t Hq, int64_t Hkv, const Tensor& workspace) {
   check_bf16_rows(q, "q");
   check_bf16_rows(out, "out");
   check_i32(block_tables, "block_tables");
@@ -228,19 +232,25 @@ void paged_attention_decode_worklist(Tensor out, const Tensor& q, const Tensor& 
   TORCH_CHECK(workspace.is_cuda() && workspace.scalar_type() == at::kFloat && workspace.is_contiguous());
   TORCH_CHECK(workspace.numel() >= max_parts * Hq * (128 + 2), "decode workspace too small for ", max_parts, " partials");
   float* part_o = workspace.data_ptr<float>();
-  float* part_ml = part_o + max_parts * Hq * 128;
+  return {part_o, part_o + max_parts * Hq * 128};
+}
+
+void paged_attention_decode_worklist(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
+                                     const Tensor& block_tables, const Tensor& seq_lens, const Tensor& work, const Tensor& red,
+                                     const Tensor& counts, int64_t items, int64_t reds, int64_t max_parts, int64_t Hq, int64_t Hkv,
+                                     double scale, const Tensor& workspace, double k_scale, double v_scale,
+                                     const c10::optional<Tensor>& kv_scales) {
+  const DecodeParts parts = check_decode_worklist(out, q, k_cache, v_cache, block_tables, seq_lens, work, red, counts, items, reds, max_parts, Hq, Hkv, workspace);
   dli::launch_paged_decode_worklist(q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr<int>(),
-                                    (int)block_tables.size(1), seq_lens.data_ptr<int>(), out.data_ptr(), out.stride(0), part_o,
-                                    part_ml, work.data_ptr<int>(), red.data_ptr<int>(), counts.data_ptr<int>(), (int)items,
+                                    (int)block_tables.size(1), seq_lens.data_ptr<int>(), out.data_ptr(), out.stride(0), parts.o,
+                                    parts.ml, work.data_ptr<int>(), red.data_ptr<int>(), counts.data_ptr<int>(), (int)items,
                                     (int)reds, (int)Hq, (int)Hkv, (float)scale, is_fp8(k_cache), (float)k_scale, (float)v_scale,
                                     scales_ptr(kv_scales, Hkv), cur_stream(q));
 }
 
-void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
-                             const Tensor& seq_lens, const Tensor& query_start_loc, const Tensor& tile_seq, const Tensor& tile_q0,
-                             int64_t num_tiles, int64_t Hq, int64_t Hkv, double scale, double k_scale, double v_scale,
-                             const c10::optional<Tensor>& kv_scales, const c10::optional<Tensor>& counts, int64_t longest,
-                             int64_t sequences) {
+static void check_prefill(const Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                          const Tensor& seq_lens, const Tensor& query_start_loc, const Tensor& tile_seq, const Tensor& tile_q0,
+                          int64_t num_tiles, int64_t Hq, int64_t Hkv) {
   check_bf16_rows(q, "q");
   check_bf16_rows(out, "out");
   check_i32(block_tables, "block_tables");
@@ -253,6 +263,14 @@ void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache,
   TORCH_CHECK(Hq % Hkv == 0 && (G == 1 || G == 2 || G == 4 || G == 8), "prefill kernel supports 1, 2, 4 or 8 query heads per KV head");
   TORCH_CHECK(q.size(1) == Hq * 128 && out.size(1) == Hq * 128 && out.size(0) == q.size(0));
   TORCH_CHECK(tile_seq.numel() >= num_tiles && tile_q0.numel() >= num_tiles && block_tables.dim() == 2);
+}
+
+void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                             const Tensor& seq_lens, const Tensor& query_start_loc, const Tensor& tile_seq, const Tensor& tile_q0,
+                             int64_t num_tiles, int64_t Hq, int64_t Hkv, double scale, double k_scale, double v_scale,
+                             const c10::optional<Tensor>& kv_scales, const c10::optional<Tensor>& counts, int64_t longest,
+                             int64_t sequences) {
+  check_prefill(out, q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, tile_seq, tile_q0, num_tiles, Hq, Hkv);
   const int* cnt = nullptr;                 // device-side tile count (counts[2]); num_tiles is then the grid's upper bound
   if (counts.has_value()) {
     check_i32(*counts, "counts");
@@ -264,6 +282,34 @@ void paged_attention_prefill(Tensor out, const Tensor& q, const Tensor& k_cache,
                             tile_seq.data_ptr<int>(), tile_q0.data_ptr<int>(), (int)num_tiles, out.data_ptr(), out.stride(0),
                             (int)Hq, (int)Hkv, (float)scale, is_fp8(k_cache), (float)k_scale, (float)v_scale,
                             scales_ptr(kv_scales, Hkv), cnt, (int)longest, (int)sequences, cur_stream(q));
+}
+
+// Decode rows and prompt tiles in one launch: `work`, `red` and what goes with them as for paged_attention_decode_worklist, or none of them and `num_seqs`,
+// `num_splits` as for paged_attention_decode (num_seqs: decode rows in
+// either form).  tiles_on_device: num_tiles is a bound, counts[2] the number.
+void paged_attention_mixed(Tensor out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                           const Tensor& seq_lens, const Tensor& query_start_loc, const Tensor& tile_seq, const Tensor& tile_q0, int64_t num_tiles,
+                           const c10::optional<Tensor>& work, const c10::optional<Tensor>& red, const c10::optional<Tensor>& counts, int64_t items,
+                           int64_t reds, int64_t max_parts, int64_t num_seqs, int64_t num_splits, int64_t Hq, int64_t Hkv, double scale,
+                           const c10::optional<Tensor>& workspace, double k_scale, double v_scale, const c10::optional<Tensor>& kv_scales,
+                           bool tiles_on_device, int64_t longest, int64_t sequences) {
+  const bool list = work.has_value();
+  TORCH_CHECK(list == red.has_value() && (!(list || tiles_on_device) || counts.has_value()) && (!list || workspace.has_value()));
+  const DecodeParts parts = list ? check_decode_worklist(out, q, k_cache, v_cache, block_tables, seq_lens, *work, *red, *counts, items, reds, max_parts, Hq, Hkv, *workspace)
+                                 : check_decode(out, q, k_cache, v_cache, block_tables, seq_lens, num_seqs, Hq, Hkv, num_splits, workspace);
+  check_prefill(out, q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, tile_seq, tile_q0, num_tiles, Hq, Hkv);
+  if (tiles_on_device) {
+    check_i32(*counts, "counts");
+    TORCH_CHECK(counts->numel() >= 4);
+  }
+  TORCH_CHECK(num_tiles >= 0 && (num_tiles + (list ? items : num_seqs * num_splits) + 16) * Hkv < (int64_t)1 << 24, "too many workgroups for one launch");
+  dli::launch_paged_mixed(q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr<int>(),
+                          (int)block_tables.size(1), seq_lens.data_ptr<int>(), query_start_loc.data_ptr<int>(), tile_seq.data_ptr<int>(),
+                          tile_q0.data_ptr<int>(), (int)num_tiles, out.data_ptr(), out.stride(0), parts.o, parts.ml,
+                          list ? work->data_ptr<int>() : nullptr, list ? red->data_ptr<int>() : nullptr,
+                          counts.has_value() ? counts->data_ptr<int>() : nullptr, (int)items, (int)reds, (int)num_seqs, (int)num_splits, (int)Hq,
+                          (int)Hkv, (float)scale, is_fp8(k_cache), (float)k_scale, (float)v_scale, scales_ptr(kv_scales, Hkv), tiles_on_device,
+                          (int)longest, (int)sequences, cur_stream(q));
 }
 
 void sample(Tensor out, const Tensor& logits, const Tensor& temperature, const Tensor& top_p, const Tensor& top_k,
@@ -819,11 +865,19 @@ TORCH_LIBRARY(dli, m) {
         "Tensor query_start_loc, Tensor tile_seq, Tensor tile_q0, int num_tiles, int num_heads, int num_kv_heads, float scale, "
         "float k_scale, float v_scale, Tensor? kv_scales=None, Tensor? counts=None, int longest=0, int sequences=0) -> ()", &paged_attention_prefill);
   m.def("rm_conv_by_runs(int rows, int channels) -> bool", [](int64_t rows, int64_t c) -> bool { return dli::rm_conv_by_runs((int)rows, (int)c); });
+  m.def("mixed_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences, int rows, bool kv_fp8) -> int",
+        [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s, int64_t r, bool f) -> int64_t {
+          return dli::mixed_page_groups((int)t, (int)h, (int)g, (int)l, (int)s, (int)r, f);
+        });
   m.def("prefill_page_groups(int num_tiles, int num_kv_heads, int group, int longest, int sequences, bool kv_fp8=False) -> int",
         [](int64_t t, int64_t h, int64_t g, int64_t l, int64_t s, bool f) -> int64_t { return dli::prefill_page_groups((int)t, (int)h, (int)g, (int)l, (int)s, f); });
   m.def("paged_attention_decode_worklist(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor seq_lens, Tensor work, Tensor red, Tensor counts, int items, int reds, int max_parts, int Hq, int Hkv, float scale, "
         "Tensor workspace, float k_scale, float v_scale, Tensor? kv_scales=None) -> ()", &paged_attention_decode_worklist);
+  m.def("paged_attention_mixed(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor seq_lens, "
+        "Tensor query_start_loc, Tensor tile_seq, Tensor tile_q0, int num_tiles, Tensor? work, Tensor? red, Tensor? counts, int items, int reds, "
+        "int max_parts, int num_seqs, int num_splits, int Hq, int Hkv, float scale, Tensor? workspace, float k_scale, float v_scale, "
+        "Tensor? kv_scales, bool tiles_on_device, int longest=0, int sequences=0) -> ()", &paged_attention_mixed);
   m.def("gather_sampled(Tensor(a!) input, Tensor src, Tensor sampled) -> ()", &gather_sampled);
   m.def("sample(Tensor(a!) out, Tensor logits, Tensor temperature, Tensor top_p, Tensor top_k, Tensor seeds, Tensor steps, "
         "Tensor? noise) -> ()", &sample);

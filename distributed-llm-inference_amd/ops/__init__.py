@@ -522,6 +522,9 @@ def rope_and_cache(qkv: torch.Tensor, positions: torch.Tensor, cos_sin: Optional
 # Captured mixed steps: prefill tiles next to the decode rows on a side stream (same-box serving A/B: TPOT p50 39.4 → 38.4 ms,
 # profiles/bench_r3aj_concurrent_attention_{0,1}.json).  DLI_CONCURRENT_ATTN=0: one after the other.
 CONCURRENT_ATTN = os.environ.get("DLI_CONCURRENT_ATTN", "1") != "0"
+# Mixed steps: prompt tiles and decode rows in one launch (csrc/kernels/attention.hip, paged_mixed_kernel).  DLI_ATTN_ONE_LAUNCH=0: launches of their own, on
+# two streams where ``attention_beside`` or a capture says so.
+ONE_LAUNCH_ATTN = CONCURRENT_ATTN and os.environ.get("DLI_ATTN_ONE_LAUNCH", "1") != "0"
 _ATTN_STREAMS: dict = {}
 
 
@@ -551,6 +554,15 @@ def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page
                                      page_element_bytes == 1) == 1
 
 
+def attention_in_one_launch(meta: AttnMetadata, num_heads: int, num_kv_heads: int, kv_fp8: bool) -> bool:
+    """Do a mixed step's prompt tiles and decode rows share a launch?  (``mixed_page_groups``: nearly always.  The launch has a grid of one dimension,
+    whose bound no step of a server comes near.)"""
+    if meta.num_prefill_tiles + max(meta.decode_items, meta.num_decode * meta.decode_splits) >= (1 << 23) // max(num_kv_heads, 1):
+        return False
+    longest, sequences = (0, 0) if meta.counts_on_device else (meta.max_seq_len, meta.num_prefill)
+    return hip().mixed_page_groups(meta.num_prefill_tiles, num_kv_heads, num_heads // num_kv_heads, longest, sequences, meta.num_decode, kv_fp8) > 0
+
+
 def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, meta: AttnMetadata,
                     num_heads: int, num_kv_heads: int, head_dim: int, scale: float,
                     k_scale: float = 1.0, v_scale: float = 1.0, out: Optional[torch.Tensor] = None,
@@ -567,6 +579,15 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         lib = hip()
         side = None
         known = (0, 0) if meta.counts_on_device else (meta.max_seq_len, meta.num_prefill)    # a captured launch has bounds only
+        listed = meta.decode_items > 0
+        if (ONE_LAUNCH_ATTN and meta.num_prefill_tiles > 0 and (listed or (meta.num_decode > 0 and meta.decode_work is None))
+                and attention_in_one_launch(meta, num_heads, num_kv_heads, k_cache.element_size() == 1)):
+            lib.paged_attention_mixed(out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.query_start_loc, meta.prefill_tile_seq,
+                                      meta.prefill_tile_q0, meta.num_prefill_tiles, meta.decode_work if listed else None,
+                                      meta.decode_red if listed else None, meta.counts if listed or meta.counts_on_device else None,
+                                      meta.decode_items, meta.decode_reds, meta.decode_max_parts, meta.num_decode, meta.decode_splits, num_heads,
+                                      num_kv_heads, scale, meta.decode_workspace, k_scale, v_scale, kv_scales, meta.counts_on_device, *known)
+            return out
         if (CONCURRENT_ATTN and meta.num_prefill_tiles > 0 and (meta.decode_items > 0 or meta.num_decode > 0)
                 and (torch.cuda.is_current_stream_capturing()
                      or attention_beside(meta, num_heads, num_kv_heads, k_cache.element_size()))):
