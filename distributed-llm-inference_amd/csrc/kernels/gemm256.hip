@@ -57,7 +57,7 @@ constexpr int STAGE_BYTES = 2 * TILE_BYTES;    // A + B
 #endif
 constexpr int G256_W_AUX = DLI_G256_W_AUX;     // cache policy of the W-operand DMA; 2 = nt was measured: neutral for one row tile, 3 % SLOWER at M ≥ 2304 (the panel IS re-used by the row tiles of an XCD: profiles/ab_g256_wnt_r3.txt)
 
-enum { EPI_SWIGLU = 0, EPI_SCATTER = 1, EPI_SCATTER_SPLITK = 2, EPI_PLAIN = 3, EPI_PLAIN_SPLITK = 4, EPI_SWIGLU_SPLITK = 5 };
+enum { EPI_SWIGLU = 0, EPI_SCATTER = 1, EPI_SCATTER_F32 = 2, EPI_PLAIN = 3, EPI_PLAIN_SPLITK = 4, EPI_SWIGLU_SPLITK = 5 };
 // The two dense split-K epilogues (mid-M GEMMs: one or two row tiles cannot fill 256 CUs, so K is cut into slices) store
 // raw fp32 partial sums into slab `split` of a workspace [k_splits][M][ldc]; splitk_reduce_kernel adds the slabs in
 // fixed order and applies the real epilogue (bf16 store, or silu(gate)·up over the [gate | up] halves of a row).
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(
     const uint16_t* __restrict__ A, int64_t a_stride, const uint16_t* __restrict__ W, int64_t w_expert_stride,
     const int* __restrict__ sorted_ids, const int* __restrict__ tile_expert, const int* __restrict__ meta,
     const float* __restrict__ topk_w, int top_k, void* __restrict__ out_, int64_t out_stride, int M, int K, int N_half,
-    int n_col_blocks, int k_splits, int64_t slab_elems, int lin_begin, int lin_count, float act_limit) {
+    int n_col_blocks, int k_splits, int64_t slab_elems, int lin_begin, int lin_count, float act_limit, float* __restrict__ cut_slabs) {
   uint16_t* out = reinterpret_cast<uint16_t*>(out_);
   __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE_BYTES];
 
@@ -91,11 +91,31 @@ __global__ __launch_bounds__(512) void gemm256_kernel(
   const int n_tiles = GROUPED ? meta[0] : (M + TM - 1) / TM;
   const int n_virtual = ranged ? n_col_blocks : n_col_blocks * k_splits;   // split-K slices are extra "columns" (slowest index)
   const int total = ranged ? lin_count * k_splits : n_tiles * n_virtual;
-  const int per_xcd = (total + 7) >> 3;
-  const int in_xcd = blockIdx.x >> 3;
+  // CUT (grouped down projections): meta[2] tiles of that order, a multiple of the CU count, are whole rounds, the tiles behind them are cut
+  // into meta[3] K-slices each (moe_align's cut_plan), whose sums go to compact slabs as in RANGE mode.
+  constexpr bool CUT = GROUPED && (EPI == EPI_SCATTER || EPI == EPI_SCATTER_F32);
+  const int plain = CUT ? meta[2] : 0, slices = CUT ? meta[3] : 1, rest = total - plain;
+  int in_xcd = blockIdx.x >> 3, count = total, begin = 0;
+  if (CUT) {
+    if (in_xcd < plain >> 3) {
+      count = plain;
+    } else {
+      in_xcd -= plain >> 3;
+      begin = plain;
+      count = rest * slices;
+    }
+  }
+  const int per_xcd = (count + 7) >> 3;
   const int j_lin = (blockIdx.x & 7) * per_xcd + in_xcd;
-  if (in_xcd >= per_xcd || j_lin >= total) return;
-  int split = 0, lin = j_lin, lin_local = 0;
+  if (in_xcd >= per_xcd || j_lin >= count) return;
+  const bool cut = CUT && slices > 1 && begin == plain;      // (plain = 0: there is no workgroup of whole rounds)
+  int split = 0, lin = begin + j_lin, lin_local = 0;
+  if (cut) {
+    split = j_lin / rest;
+    lin_local = j_lin - split * rest;
+    lin = plain + lin_local;
+    k_splits = slices;
+  }
   if (ranged) {
     split = j_lin / lin_count;
     lin_local = j_lin - split * lin_count;
@@ -106,8 +126,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(
   const int gw = min(GW, n_virtual - grp * GW);              // the last group may be narrower
   const int tile = within / gw;
   const int col_virtual = grp * GW + (within - tile * gw);
-  if (!ranged) split = col_virtual / n_col_blocks;
-  const int col_block = ranged ? col_virtual : col_virtual - split * n_col_blocks;
+  if (!ranged && !CUT) split = col_virtual / n_col_blocks;
+  const int col_block = ranged || CUT ? col_virtual : col_virtual - split * n_col_blocks;
   const int e = GROUPED ? tile_expert[tile] : 0;
   const uint16_t* We = W + (int64_t)e * w_expert_stride;
   const int n0 = col_block * (is_swiglu(EPI) ? TN / 2 : TN);
@@ -344,10 +364,11 @@ __global__ __launch_bounds__(512) void gemm256_kernel(
           *reinterpret_cast<bf16x4*>(dst + n * 16) = o;        // grouped padding rows hold finite junk, never read back
         }
       }
-    } else if (EPI == EPI_SCATTER_SPLITK) {
+    } else if (CUT && (EPI == EPI_SCATTER_F32 || cut)) {
       if (sid >= 0) {
         const float w = topk_w[sid];
-        float* dst = reinterpret_cast<float*>(out_) + split * slab_elems + (int64_t)sid * out_stride + n0 + wc * 64 + 4 * g;
+        float* dst = (cut ? cut_slabs + ((int64_t)split * rest + lin_local) * (TM * TN) + lrow * TN : reinterpret_cast<float*>(out_) + (int64_t)sid * out_stride + n0) +
+                     wc * 64 + 4 * g;
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
           f32x4 o;
@@ -372,11 +393,11 @@ __global__ __launch_bounds__(512) void gemm256_kernel(
 
 }  // namespace g256
 
-// epilogue: 0 SwiGLU, 1 scatter (MoE down), 2 scatter split-K (fp32 slabs).  Same contract as launch_grouped_gemm,
-// 256-row tiles (moe_align must have padded the expert segments to 256).
+// epilogue: 0 SwiGLU, 1 scatter (MoE down), 2 the same with fp32 rows.  Same contract as launch_grouped_gemm, 256-row tiles (moe_align must
+// have padded the expert segments to 256).  1 and 2: meta holds a cut plan, `cut_slabs` grouped_cut_slabs(…) tiles of 256 × 256 floats.
 void launch_grouped_gemm256(int epilogue, const void* A, int64_t a_stride, const void* W, int64_t w_expert_stride,
                             const int* sorted_ids, const int* tile_expert, const int* meta, const float* topk_w, int top_k,
-                            void* out, int64_t out_stride, int K, int N_out, int max_tiles, int k_splits, int64_t slab_elems,
+                            void* out, int64_t out_stride, int K, int N_out, int max_tiles, float* cut_slabs,
                             hipStream_t stream, float act_limit) {
   using namespace g256;
   if (max_tiles == 0) return;
@@ -385,15 +406,15 @@ void launch_grouped_gemm256(int epilogue, const void* A, int64_t a_stride, const
     return (v && v[0] == '0') ? 0 : 1;
   }();
   const int n_col_blocks = N_out / (epilogue == EPI_SWIGLU ? TN / 2 : TN);
-  const int n_virtual = n_col_blocks * k_splits;
-  dim3 grid((max_tiles * n_virtual + 7) / 8 * 8);                            // surplus blocks exit on meta[0]
+  const int blocks = max_tiles * n_col_blocks;
+  dim3 grid((blocks + (epilogue == EPI_SWIGLU ? 0 : grouped_cut_slabs(blocks)) + 7) / 8 * 8);      // surplus blocks exit on meta
 #define G256_GO(EPI)                                                                                                       \
   hipLaunchKernelGGL((gemm256_kernel<EPI, true>), grid, dim3(512), 0, stream, (const uint16_t*)A, a_stride, (const uint16_t*)W, \
                      w_expert_stride, sorted_ids, tile_expert, meta, topk_w, top_k, out, out_stride, 0, K, N_out, n_col_blocks, \
-                     k_splits, slab_elems, half_tiles, 0, act_limit)
+                     1, 0, half_tiles, 0, act_limit, cut_slabs)
   if (epilogue == EPI_SWIGLU) G256_GO(EPI_SWIGLU);
   else if (epilogue == EPI_SCATTER) G256_GO(EPI_SCATTER);
-  else G256_GO(EPI_SCATTER_SPLITK);
+  else G256_GO(EPI_SCATTER_F32);
 #undef G256_GO
 }
 
@@ -499,7 +520,7 @@ void launch_dense_gemm256(bool swiglu, const void* x, int64_t x_stride, const vo
 #define G256_DENSE(EPI, grid_, out_ptr_, ld_, splits_, slab_, begin_, count_)                                                    \
   hipLaunchKernelGGL((gemm256_kernel<EPI, false>), dim3(grid_), dim3(512), 0, stream, (const uint16_t*)x, x_stride,              \
                      (const uint16_t*)W, (int64_t)0, nullptr, nullptr, nullptr, nullptr, 1, out_ptr_, ld_, M, K, N_out,          \
-                     n_col_blocks, splits_, slab_, begin_, count_, 0.f)
+                     n_col_blocks, splits_, slab_, begin_, count_, 0.f, nullptr)
   if (k_splits > 1) {
     const int64_t ldc = (int64_t)N_out * (swiglu ? 2 : 1), slab = (int64_t)M * ldc;
     const int grid = (n_tiles * n_col_blocks * k_splits + 7) / 8 * 8;

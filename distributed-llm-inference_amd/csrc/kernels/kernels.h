@@ -61,7 +61,8 @@ size_t sample_workspace_bytes(int B, int V);
 // mixture of experts (moe.hip)
 void launch_moe_route(const void* logits, int T, int E, int K, int* ids, float* weights, hipStream_t stream);
 void launch_moe_align(const int* ids, int n, int expert_offset, int E_local, int* sorted_ids, int* tile_expert, int* meta,
-                      int capacity_rows, int tile_rows, hipStream_t stream);
+                      int capacity_rows, int tile_rows, hipStream_t stream, int n_col_blocks = 0, int nk = 0, int* pos_of = nullptr);
+int grouped_cut_slabs(int blocks);
 void launch_grouped_gemm(int epilogue, const void* A, int64_t a_stride, const void* W, int64_t w_expert_stride,
                          const int* sorted_ids, const int* tile_expert, const int* meta, const float* topk_w, int top_k,
                          void* out, int64_t out_stride, int K, int N_out, int max_tiles, int k_splits, int64_t slab_elems,
@@ -69,8 +70,8 @@ void launch_grouped_gemm(int epilogue, const void* A, int64_t a_stride, const vo
 // 256×256×64 tile (gemm256.hip): large-M grouped GEMM and dense GEMM with optional SwiGLU epilogue
 void launch_grouped_gemm256(int epilogue, const void* A, int64_t a_stride, const void* W, int64_t w_expert_stride,
                             const int* sorted_ids, const int* tile_expert, const int* meta, const float* topk_w, int top_k,
-                            void* out, int64_t out_stride, int K, int N_out, int max_tiles, int k_splits, int64_t slab_elems,
-                            hipStream_t stream, float act_limit = 0.f);
+                            void* out, int64_t out_stride, int K, int N_out, int max_tiles, float* cut_slabs, hipStream_t stream,
+                            float act_limit = 0.f);
 void launch_dense_gemm256(bool swiglu, const void* x, int64_t x_stride, const void* W, void* out, int64_t out_stride, int M,
                           int K, int N_out, int k_splits, float* workspace, bool split_tail, hipStream_t stream);
 void dense_gemm256_tail_plan(int M, int K, int N_out, bool swiglu, int* tail_tiles, int* tail_slices);
@@ -89,6 +90,8 @@ void launch_grouped_stream_gemm(int epilogue, int tile_rows, const void* A, int6
 void launch_splitk_reduce(bool swiglu, const float* slabs, int n_slabs, int M, int N, void* out, int64_t out_stride, hipStream_t stream);
 void launch_moe_sum(const void* y, bool y_fp32, int n_slabs, int64_t slab_elems, const int* ids, int expert_offset, int E_local,
                     int top_k, int T, int H, void* out, hipStream_t stream);
+void launch_moe_sum_cut(const void* y, bool y_fp32, const float* slabs, const int* pos_of, const int* meta, const int* ids, int expert_offset, int E_local,
+                        int top_k, int T, int H, void* out, hipStream_t stream);
 
 // heterogeneous decoder stacks (seqmix.hip): fp32 stream / statistics / state, activations bf16 or fp32 (the *_bf16 flags)
 void launch_sm_layer_norm(const float* x, const float* w, const float* b, float eps, int rows, int W, void* out, bool out_bf16,

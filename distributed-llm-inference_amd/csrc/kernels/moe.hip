@@ -15,6 +15,8 @@
 //                  EPI_SCATTER: rows are scaled by their routing weight and stored at (token·k + slot).
 //   moe_sum        out[t] = Σ_slots y[t·k + slot] over the slots served by local experts (no atomics:
 //                  bitwise reproducible; non-local slots are summed in by the caller's all-reduce).
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -56,10 +58,37 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const uint16_t* __restri
 }
 
 // ------------------------------------------------------------------------------------------ alignment
-// meta[0] = number of row tiles, meta[1] = padded row count
+// Down projection on 256 × 256 tiles, one workgroup a compute unit: whole rounds of 256 tiles, and what is left over (all of it, if that is less than a
+// round) in K-slices, so that a last round of few tiles does not leave most of the chip idle.  Only the device knows the number of tiles.
+// → {tiles in whole rounds, slices of each of the others}.  µs, measured at K = 14336, 4096 columns: a K-step of a tile 1.7 (`full`: a tile's share of that on
+// average, tiles of up to 128 rows take 0.58), a workgroup's start and end 6, a slice's 256 KB of sums written and read 0.1.  Slices that are more than a round end
+// half a slice apart.  Mixtral's layer, µs, slices by the largest possible number of tiles and fp32 rows for all of them / this: 300 tokens 636 / 592, 777 731 /
+// 680, 2048 1403 / 1343; whole rounds only / this: 4096 2415 / 2321 (tiles for a round and a quarter, say, take that and not two).
+constexpr int CUT_CUS = 256, CUT_MAX_SLICES = 8, CUT_MAX_TILES = 512;
+int grouped_cut_slabs(int blocks) { return std::min(CUT_MAX_TILES, CUT_MAX_SLICES * std::min(blocks, CUT_CUS - 1)); }
+__host__ __device__ inline int2 cut_plan(int blocks, int nk, float full) {
+  const int rest = blocks % CUT_CUS;
+  int best = 1;
+  const float top = full < 0.59f ? full : 1.f;              // the longest of the tiles
+  float best_us = top * 1.7f * nk + 6.f;
+  for (int k = 2; k <= CUT_MAX_SLICES && 4 * k <= nk && rest * k <= CUT_MAX_TILES; ++k) {
+    const int waves = (rest * k + CUT_CUS - 1) / CUT_CUS;
+    const float rounds = waves == 1 ? top / k : fminf(waves * top / k, rest * full / CUT_CUS + 0.5f * top / k);
+    const float us = rounds * 1.7f * nk + waves * 6.f + 0.1f * rest * k * full;
+    if (us < best_us) {
+      best_us = us;
+      best = k;
+    }
+  }
+  return rest > 0 && best > 1 ? make_int2(blocks - rest, best) : make_int2(0, 1);
+}
+
+// meta[0] = number of row tiles, meta[1] = padded row count; n_col_blocks > 0: meta[2], meta[3] = cut_plan of that many column blocks and nk
+// K-steps, pos[i] = row of pair i in the sorted order
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int n, int expert_offset, int E_local,
                                                          int* __restrict__ sorted_ids, int* __restrict__ tile_expert,
-                                                         int* __restrict__ meta, int capacity_rows, int tile_rows) {
+                                                         int* __restrict__ meta, int capacity_rows, int tile_rows, int n_col_blocks, int nk,
+                                                         int* __restrict__ pos_of) {
   const int BM = tile_rows;                               // row tile of the GEMM that consumes the alignment (32, 64, 128 or 256)
   __shared__ int cnt[MOE_MAX_E], off[MOE_MAX_E + 1], pos[MOE_MAX_E];
   for (int e = threadIdx.x; e < MOE_MAX_E; e += blockDim.x) { cnt[e] = 0; pos[e] = 0; }
@@ -71,13 +100,21 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   __syncthreads();
   if (threadIdx.x == 0) {
     off[0] = 0;
+    int half = 0;
     for (int e = 0; e < E_local; ++e) {
       const int padded = (cnt[e] + BM - 1) / BM * BM;
+      half += padded - cnt[e] >= BM / 2 ? 1 : 0;
       for (int t = off[e] / BM; t < (off[e] + padded) / BM; ++t) tile_expert[t] = e;
       off[e + 1] = off[e] + padded;
     }
-    meta[0] = off[E_local] / BM;
+    const int tiles = off[E_local] / BM;
+    meta[0] = tiles;
     meta[1] = off[E_local];
+    if (n_col_blocks > 0) {
+      const int2 plan = cut_plan(tiles * n_col_blocks, nk, 1.f - 0.42f * half / max(tiles, 1));
+      meta[2] = plan.x;
+      meta[3] = plan.y;
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < capacity_rows; i += blockDim.x) sorted_ids[i] = -1;
@@ -123,6 +160,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
       int before = run[par][e];
       for (int w = 0; w < wave; ++w) before += wcnt[par][w][e];
       sorted_ids[off[e] + before + rank] = i;
+      if (n_col_blocks > 0) pos_of[i] = off[e] + before + rank;
     }
     if (threadIdx.x < E_local) {                            // positions for the next chunk, read after ITS barrier
       int add = run[par][threadIdx.x];
@@ -342,6 +380,42 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const void* __restrict__ y
   }
 }
 
+// The same behind a down projection on 256 × 256 tiles: y bf16 or fp32 rows (F32) of the tiles in whole rounds; the sums of a cut tile (meta[2], meta[3]) are
+// those of its slices, [slice][tile][256][256] fp32.
+template <bool F32>
+__global__ __launch_bounds__(256) void moe_sum_cut_kernel(const void* __restrict__ y_, const float* __restrict__ slabs, const int* __restrict__ pos_of,
+                                                          const int* __restrict__ meta, const int* __restrict__ ids, int expert_offset, int E_local,
+                                                          int top_k, int H, uint16_t* __restrict__ out) {
+  const int t = blockIdx.x, n_tiles = meta[0], plain = meta[2], slices = meta[3], n_col = H >> 8, rest = n_tiles * n_col - plain;
+  for (int v = threadIdx.x; v < H / 8; v += blockDim.x) {
+    // this column block's tiles in the order in which the kernel deals them: groups of 8 column blocks, row tile, column block
+    const int cb = v >> 5, first = cb & ~7, width = min(8, n_col - first), lin0 = first * n_tiles + cb - first - plain;
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int s = 0; s < top_k; ++s) {
+      const int pair = t * top_k + s, e = ids[pair] - expert_offset;
+      if (e < 0 || e >= E_local) continue;
+      const int row = pos_of[pair], lin = lin0 + (row >> 8) * width;
+      const bool cut = slices > 1 && lin >= 0;
+      if (F32 || cut) {
+        const float* y = cut ? slabs + (int64_t)lin * 65536 + (row & 255) * 256 + (v & 31) * 8 : reinterpret_cast<const float*>(y_) + (int64_t)pair * H + v * 8;
+        for (int k = 0; k < (cut ? slices : 1); ++k, y += (int64_t)rest * 65536) {        // fixed order: bitwise reproducible
+          const f32x4 a = *reinterpret_cast<const f32x4*>(y), b = *reinterpret_cast<const f32x4*>(y + 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) { acc[j] += a[j]; acc[4 + j] += b[j]; }
+        }
+      } else {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint16_t*>(y_) + (int64_t)pair * H + v * 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += bf2f((uint16_t)a[j]);
+      }
+    }
+    bf16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = (short)f2bf(acc[j]);
+    *reinterpret_cast<bf16x8*>(out + (int64_t)t * H + v * 8) = o;
+  }
+}
+
 // ------------------------------------------------------------------------------------------ launchers
 void launch_moe_route(const void* logits, int T, int E, int K, int* ids, float* weights, hipStream_t stream) {
   if (T == 0) return;
@@ -349,9 +423,9 @@ void launch_moe_route(const void* logits, int T, int E, int K, int* ids, float* 
 }
 
 void launch_moe_align(const int* ids, int n, int expert_offset, int E_local, int* sorted_ids, int* tile_expert, int* meta,
-                      int capacity_rows, int tile_rows, hipStream_t stream) {
+                      int capacity_rows, int tile_rows, hipStream_t stream, int n_col_blocks, int nk, int* pos_of) {
   hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), 0, stream, ids, n, expert_offset, E_local, sorted_ids, tile_expert,
-                     meta, capacity_rows, tile_rows);
+                     meta, capacity_rows, tile_rows, n_col_blocks, nk, pos_of);
 }
 
 void launch_grouped_gemm(int epilogue, const void* A, int64_t a_stride, const void* W, int64_t w_expert_stride,
@@ -383,6 +457,13 @@ void launch_moe_sum(const void* y, bool y_fp32, int n_slabs, int64_t slab_elems,
   else
     hipLaunchKernelGGL(moe_sum_kernel<false>, dim3(T), dim3(256), 0, stream, y, ids, expert_offset, E_local, top_k, H, 1,
                        slab_elems, (uint16_t*)out);
+}
+
+void launch_moe_sum_cut(const void* y, bool y_fp32, const float* slabs, const int* pos_of, const int* meta, const int* ids, int expert_offset, int E_local,
+                        int top_k, int T, int H, void* out, hipStream_t stream) {
+  if (T == 0) return;
+  hipLaunchKernelGGL((y_fp32 ? moe_sum_cut_kernel<true> : moe_sum_cut_kernel<false>), dim3(T), dim3(256), 0, stream, y, slabs, pos_of, meta, ids,
+                     expert_offset, E_local, top_k, H, (uint16_t*)out);
 }
 
 }  // namespace dli

@@ -475,36 +475,46 @@ void moe_experts_forward(const Tensor& x, const Tensor& ids, const Tensor& wts, 
   auto i32 = x.options().dtype(at::kInt);
   const int64_t capacity = (n + TR - 1) / TR * TR + El * TR;
   const int64_t max_tiles = capacity / TR;
-  Tensor sorted = at::empty({capacity}, i32), tile_expert = at::empty({max_tiles}, i32), meta = at::empty({2}, i32);
+  Tensor sorted = at::empty({capacity}, i32), tile_expert = at::empty({max_tiles}, i32), meta = at::empty({4}, i32);
   Tensor act = at::empty({capacity, I}, x.options());
+  int *ids_ = ids.data_ptr<int>(), *sorted_ = sorted.data_ptr<int>(), *te = tile_expert.data_ptr<int>(), *mt = meta.data_ptr<int>();
+  float* tw = wts.data_ptr<float>();
   // Down projection: with few row tiles a (row tile × 128 columns) grid cannot fill 256 CUs, so K is cut into slices whose fp32
   // partial slabs are summed (in fixed order) by moe_sum.  The slice count depends on T only: static under hipGraph.
-  // (512-thread 256² tiles run one per CU: two full rounds of the chip are enough; the 128² tiles run 2–3 per CU; of the streaming tiles
-  // about one an expert has rows)
+  // (512-thread 256² tiles run one per CU, and the device decides by their number which of them are cut: moe.hip, cut_plan.  Their rows are fp32 where
+  // fewer than two rounds of them are possible.  The 128² tiles run 2–3 per CU; of the streaming tiles about one an expert has rows)
   const int64_t nk2 = I / 64;
   const bool stream_tiles = TR <= 64;
   // (no local expert, or a capacity of no rows: nothing to fill)
   const int64_t blocks = std::max<int64_t>(1, stream_tiles ? (std::min(n, El) + n / TR) * (H / 128) : max_tiles * (H / TR));
   const int64_t want_blocks = stream_tiles ? g_moe_stream_min_blocks : TR == 256 ? g_moe_splitk_min_blocks256 : 1024;
+  if (TR == 256) {
+    const bool f32 = blocks < want_blocks;
+    Tensor y = at::empty({n, H}, f32 ? x.options().dtype(at::kFloat) : x.options()), pos = at::empty({n}, i32);
+    Tensor slabs = at::empty({(int64_t)dli::grouped_cut_slabs((int)blocks) * 65536}, x.options().dtype(at::kFloat));
+    dli::launch_moe_align(ids_, (int)n, (int)expert_offset, (int)El, sorted_, te, mt, (int)capacity, (int)TR, stream, (int)(H / 256), (int)nk2, pos.data_ptr<int>());
+    dli::launch_grouped_gemm256(0, x.data_ptr(), H, w13.data_ptr(), 2 * I * H, sorted_, te, mt, tw, (int)top_k, act.data_ptr(), I, (int)H, (int)I,
+                                (int)max_tiles, nullptr, stream, act_limit);
+    dli::launch_grouped_gemm256(f32 ? 2 : 1, act.data_ptr(), I, w2.data_ptr(), H * I, sorted_, te, mt, tw, (int)top_k, y.data_ptr(), H, (int)I, (int)H,
+                                (int)max_tiles, slabs.data_ptr<float>(), stream);
+    dli::launch_moe_sum_cut(y.data_ptr(), f32, slabs.data_ptr<float>(), pos.data_ptr<int>(), mt, ids_, (int)expert_offset, (int)El, (int)top_k, (int)T,
+                            (int)H, out, stream);
+    return;
+  }
   int64_t k_splits = 1;
   if (blocks < want_blocks)
     k_splits = std::max<int64_t>(1, std::min<int64_t>({(want_blocks + blocks - 1) / blocks, 16, stream_tiles ? nk2 / 8 : nk2}));
   const bool split = k_splits > 1 || stream_tiles;           // (few rows: the slots of a token are added in fp32 whatever the slice count)
   Tensor y = split ? at::empty({k_splits, n, H}, x.options().dtype(at::kFloat)) : at::empty({n, H}, x.options());
-  dli::launch_moe_align(ids.data_ptr<int>(), (int)n, (int)expert_offset, (int)El, sorted.data_ptr<int>(),
-                        tile_expert.data_ptr<int>(), meta.data_ptr<int>(), (int)capacity, (int)TR, stream);
-  auto gg = [&](int epi, const void* A, int64_t a_stride, const void* W, int64_t w_stride, const int* ids_, const int* te, const int* mt,
-                const float* tw, int k_, void* o, int64_t os, int K, int N_out, int tiles, int splits, int64_t slab, hipStream_t st, float limit) {
-    if (TR == 256) dli::launch_grouped_gemm256(epi, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
-    else if (TR == 128) dli::launch_grouped_gemm(epi, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
-    else dli::launch_grouped_stream_gemm(epi, (int)TR, A, a_stride, W, w_stride, ids_, te, mt, tw, k_, o, os, K, N_out, tiles, splits, slab, st, limit);
+  dli::launch_moe_align(ids_, (int)n, (int)expert_offset, (int)El, sorted_, te, mt, (int)capacity, (int)TR, stream);
+  auto gg = [&](int epi, const void* A, int64_t a_stride, const void* W, int64_t w_stride, void* o, int64_t os, int K, int N_out, int splits,
+                int64_t slab, float limit) {
+    if (TR == 128) dli::launch_grouped_gemm(epi, A, a_stride, W, w_stride, sorted_, te, mt, tw, (int)top_k, o, os, K, N_out, (int)max_tiles, splits, slab, stream, limit);
+    else dli::launch_grouped_stream_gemm(epi, (int)TR, A, a_stride, W, w_stride, sorted_, te, mt, tw, (int)top_k, o, os, K, N_out, (int)max_tiles, splits, slab, stream, limit);
   };
-  gg(0, x.data_ptr(), H, w13.data_ptr(), 2 * I * H, sorted.data_ptr<int>(), tile_expert.data_ptr<int>(), meta.data_ptr<int>(),
-     wts.data_ptr<float>(), (int)top_k, act.data_ptr(), I, (int)H, (int)I, (int)max_tiles, 1, 0, stream, act_limit);
-  gg(split ? 2 : 1, act.data_ptr(), I, w2.data_ptr(), H * I, sorted.data_ptr<int>(), tile_expert.data_ptr<int>(),
-     meta.data_ptr<int>(), wts.data_ptr<float>(), (int)top_k, y.data_ptr(), H, (int)I, (int)H, (int)max_tiles, (int)k_splits,
-     n * H, stream, 0.f);
-  dli::launch_moe_sum(y.data_ptr(), split, (int)k_splits, n * H, ids.data_ptr<int>(), (int)expert_offset, (int)El, (int)top_k,
+  gg(0, x.data_ptr(), H, w13.data_ptr(), 2 * I * H, act.data_ptr(), I, (int)H, (int)I, 1, 0, act_limit);
+  gg(split ? 2 : 1, act.data_ptr(), I, w2.data_ptr(), H * I, y.data_ptr(), H, (int)I, (int)H, (int)k_splits, n * H, 0.f);
+  dli::launch_moe_sum(y.data_ptr(), split, (int)k_splits, n * H, ids_, (int)expert_offset, (int)El, (int)top_k,
                       (int)T, (int)H, out, stream);
 }
 
