@@ -85,87 +85,106 @@ __host__ __device__ inline int2 cut_plan(int blocks, int nk, float full) {
 
 // meta[0] = number of row tiles, meta[1] = padded row count; n_col_blocks > 0: meta[2], meta[3] = cut_plan of that many column blocks and nk
 // K-steps, pos[i] = row of pair i in the sorted order
+// A wave has a run of neighbouring pairs: it counts them, learns where its share of each expert's rows begins, and places them, in the order of the pair
+// index and without atomics: every launch produces the same sorted_ids, so WHICH rows share an expert's last tile never
+// changes from launch to launch and a step replays bit-identically whatever the tile variants do with a partly filled tile.  Two barriers in all.  Bound by
+// the instructions that one compute unit issues: the pairs of a lane's expert among 64 come from a ballot for every bit of its number, once, whatever the
+// number of experts (8192 pairs of 8 experts, µs: an LDS atomic for every pair and a ballot for every expert 21, two of those 18 to 21, this 10).
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int n, int expert_offset, int E_local,
                                                          int* __restrict__ sorted_ids, int* __restrict__ tile_expert,
                                                          int* __restrict__ meta, int capacity_rows, int tile_rows, int n_col_blocks, int nk,
                                                          int* __restrict__ pos_of) {
+  static_assert(MOE_MAX_E <= 64, "a lane for every expert, six bits of its number");
+  constexpr int HELD = 8;                                  // 64 pairs each: runs of up to 512 pairs are looked at once
   const int BM = tile_rows;                               // row tile of the GEMM that consumes the alignment (32, 64, 128 or 256)
-  __shared__ int cnt[MOE_MAX_E], off[MOE_MAX_E + 1], pos[MOE_MAX_E];
-  for (int e = threadIdx.x; e < MOE_MAX_E; e += blockDim.x) { cnt[e] = 0; pos[e] = 0; }
-  __syncthreads();
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int e = ids[i] - expert_offset;
-    if (e >= 0 && e < E_local) atomicAdd(&cnt[e], 1);
+  __shared__ int wave_cnt[16][MOE_MAX_E], off[MOE_MAX_E + 1], cnt[MOE_MAX_E];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
+  const int run = ((n + n_waves - 1) / n_waves + 63) & ~63, begin = wave * run, end = min(n, begin + run);
+  const int bits = 32 - __clz(max(E_local - 1, 1));
+  // expert (-1: none of these) of pair at + 64 j + lane, how many before it among the 64 have the same one, and how many in all
+  int held[HELD], rank[HELD], same_all[HELD];
+  auto look = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) held[j] = at + 64 * j + lane < end ? ids[at + 64 * j + lane] : -1;
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) {
+      if (at + 64 * j >= end) break;
+      const int e = held[j] - expert_offset;
+      const bool here = held[j] >= 0 && e >= 0 && e < E_local;
+      const unsigned long long any = __ballot(here);
+      uint32_t lo = (uint32_t)any, hi = (uint32_t)(any >> 32);
+      for (int b = 0; b < bits; ++b) {
+        const unsigned long long set = __ballot((e >> b) & 1);
+        const uint32_t clear = ((e >> b) & 1) - 1;         // all ones where the lane's bit is 0
+        lo &= (uint32_t)set ^ clear;
+        hi &= (uint32_t)(set >> 32) ^ clear;
+      }
+      held[j] = here ? e : -1;
+      rank[j] = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+      same_all[j] = __popc(lo) + __popc(hi);
+    }
+  };
+  wave_cnt[wave][lane] = 0;                                // (a wave's row is its own until the barrier: LDS keeps its order)
+  for (int at = begin; at < end; at += 64 * HELD) {
+    look(at);
+#pragma unroll
+    for (int j = 0; j < HELD; ++j)
+      if (at + 64 * j < end && held[j] >= 0 && rank[j] == 0) wave_cnt[wave][held[j]] += same_all[j];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    off[0] = 0;
-    int half = 0;
-    for (int e = 0; e < E_local; ++e) {
-      const int padded = (cnt[e] + BM - 1) / BM * BM;
-      half += padded - cnt[e] >= BM / 2 ? 1 : 0;
-      for (int t = off[e] / BM; t < (off[e] + padded) / BM; ++t) tile_expert[t] = e;
-      off[e + 1] = off[e] + padded;
+  if (wave == 0) {                                         // per expert: the waves' counts → places before them, the sum
+    int c[16], sum = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) c[w] = w < n_waves ? wave_cnt[w][lane] : 0;
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) total += c[w];
+    const int tiles = lane < E_local ? (total + BM - 1) / BM : 0;
+    int before = tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(before, o, 64);
+      if (lane >= o) before += up;
     }
-    const int tiles = off[E_local] / BM;
-    meta[0] = tiles;
-    meta[1] = off[E_local];
-    if (n_col_blocks > 0) {
-      const int2 plan = cut_plan(tiles * n_col_blocks, nk, 1.f - 0.42f * half / max(tiles, 1));
-      meta[2] = plan.x;
-      meta[3] = plan.y;
+    const int all = __builtin_amdgcn_readlane(before, 63);
+    before -= tiles;
+    cnt[lane] = total;
+    off[lane] = before * BM;
+    if (lane == 0) off[MOE_MAX_E] = all * BM;
+    sum = before * BM;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      if (w < n_waves) wave_cnt[w][lane] = sum;            // the wave's first row of this expert
+      sum += c[w];
+    }
+    for (int t = 0; t < tiles; ++t) tile_expert[before + t] = lane;
+    const int half = __popcll(__ballot(tiles * BM - total >= BM / 2 && tiles > 0));
+    if (lane == 0) {
+      meta[0] = all;
+      meta[1] = all * BM;
+      if (n_col_blocks > 0) {
+        const int2 plan = cut_plan(all * n_col_blocks, nk, 1.f - 0.42f * half / max(all, 1));
+        meta[2] = plan.x;
+        meta[3] = plan.y;
+      }
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < capacity_rows; i += blockDim.x) sorted_ids[i] = -1;
-  // Placement in the order of the routed-row index (stable), without atomics: every launch produces the same sorted_ids,
-  // so WHICH rows share an expert's last tile never changes from launch to launch and a step replays bit-identically
-  // whatever the tile variants do with a partly filled tile (graph-vs-eager self-test, greedy reproducibility; the
-  // first half-tile version of gemm256.hip summed K in another order than a full tile and exposed the atomics' order).
-  // Per chunk of blockDim ids: rank inside the wave by ballots over the experts present in it, wave totals through
-  // LDS, then the running position of the expert.
-  // One barrier per chunk: the per-wave counts and the running positions are double-buffered by the chunk's parity.
-  __shared__ int wcnt[2][16][MOE_MAX_E], run[2][MOE_MAX_E];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
-  if (threadIdx.x < MOE_MAX_E) run[0][threadIdx.x] = 0;
-  const bool few = E_local <= 16;                          // few experts: one ballot per expert, every wave writes every count
-  __syncthreads();
-  int par = 0;
-  for (int base = 0; base < n; base += blockDim.x, par ^= 1) {
-    const int i = base + threadIdx.x;
-    int e = i < n ? ids[i] - expert_offset : -1;
-    if (e >= E_local) e = -1;
-    int rank = 0;
-    if (few) {
-      for (int t = 0; t < E_local; ++t) {
-        const unsigned long long same = __ballot(e == t);
-        if (e == t) rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (lane == 0) wcnt[par][wave][t] = __popcll(same);
+  // rows without a pair: the end of every expert's last tile, and what no tile has
+  for (int e = wave; e < E_local; e += n_waves)
+    for (int i = off[e] + cnt[e] + lane; i < (off[e] + cnt[e] + BM - 1) / BM * BM; i += 64) sorted_ids[i] = -1;
+  for (int i = off[MOE_MAX_E] + threadIdx.x; i < capacity_rows; i += blockDim.x) sorted_ids[i] = -1;
+  for (int at = begin; at < end; at += 64 * HELD) {
+    if (run > 64 * HELD) look(at);
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) {
+      const int i = at + 64 * j + lane, e = held[j];
+      if (i < end && e >= 0) {
+        const int first = wave_cnt[wave][e], to = first + rank[j];
+        if (rank[j] == 0) wave_cnt[wave][e] = first + same_all[j];
+        sorted_ids[to] = i;
+        if (n_col_blocks > 0) pos_of[i] = to;
       }
-    } else {
-      static_assert(MOE_MAX_E <= 64, "one lane per expert clears the wave's row");
-      if (lane < MOE_MAX_E) wcnt[par][wave][lane] = 0;      // this wave's own row: same-wave LDS order, no barrier needed
-      unsigned long long todo = __ballot(e >= 0);
-      while (todo) {                                        // one round per expert present in this wave
-        const int leader = __ffsll((long long)todo) - 1;
-        const int le = __builtin_amdgcn_readlane(e, leader);
-        const unsigned long long same = __ballot(e == le);
-        if (e == le) rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (lane == leader) wcnt[par][wave][le] = __popcll(same);
-        todo &= ~same;
-      }
-    }
-    __syncthreads();
-    if (e >= 0) {
-      int before = run[par][e];
-      for (int w = 0; w < wave; ++w) before += wcnt[par][w][e];
-      sorted_ids[off[e] + before + rank] = i;
-      if (n_col_blocks > 0) pos_of[i] = off[e] + before + rank;
-    }
-    if (threadIdx.x < E_local) {                            // positions for the next chunk, read after ITS barrier
-      int add = run[par][threadIdx.x];
-      for (int w = 0; w < n_waves; ++w) add += wcnt[par][w][threadIdx.x];
-      run[par ^ 1][threadIdx.x] = add;
     }
   }
 }
