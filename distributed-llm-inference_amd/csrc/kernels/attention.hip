@@ -560,6 +560,29 @@ __device__ __forceinline__ void prefill_tile(
     for (int p = 0; p < NPG; ++p)
       if (p == 0 || NPG * turn + p < nblk) stage_page(NPG * turn + p, smem + at * STAGE + p * 2 * PAGE_BYTES);
   };
+  // SPREAD (two groups): the pieces of the turn that is fetched are asked for behind the first score products, whose fragments are read before them, and its
+  // block table entries a turn before.  At the start of a turn, where all waves have just passed the barrier, the pieces queue up for the unit's one path to memory while
+  // the matrix cores are idle, and a scalar load that is waited for where it is made stops the wave for its latency.  Whole calls, µs, at the start / spread: bf16, 32/8 heads,
+  // one prompt of 1000 tokens 41.6 / 39.1, of 2000 81.0 / 75.5, 8/1 heads 59.0 / 51.9, of 3500 97.8 / 84.0; e4m3 79.5 / 77.2, 8/1 heads 56.0 / 54.4, of 3500 92.2 / 88.5.
+  // One group, whose unit has three workgroups at different places, loses 1 to 4 %.
+  constexpr bool SPREAD = GROUPS == 2;
+  int entry[NPG];
+  auto look_up = [&](int turn) {
+#pragma unroll
+    for (int p = 0; p < NPG; ++p) entry[p] = bt[min(NPG * turn + p, nblk - 1)];
+  };
+  // quarter `part` of a turn's pieces
+  auto stage_part = [&](int turn, int at, int part) __attribute__((always_inline)) {
+    constexpr int PIECES = 2 * NCH;                         // a wave's DMA instructions for a page
+#pragma unroll
+    for (int i = NPG * PIECES * part / 4; i < NPG * PIECES * (part + 1) / 4; ++i) {
+      if (i >= PIECES && NPG * turn + 1 >= nblk) break;
+      const int64_t page = ((int64_t)entry[i / PIECES] * Hkv + kvh) * PAGE_BYTES;
+      char* dst = smem + at * STAGE + i / PIECES * 2 * PAGE_BYTES + (wave + 4 * (i % PIECES >> 1)) * 1024;
+      if (i & 1) __builtin_amdgcn_global_load_lds((gptr_t)(vc + page + src_v[i % PIECES >> 1]), (lptr_t)(dst + PAGE_BYTES), 16, 0, 0);
+      else __builtin_amdgcn_global_load_lds((gptr_t)(kc + page + src_k[i % PIECES >> 1]), (lptr_t)dst, 16, 0, 0);
+    }
+  };
   // Lane offsets inside a staged page.  Rows of 64 bytes (K: token rows of a d chunk; bf16 V: d rows) carry the slot
   // swizzle of their row; it depends on (row >> 2) & 3 only, and every row this lane reads is c32 + a multiple of 32.
   const int swz = slot_swizzle(c32);
@@ -569,21 +592,33 @@ __device__ __forceinline__ void prefill_tile(
   const int v_off0 = c32 * 64 + ((hi ^ swz) << 4), v_off1 = c32 * 64 + (((2 + hi) ^ swz) << 4);
   const int v8_off = c32 * 32 + 16 * hi;
 
-  // NP pages from b on, staged at `kb`: scores, maxima, weights, P·V
-  auto pages = [&](auto np, int b, const char* kb) __attribute__((always_inline)) {
+  // NP pages from b on, staged at `kb`: scores, maxima, weights, P·V; between(0 … 3) behind the first four pairs of products
+  auto pages = [&](auto np, int b, const char* kb, auto&& between) __attribute__((always_inline)) {
     constexpr int NP = decltype(np)::value;
     f32x16 s[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[p][r] = 0.f;
-    if constexpr (!KV8) {
+    if constexpr (!SPREAD && !KV8) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int p = 0; p < NP; ++p)
           s[p] = mfma32(*reinterpret_cast<const bf16x8*>(kb + p * 2 * PAGE_BYTES + (j >> 1) * 2048 + k_off[j & 1]), qf[j], s[p]);
-    } else {
+    } else if constexpr (!KV8) {
+      bf16x8 kf[NP][8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) kf[p][j] = *reinterpret_cast<const bf16x8*>(kb + p * 2 * PAGE_BYTES + (j >> 1) * 2048 + k_off[j & 1]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) s[p] = mfma32(kf[p][j], qf[j], s[p]);
+        if (j < 4) between(j);
+      }
+    } else if constexpr (!SPREAD) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -597,6 +632,26 @@ __device__ __forceinline__ void prefill_tile(
           s[p] = mfma32(k0, qf[2 * j], s[p]);
           s[p] = mfma32(k1, qf[2 * j + 1], s[p]);
         }
+    } else {
+      u32x4 raw[NP][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) raw[p][j] = *reinterpret_cast<const u32x4*>(kb + p * 2 * PAGE_BYTES + (j >> 1) * 2048 + k_off[j & 1]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          bf16x8 k0, k1;
+          fp8x4_to_bf16(raw[p][j][0], k0, 0);
+          fp8x4_to_bf16(raw[p][j][1], k0, 4);
+          fp8x4_to_bf16(raw[p][j][2], k1, 0);
+          fp8x4_to_bf16(raw[p][j][3], k1, 4);
+          s[p] = mfma32(k0, qf[2 * j], s[p]);
+          s[p] = mfma32(k1, qf[2 * j + 1], s[p]);
+        }
+        between(j);
+      }
     }
     const int tok0 = b * 32 + 4 * hi;
     // The maximum moves with every page that raises it in some lane, so a column's largest weight is 1, exact in bf16.  (A maximum that lags by up to
@@ -685,16 +740,25 @@ __device__ __forceinline__ void prefill_tile(
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  if (SPREAD) look_up(start + (NSTAGE - 1) * step);
   __syncthreads();
   if (alone) turns = max(turns_of[0], turns_of[1]);
   int st = 0;
   for (int t = 0; t < turns; ++t) {
     const int turn = step * t + start;
-    const bool ahead = turn + (NSTAGE - 1) * step < nturn;
-    if (ahead) stage(turn + (NSTAGE - 1) * step, st == 0 ? NSTAGE - 1 : st - 1);
+    const int later = turn + (NSTAGE - 1) * step, to = st == 0 ? NSTAGE - 1 : st - 1;
+    const bool ahead = later < nturn;
+    auto between = [&](int part) __attribute__((always_inline)) {
+      if (SPREAD && ahead) stage_part(later, to, part);
+    };
+    if (!SPREAD && ahead) stage(later, to);
     const char* kb = smem + st * STAGE;
-    if (NPG == 2 && 2 * turn + 1 < my_nblk) pages(std::integral_constant<int, 2>{}, 2 * turn, kb);
-    else if (NPG * turn < my_nblk) pages(std::integral_constant<int, 1>{}, NPG * turn, kb);
+    if (NPG == 2 && 2 * turn + 1 < my_nblk) pages(std::integral_constant<int, 2>{}, 2 * turn, kb, between);
+    else if (NPG * turn < my_nblk) pages(std::integral_constant<int, 1>{}, NPG * turn, kb, between);
+    else
+#pragma unroll
+      for (int part = 0; part < 4; ++part) between(part);
+    if (SPREAD && ahead) look_up(later + step);
     if (NSTAGE == 3 && ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FLIGHT) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -933,21 +997,22 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
 }
 
 // Page groups of a mixed step's tiles (paged_mixed_kernel), 0: launches of their own.  rows: decode rows; longest, sequences as in prefill_page_groups.
-// µs of the longest tile's chain with one and two groups as there (one group on e4m3 pages 4 more); decode rows by themselves take 5 µs and their pages' bytes
-// at 5.5 TB/s (half the longest context each), a unit without a tile reads at 2.2 of its share.  One launch of one group then takes its chain and 0.4 of
+// µs of the longest tile's chain with one and two groups measured as there (8/1 heads, 250 to 3500 tokens); decode rows by themselves take 5 µs and their pages' bytes
+// at 5.5 TB/s (half the longest context each, at most 800 tokens: the longest may be a prompt's), a unit without a tile reads at 2.2 of its share.  One launch of one group then takes its chain and 0.4 of
 // the rows' time, or what the rows take; one of two groups its chain, 0.15 of the rows' time, and what the units without a tile leave, or 1.15 of the rows' time.  Measured, after each other / one
 // group / two — 8/1 heads, 16 bf16 rows of up to 1500 and one of 2000 behind 500 (125 tiles) 66.5 / 74.4 / 61.2, e4m3 65.2 / 80.4 / 61.6, 400 bf16 rows 94.8 /
 // 86.8 / 67.5; 64/8 heads and one of 500 behind 1500 (256), bf16, 16 rows 71.8 / 68.9 / 61.5, 96 107.7 / 83.8 / 106.5; of 400 behind 500 (200), e4m3, 48 48.9 /
 // 40.1 / 38.4, 96 58.1 / 40.0 / 48.9.  Past 256 tiles, where their own launch has two groups, one launch pays if it hides
 // rows of some length: 32/8 heads, e4m3, two of up to 1024 behind
-// up to 1024 (296), 16 rows 49.4 / 50.0, 96 67.2 / 49.4.  (More: profiles/mixed_steps_one_launch.txt.)
+// up to 1024 (296), 16 rows 49.4 / 50.0, 96 67.2 / 49.4.  (With the pieces of two groups still at the start of their turns.  More:
+// profiles/mixed_steps_one_launch.txt.)
 int mixed_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, int rows, bool kv_fp8) {
   const int blocks = num_tiles * Hkv;
   const bool two = prefill_page_groups(num_tiles, Hkv, G, longest, sequences, kv_fp8) != 1;
   if (longest == 0) return two ? 2 : 1;                       // (up to 256 tiles: at most 1.05 of launches of their own)
-  const float one_us = 5.f + 0.0285f * longest + (kv_fp8 ? 4.f : 0.f);
-  const float two_us = longest > 224 ? 5.5f + 0.0225f * longest : one_us;      // short tiles are done by one group in either form
-  const float rows_us = 5.f + (float)rows * longest * Hkv * (kv_fp8 ? 128.f : 256.f) / 5.5e6f;
+  const float one_us = 5.f + (kv_fp8 ? 0.03f : 0.0277f) * longest;
+  const float two_us = longest > 224 ? 5.5f + 0.0207f * longest : one_us;      // short tiles are done by one group in either form
+  const float rows_us = 5.f + (float)rows * std::min(longest / 2, 800) * Hkv * (kv_fp8 ? 256.f : 512.f) / 5.5e6f;
   if (blocks > PREFILL_UNITS) return two && rows_us < one_us / 2.2f ? 0 : 1;
   const float idle = (float)(PREFILL_UNITS - blocks) / PREFILL_UNITS;
   const float with_two = std::max(two_us + 0.15f * rows_us + std::max(0.f, rows_us - 2.2f * idle * two_us), 1.15f * rows_us);
