@@ -338,6 +338,31 @@ def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor
     return (plan is None or plan == _STREAM) and _stream_operands_ok(x, weight, out)
 
 
+def tile_slices(m: int, n: int, k: int, swiglu: bool = False) -> int:
+    """K slices with which the own 256² tiles (``csrc/kernels/gemm256.hip``) beat the library GEMM (and its activation pass) where the start-up measurement
+    says nothing; 0: the library.  Rows past 256 whose tiles are at most half as many as the 256 compute units, long K: the library leaves units idle, the
+    slices fill them.  µs, library / sliced:
+
+    * plain, K from 14336 on (4096 × 14336 at 257 rows 81 / 61, 512 93 / 65, 768 109 / 90, 1024 132 / 106, 2048 207 / 180; 8192 × 28672 at 512 313 / 188;
+      2048 × 28672 at 1024 277 / 100), but not at 8192 (8192 × 8192 at 512 82 / 72, at 768 98 / 100, 4096 × 8192 68 / 69 at 1024) or 4096 (1.15 – 1.4);
+    * with SwiGLU, which saves the activation pass too, from 8192 on (7168 × 8192 at 257 72 / 60, 512 83 / 65, 1024 117 / 106; 3584 × 8192 at 1024 70 / 62; more columns
+      are not measured), but not at 4096 (7168 × 4096 1.0 – 1.12);
+    * where tiles and slices fill 210 units (4096 × 14336 with 32 to 128 tiles; 96 tiles in two slices leave a quarter idle: 8192 × 28672 at 700 rows
+      285 / 296), or half of them with eight slices, plain (2048 × 28672 at 512 184 / 88, 1024 × 14336 at 1024 53 / 50, but 45 / 46 with 12 tiles)."""
+    if m <= 256 or n < 256 or n % 256 or k % 64 or k < (8192 if swiglu else 14336) or (swiglu and n > 7168):
+        return 0
+    tiles = (m + 255) // 256 * (n // 256)
+    s = min(8, 256 // tiles)
+    return s if s >= 2 and (tiles * s >= 210 or (not swiglu and s == 8 and tiles >= 16)) else 0
+
+
+def _tile_slices(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False) -> int:
+    if x.dim() != 2 or weight.dim() != 2:
+        return 0
+    s = tile_slices(x.shape[0], *weight.shape, swiglu)
+    return s if s and _stream_operands_ok(x, weight, out) and _tile_operand_ok(x, weight) else 0
+
+
 def _planned(x: torch.Tensor, weight: torch.Tensor, swiglu: bool) -> Optional[int]:
     if not (_PLAN.table and x.is_cuda and x.dim() == 2):
         return None
@@ -349,7 +374,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """``x @ weightᵀ + bias``.  Decode-sized GPU inputs take the weight-streaming MFMA kernel
     (``csrc/kernels/skinny_gemm.hip``); above that the start-up measurement (``ops/gemm_plan.py``) says, per layer shape and row count, whether
     the library GEMM (hipBLASLt through torch), the streaming tiles or the own 256² tile — with K cut into slices at mid-M — runs; what it
-    never measured goes to the streaming tiles where ``stream_rows_ok`` says so, else to the library.  ``out``: 2-D result buffer to write into (the row-parallel
+    never measured goes to the streaming tiles where ``stream_rows_ok`` says so, to sliced tiles where ``tile_slices`` does, else to the library.  ``out``: 2-D result buffer to write into (the row-parallel
     layers pass a view of the all-reduce's IPC staging buffer)."""
     if _skinny_ok(x, weight, 16):
         return hip().skinny_linear(x, weight, bias, False, out)
@@ -359,6 +384,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
             return hip().stream_gemm(x, weight, False, 0, out)
         if s and s != _STREAM and _tile_operand_ok(x, weight):
             return hip().dense_gemm256(x, weight, False, 1, out, True) if s == _TAIL else hip().dense_gemm256(x, weight, False, s, out)
+        if s is None:
+            s = _tile_slices(x, weight, out)
+            if s:
+                return hip().dense_gemm256(x, weight, False, s, out)
     if out is not None:
         return torch.mm(x, weight.t(), out=out) if bias is None else torch.addmm(bias, x, weight.t(), out=out)
     return torch.nn.functional.linear(x, weight, bias)
@@ -493,11 +522,16 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         if s and s != _STREAM and _tile_operand_ok(x, weight):
             return hip().dense_gemm256(x, weight, True, 1, None, True) if s == _TAIL else hip().dense_gemm256(x, weight, True, s)
         return silu_and_mul(torch.nn.functional.linear(x, weight))
+    s = _tile_slices(x, weight, swiglu=True)
+    if s:
+        return hip().dense_gemm256(x, weight, True, s)
     if (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_contiguous()
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and gemm256_swiglu_ok(x.shape[0], weight.shape[0] // 2, weight.shape[1])
             and x.shape[0] * x.stride(0) * 2 < 2 ** 32 and weight.numel() * 2 < 2 ** 32):
-        return hip().dense_gemm256(x, weight, True)
+        # what is left over after whole rounds in K slices (28672 × 4096 at 700 rows, µs, without / with: 165 / 150, 1200 253 / 236, 1700 338 / 321; 7168 × 8192 at 2500
+        # 299 / 232; where nothing is cut the same)
+        return hip().dense_gemm256(x, weight, True, 1, None, True)
     return silu_and_mul(torch.nn.functional.linear(x, weight))
 
 

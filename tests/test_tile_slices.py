@@ -1,0 +1,28 @@
+"""Rows past 256 with long K: the rule that sends them to sliced own tiles, at sizes timed both ways, and the products at its edges."""
+import pytest
+import torch
+
+from dli_amd import ops
+
+
+def test_sizes_on_both_sides_of_the_line():
+    f = ops.tile_slices
+    assert [f(*s) for s in ((257, 4096, 14336), (512, 4096, 14336), (768, 4096, 14336), (1024, 4096, 14336), (2048, 4096, 14336), (512, 8192, 28672),
+                            (512, 2048, 28672), (1024, 1024, 14336))] == [8, 8, 5, 4, 2, 4, 8, 8]
+    assert [f(*s, True) for s in ((257, 7168, 8192), (768, 7168, 8192), (1024, 7168, 8192), (1024, 3584, 8192))] == [4, 3, 2, 4]
+    assert not any(f(*s) for s in ((256, 4096, 14336), (2049, 4096, 14336), (700, 8192, 28672), (512, 8192, 8192), (1024, 4096, 4096), (257, 1024, 14336),
+                                   (512, 4096, 14336 + 32), (512, 4000, 14336), (512, 0, 14336), (0, 4096, 14336), (512, 7168, 8192), (512, 7168, 4096, True)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,swiglu", [(257, 1024, 14336, False), (1025, 1024, 14336, False), (520, 4096, 14336, False), (300, 7168, 8192, True),
+                                          (769, 3584, 8192, True)])
+def test_products_match_fp32(m, n, k, swiglu):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).bfloat16()
+    got = (ops.linear_swiglu(x, w) if swiglu else ops.linear(x, w)).float()
+    want = x.float() @ w.float().t()
+    if swiglu:
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2e-2)      # one rounding to bf16 (and the fast exponential); sums of K products in fp32
