@@ -439,10 +439,11 @@ __device__ __forceinline__ void solve_tiles(const float* Mn, f32x4 (&x)[N][4], i
     }
   }
 }
-// The end of both block kernels: Mn complete in LDS, the W region holding diag(w e^P) K, wt the weights.  Column tiles of W, then of U0.
-template <typename A>
-__device__ __forceinline__ void solve_block(float* Mn, const float* wt, float* wa, const DeltaSpace& sp, const A* __restrict__ v,
-                                            int64_t v_stride, int n, int Dv, int wave, int lane) {
+// The end of both block kernels: Mn complete in LDS, diag(w e^P) K in the W region, or with KEPT in LDS as tiles [4][KEPT], wt the weights.
+// Column tiles of W, then of U0.
+template <typename A, int KEPT = 0>
+__device__ __forceinline__ void solve_block(float* Mn, const float* wt, const float* kept, float* wa, const DeltaSpace& sp,
+                                            const A* __restrict__ v, int64_t v_stride, int n, int Dv, int wave, int lane) {
   const int c = lane & 15, g4 = lane >> 4;
   __syncthreads();
   diagonal_inverse(Mn, wave, lane);
@@ -453,18 +454,23 @@ __device__ __forceinline__ void solve_block(float* Mn, const float* wt, float* w
   for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
     f32x4 x[2][4];
     // All loads in flight together, the values' at clamped places: a branch around each of them made every one of 32 wait for itself.
+    constexpr bool SAME = std::is_same<A, float>::value;    // fp32 values land where they are used
     A raw[2][4][4];
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
       const int t = min(t0 + y, tiles - 1), e = (t - sp.DT) * 16 + c;
       if (t < sp.DT) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[y][i] = *reinterpret_cast<const f32x4*>(ww + (i * sp.DT + t) * TILE + lane * 4);
+        for (int i = 0; i < 4; ++i) x[y][i] = *reinterpret_cast<const f32x4*>((KEPT ? kept + (i * KEPT + t) * TILE : ww + (i * sp.DT + t) * TILE) + lane * 4);
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) raw[y][i][r] = v[min(16 * i + 4 * g4 + r, n - 1) * v_stride + min(e, Dv - 1)];
+          for (int r = 0; r < 4; ++r) {
+            const A value = v[min(16 * i + 4 * g4 + r, n - 1) * v_stride + min(e, Dv - 1)];
+            if constexpr (SAME) x[y][i][r] = value;
+            else raw[y][i][r] = value;
+          }
       }
     }
 #pragma unroll
@@ -472,13 +478,18 @@ __device__ __forceinline__ void solve_block(float* Mn, const float* wt, float* w
       const int t = min(t0 + y, tiles - 1), e = (t - sp.DT) * 16 + c;
       if (t < sp.DT) continue;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 w4 = *reinterpret_cast<const f32x4*>(wt + 16 * i + 4 * g4);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = 16 * i + 4 * g4 + r;
-          const float u = wt[row] * ldf<A>(&raw[y][i][r]);
+          float value;
+          if constexpr (SAME) value = x[y][i][r];
+          else value = ldf<A>(&raw[y][i][r]);
+          const float u = w4[r] * value;
           x[y][i][r] = row < n && e < Dv ? u : 0.f;
         }
+      }
     }
     solve_tiles<2>(Mn, x, lane);
 #pragma unroll
@@ -585,7 +596,7 @@ __global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict_
                                                          int G, int D, int Dv, int wide, float q_scale, const int* __restrict__ first_row,
                                                          float* __restrict__ ws) {
   __shared__ double P[BT];
-  __shared__ float wt[BT];
+  __shared__ __align__(16) float wt[BT];
   __shared__ __align__(16) float M[BT * BS];
   const int tile = blockIdx.x, h = blockIdx.y;
   if (tile >= min(counts[2], num_tiles)) return;
@@ -667,7 +678,7 @@ __global__ __launch_bounds__(NT, 3) void delta_block_kernel(const A* __restrict_
       }
       *reinterpret_cast<f32x4*>(wa + (wave * 4 + s) * TILE + lane * 4) = turned(a, unit);
     }
-  solve_block<A>(M, wt, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
+  solve_block<A>(M, wt, nullptr, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
 }
 
 // Channel decays.  With P_t[d] the log decays summed to token t inside the block, the same block form reads
@@ -735,7 +746,12 @@ template <typename A> __device__ __forceinline__ typename Raw<A>::v4 raw4(const 
 }
 // WIDE: D a multiple of 16, all rows 16-byte aligned: the next channels' fetches have no condition, so the compiler can count them and the
 // current channels' arithmetic does not wait for them.
-template <typename Z, bool WIDE>
+// KEPT: up to that many 16-channel tiles of diag(w e^P) K wait in LDS for the solve instead of in the workspace, with the loop's fragments in the
+// place that M takes behind it: 50 KB, still three workgroups a compute unit.  A block writes 148 KB where it wrote 180 and read 32 back.  The whole
+// step of a layer with heads of 128, µs: 16 heads, four prompts of 512 to 1069 tokens 181.2 → 177.8; 32 heads 325.8 → 317.8, one prompt of 2000
+// 234.6 → 228.0; equal below a chip full of blocks.  Longer heads would leave two workgroups a unit.  Four of them (128 registers, the next
+// channels fetched behind the stores, which loads then wait for) were slower: 191.8.
+template <typename Z, bool WIDE, int KEPT>
 __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k,
                                                            int64_t k_stride, const float* __restrict__ v, int64_t v_stride,
                                                            ChannelArgs<Z> ch, const float* __restrict__ weight,
@@ -743,9 +759,13 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
                                                            const int* __restrict__ counts, const int* __restrict__ tile_seq,
                                                            const int* __restrict__ tile_q0, int num_tiles, int H, int G, int D, int Dv, int wide,
                                                            const int* __restrict__ first_row, float* __restrict__ ws) {
-  __shared__ float wt[BT];
+  __shared__ __align__(16) float wt[BT];
   __shared__ __align__(16) float M[BT * BS];
-  __shared__ __align__(16) float KR[2][BT][20], EM[2][4][16];
+  constexpr int LOOP = 2 * BT * 20 + 2 * 4 * 16;
+  static_assert(LOOP <= BT * BS);
+  __shared__ __align__(16) float own[KEPT ? 4 : LOOP], kept[KEPT ? 4 * KEPT * TILE : 4];
+  auto KR = reinterpret_cast<float (*)[BT][20]>(KEPT ? M : own);
+  auto EM = reinterpret_cast<float (*)[4][16]>((KEPT ? M : own) + 2 * BT * 20);
   const int tile = blockIdx.x, h = blockIdx.y;
   if (tile >= min(counts[2], num_tiles)) return;
   const int seq = tile_seq[tile];
@@ -799,7 +819,8 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
     f32x4 gd, L, R, ql, kl, kR;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      gd[j] = live && d + j < D ? channel_decay<Z>(zc[j] + bc[j], rate) : 1.f;
+      const float decay = channel_decay<Z>(zc[j] + bc[j], rate);
+      gd[j] = live && (WIDE || d + j < D) ? decay : 1.f;
       float p = gd[j];
       p *= row_shr<1>(p, 1.f);
       p *= row_shr<2>(p, 1.f);
@@ -848,12 +869,13 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
     }
     const int at = (wave * sp.DT + it) * TILE + lane * 4;
     *reinterpret_cast<f32x4*>(wa + sp.q() + at) = oq;
-    *reinterpret_cast<f32x4*>(wa + sp.w() + at) = turned(ok, unit);
+    *reinterpret_cast<f32x4*>(KEPT ? kept + (wave * KEPT + it) * TILE + lane * 4 : wa + sp.w() + at) = turned(ok, unit);
     *reinterpret_cast<f32x4*>(wa + sp.kt() + (it * 4 + wave) * TILE + lane * 4) = turned(ot, unit);
     if (wave == 3 && c == 15)
       *reinterpret_cast<f32x4*>(wa + sp.pe() + d) = f32x4{L[0] * before[0], L[1] * before[1], L[2] * before[2], L[3] * before[3]};
     all_near_pairs(std::make_integer_sequence<int, 15>{}, qc, kc, gd, aq, ak);
   }
+  if (KEPT) lds_barrier();                                // M overwrites the loop's fragments
   // off-diagonal tiles
 #pragma unroll
   for (int b = 0; b < 3; ++b)
@@ -874,13 +896,13 @@ __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __res
     wa[(wave * 4 + wave) * TILE + (c + 16 * (col >> 2)) * 4 + (col & 3)] = c >= s ? x : 0.f;
     M[row * BS + 16 * wave + col] = s > 0 && c >= s ? -(wr * y) : 0.f;
   }
-  solve_block<float>(M, wt, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
+  solve_block<float, KEPT>(M, wt, kept, wa, sp, v + (int64_t)t0 * v_stride + (int64_t)h * Dv, v_stride, n, Dv, wave, lane);
 }
 
 // The walk of the delta rule: per (sequence, head, 16·CT state columns) over its blocks in order, the state on the accumulators.  A block is
 //   [o | x] = [Q̃ | W] S, u = U0 - x → LDS → o += A u, S = e^{P_end} ⊙ S + K̃ᵀ u → LDS,
 // two barriers.  16 heads of 128, four sequences of 512 to 1069 tokens: the walk 146 → 75 µs (36 of them fp32 matrix instructions, were they spread
-// evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83 (79 now that its loads are asked for at once).  The next block's tiles are fetched as soon as
+// evenly), channel_block_kernel with the solve in place of its one-wave inverse 76 → 83 (79 with its loads asked for at once, less with its keys kept in LDS).  The next block's tiles are fetched as soon as
 // their registers are free and without a condition (the last block fetches itself again), so they land during the products; the compiler
 // still waits for all of them at the end of a block, where some change registers.  Sums that a block adds up are kept apart until they are complete: the state's error against 64 bits stays
 // below that of the walk before (2.7e-7 against 2.9e-7 of its norm).
@@ -1432,7 +1454,7 @@ void launch_gm_channel_scan(const float* q, int64_t q_stride, const float* k, in
 #undef GM_STEP
   if (!blocks) return;
   const int wide = D % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && z_stride % 4 == 0 && al16(q) && al16(k) && al16(z) && al16(bias);
-  GM_BF16(z_bf16, Z, hipLaunchKernelGGL((wide && D % 16 == 0 ? channel_block_kernel<Z, true> : channel_block_kernel<Z, false>), dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride,
+  GM_BF16(z_bf16, Z, hipLaunchKernelGGL((!wide || D % 16 ? channel_block_kernel<Z, false, 0> : D <= 128 ? channel_block_kernel<Z, true, 8> : channel_block_kernel<Z, true, 0>), dim3(num_tiles, H), dim3(NT), 0, stream, q, q_stride, k, k_stride, v, v_stride,
                                         (ChannelArgs<Z>{(const Z*)z, z_stride, rate, bias}), weight, qsl, state_slots, counts, tile_seq,
                                         tile_q0, num_tiles, H, G, D, Dv, wide, first_row, ws));
   delta_walk(state, positions, qsl, state_slots, counts, seqs, num_tiles, H, D, Dv, first_row, ws, out, stream);
