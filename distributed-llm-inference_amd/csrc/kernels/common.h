@@ -97,6 +97,14 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// What the lanes of a wave wrote to LDS before it is what they read after it.  The hardware keeps a wave's LDS accesses in order anyway (no instruction
+// comes of this); the compiler, which knows one lane only, need not.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Block-wide sum for blockDim.x = NT (multiple of 64).  `red` is NT/64 floats of LDS.
 template <int NT>
 __device__ __forceinline__ float block_sum(float v, float* red) {

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
                                                          int* __restrict__ sorted_ids, int* __restrict__ tile_expert,
                                                          int* __restrict__ meta, int capacity_rows, int tile_rows, int n_col_blocks, int nk,
                                                          int* __restrict__ pos_of) {
-  static_assert(MOE_MAX_E <= 64, "a lane for every expert, six bits of its number");
+  static_assert(MOE_MAX_E == 64, "a lane for every expert, six bits of its number");
   constexpr int HELD = 8;                                  // 64 pairs each: runs of up to 512 pairs are looked at once
   const int BM = tile_rows;                               // row tile of the GEMM that consumes the alignment (32, 64, 128 or 256)
   __shared__ int wave_cnt[16][MOE_MAX_E], off[MOE_MAX_E + 1], cnt[MOE_MAX_E];
@@ -124,12 +124,14 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
       same_all[j] = __popc(lo) + __popc(hi);
     }
   };
-  wave_cnt[wave][lane] = 0;                                // (a wave's row is its own until the barrier: LDS keeps its order)
+  wave_cnt[wave][lane] = 0;                                // (a wave's row is its own until the barrier)
   for (int at = begin; at < end; at += 64 * HELD) {
     look(at);
 #pragma unroll
-    for (int j = 0; j < HELD; ++j)
+    for (int j = 0; j < HELD; ++j) {
+      wave_lds_order();                                    // the expert's last count may be another lane's
       if (at + 64 * j < end && held[j] >= 0 && rank[j] == 0) wave_cnt[wave][held[j]] += same_all[j];
+    }
   }
   __syncthreads();
   if (wave == 0) {                                         // per expert: the waves' counts → places before them, the sum
@@ -178,10 +180,12 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
     if (run > 64 * HELD) look(at);
 #pragma unroll
     for (int j = 0; j < HELD; ++j) {
-      const int i = at + 64 * j + lane, e = held[j];
-      if (i < end && e >= 0) {
-        const int first = wave_cnt[wave][e], to = first + rank[j];
-        if (rank[j] == 0) wave_cnt[wave][e] = first + same_all[j];
+      const int i = at + 64 * j + lane, e = held[j];       // (e < 0 from the run's end on)
+      const int first = e >= 0 ? wave_cnt[wave][e] : 0, to = first + rank[j];
+      wave_lds_order();                                    // all lanes have read before the first of an expert moves its place on …
+      if (e >= 0 && rank[j] == 0) wave_cnt[wave][e] = first + same_all[j];
+      wave_lds_order();                                    // … and the next pairs' lanes read after it
+      if (e >= 0) {
         sorted_ids[to] = i;
         if (n_col_blocks > 0) pos_of[i] = to;
       }
