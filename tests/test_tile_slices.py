@@ -14,6 +14,26 @@ def test_sizes_on_both_sides_of_the_line():
                                    (512, 4096, 14336 + 32), (512, 4000, 14336), (512, 0, 14336), (0, 4096, 14336), (512, 7168, 8192), (512, 7168, 4096, True)))
 
 
+def test_short_products_keep_their_last_round_whole():
+    """K timed with the last round cut and whole, on both sides of the line."""
+    assert not any(ops.swiglu_tail_cut(k) for k in (512, 1024, 2048, 2560))
+    assert all(ops.swiglu_tail_cut(k) for k in (3072, 4096, 8192))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [512, 3072])
+def test_last_round_of_the_untuned_gate_up(monkeypatch, k):
+    """300 tiles: a whole round and 44 more, whole behind a short K, in slices behind a long one.  Against fp32 products; and the call is asked for as the line says."""
+    asked, op = [], ops.hip().dense_gemm256
+    monkeypatch.setattr(ops.hip(), "dense_gemm256", lambda x, w, *a: (asked.append(a[-1]), op(x, w, *a))[1], raising=False)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(730, k, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(25600, k, generator=g, device="cuda") * k ** -0.5).bfloat16()
+    got, y = ops.linear_swiglu(x, w).float(), x.float() @ w.float().t()
+    torch.testing.assert_close(got, torch.nn.functional.silu(y[:, :12800]) * y[:, 12800:], rtol=2 ** -7, atol=2e-2)      # as below
+    assert asked == [k >= 3072]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,swiglu", [(257, 1024, 14336, False), (1025, 1024, 14336, False), (520, 4096, 14336, False), (300, 7168, 8192, True),
                                           (769, 3584, 8192, True)])
