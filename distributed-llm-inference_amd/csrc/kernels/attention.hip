@@ -440,6 +440,7 @@ __device__ __forceinline__ void value_fragments(const char* vb, int n, int off0,
   }
 }
 
+static constexpr int PREFILL_UNITS = 256;                      // workgroups of two groups that run at once: one a compute unit
 template <bool KV8, int GROUPS, int NPG> struct PrefillShape {
   static constexpr int PAGE_BYTES = PAGE_ELEMS * (KV8 ? 1 : 2);
   static constexpr int STAGE = NPG * 2 * PAGE_BYTES;        // K and V of a turn's pages
@@ -838,24 +839,31 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
 // instructions, decode rows by the cache's bytes, so a compute unit that holds both does one while the other waits; one after the other, 96 e4m3 rows of
 // up to 1500 tokens and two chunks of up to 1024 behind up to 1024 (32/8 heads) take 67 µs, here 49, and in bf16 99 → 65.  (Two streams or two branches of a
 // graph reach part of it: their launches compete for the units as they come, a captured branch costs 5 µs where the step is small, an event on an eager
-// stream 10 and 30 to 55 of the host.  In 88 captured steps this launch takes 0.86 of the branches' time on average, 0.60 to 1.04.)
+// stream 10 and 30 to 55 of the host.)
 // Three workgroups share a unit (145 registers, 48 KB of LDS).  Octets of workgroups, one for each XCD so that a head's pages stay in one L2:
-//   * `period` = 3: every third octet is one of decode rows, as long as there are both, then what is left.  For many tiles, which would fill all units and
+//   * more than 512 tiles: every third octet is one of decode rows, as long as there are both, then what is left.  So many tiles would fill all units and
 //     leave the decode rows for the end (96 bf16 rows, one fresh prompt of 3500 tokens, 880 tiles: prompts first 152 µs, every second 185, every third 138,
 //     every fourth 152; e4m3 rows, four of 1000 behind 500, 672 tiles 68 / 78 / 58 / 65);
-//   * 0: all prompts first, whose longest chain the launch has to wait for anyway, where they leave a third of the units' room (e4m3, 504 tiles: 85 / 115 /
-//     94 / 91; 200 tiles 50 / 47 / 49 / 48).
-// GROUPS = 2: tiles by two page groups and decode items by as many waves as in their own launch
-// (both give the same bits), a workgroup a compute unit.
+//   * up to 512: all prompts first, whose longest chain the launch has to wait for anyway, where they leave a third of the units' room (e4m3, 504 tiles:
+//     85 / 115 / 94 / 91; 200 tiles 50 / 47 / 49 / 48).
+// A captured launch deals the step's own tiles and rows, which the device knows, not the bounds of its grid: by the bounds, 256 tiles among 2304 had decode rows
+// between them, which left units with two of the longest tiles beside units without any (e4m3, 16 rows and 1000 tokens behind 6000: branches 245 µs, dealt
+// by bounds 258, by what there is 205).
+// GROUPS = 2: tiles by two page groups and decode items by as many waves as in their own launch (both give the same bits), a workgroup a compute unit.
 template <bool KV8, bool WL, int GROUPS>
 __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void paged_mixed_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ query_start_loc,
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, uint16_t* __restrict__ out, int64_t out_stride,
     float* __restrict__ part_o, float* __restrict__ part_ml, int Hq, int Hkv, int num_tiles, int items, int num_splits, float scale_log2, float v_scale,
-    const float* __restrict__ kv_scales, const int4* __restrict__ work, const int* __restrict__ counts, int tiles_on_device, int period) {
+    const float* __restrict__ kv_scales, const int4* __restrict__ work, const int* __restrict__ counts, int on_device) {
   constexpr int NPG = GROUPS == 2 && KV8 ? 2 : 1, NW = GROUPS == 2 && !KV8 ? 8 : 4, IPW = 4 * GROUPS / NW;      // IPW: decode items a workgroup
   __shared__ __attribute__((aligned(16))) char smem[PrefillShape<KV8, GROUPS, NPG>::LDS];      // (a decode item of up to 8 heads a group takes 17 KB of it, 34 by eight waves)
+  if (on_device) {                                          // the launched numbers are bounds
+    num_tiles = min(num_tiles, counts[2]);
+    if (WL) items = min(items, counts[0]);
+  }
+  const int period = num_tiles * Hkv > 2 * PREFILL_UNITS ? 3 : 0;
   const int octets = (num_tiles * Hkv + 7) >> 3, rows = ((items + IPW - 1) / IPW * Hkv + 7) >> 3;
   const int octet = (int)blockIdx.x >> 3, in = (int)blockIdx.x & 7;
   const int turns = period > 1 ? min(rows, octets / (period - 1)) : 0;
@@ -868,7 +876,6 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void paged_mixed
     row = octet - octets;
   }
   if (row < 0) {
-    if (tiles_on_device) num_tiles = counts[2];             // (the launched number is a bound)
     prefill_tile<KV8, GROUPS, NPG>(8 * tile + in, smem, q, q_stride, k_cache, v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq,
                                    tile_q0, out, out_stride, Hq, Hkv, num_tiles, scale_log2, v_scale, kv_scales, 0x7fffffff);
     return;
@@ -948,7 +955,6 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
                        out_stride, Hq, 1, kv_fp8 ? v_scale : 1.f, kv_fp8 ? kv_scales : nullptr, Hkv, (const int4*)red, counts);
 }
 
-static constexpr int PREFILL_UNITS = 256;                      // workgroups of two groups that run at once: one a compute unit
 // Two groups where a compute unit gets one workgroup: a tile's pages are a serial chain of 0.7 µs each, and what the chip
 // has no second tile for, a second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: prompts of 1000 tokens (256
 // workgroups) 32.3 / 26.9, of 2000 with 8/1 heads (250) 57.8 / 45.7, 8 × 128 tokens behind 1000 (256) 37.9 / 34.5, 32 × 16 behind 300 15.0 / 15.3.
@@ -1035,12 +1041,11 @@ void launch_paged_mixed(const void* q, int64_t q_stride, const void* k_cache, co
   if (octets == 0) return;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-  const int period = (int64_t)num_tiles * Hkv > 2 * PREFILL_UNITS ? 3 : 0;
 #define DLI_MIXED_GO(KV8_, WL_, G_)                                                                                                      \
   hipLaunchKernelGGL((paged_mixed_kernel<KV8_, WL_, G_>), dim3((unsigned)(8 * octets)), dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, \
                      v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, part_o, part_ml, \
                      Hq, Hkv, num_tiles, items, wl ? 1 : num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work,  \
-                     counts, tiles_on_device ? 1 : 0, period)
+                     counts, tiles_on_device ? 1 : 0)
 #define DLI_MIXED_WL(KV8_, G_) do { if (wl) DLI_MIXED_GO(KV8_, true, G_); else DLI_MIXED_GO(KV8_, false, G_); } while (0)
   if (groups == 2) { if (kv_fp8) DLI_MIXED_WL(true, 2); else DLI_MIXED_WL(false, 2); }
   else { if (kv_fp8) DLI_MIXED_WL(true, 1); else DLI_MIXED_WL(false, 1); }

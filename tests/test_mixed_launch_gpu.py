@@ -15,7 +15,7 @@ def _i32(a):
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).cuda()
 
 
-def _step(heads, kv_heads, dtype, decode, prompts, listed=True, bounds=False, seed=3):
+def _step(heads, kv_heads, dtype, decode, prompts, listed=True, bounds=False, seed=3, extra=40, items=700):
     lens = np.array(decode + [length for length, _ in prompts])
     new = np.array([1] * len(decode) + [n for _, n in prompts])
     pages = (lens + 31) // 32
@@ -30,12 +30,11 @@ def _step(heads, kv_heads, dtype, decode, prompts, listed=True, bounds=False, se
     meta = ops.AttnMetadata(len(decode), len(prompts), int(new.sum()), None, None, _i32(bt), _i32(lens), _i32(np.concatenate([[0], np.cumsum(new)])),
                             max_seq_len=int(lens.max()), prefill_tile_seq=_i32(ts), prefill_tile_q0=_i32(t0), num_prefill_tiles=len(ts))
     if listed:
-        ops.attach_decode_worklist(meta, lens[:len(decode)], heads, kv_heads, "cuda", launch_items=700 if bounds else 0)
+        ops.attach_decode_worklist(meta, lens[:len(decode)], heads, kv_heads, "cuda", launch_items=items if bounds else 0)
     else:
         meta.decode_splits = 3
         meta.decode_workspace = torch.empty(len(decode) * heads * 3 * 130, dtype=torch.float32, device="cuda")
     if bounds:                                              # what a captured step launches: more tiles than there are, their number on the device
-        extra = 40
         meta.prefill_tile_seq, meta.prefill_tile_q0 = _i32(np.concatenate([ts, np.zeros(extra)])), _i32(np.concatenate([t0, np.zeros(extra)]))
         meta.num_prefill_tiles, meta.counts_on_device = len(ts) + extra, True
     qkv = torch.randn(int(new.sum()), (heads + 2 * kv_heads) * 128, generator=g, device="cuda", dtype=torch.bfloat16)
@@ -71,6 +70,28 @@ def test_mixed_launch_matches_reference(monkeypatch, name, dtype, form):
     got = ops.paged_attention(qkv, kc, vc, meta, heads, kv_heads, 128, 0.088, out=out).float()
     want = ref.paged_attention_ref(qkv[:, :heads * 128].reshape(T, heads, 128), kc, vc, meta.block_tables, meta.seq_lens, meta.query_start_loc, 0.088).float()
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)      # (both round to bf16; the weights are bf16 in the products)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("extra,items", [(0, 100), (60, 2000), (700, 100), (700, 2000)])
+@pytest.mark.parametrize("empty", ["", "rows", "tiles", "both"])
+def test_bounds_far_from_the_step(dtype, extra, items, empty):
+    """A captured launch deals the tiles and rows that there are, by the numbers on the device: grids of many times as many, steps without rows or tiles."""
+    decode = ROWS * 2
+    kc, vc, meta, qkv = _step(32, 8, dtype, decode, [(300, 290), (90, 17)], True, True, extra=extra, items=items)
+    T, nd = qkv.shape[0], len(decode)
+    want = ref.paged_attention_ref(qkv[:, :4096].reshape(T, 32, 128), kc, vc, meta.block_tables, meta.seq_lens, meta.query_start_loc, 0.088).float()
+    if empty in ("rows", "both"):
+        meta.counts[:2] = 0
+    if empty in ("tiles", "both"):
+        meta.counts[2] = 0
+    out = torch.full((T, 4096), float("nan"), dtype=torch.bfloat16, device="cuda")
+    got = ops.paged_attention(qkv, kc, vc, meta, 32, 8, 128, 0.088, out=out).float()
+    for part, left_out in ((slice(0, nd), empty in ("rows", "both")), (slice(nd, T), empty in ("tiles", "both"))):
+        if left_out:
+            assert bool(torch.isnan(got[part]).all())
+        else:
+            torch.testing.assert_close(got[part], want[part], rtol=2e-2, atol=2e-2)      # as above
 
 
 def test_mixed_launch_replayed_from_a_graph():
