@@ -325,7 +325,9 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
   const int qh = blockIdx.y, d = threadIdx.x, lane = threadIdx.x & 63;
   if (kv_scales != nullptr) v_scale = kv_scales[Hkv + qh / (Hq / Hkv)];
   // 64 partials at a time, a lane each: their (m, l) arrive together and the rows' loads do not wait for one another.  (One after the
-  // other — a load's latency per partial, twice — five partials took 4.5 µs.)
+  // other — a load's latency per partial, twice — five partials took 4.5 µs.)  The rows come 8 at a time, 32 where there are many: behind one row of 16000 tokens
+  // of one key head, in 126 ranges, the whole call 19.3 → 15.6 µs (beside a prompt's chunk of 400 tokens, which cannot hide it, 48.2 → 45.5); up to 16
+  // ranges 24 loads too many cost up to 0.4.
   float M = NEG_BIG, num = 0.f, den = 0.f;
   for (int s0 = 0; s0 < n; s0 += 64) {
     const int k = min(n - s0, 64);
@@ -337,13 +339,18 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(const float* __restr
     den = den * old + wave_sum(f * ml[1]);
     num *= old;
     M = Mn;
-    for (int s = 0; s < k; s += 8) {
-      float x[8];
+    auto add = [&](auto rows, int s) __attribute__((always_inline)) {
+      constexpr int N = decltype(rows)::value;
+      float x[N];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = part_o[(slot0 + (int64_t)min(s + j, k - 1) * Hq) * HD + d];
+      for (int j = 0; j < N; ++j) x[j] = part_o[(slot0 + (int64_t)min(s + j, k - 1) * Hq) * HD + d];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) num += s + j < k ? __shfl(f, s + j, 64) * x[j] : 0.f;
-    }
+      for (int j = 0; j < N; ++j) num += s + j < k ? __shfl(f, s + j, 64) * x[j] : 0.f;
+    };
+    if (k <= 16)
+      for (int s = 0; s < k; s += 8) add(std::integral_constant<int, 8>{}, s);
+    else
+      for (int s = 0; s < k; s += 32) add(std::integral_constant<int, 32>{}, s);
   }
   const float r = den > 0.f ? v_scale / den : 0.f;
   out[(int64_t)seq * out_stride + qh * HD + d] = f2bf(num * r);
