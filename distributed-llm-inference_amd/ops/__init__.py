@@ -341,19 +341,25 @@ def _stream_ok(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor
 def tile_slices(m: int, n: int, k: int, swiglu: bool = False) -> int:
     """K slices with which the own 256² tiles (``csrc/kernels/gemm256.hip``) beat the library GEMM (and its activation pass) where the start-up measurement
     says nothing; 0: the library.  Rows past 256 whose tiles are at most half as many as the 256 compute units, long K: the library leaves units idle, the
-    slices fill them.  µs, library / sliced:
+    slices fill them.  2700 sizes of 257 to 4200 rows, 256 to 18432 columns, K up to 28672, weights that no cache holds; sliced over library:
 
-    * plain, K from 14336 on (4096 × 14336 at 257 rows 81 / 61, 512 93 / 65, 768 109 / 90, 1024 132 / 106, 2048 207 / 180; 8192 × 28672 at 512 313 / 188;
-      2048 × 28672 at 1024 277 / 100), but not at 8192 (8192 × 8192 at 512 82 / 72, at 768 98 / 100, 4096 × 8192 68 / 69 at 1024) or 4096 (1.15 – 1.4);
-    * with SwiGLU, which saves the activation pass too, from 8192 on (7168 × 8192 at 257 72 / 60, 512 83 / 65, 1024 117 / 106; 3584 × 8192 at 1024 70 / 62; more columns
-      are not measured), but not at 4096 (7168 × 4096 1.0 – 1.12);
-    * where tiles and slices fill 210 units (4096 × 14336 with 32 to 128 tiles; 96 tiles in two slices leave a quarter idle: 8192 × 28672 at 700 rows
-      285 / 296), or half of them with eight slices, plain (2048 × 28672 at 512 184 / 88, 1024 × 14336 at 1024 53 / 50, but 45 / 46 with 12 tiles)."""
-    if m <= 256 or n < 256 or n % 256 or k % 64 or k < (8192 if swiglu else 14336) or (swiglu and n > 7168):
+    * plain, K from 12288 on: 12288 – 14335 0.80 on average, from 14336 0.68; shorter sums lose at some sizes (10240 – 12287 0.91, up to 1.14; 8192 – 9215
+      1.00, up to 1.28).  4096 × 12288 at 512 rows 82 / 61 µs, 8192 × 12288 at 1024 171 / 158, 4096 × 14336 at 512 93 / 65, 2560 × 20480 at 300 145 / 64;
+    * with SwiGLU, which saves the activation pass too, from 7168 on: 7168 – 8192 0.88 (8 of 470 sizes 1.02 to 1.06), longer 0.71; below, 6144 – 7167 1.00,
+      up to 1.25, 5120 – 6143 1.01.  7168 × 8192 at 512 rows 79 / 70, 7168 × 12288 at 512 120 / 90;
+    * where tiles and slices fill 210 units (96 tiles in two slices leave a quarter idle: 8192 × 28672 at 700 rows 285 / 296), or half of them with eight
+      slices, plain (2048 × 28672 at 512 184 / 88, 1024 × 14336 at 1024 53 / 50, but 45 / 46 with 12 tiles);
+    * not where wide weights meet a half empty row tile, whose products are as long as a full one's: two slices (rows up to 0.6 of their tiles: plain 0.97, up to
+      1.20, SwiGLU 0.98, up to 1.15; to 0.8 up to 1.10; above at most 1.01) or three (to 0.6 up to 1.12, above at most 0.95).  16384 × 16384
+      at 257 rows 178 / 213, at 512 227 / 221; with SwiGLU 10240 × 8192 at 257 69 / 78, at 512 97 / 87.  Four and more win at any number of rows."""
+    if m <= 256 or n < 256 or n % 256 or k % 64 or k < (7168 if swiglu else 12288):
         return 0
-    tiles = (m + 255) // 256 * (n // 256)
+    row_tiles = (m + 255) // 256
+    tiles = row_tiles * (n // 256)
     s = min(8, 256 // tiles)
-    return s if s >= 2 and (tiles * s >= 210 or (not swiglu and s == 8 and tiles >= 16)) else 0
+    if s < 2 or (s <= 3 and m < (0.8 if s == 2 else 0.6) * 256 * row_tiles):
+        return 0
+    return s if tiles * s >= 210 or (not swiglu and s == 8 and tiles >= 16) else 0
 
 
 def _tile_slices(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False) -> int:

@@ -14,6 +14,22 @@ def test_sizes_on_both_sides_of_the_line():
                                    (512, 4096, 14336 + 32), (512, 4000, 14336), (512, 0, 14336), (0, 4096, 14336), (512, 7168, 8192), (512, 7168, 4096, True)))
 
 
+def test_wide_weights_and_half_empty_row_tiles():
+    """Two or three slices lose to the library where the last row tile is nearly empty (16384 × 16384 at 257 rows 178 µs / 213), four do not."""
+    f = ops.tile_slices
+    assert not any(f(*s) for s in ((257, 16384, 16384), (400, 16384, 16384), (310, 13824, 18240), (569, 10496, 13504), (257, 10240, 16384), (300, 9728, 15616)))
+    assert not any(f(*s, True) for s in ((257, 16384, 7680), (315, 15616, 11648), (257, 10240, 8576)))
+    assert [f(*s) for s in ((512, 16384, 16384), (1024, 8192, 14336), (330, 10240, 14336), (257, 8192, 14336), (257, 7168, 18432))] == [2, 2, 3, 4, 4]
+    assert [f(*s, True) for s in ((512, 16384, 8192), (330, 10240, 8576), (257, 8192, 8192))] == [2, 3, 4]
+
+
+def test_long_enough_sums():
+    """K on both sides of the lines, at sizes that are no preset's: below them the library wins at some sizes."""
+    f = ops.tile_slices
+    assert [f(512, 4096, k) > 0 for k in (9216, 11008, 12224, 12288, 13824)] == [False, False, False, True, True]
+    assert [f(512, 5120, k, True) > 0 for k in (5120, 6144, 7104, 7168, 9216)] == [False, False, False, True, True]
+
+
 def test_short_products_keep_their_last_round_whole():
     """K timed with the last round cut and whole, on both sides of the line."""
     assert not any(ops.swiglu_tail_cut(k) for k in (512, 1024, 2048, 2560))
