@@ -346,13 +346,14 @@ def tile_slices(m: int, n: int, k: int, swiglu: bool = False) -> int:
     * plain, K from 12288 on: 12288 – 14335 0.80 on average, from 14336 0.68; shorter sums lose at some sizes (10240 – 12287 0.91, up to 1.14; 8192 – 9215
       1.00, up to 1.28).  4096 × 12288 at 512 rows 82 / 61 µs, 8192 × 12288 at 1024 171 / 158, 4096 × 14336 at 512 93 / 65, 2560 × 20480 at 300 145 / 64;
     * with SwiGLU, which saves the activation pass too, from 7168 on: 7168 – 8192 0.88 (8 of 470 sizes 1.02 to 1.06), longer 0.71; below, 6144 – 7167 1.00,
-      up to 1.25, 5120 – 6143 1.01.  7168 × 8192 at 512 rows 79 / 70, 7168 × 12288 at 512 120 / 90;
+      up to 1.25, 5120 – 6143 1.01.  More columns than 7168 from K above 8192 on (8192 × 8192 0.94 – 1.05, 16384 × 8192 at 512 rows 1.05, but
+      16384 × 16384 245 / 213).  7168 × 8192 at 512 rows 79 / 70, 7168 × 12288 at 512 120 / 90;
     * where tiles and slices fill 210 units (96 tiles in two slices leave a quarter idle: 8192 × 28672 at 700 rows 285 / 296), or half of them with eight
       slices, plain (2048 × 28672 at 512 184 / 88, 1024 × 14336 at 1024 53 / 50, but 45 / 46 with 12 tiles);
     * not where wide weights meet a half empty row tile, whose products are as long as a full one's: two slices (rows up to 0.6 of their tiles: plain 0.97, up to
       1.20, SwiGLU 0.98, up to 1.15; to 0.8 up to 1.10; above at most 1.01) or three (to 0.6 up to 1.12, above at most 0.95).  16384 × 16384
       at 257 rows 178 / 213, at 512 227 / 221; with SwiGLU 10240 × 8192 at 257 69 / 78, at 512 97 / 87.  Four and more win at any number of rows."""
-    if m <= 256 or n < 256 or n % 256 or k % 64 or k < (7168 if swiglu else 12288):
+    if m <= 256 or n < 256 or n % 256 or k % 64 or k < (7168 if swiglu else 12288) or (swiglu and n > 7168 and k <= 8192):
         return 0
     row_tiles = (m + 255) // 256
     tiles = row_tiles * (n // 256)

@@ -20,7 +20,8 @@ def test_wide_weights_and_half_empty_row_tiles():
     assert not any(f(*s) for s in ((257, 16384, 16384), (400, 16384, 16384), (310, 13824, 18240), (569, 10496, 13504), (257, 10240, 16384), (300, 9728, 15616)))
     assert not any(f(*s, True) for s in ((257, 16384, 7680), (315, 15616, 11648), (257, 10240, 8576)))
     assert [f(*s) for s in ((512, 16384, 16384), (1024, 8192, 14336), (330, 10240, 14336), (257, 8192, 14336), (257, 7168, 18432))] == [2, 2, 3, 4, 4]
-    assert [f(*s, True) for s in ((512, 16384, 8192), (330, 10240, 8576), (257, 8192, 8192))] == [2, 3, 4]
+    assert [f(*s, True) for s in ((512, 16384, 16384), (330, 10240, 8576), (257, 8192, 8576), (257, 7168, 8192))] == [2, 3, 4, 4]
+    assert not any(f(*s, True) for s in ((345, 8192, 8192), (512, 16384, 8192)))       # (at this K the wide ones are no faster however full)
 
 
 def test_long_enough_sums():
