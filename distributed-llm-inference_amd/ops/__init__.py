@@ -364,7 +364,7 @@ def tile_slices(m: int, n: int, k: int, swiglu: bool = False) -> int:
 
 
 def _tile_slices(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False) -> int:
-    if x.dim() != 2 or weight.dim() != 2:
+    if x.dim() != 2 or weight.dim() != 2 or (swiglu and not GEMM256_SWIGLU):
         return 0
     s = tile_slices(x.shape[0], *weight.shape, swiglu)
     return s if s and _stream_operands_ok(x, weight, out) and _tile_operand_ok(x, weight) else 0

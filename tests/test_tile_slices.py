@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from dli_amd import ops
+from test_dispatch import _Recorder
 
 
 def test_sizes_on_both_sides_of_the_line():
@@ -29,6 +30,23 @@ def test_long_enough_sums():
     f = ops.tile_slices
     assert [f(512, 4096, k) > 0 for k in (9216, 11008, 12224, 12288, 13824)] == [False, False, False, True, True]
     assert [f(512, 5120, k, True) > 0 for k in (5120, 6144, 7104, 7168, 9216)] == [False, False, False, True, True]
+
+
+def test_gate_up_goes_to_the_library_where_the_switch_says_so(monkeypatch):
+    """DLI_NO_GEMM256_SWIGLU=1 names every untuned gate/up product on the own 256² tiles, the sliced ones too; down projections are none of its business."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    monkeypatch.setattr(ops, "hip", _Recorder)
+    monkeypatch.setattr(ops, "_plain", lambda *t: True)
+
+    def route(f, m, n, k):
+        with FakeTensorMode(), pytest.raises(RuntimeError) as e:
+            f(*(torch.empty(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n)))
+        return str(e.value)
+    sizes = ((512, 7168, 8192), (300, 7168, 12288), (700, 28672, 4096))
+    assert [route(ops.linear_swiglu, *s) for s in sizes] == ["dense_gemm256"] * 3
+    monkeypatch.setattr(ops, "GEMM256_SWIGLU", False)
+    assert [route(ops.linear_swiglu, *s) for s in sizes] == ["silu_and_mul"] * 3
+    assert route(ops.linear, 512, 4096, 14336) == "dense_gemm256"
 
 
 def test_short_products_keep_their_last_round_whole():
