@@ -857,7 +857,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void paged_prefill_kernel(
 // between them, which left units with two of the longest tiles beside units without any (e4m3, 16 rows and 1000 tokens behind 6000: branches 245 µs, dealt
 // by bounds 258, by what there is 205).
 // GROUPS = 2: tiles by two page groups and decode items by as many waves as in their own launch (both give the same bits), a workgroup a compute unit.
-template <bool KV8, bool WL, int GROUPS>
+template <bool KV8, bool WL, int GROUPS, bool NT>
 __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void paged_mixed_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ query_start_loc,
@@ -891,7 +891,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void paged_mixed
   const int id = 8 * row + in, group = id / Hkv, kvh = id - group * Hkv, item = group * IPW + sub;
   if (item >= items) return;                                // the last octet, the last item's neighbour
   const int seq = WL ? item : item / num_splits, split = WL ? 0 : item - seq * num_splits;
-  decode_item<KV8, WL, NW, true>((int)threadIdx.x - 256 * sub, kvh, seq, split, reinterpret_cast<float*>(smem + sub * (int)(sizeof(smem) / 2)), q, q_stride,
+  decode_item<KV8, WL, NW, NT>((int)threadIdx.x - 256 * sub, kvh, seq, split, reinterpret_cast<float*>(smem + sub * (int)(sizeof(smem) / 2)), q, q_stride,
                                  k_cache, v_cache, block_tables, max_blocks, seq_lens, out, out_stride, part_o, part_ml, Hq, Hkv, num_splits,
                                  scale_log2, v_scale, kv_scales, work, counts);
 }
@@ -1048,15 +1048,17 @@ void launch_paged_mixed(const void* q, int64_t q_stride, const void* k_cache, co
   if (octets == 0) return;
   if (kv_scales != nullptr) k_scale = v_scale = 1.f;
   const float scale_log2 = scale * 1.4426950408889634f * (kv_fp8 ? k_scale : 1.f);
-#define DLI_MIXED_GO(KV8_, WL_, G_)                                                                                                      \
-  hipLaunchKernelGGL((paged_mixed_kernel<KV8_, WL_, G_>), dim3((unsigned)(8 * octets)), dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride, k_cache, \
-                     v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, part_o, part_ml, \
+#define DLI_MIXED_GO(KV8_, WL_, G_, NT_)                                                                                                 \
+  hipLaunchKernelGGL((paged_mixed_kernel<KV8_, WL_, G_, NT_>), dim3((unsigned)(8 * octets)), dim3(256 * G_), 0, stream, (const uint16_t*)q, q_stride,  \
+                     k_cache, v_cache, block_tables, max_blocks, seq_lens, query_start_loc, tile_seq, tile_q0, (uint16_t*)out, out_stride, part_o, part_ml, \
                      Hq, Hkv, num_tiles, items, wl ? 1 : num_splits, scale_log2, KV8_ ? v_scale : 1.f, KV8_ ? kv_scales : nullptr, (const int4*)work,  \
                      counts, tiles_on_device ? 1 : 0)
-#define DLI_MIXED_WL(KV8_, G_) do { if (wl) DLI_MIXED_GO(KV8_, true, G_); else DLI_MIXED_GO(KV8_, false, G_); } while (0)
+#define DLI_MIXED_NT(KV8_, WL_, G_) do { if (g_decode_nt) DLI_MIXED_GO(KV8_, WL_, G_, true); else DLI_MIXED_GO(KV8_, WL_, G_, false); } while (0)
+#define DLI_MIXED_WL(KV8_, G_) do { if (wl) DLI_MIXED_NT(KV8_, true, G_); else DLI_MIXED_NT(KV8_, false, G_); } while (0)
   if (groups == 2) { if (kv_fp8) DLI_MIXED_WL(true, 2); else DLI_MIXED_WL(false, 2); }
   else { if (kv_fp8) DLI_MIXED_WL(true, 1); else DLI_MIXED_WL(false, 1); }
 #undef DLI_MIXED_WL
+#undef DLI_MIXED_NT
 #undef DLI_MIXED_GO
   if (wl ? reds > 0 : num_splits > 1)
     hipLaunchKernelGGL(decode_reduce_kernel, dim3(wl ? reds : num_seqs, Hq), dim3(128), 0, stream, part_o, part_ml, (uint16_t*)out,
