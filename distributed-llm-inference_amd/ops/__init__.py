@@ -313,10 +313,11 @@ def stream_rows_ok(m: int, n: int, k: int, swiglu: bool = False) -> bool:
 
 def _plain(*tensors: torch.Tensor) -> bool:
     """Ordinary tensors that nothing but the call looks at: no fake or other subclass, no trace, vmap, functional or forward-mode transform,
-    no gradient.  A kernel that takes addresses sees through all of these."""
+    no gradient, no autocast to another type than the bf16 of these paths.  A kernel that takes addresses sees through all of these."""
     return (not torch.compiler.is_compiling() and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._get_tracing_state() is None and torch.autograd.forward_ad._current_level < 0
+            and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 

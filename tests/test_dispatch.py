@@ -171,6 +171,27 @@ def test_plain_tensors():
     assert seen == [False] * 5 and ops._plain(t)
 
 
+@pytest.mark.parametrize("dtype,plain", [(torch.float16, False), (torch.bfloat16, True)])
+def test_autocast_to_another_type_is_the_librarys(dtype, plain):
+    """``torch.nn.functional.linear`` casts its operands there and returns that type; a kernel would return bf16."""
+    before = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    try:
+        torch.set_autocast_enabled("cuda", True)
+        torch.set_autocast_dtype("cuda", dtype)
+        assert ops._plain(torch.ones(2, 2, dtype=torch.bfloat16)) is plain
+    finally:
+        torch.set_autocast_enabled("cuda", before[0])
+        torch.set_autocast_dtype("cuda", before[1])
+
+
+@pytest.mark.gpu
+def test_long_sums_under_autocast():
+    x, w = torch.ones(512, 14336, device="cuda", dtype=torch.bfloat16), torch.ones(4096, 14336, device="cuda", dtype=torch.bfloat16) / 64
+    assert ops.tile_slices(512, 4096, 14336) and ops.linear(x, w).dtype == torch.bfloat16
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ops.linear(x, w).dtype == torch.nn.functional.linear(x, w).dtype == torch.float16
+
+
 def test_short_decode_rows_stay_whole():
     """Sizes timed with rows cut into ranges and whole: (rows, heads, pages of the longest) on both sides of the line."""
     cut = lambda n, heads, pages: len(ops.build_decode_work(np.full(n, 32 * pages), heads)[1]) > 0
