@@ -567,11 +567,10 @@ def rope_and_cache(qkv: torch.Tensor, positions: torch.Tensor, cos_sin: Optional
                                head_dim, k_scale, v_scale)
 
 
-# Captured mixed steps: prefill tiles next to the decode rows on a side stream (same-box serving A/B: TPOT p50 39.4 → 38.4 ms,
-# profiles/bench_r3aj_concurrent_attention_{0,1}.json).  DLI_CONCURRENT_ATTN=0: one after the other.
+# Mixed steps: prompt tiles and decode rows in one launch (csrc/kernels/attention.hip, paged_mixed_kernel).  DLI_ATTN_ONE_LAUNCH=0: launches of their own,
+# captured ones on two branches of the graph (DLI_CONCURRENT_ATTN=0, which turns both off: one after the other), eager ones on two streams where
+# ``attention_beside`` says so.
 CONCURRENT_ATTN = os.environ.get("DLI_CONCURRENT_ATTN", "1") != "0"
-# Mixed steps: prompt tiles and decode rows in one launch (csrc/kernels/attention.hip, paged_mixed_kernel).  DLI_ATTN_ONE_LAUNCH=0: launches of their own, on
-# two streams where ``attention_beside`` or a capture says so.
 ONE_LAUNCH_ATTN = CONCURRENT_ATTN and os.environ.get("DLI_ATTN_ONE_LAUNCH", "1") != "0"
 _ATTN_STREAMS: dict = {}
 
@@ -584,7 +583,9 @@ def _attn_stream(device):
 
 
 def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page_element_bytes: int) -> bool:
-    """Does an eager mixed step pay for a second stream?  Its events cost 30 to 55 µs of host time and, where the host keeps up, 10 of the GPU's; a captured
+    """Does an eager mixed step whose rows and tiles have launches of their own pay for a second stream?  (With DLI_ATTN_ONE_LAUNCH=0, or past the grid of one
+    launch.  Where the rule for one launch keeps them apart, the tiles take two page groups and the answer is no; so nothing else comes to the second stream by default.)
+    Its events cost 30 to 55 µs of host time and, where the host keeps up, 10 of the GPU's; a captured
     graph's branches cost neither.  And the two launches only run beside each other where their registers fit a compute unit together: prompts of one
     page group, not of two.  Then it pays from about 0.7 GB of cache pages on (rows × longest context), in bf16 from half of that where up to two
     prompt workgroups a unit leave room.  µs, beside / one after the other, 32/8 heads: 2 rows of up to 400 tokens and a prompt of 40 42.4 / 19.9; e4m3
@@ -592,8 +593,8 @@ def attention_beside(meta: AttnMetadata, num_heads: int, num_kv_heads: int, page
     1000 behind 500 105 / 94, 200 140 / 150; two groups, 160 of up to 2000 and one of 800 behind 300 159 / 165, 300 of up to 1500 and one of 200 behind
     500 203 / 198; 64/8 heads, 400 of up to 1500 and one of 1500 bf16 286 / 313, e4m3 178 / 204; 8/1 heads 0.41 to 0.97, but for 400 rows
     of up to 1500 with one prompt of 1500 in bf16, 81.9 after and 74.1 beside (more sizes: ``profiles/mixed_steps_eager.txt``).  Captured
-    steps, with the launch extents that the runner captures (``profiles/mixed_steps_captured.txt``, 88 sizes): branches take 0.95 of the time one after the
-    other on average, 0.74 to 1.12 but for 256 tokens of four fresh prompts (1.07 to 1.24), so all of them have branches."""
+    steps in launches of their own, with the launch extents that the runner captures (``profiles/mixed_steps_captured.txt``, 88 sizes): branches take 0.95 of
+    the time one after the other on average, 0.74 to 1.12 but for 256 tokens of four fresh prompts (1.07 to 1.24), so there all of them have branches."""
     longest = meta.max_seq_len or 1024                       # (0: not known)
     room = page_element_bytes == 2 and meta.num_prefill_tiles * num_kv_heads <= 512
     if meta.num_decode * longest * num_kv_heads * 256 * page_element_bytes < (350_000_000 if room else 700_000_000):
@@ -639,7 +640,7 @@ def paged_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         if (CONCURRENT_ATTN and meta.num_prefill_tiles > 0 and (meta.decode_items > 0 or meta.num_decode > 0)
                 and (torch.cuda.is_current_stream_capturing()
                      or attention_beside(meta, num_heads, num_kv_heads, k_cache.element_size()))):
-            # mixed step: the prefill tiles (MFMA / VALU-bound, a few hundred workgroups) run on a side stream next to the
+            # mixed step in launches of its own: the prefill tiles (MFMA / VALU-bound, a few hundred workgroups) run on a side stream next to the
             # decode rows (HBM-bound) — disjoint rows of `out`; inside a capture the side stream forks from and joins the
             # capturing stream, so the step's graph gets two parallel branches per layer
             main = torch.cuda.current_stream()

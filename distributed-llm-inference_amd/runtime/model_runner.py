@@ -140,7 +140,8 @@ class ModelRunner:
                        + 3 * m.intermediate_size // tp * max(m.top_k_experts, 1))
         logits = sched.max_num_seqs * m.vocab_size * 8
         scan = scan_workspace_bytes(m.layer_specs, T, sched.max_num_seqs) if self.stateful else 0
-        # + graph pools; the scans' workspace once for eager steps and once in the captured ones' pool
+        # + graph pools, and in them and beside them, once each, the partial sums of products cut along K: up to 134 MB for routed experts on 256-row tiles (as many
+        # slabs as any plan of the device can ask for), 67 MB for dense layers; the scans' workspace once for eager steps and once in the captured ones' pool
         return max(3 * (act + logits), 4 << 30) + (2 << 30) + 2 * scan
 
     @property
