@@ -570,8 +570,9 @@ __device__ __forceinline__ void prefill_tile(
   };
   // SPREAD (two groups): the pieces of the turn that is fetched are asked for behind the first score products, whose fragments are read before them, and its
   // block table entries a turn before.  At the start of a turn, where all waves have just passed the barrier, the pieces queue up for the unit's one path to memory while
-  // the matrix cores are idle, and a scalar load that is waited for where it is made stops the wave for its latency.  Whole calls, µs, at the start / spread: bf16, 32/8 heads,
-  // one prompt of 1000 tokens 41.6 / 39.1, of 2000 81.0 / 75.5, 8/1 heads 59.0 / 51.9, of 3500 97.8 / 84.0; e4m3 79.5 / 77.2, 8/1 heads 56.0 / 54.4, of 3500 92.2 / 88.5.
+  // the matrix cores are idle, and a scalar load that is waited for where it is made stops the wave for its latency.  Whole calls with rotation and cache
+  // write, µs, at the start / spread: bf16, 32/8 heads, one prompt of 1000 tokens 41.4 / 39.7, of 2000 80.4 / 76.4, 8/1 heads 58.8 / 51.5, of 3500 95.9 / 83.7;
+  // e4m3, 32/8 heads, 2000 77.6 / 76.7, 8/1 heads 55.8 / 53.9, of 3500 90.5 / 86.2.
   // One group, whose unit has three workgroups at different places, loses 1 to 4 %.
   constexpr bool SPREAD = GROUPS == 2;
   int entry[NPG];
@@ -962,20 +963,22 @@ void launch_paged_decode_worklist(const void* q, int64_t q_stride, const void* k
                        out_stride, Hq, 1, kv_fp8 ? v_scale : 1.f, kv_fp8 ? kv_scales : nullptr, Hkv, (const int4*)red, counts);
 }
 
-// Two groups where a compute unit gets one workgroup: a tile's pages are a serial chain of 0.7 µs each, and what the chip
-// has no second tile for, a second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: prompts of 1000 tokens (256
-// workgroups) 32.3 / 26.9, of 2000 with 8/1 heads (250) 57.8 / 45.7, 8 × 128 tokens behind 1000 (256) 37.9 / 34.5, 32 × 16 behind 300 15.0 / 15.3.
+// Two groups where a compute unit gets one workgroup: a tile's pages are a serial chain of 0.7 µs each, and what the chip has no second tile for, a
+// second half of the same tile can fill.  Causal tiles of 32/8 heads, µs, one / two groups: prompts of 1000 tokens (256 workgroups) 34.1 / 29.6, of 2000
+// with 8/1 heads (125) 58.2 / 45.8, 8 × 128 tokens behind 1000 (256) 40.9 / 34.5, 32 × 16 behind 300 15.5 / 15.1.
 // A unit holds one workgroup of two groups (100 KB of LDS; e4m3 68 KB, but its registers leave room for one too), and three of one.  Past 256 tiles:
-//   * the shortest share workgroups, a group each (SHARED).  Both pass the same barriers, so they wait for their loads and products at the same time
-//     and take 1.25 of what they take in workgroups of their own; the longest take 0.8.  It pays where the shared ones are the shorter ones: 2 × 600
-//     tokens (304 tiles) 24.1 / 20.7, 4 × 300 (320) 16.1 / 14.7, one of 1100 behind 500 (280) 51.0 / 39.9, but 3 × 400 behind 1000 (312) 48.6 / 55.9,
-//     2 × 1024 (512, all shared) 37.4 / 46.6.  e4m3, whose two groups take two pages a turn: 2 × 600 behind 600 42.2 / 41.5, 1100 behind 2000 (280) 100.0 /
-//     96.2, 4 × 1500 behind 500 with 8/1 heads (376) 63.1 / 61.8, a mixed step of 96 rows and two chunks of up to 1024 behind up to 1024 (296), called
-//     eagerly and with the decode rows, 89.2 / 75.6 (in bf16 94 / 99).
-//   * or the rest comes in a second round (ROUNDS), whose workgroups all start with 5 µs of latencies: 16 × 100 tokens (512) 12.5 / 17.2, 9 × 128 behind
-//     1000 (288) 46.3 / 60.4.  It pays only if that is made of short tiles: one prompt of 2000 (504) 63.5 / 58.1.  With 5 µs + 0.0285 µs a token for
-//     one group, 5.5 + 0.0225 for two, and the first tile of the second round at `second` tokens of context, that is what the last line says
-//     (fitted on 190 steps of equal prompts).
+//   * the shortest share workgroups, a group each (SHARED).  Both pass the same barriers, so they wait for their loads and products at the same time and
+//     take 1.25 of what they take in workgroups of their own; the longest take 0.8.  It pays where the shared ones are the shorter ones: 2 × 600 tokens
+//     (304 tiles) 24.1 / 20.6, 4 × 300 (320) 15.8 / 14.9, one of 1100 behind 500 (280) 51.2 / 39.4, but 3 × 400 behind 1000 (312) 50.2 / 54.8, 2 × 1024
+//     (512, all shared) 38.6 / 45.1.  e4m3, whose two groups take two pages a turn: 2 × 600 behind 600 42.8 / 41.2, 1100 behind 2000 (280) 100 / 93.8,
+//     4 × 1500 behind 500 with 8/1 heads (376) 62.8 / 61.9.
+//   * or the rest comes in a second round (ROUNDS), whose workgroups all start with 5 µs of latencies: 16 × 100 tokens (512) 13.0 / 16.6, 9 × 128 behind
+//     1000 (288) 49.5 / 57.8.  It pays only if that is made of short tiles: one prompt of 2000 (504) 65.1 / 58.0.  With 5 µs + 0.0285 µs a token for
+//     one group, 5.5 + 0.0225 for two, and the first tile of the second round at `second` tokens of context, that is what the last line says.
+// The lines were fitted on 190 steps of equal prompts before two groups spread their fetches, which takes a token of theirs from 0.0225 to 0.0207 µs.  At 47
+// sizes timed since (profiles/prefill_page_groups.txt) the form taken is the fastest or within 3 % for equal prompts, but for one of 2000 behind 500
+// (1.06) and, 8/1 heads, of several long ones that would rather have a second round than share (1.06 to 1.09).  `mean` speaks of equal prompts: of uneven
+// ones, a long one beside short ones is kept at one group where two would take 0.78.
 // longest: tokens of context (new ones included) of the longest sequence, sequences: with new tokens; 0: not known, as for a captured launch of bounds.
 int prefill_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, bool kv_fp8) {
   constexpr int ONE = 1, ROUNDS = 2, SHARED = 3;
@@ -1010,15 +1013,22 @@ void launch_paged_prefill(const void* q, int64_t q_stride, const void* k_cache, 
 }
 
 // Page groups of a mixed step's tiles (paged_mixed_kernel), 0: launches of their own.  rows: decode rows; longest, sequences as in prefill_page_groups.
-// µs of the longest tile's chain with one and two groups measured as there (8/1 heads, 250 to 3500 tokens); decode rows by themselves take 5 µs and their pages' bytes
-// at 5.5 TB/s (half the longest context each, at most 800 tokens: the longest may be a prompt's), a unit without a tile reads at 2.2 of its share.  One launch of one group then takes its chain and 0.4 of
-// the rows' time, or what the rows take; one of two groups its chain, 0.15 of the rows' time, and what the units without a tile leave, or 1.15 of the rows' time.  Measured, after each other / one
-// group / two — 8/1 heads, 16 bf16 rows of up to 1500 and one of 2000 behind 500 (125 tiles) 66.5 / 74.4 / 61.2, e4m3 65.2 / 80.4 / 61.6, 400 bf16 rows 94.8 /
-// 86.8 / 67.5; 64/8 heads and one of 500 behind 1500 (256), bf16, 16 rows 71.8 / 68.9 / 61.5, 96 107.7 / 83.8 / 106.5; of 400 behind 500 (200), e4m3, 48 48.9 /
-// 40.1 / 38.4, 96 58.1 / 40.0 / 48.9.  Past 256 tiles, where their own launch has two groups, one launch pays if it hides
-// rows of some length: 32/8 heads, e4m3, two of up to 1024 behind
-// up to 1024 (296), 16 rows 49.4 / 50.0, 96 67.2 / 49.4.  (With the pieces of two groups still at the start of their turns.  More:
-// profiles/mixed_steps_one_launch.txt.)
+// The rule compares what the forms should take, in µs:
+//   * the longest tile's chain, with one and two groups as measured with 8/1 heads at 250 to 3500 tokens;
+//   * the decode rows by themselves: 5, and their pages' bytes at 5.5 TB/s.  `longest` may be a prompt's, so the rows are taken for half of it, 800 tokens at most;
+//   * one launch of one group: its chain and 0.4 of the rows' time, or what the rows take;
+//   * one of two groups, a workgroup a unit: its chain, 0.15 of the rows' time and what the units without a tile leave of them (such a unit reads 2.2 of its
+//     share), or 1.15 of the rows' time.
+// Past 256 tiles, where their own launch may have two groups, one launch of one group pays if it hides rows of some length.
+// Measured, after each other / one group / two:
+//   8/1 heads, one prompt of 2000 behind 500 (125 tiles): 16 bf16 rows of up to 1500 64.0 / 75.9 / 59.6, e4m3 65.8 / 80.6 / 61.4, 400 bf16 89.2 / 86.8 / 60.7;
+//   64/8, one of 500 behind 1500 (256), bf16: 16 rows 68.7 / 67.9 / 60.3, 96 104 / 82.9 / 103;
+//   64/8, one of 400 behind 500 (200), e4m3: 48 rows 49.5 / 40.8 / 39.3, 96 58.3 / 40.2 / 49.1 (two are taken);
+//   32/8, two of up to 1024 behind up to 1024 (296), e4m3: 16 rows 49.4 / 50.6 / 41.1, 96 66.9 / 49.8 / 60.7.
+// Long rows are taken for short ones, and a long row's context for the chain of a short chunk's tiles.  That costs no step more than launches of its own
+// would (336 steps with rows of 4000 to 16000 tokens: 0.83 of them on average, at most 1.03), but it is not the best form: 64 rows of up to 16000 beside 1000
+// behind 6000 (256 tiles), where two groups are taken, bf16 532 / 418 / 498, e4m3 362 / 245 / 355; beside 40 behind 3000, e4m3 278 / 209 / 214.
+// (More: profiles/mixed_steps_one_launch.txt.)
 int mixed_page_groups(int num_tiles, int Hkv, int G, int longest, int sequences, int rows, bool kv_fp8) {
   const int blocks = num_tiles * Hkv;
   const bool two = prefill_page_groups(num_tiles, Hkv, G, longest, sequences, kv_fp8) != 1;

@@ -749,7 +749,7 @@ template <typename A> __device__ __forceinline__ typename Raw<A>::v4 raw4(const 
 // KEPT: up to that many 16-channel tiles of diag(w e^P) K wait in LDS for the solve instead of in the workspace, with the loop's fragments in the
 // place that M takes behind it: 50 KB, still three workgroups a compute unit.  A block writes 148 KB where it wrote 180 and read 32 back.  The whole
 // step of a layer with heads of 128, µs: 16 heads, four prompts of 512 to 1069 tokens 181.2 → 177.8; 32 heads 325.8 → 317.8, one prompt of 2000
-// 234.6 → 228.0; equal below a chip full of blocks.  Longer heads would leave two workgroups a unit.  Four of them (128 registers, the next
+// 234.6 → 228.0; equal below a chip full of blocks; this kernel alone, both in turn, 76.5 → 73.5, 131 → 125, 79.4 → 73.8.  Longer heads would leave two workgroups a unit.  Four of them (128 registers, the next
 // channels fetched behind the stores, which loads then wait for) were slower: 191.8.
 template <typename Z, bool WIDE, int KEPT>
 __global__ __launch_bounds__(NT, 3) void channel_block_kernel(const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k,

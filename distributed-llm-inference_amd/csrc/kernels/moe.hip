@@ -64,6 +64,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const uint16_t* __restri
 // average, tiles of up to 128 rows take 0.58), a workgroup's start and end 6, a slice's 256 KB of sums written and read 0.1.  Slices that are more than a round end
 // half a slice apart.  Mixtral's layer, µs, slices by the largest possible number of tiles and fp32 rows for all of them / this: 300 tokens 636 / 592, 777 731 /
 // 680, 2048 1403 / 1343; whole rounds only / this: 4096 2415 / 2321 (tiles for a round and a quarter, say, take that and not two).
+// (The times are one layer's; at 63 steps of 13 layers, 512 to 8192 columns, K 1024 to 28672, 2 to 16 experts, 0.93 of the former's on average, at most 1.02.)
 constexpr int CUT_CUS = 256, CUT_MAX_SLICES = 8, CUT_MAX_TILES = 512;
 int grouped_cut_slabs(int blocks) { return std::min(CUT_MAX_TILES, CUT_MAX_SLICES * std::min(blocks, CUT_CUS - 1)); }
 __host__ __device__ inline int2 cut_plan(int blocks, int nk, float full) {
